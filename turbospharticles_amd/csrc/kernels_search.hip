@@ -1199,21 +1199,17 @@ namespace tsp
 
     constexpr uint32_t kHashSlots = 2048;   // > kHaloMax + kBlock: probes always end
 
-    // With TSP_TUNE_SLOT16 the halo slots of a u32 slice are stored as u16 in the first half of
+    // The halo slots of a u32 slice are stored as u16 in the first half of
     // its storage (entry k of lane l at u16 position k * kSlice + l, which the lanes reach only
     // after reading the u32 entries there), and the slice turns u16 once its entries are written.
     __device__ __forceinline__ void slotsToU16(const Dev& d, uint32_t i, const SliceMeta& m)
     {
-#if TSP_TUNE_SLOT16
         if (i < d.nF && (i & (kSlice - 1)) == 0 && m.format != kFmtDelta16)
         {
             SliceMeta& w = d.meta[REL_FF][i / kSlice];
             w.format = kFmtDelta16;
             w.base = 0;
         }
-#else
-        (void)d; (void)i; (void)m;
-#endif
     }
     constexpr uint32_t kSortKeys = kHaloMax <= 1024 ? 1024 : 2048;    // power of two >= kHaloMax
 
@@ -1365,8 +1361,7 @@ namespace tsp
             }
             const uint32_t q = lastSlot * kPageWords + ((j >> 5) & (kPageWords - 1u));
             const uint32_t slot = (wrank[q] + static_cast<uint32_t>(__popc(bits[q] & ((1u << (j & 31u)) - 1u)))) << kSlotShift;
-            if (m.format == kFmtDelta16 || TSP_TUNE_SLOT16) { d.pool[REL_FF][m.offset + k * kSlice + lane] = static_cast<uint16_t>(slot); }
-            else { reinterpret_cast<uint32_t*>(d.pool[REL_FF] + m.offset)[k * kSlice + lane] = slot; }
+            d.pool[REL_FF][m.offset + k * kSlice + lane] = static_cast<uint16_t>(slot);
         }
         slotsToU16(d, i, m);
     }
@@ -1382,7 +1377,7 @@ namespace tsp
         const uint32_t blk = blockIdx.x;
         const uint32_t t = threadIdx.x;
         const uint32_t i = blk * kBlock + t;
-        if (t == 0) { unique = 0; filled = 0; bmin = kEmpty32; notDelta = 0; outOfSpan = 0; }
+        if (t == 0) { unique = 0; filled = 0; bmin = kEmpty32; notDelta = 0; outOfSpan = 0; d.haloUlps[blk] = 1u; }
         __syncthreads();
         uint32_t n = 0;
         SliceMeta m{};
@@ -1534,8 +1529,7 @@ namespace tsp
         {
             const uint32_t j = sellRead(d.pool[REL_FF], m, lane, k);
             const uint32_t slot = rank[haloFind(table, j)] << kSlotShift;
-            if (m.format == kFmtDelta16 || TSP_TUNE_SLOT16) { d.pool[REL_FF][m.offset + k * kSlice + lane] = static_cast<uint16_t>(slot); }
-            else { reinterpret_cast<uint32_t*>(d.pool[REL_FF] + m.offset)[k * kSlice + lane] = slot; }
+            d.pool[REL_FF][m.offset + k * kSlice + lane] = static_cast<uint16_t>(slot);
         }
         slotsToU16(d, i, m);
     }

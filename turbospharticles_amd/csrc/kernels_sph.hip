@@ -178,18 +178,9 @@ namespace tsp
         const float xi = pi.x, yi = pi.y, zi = pi.z, vxi = vi.x, vyi = vi.y, vzi = vi.z;
         float sF = 0.0f, cFx = 0.0f, cFy = 0.0f, cFz = 0.0f, g2 = 0.0f;
         const List ff = listAt(d, REL_FF, p, i);
-        const auto ffTerm = [&](const float4& pj, const float4& vj, uint32_t e)
+        const auto ffSum = [&](float dx, float dy, float dz, float d2, float kg, const float4& vj)
         {
-            const float dx = xi - pj.x, dy = yi - pj.y, dz = zi - pj.z;
             const float dvx = vxi - vj.x, dvy = vyi - vj.y, dvz = vzi - vj.z;
-            const float d2 = dist2(dx, dy, dz);
-            const float kg = kgFactor<kFast>(d2, k);
-#if TSP_TUNE_KG_STORE
-            // the sweeps of this step read the pair's gradient factor instead of recomputing it
-            d.kgFF[e] = kg;
-#else
-            (void)e;
-#endif
             const float st = __builtin_fmaf(dvx, dx, __builtin_fmaf(dvy, dy, dvz * dz));
             sF = __builtin_fmaf(kg, st, sF);
             cFx = __builtin_fmaf(kg, dx, cFx);
@@ -197,8 +188,30 @@ namespace tsp
             cFz = __builtin_fmaf(kg, dz, cFz);
             g2 = __builtin_fmaf(kg, kg * d2, g2);
         };
-        visitFF(ff, hc <= kHaloMax, [&](uint32_t q, uint32_t e) { ffTerm(recAt(hp, q), recAt(hv, q), e); },
-                [&](uint32_t j, uint32_t e) { ffTerm(d.pos[j], d.vp[j], e); });
+        uint32_t far = 0;   // a correction of this list does not fit its four bits
+        visitFF(ff, hc <= kHaloMax, [&](uint32_t q, uint32_t e)
+                {
+                    const float4& pj = recAt(hp, q);
+                    const float dx = xi - pj.x, dy = yi - pj.y, dz = zi - pj.z;
+                    const float d2 = dist2(dx, dy, dz);
+                    const float kg = kgFactor<kFast>(d2, k);
+                    if (kFast)
+                    {
+                        // the pair's kgShort correction for this step's sweeps
+                        const uint32_t ulps = static_cast<uint32_t>(__float_as_int(kg) - __float_as_int(kgShort(d2, k)));
+                        far |= (ulps + 8u) & ~15u;
+                        d.pool[REL_FF][e] = static_cast<uint16_t>(q | (ulps & 15u));
+                    }
+                    ffSum(dx, dy, dz, d2, kg, recAt(hv, q));
+                },
+                [&](uint32_t j, uint32_t)
+                {
+                    const float4 pj = d.pos[j];
+                    const float dx = xi - pj.x, dy = yi - pj.y, dz = zi - pj.z;
+                    const float d2 = dist2(dx, dy, dz);
+                    ffSum(dx, dy, dz, d2, kgFactor<kFast>(d2, k), d.vp[j]);
+                });
+        if (far) { d.haloUlps[blk] = 0u; }
         float sB = 0.0f, cBx = 0.0f, cBy = 0.0f, cBz = 0.0f;
         const List fb = listAt(d, REL_FB, p, i);
         visit(fb, [&](uint32_t j, uint32_t)
@@ -429,6 +442,7 @@ namespace tsp
             if (skip) { return; }
         }
         const uint32_t hc = d.haloCount[blk];
+        const bool ulps = hc <= kHaloMax && d.haloUlps[blk] != 0u;
         stageHalo(d, blk, hc, [&](uint32_t q, uint32_t j) { hp[q] = d.pos[j]; });
         for (uint32_t r = 0; r < kBlock / kSweepThreads; r++)
         {
@@ -447,22 +461,28 @@ namespace tsp
         const auto sumFF = [&](auto dictFlag)
         {
             constexpr bool kDict = decltype(dictFlag)::value;
-            const auto ffTerm = [&](const float4& pj, uint32_t e)
+            // q: the pair's halo entry where its low bits correct kgShort (kShort)
+            const auto ffTerm = [&](const float4& pj, uint32_t q, auto shortFlag)
             {
+                constexpr bool kShort = decltype(shortFlag)::value;
                 const float dx = xi - pj.x, dy = yi - pj.y, dz = zi - pj.z;
-#if TSP_TUNE_KG_STORE
-                const float kg = d.kgFF[e];
-#else
-                (void)e;
-                const float kg = kgFactor<kFast>(dist2(dx, dy, dz), k);
-#endif
+                const float d2 = dist2(dx, dy, dz);
+                const float kg = kShort ? addUlps(kgShort(d2, k), q) : kgFactor<kFast>(d2, k);
                 const float coeff = (kDict ? pi + pj.w : outerF + k.mass * pj.w * k.presDis) * kg;
                 sx = __builtin_fmaf(coeff, dx, sx);
                 sy = __builtin_fmaf(coeff, dy, sy);
                 sz = __builtin_fmaf(coeff, dz, sz);
             };
-            visitFFSplit(ff, hc <= kHaloMax, [&](uint32_t q) { return recAt(hp, q); }, ffTerm,
-                         [&](uint32_t j, uint32_t e) { ffTerm(d.pos[j], e); });
+            if (kFast && ulps)
+            {
+                visitSlots(ff, [&](uint32_t q) { return recAt(hp, q & kSlotMask); },
+                           [&](const float4& pj, uint32_t q) { ffTerm(pj, q, Flag<true>{}); });
+            }
+            else
+            {
+                visitFF(ff, hc <= kHaloMax, [&](uint32_t q, uint32_t) { ffTerm(recAt(hp, q & kSlotMask), q, Flag<false>{}); },
+                        [&](uint32_t j, uint32_t) { ffTerm(d.pos[j], 0u, Flag<false>{}); });
+            }
         };
         if (dict) { sumFF(Flag<true>{}); } else { sumFF(Flag<false>{}); }
         float ax = dict ? sx * k.presOuterFF : sx, ay = dict ? sy * k.presOuterFF : sy, az = dict ? sz * k.presOuterFF : sz;
@@ -525,6 +545,7 @@ namespace tsp
         const bool compute = d.solve[sc].compute != 0u;
         if (blk == S.blk0 && threadIdx.x == 0) { d.solve[sc].pending = 1u; }
         const uint32_t hc = d.haloCount[blk];
+        const bool ulps = hc <= kHaloMax && d.haloUlps[blk] != 0u;
         // (positions only: the pressures this launch writes into pos.w are not read here)
 #if TSP_TUNE_JACOBI_REC24
         stageHalo(d, blk, hc, [&](uint32_t q, uint32_t j)
@@ -547,15 +568,12 @@ namespace tsp
             const float xi = pi.x, yi = pi.y, zi = pi.z, axi = ai.x, ayi = ai.y, azi = ai.z;
             float sf = 0.0f;
             const List ff = listAt(d, REL_FF, p, i);
-            const auto ffTerm = [&](float xj, float yj, float zj, float axj, float ayj, float azj, uint32_t e)
+            const auto ffTerm = [&](float xj, float yj, float zj, float axj, float ayj, float azj, uint32_t q, auto shortFlag)
             {
+                constexpr bool kShort = decltype(shortFlag)::value;
                 const float dx = xi - xj, dy = yi - yj, dz = zi - zj;
-#if TSP_TUNE_KG_STORE
-                const float kg = d.kgFF[e];
-#else
-                (void)e;
-                const float kg = kgFactor<kFast>(dist2(dx, dy, dz), k);
-#endif
+                const float d2 = dist2(dx, dy, dz);
+                const float kg = kShort ? addUlps(kgShort(d2, k), q) : kgFactor<kFast>(d2, k);
                 const float sv = __builtin_fmaf(axi - axj, dx, __builtin_fmaf(ayi - ayj, dy, (azi - azj) * dz));
                 sf = __builtin_fmaf(kg, sv, sf);
             };
@@ -578,13 +596,25 @@ namespace tsp
                 return Rec{ pj.x, pj.y, pj.z, aj.x, aj.y, aj.z };
             };
 #endif
-            visitFFSplit(ff, hc <= kHaloMax, haloLoad,
-                         [&](const Rec& r, uint32_t e) { ffTerm(r.x, r.y, r.z, r.ax, r.ay, r.az, e); },
-                         [&](uint32_t j, uint32_t e)
-                         {
-                             const float4 pj = d.pos[j], aj = d.ap[j];
-                             ffTerm(pj.x, pj.y, pj.z, aj.x, aj.y, aj.z, e);
-                         });
+            if (kFast && ulps)
+            {
+                visitSlots(ff, [&](uint32_t q) { return haloLoad(q & kSlotMask); },
+                           [&](const Rec& r, uint32_t q) { ffTerm(r.x, r.y, r.z, r.ax, r.ay, r.az, q, Flag<true>{}); });
+            }
+            else
+            {
+                visitFF(ff, hc <= kHaloMax,
+                        [&](uint32_t q, uint32_t)
+                        {
+                            const Rec r = haloLoad(q & kSlotMask);
+                            ffTerm(r.x, r.y, r.z, r.ax, r.ay, r.az, 0u, Flag<false>{});
+                        },
+                        [&](uint32_t j, uint32_t)
+                        {
+                            const float4 pj = d.pos[j], aj = d.ap[j];
+                            ffTerm(pj.x, pj.y, pj.z, aj.x, aj.y, aj.z, 0u, Flag<false>{});
+                        });
+            }
             sf *= k.mass;
             float sb = 0.0f;
             const List fb = listAt(d, REL_FB, p, i);

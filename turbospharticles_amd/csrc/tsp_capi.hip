@@ -465,11 +465,6 @@ struct tsp_ctx
         }
         d.rfCap = rfCap;
         d.rfIdx = alloc<uint32_t>(rfCap, poolAllocs, MEM_LR);
-#if TSP_TUNE_KG_STORE
-        d.kgFF = alloc<float>(cap[REL_FF], poolAllocs, MEM_LF);
-#else
-        d.kgFF = nullptr;
-#endif
     }
 
     // --- a planned scene's fluid and boundary generated in the new arena (n) at h's offsets ---
@@ -866,6 +861,7 @@ struct tsp_ctx
             const uint64_t nBlocks = nF / kBlock;
             d.haloIdx = alloc<uint32_t>(nBlocks * kHaloMax, work, MEM_LF);
             d.haloCount = alloc<uint32_t>(nBlocks, work, MEM_LF);
+            d.haloUlps = alloc<uint32_t>(nBlocks, work, MEM_LF);
             // no block has a halo until the first search builds one
             hipCheck(hipMemsetAsync(d.haloCount, 0xff, sizeof(uint32_t) * std::max<uint64_t>(nBlocks, 1), stream), "memset");
         }

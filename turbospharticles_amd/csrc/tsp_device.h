@@ -40,7 +40,6 @@
 //   TSP_TUNE_STEP_GRAPH    a step runs as one captured graph launch with one status read (1), or
 //                          launch by launch with the host reading the status between phases (0)
 //   TSP_TUNE_JACOBI_REC24  kJacobi's halo records take 24 bytes instead of 32 (six blocks per CU)
-//   TSP_TUNE_KG_STORE      kSourceDiag stores each FF pair's gradient factor; the sweeps read it
 //   TSP_TUNE_HALO_MAX      FF halo records per 256-particle block (LDS per sweep block)
 //   TSP_TUNE_GRAPHS        each group of solver sweeps runs as one instantiated HIP graph
 //   TSP_TUNE_PA_WAVES, TSP_TUNE_JACOBI_WAVES   waves per SIMD the compiler must leave room for
@@ -51,8 +50,6 @@
 //   TSP_TUNE_RADIX_BITS    digit width of the LSD radix sorts (8: 256 buckets, 6, 4)
 //   TSP_TUNE_SWEEP_THREADS threads per 256-particle tile of the solver sweeps (256, or 128: two
 //                          particles per thread)
-//   TSP_TUNE_SLOT16        the halo build stores the halo slots of u32 slices as u16 (1), or keeps
-//                          their u32 storage (0)
 //   TSP_TUNE_LANE_SORT     the lists of each 256-particle block take its list positions longest
 //                          first, so a wave's lanes walk lists of similar length (1: by FF count,
 //                          2: by FB count, then FF count; 0: positions in particle order)
@@ -93,9 +90,6 @@
 #ifndef TSP_TUNE_JACOBI_REC24
 #define TSP_TUNE_JACOBI_REC24 1
 #endif
-#ifndef TSP_TUNE_KG_STORE
-#define TSP_TUNE_KG_STORE 0
-#endif
 #ifndef TSP_TUNE_HALO_MAX
 #define TSP_TUNE_HALO_MAX 1000
 #endif
@@ -116,9 +110,6 @@
 #endif
 #ifndef TSP_TUNE_SEARCH_FLAT
 #define TSP_TUNE_SEARCH_FLAT 0
-#endif
-#ifndef TSP_TUNE_SLOT16
-#define TSP_TUNE_SLOT16 1
 #endif
 #ifndef TSP_TUNE_LANE_SORT
 #define TSP_TUNE_LANE_SORT 1
@@ -392,7 +383,6 @@ namespace tsp
         SliceMeta *meta[3];
         uint16_t *pool[3];
         uint64_t poolCap[3];     // u16 units
-        float *kgFF;             // per FF entry (by its u16 position): gradient factor of the step (build variant)
         uint8_t *laneRank;       // per particle: its list position within its block (lane sorting)
         uint8_t *rankWho;        // per list position: the particle's index within the block (lane sorting)
         uint32_t *ffMin;         // per particle: smallest FF neighbor index (0 without FF neighbors), with
@@ -402,6 +392,7 @@ namespace tsp
                                  // is an FF neighbor; then the rows the masks do not cover
         uint32_t *haloIdx;       // per block: kHaloMax particle indices, ascending
         uint32_t *haloCount;     // per block: halo size, or kNoHalo
+        uint32_t *haloUlps;      // per block: 1 while every halo entry's low bits correct kgShort exactly
         // rigid-source CSR (RF), counts of RB and RR
         uint32_t *rfCnt, *rfOff, *rfIdx;
         uint32_t *rbCnt, *rrCnt;
@@ -556,15 +547,14 @@ namespace tsp
         return static_cast<uint32_t>(__float_as_int(d2)) - 1u < 0x0f800000u - 1u;
     }
 
-    // a / b: the reciprocal estimate refined by one Newton step, then two residual corrections
-    // of the quotient -- the general lowering's core, which is the whole computation when it
-    // needs no operand scaling. Callers guarantee 2^-60 <= |a| <= 2^60 and
+    // a / b from an estimate y of 1 / b: the estimate refined by one Newton step, then two residual
+    // corrections of the quotient -- the general lowering's core, which is the whole computation
+    // when it needs no operand scaling. Callers guarantee 2^-60 <= |a| <= 2^60 and
     // 2^-30 <= |b| <= 2^31 (the exponents then differ by less than the 96 that trigger
     // scaling, and every intermediate is a normal number); checked bit for bit against the
     // general lowering over such operands.
-    __device__ __forceinline__ float divCR(float a, float b)
+    __device__ __forceinline__ float quotFrom(float a, float b, float y)
     {
-        float y = __builtin_amdgcn_rcpf(b);
         const float e = __builtin_fmaf(-b, y, 1.0f);
         y = __builtin_fmaf(e, y, y);
         float q = a * y;
@@ -572,6 +562,21 @@ namespace tsp
         q = __builtin_fmaf(r, y, q);
         r = __builtin_fmaf(-b, q, a);
         return __builtin_fmaf(r, y, q);
+    }
+
+    __device__ __forceinline__ float divCR(float a, float b) { return quotFrom(a, b, __builtin_amdgcn_rcpf(b)); }
+
+    // sqrt(x) for x = 0 or 2^-96 <= x < inf, and an estimate y of 1 / sqrt(x) (2^60 for x = 0):
+    // the root from the reciprocal root and one residual correction. It rounds correctly because
+    // the correction's error is 2^-22 of an ulp and no such root of a float lies that near a
+    // midpoint; checked for every mantissa and exponent against the general lowering. One quarter-rate
+    // instruction and five others, against two and fifteen for sqrtCR and divCR, whose reciprocal
+    // estimate y takes the place of.
+    __device__ __forceinline__ float rootRcp(float x, float& y)
+    {
+        y = __builtin_fminf(__builtin_amdgcn_rsqf(x), 0x1p60f);
+        const float s = x * y;
+        return __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * y, s);
     }
 
     // KernelWeight_CubicSpline_SIMD, CPU/simd.h:279-309 (with kFast the root takes sqrtCR)
@@ -600,19 +605,45 @@ namespace tsp
     }
 
     // KernelGradientFactorNoMinDist_CubicSpline_SIMD, CPU/simd.h:374-388. With kFast the root
-    // and the quotient take sqrtCR and divCR. The host allows it for a launch when no FF or FB
-    // pair of the search has 0 < d2 < 2^-96 and every scene has |koutScale| and h in divCR's
+    // and the quotient take rootRcp and quotFrom. The host allows it for a launch when no FF or FB
+    // pair of the search has 0 < d2 < 2^-96 and every scene has |koutScale| and h in quotFrom's
     // range (the quotient's operands are koutScale and dist, and it only matters where
     // dist >= h). FR pairs keep the general lowering: rigid particles move within a step, after
     // the search has seen their distances.
     template <bool kFast = false>
     __device__ __forceinline__ float kgFactor(float d2, const Consts& k)
     {
-        const float dist = kFast ? sqrtCR(d2) : __builtin_sqrtf(d2);
+        float y = 0.0f;
+        const float dist = kFast ? rootRcp(d2, y) : __builtin_sqrtf(d2);
         const float inner = __builtin_fmaf(k.kinSlope, dist, k.kinOff);
         const float t2 = vmax(k.ktwo - dist, 0.0f);
-        const float outer = (t2 * t2) * (kFast ? divCR(k.koutScale, dist) : k.koutScale / dist);
+        const float outer = (t2 * t2) * (kFast ? quotFrom(k.koutScale, dist, y) : k.koutScale / dist);
         return dist < k.ksize ? inner : outer;
+    }
+
+    // The gradient factor of a pair whose exact value is known to lie a few ulps from a cheaper one.
+    // kgShort replaces the exact quotient by koutScale * y (at most 2 ulps off, the factor then at
+    // most 4) and drops the clamp of t2. Positions do not move within a step, so kSourceDiag, which
+    // computes the exact factor of every pair anyway, stores the difference in ulps in the four low
+    // bits of the pair's halo entry (zero in a byte offset of 16-byte records), and the solver sweeps
+    // add it back with one dot-product instruction: the same bits for 8 issue slots less. A block
+    // with a difference outside [-8, 7] keeps the exact form (Dev::haloUlps). Measured with rootRcp
+    // on the 1M cube drop: kJacobi 1,529 to 1,247 VALU instructions per wave, 49.2 to 47.4 us;
+    // kPressureAcc 40.2 to 38.0 us; kSourceDiag, which stores the corrections, 66.8 to 69.8 us.
+    __device__ __forceinline__ float kgShort(float d2, const Consts& k)
+    {
+        float y;
+        const float dist = rootRcp(d2, y);
+        const float inner = __builtin_fmaf(k.kinSlope, dist, k.kinOff);
+        const float t2 = k.ktwo - dist;
+        const float outer = (t2 * t2) * (k.koutScale * y);
+        return dist < k.ksize ? inner : outer;
+    }
+
+    // the bits of f moved by the signed low nibble of a halo entry
+    __device__ __forceinline__ float addUlps(float f, uint32_t entry)
+    {
+        return __int_as_float(__builtin_amdgcn_sdot8(static_cast<int>(entry), 1, __float_as_int(f), false));
     }
 
     // KernelGradient_CubicSpline_Scalar, CPU/simd.h:311-347 (rigid reaction forces)
@@ -660,7 +691,9 @@ namespace tsp
     }
     // FF entries of a block with a halo hold the byte offset of the neighbor's 16-byte record in
     // the block's LDS halo (slot << kSlotShift), so a sweep addresses the record without a shift
+    // (kSourceDiag puts each pair's kgShort correction into the four low bits: kSlotMask)
     constexpr uint32_t kSlotShift = 4;
+    constexpr uint32_t kSlotMask = 0xfff0u;
     static_assert((TSP_TUNE_HALO_MAX << 4) <= 0x10000u, "halo byte offsets fit the u16 entries");
 
     // the record of a halo entry in an LDS array: 16-byte records at the entry's byte offset,
@@ -796,17 +829,21 @@ namespace tsp
         else { visitEntries<false>(l, fg); }
     }
 
-    // the same with the halo records read as load(slot) and summed as use(record, e): with
-    // TSP_TUNE_GATHER4 the four LDS reads of a group issue before its four sums
-    template <typename HLoad, typename HUse, typename FromGlobal>
-    __device__ __forceinline__ void visitFFSplit(const List& l, bool halo, HLoad&& hl, HUse&& hu, FromGlobal&& fg)
+    // the entries of a list in a block with a halo, as use(load(q), q): q the stored halo entry, load
+    // its record. With TSP_TUNE_GATHER4 the four LDS reads of a group issue before its four sums.
+    template <typename Load, typename Use>
+    __device__ __forceinline__ void visitSlots(const List& l, Load&& load, Use&& use)
     {
 #if TSP_TUNE_GATHER4
-        if (halo) { visitSplit<true>(l, hl, hu); }
+        struct Got
+        {
+            decltype(load(0u)) r;
+            uint32_t q;
+        };
+        visitSplit<true>(l, [&](uint32_t q) { return Got{ load(q), q }; }, [&](const Got& g, uint32_t) { use(g.r, g.q); });
 #else
-        if (halo) { visitEntries<true>(l, [&](uint32_t q, uint32_t e) { hu(hl(q), e); }); }
+        visitEntries<true>(l, [&](uint32_t q, uint32_t) { use(load(q), q); });
 #endif
-        else { visitEntries<false>(l, fg); }
     }
 
     // --- rigid bodies, one body or particle (shared by the rigid kernels and the contact solve) ---

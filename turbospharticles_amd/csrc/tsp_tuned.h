@@ -23,9 +23,6 @@
 #ifndef TSP_TUNE_JACOBI_WAVES
 #define TSP_TUNE_JACOBI_WAVES 6
 #endif
-#ifndef TSP_TUNE_KG_STORE
-#define TSP_TUNE_KG_STORE 0
-#endif
 #ifndef TSP_TUNE_PA_WAVES
 #define TSP_TUNE_PA_WAVES 6
 #endif
@@ -64,9 +61,6 @@
 #endif
 #ifndef TSP_TUNE_LANE_SORT
 #define TSP_TUNE_LANE_SORT 1
-#endif
-#ifndef TSP_TUNE_SLOT16
-#define TSP_TUNE_SLOT16 1
 #endif
 #ifndef TSP_TUNE_SEARCH_FLAT
 #define TSP_TUNE_SEARCH_FLAT 0

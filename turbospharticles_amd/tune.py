@@ -5,8 +5,7 @@ height (32 or 64 particles per slice), the radix sort's digit width (8, 6 or 4 b
 over 28-bit keys), the threads of a solver sweep tile (256, or 128 with two particles each), the
 sweeps' LDS reads of four halo records ahead of their sums, the size of a step's first sweep
 group against the previous step's sweep count, the whole step as one graph launch or launch by
-launch, the FF halo built from page bitmaps or a window bitmap and hash set, prefetched list entries, 24- or 32-byte Jacobi halo records, stored or
-recomputed gradient factors, the halo cap (LDS per sweep block), register budgets of the sweep
+launch, the FF halo built from page bitmaps or a window bitmap and hash set, prefetched list entries, 24- or 32-byte Jacobi halo records, the halo cap (LDS per sweep block), register budgets of the sweep
 kernels, sweep groups as HIP graphs, the neighbor query's walk of the stencil (cell by cell, or
 rows of three cells) and its candidate loads in flight. The
 tuner walks the switches one at a time from the current settings (coordinate descent), keeping a
@@ -50,14 +49,12 @@ SPACE = {
     "TSP_TUNE_RANGE_LOADS": [0, 1],
     "TSP_TUNE_BOX_CELLS": [0, 512, 768, 1024],
     "TSP_TUNE_JACOBI_REC24": [1, 0],
-    "TSP_TUNE_KG_STORE": [0, 1],
     "TSP_TUNE_HALO_MAX": [1000, 960, 1024, 1064],
     "TSP_TUNE_GRAPHS": [1, 0],
     "TSP_TUNE_PA_WAVES": [0, 6, 8],
     "TSP_TUNE_JACOBI_WAVES": [0, 6],
     "TSP_TUNE_SEARCH_ROW": [1, 0, 2],
     "TSP_TUNE_LANE_SORT": [1, 0, 2],
-    "TSP_TUNE_SLOT16": [1, 0],
     "TSP_TUNE_SEARCH_FLAT": [0, 1, 2],
     "TSP_TUNE_SEARCH_BATCH": [4, 8],
     "TSP_TUNE_PERSISTENT": [0, 1],
