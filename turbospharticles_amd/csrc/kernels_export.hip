@@ -27,10 +27,10 @@ namespace tsp
         flags[local] = 1u;
         const List ff = listOf(d, REL_FF, i);
         const uint32_t blk = i / kBlock;
-        const uint32_t hc = d.haloCount[blk];
+        const uint32_t hc = d.haloInfo[blk].count;
         const uint32_t* halo = d.haloIdx + static_cast<size_t>(blk) * kHaloMax;
-        visitFF(ff, hc <= kHaloMax, [&](uint32_t q, uint32_t) { flags[halo[q >> kSlotShift] - off] = 1u; },
-                [&](uint32_t j, uint32_t) { flags[j - off] = 1u; });
+        if (hc <= kHaloMax) { visitEntries<true>(ff, [&](uint32_t q) { flags[halo[q >> kSlotShift] - off] = 1u; }); }
+        else { visit(ff, [&](uint32_t j) { flags[j - off] = 1u; }); }
     }
 
     // the exported particles at their scanned slots: position triples and speed

@@ -888,17 +888,15 @@ namespace tsp
                 if (wideHere) { d.wideList[base + static_cast<uint32_t>(__popcll(ballot & ((1ull << lane64) - 1ull)))] = i; }
             }
         }
-#if TSP_TUNE_LANE_SORT
         // the block's list positions, longest lists first (ties in particle order): a thread's
         // rank is the number of the block's sort keys above its own, the keys made distinct by
         // the thread index in their low byte. The slice statistics below then run over positions.
         {
             __shared__ uint32_t sortKey[kBlock];
             __shared__ uint32_t byPos[9][kBlock];
+            __shared__ uint8_t who[kBlock];
             const uint32_t t = threadIdx.x;
-            const uint32_t nFF = min(cnt[0], 255u), nFB = min(cnt[1], 255u);
-            const uint32_t key = TSP_TUNE_LANE_SORT == 2 ? (nFB << 8) | nFF : nFF;
-            const uint32_t own = (key << 8) | (kBlock - 1u - t);
+            const uint32_t own = (min(cnt[0], 255u) << 8) | (kBlock - 1u - t);
             sortKey[t] = own;
             __syncthreads();
             uint32_t rank = 0;
@@ -907,16 +905,13 @@ namespace tsp
                 const uint4 v = *reinterpret_cast<const uint4*>(&sortKey[u]);
                 rank += (v.x > own ? 1u : 0u) + (v.y > own ? 1u : 0u) + (v.z > own ? 1u : 0u) + (v.w > own ? 1u : 0u);
             }
-            if (i < d.nF)
-            {
-                d.laneRank[i] = static_cast<uint8_t>(rank);
-                d.rankWho[blk * kBlock + rank] = static_cast<uint8_t>(t);
-            }
+            if (i < d.nF) { d.laneRank[i] = static_cast<uint8_t>(rank); }
+            who[rank] = static_cast<uint8_t>(t);
             for (int r = 0; r < 3; r++) { byPos[r][rank] = cnt[r]; byPos[3 + r][rank] = mn[r]; byPos[6 + r][rank] = mx[r]; }
             __syncthreads();
             for (int r = 0; r < 3; r++) { cnt[r] = byPos[r][t]; mn[r] = byPos[3 + r][t]; mx[r] = byPos[6 + r][t]; }
+            if (i < d.nF) { d.head[i] = make_uint2((cnt[0] & 0xffffu) | (cnt[1] << 16), (cnt[2] & 0xffffu) | (static_cast<uint32_t>(who[t]) << 16)); }
         }
-#endif
         // per slice (list positions i of the block): pitch, base (min index), format, entries
         const uint32_t slice = i / kSlice;
         for (int r = 0; r < 3; r++)
@@ -1079,7 +1074,6 @@ namespace tsp
             // (the FF lists of wide particles: kQueryFillWide)
         }
         // the staged FF entries leave as whole slice rows: column k of the slice's lanes per store
-#if TSP_TUNE_LANE_SORT
         // (thread t writes list position t of the block: the staged entries of the particle there,
         // whose count and base it reads back; a particle outside the frame has no FF entries)
         __syncthreads();
@@ -1091,12 +1085,6 @@ namespace tsp
         if (own) { mw = d.meta[REL_FF][p / kSlice]; }
         const uint32_t base = mw.format == kFmtDelta16 ? mw.base : wMin;
         const uint32_t lw = p & (kSlice - 1);
-#else
-        __syncthreads();
-        const uint32_t own = (active && staged) ? min(cF, kStage) : 0u, base = mF.base;
-        const SliceMeta mw = mF;
-        const uint32_t lw = lane;
-#endif
         const uint32_t rows = sliceMax(own);
         if (mw.format == kFmtDelta16)
         {
@@ -1289,7 +1277,7 @@ namespace tsp
         __syncthreads();
         if (full)
         {
-            if (t == 0) { d.haloCount[blk] = kNoHalo; }
+            if (t == 0) { d.haloInfo[blk].count = kNoHalo; }
             return;
         }
         // the pages in ascending order: slotOfRank[r] is the slot of the r-th smallest page
@@ -1325,7 +1313,7 @@ namespace tsp
         for (uint32_t w = 0; w < kBlock / 64; w++) { before += w < (t >> 6) ? waveSum[w] : 0u; count += waveSum[w]; }
         if (count > kHaloMax)
         {
-            if (t == 0) { d.haloCount[blk] = kNoHalo; }
+            if (t == 0) { d.haloInfo[blk].count = kNoHalo; }
             return;
         }
         uint32_t* out = d.haloIdx + static_cast<size_t>(blk) * kHaloMax;
@@ -1345,7 +1333,7 @@ namespace tsp
                 b &= b - 1u;
             }
         }
-        if (t == 0) { d.haloCount[blk] = count; }
+        if (t == 0) { d.haloInfo[blk].count = count; }
         __syncthreads();
         // entries become the byte offsets of their slots, in their storage format
         lastPage = kEmpty32;
@@ -1377,7 +1365,7 @@ namespace tsp
         const uint32_t blk = blockIdx.x;
         const uint32_t t = threadIdx.x;
         const uint32_t i = blk * kBlock + t;
-        if (t == 0) { unique = 0; filled = 0; bmin = kEmpty32; notDelta = 0; outOfSpan = 0; d.haloUlps[blk] = 1u; }
+        if (t == 0) { unique = 0; filled = 0; bmin = kEmpty32; notDelta = 0; outOfSpan = 0; d.haloInfo[blk].ulps = 1u; }
         __syncthreads();
         uint32_t n = 0;
         SliceMeta m{};
@@ -1430,7 +1418,7 @@ namespace tsp
                 for (uint32_t w = 0; w < kBlock / 64; w++) { before += w < (t >> 6) ? waveSum[w] : 0u; count += waveSum[w]; }
                 if (count > kHaloMax)
                 {
-                    if (t == 0) { d.haloCount[blk] = kNoHalo; }
+                    if (t == 0) { d.haloInfo[blk].count = kNoHalo; }
                     return;
                 }
                 uint32_t r = before + incl - sum;
@@ -1447,7 +1435,7 @@ namespace tsp
                         bits &= bits - 1u;
                     }
                 }
-                if (t == 0) { d.haloCount[blk] = count; }
+                if (t == 0) { d.haloInfo[blk].count = count; }
                 __syncthreads();
                 for (uint32_t k = 0; k < n; k++)
                 {
@@ -1487,7 +1475,7 @@ namespace tsp
         const uint32_t count = unique;
         if (count > kHaloMax)
         {
-            if (t == 0) { d.haloCount[blk] = kNoHalo; }
+            if (t == 0) { d.haloInfo[blk].count = kNoHalo; }
             return;
         }
         // compact, pad, sort ascending (bitonic over the power of two at or above the count)
@@ -1522,7 +1510,7 @@ namespace tsp
             out[q] = keys[q];
             rank[haloFind(table, keys[q])] = static_cast<uint16_t>(q);
         }
-        if (t == 0) { d.haloCount[blk] = count; }
+        if (t == 0) { d.haloInfo[blk].count = count; }
         __syncthreads();
         // entries become their rank in the sorted halo, in their storage format
         for (uint32_t k = 0; k < n; k++)

@@ -1,7 +1,14 @@
 // kernels_sph.hip -- IISPH solver kernels of the step on gfx950.
 //
-// One thread per fluid particle in Morton order; a wave64 reads two SELL-32 slices, so the list
-// loads of a neighbor column are two 64-byte rows. FF sums use the reference CPU's dict-chunk
+// One thread per fluid particle; a wave64 reads one SELL slice, so the list loads of a neighbor
+// column are one row. Every kernel first issues the loads that depend on nothing but the block (list
+// heads, slice headers, first entries, halo indices), then the ones that depend on those (the halo
+// records, the particle's own), and only then waits: a block starts its sums after two memory
+// latencies instead of eight, which also shortens the first and the last blocks of a large launch.
+// Headers, constants and scene records are scalar loads (uniformLoad). Measured against the loads in
+// order of use: 1M cube drop kJacobi 47.4 to 39.3 us, kPressureAcc 38.0 to 31.0, kDensity 36.3 to
+// 32.7, kSourceDiag 69.8 to 59.8, kNonPressure 64.2 to 62.0; 64k particles kPressureAcc 12.8 to 11.0,
+// kJacobi 12.4 to 10.4. FF sums use the reference CPU's dict-chunk
 // form (one scale after the sum), FB/FR sums its normal form, each in the list order the fill
 // wrote (CPU/backend/sph_solver.cpp):
 //   kDensity         Density_ChunkedSELL                            :734-890
@@ -20,18 +27,17 @@
 
 namespace tsp
 {
-    // copies the FF halo records of a block into LDS (load(slot, particle index)); every thread
-    // of the block calls it. A count above kHaloMax (kNoHalo) means the block has no halo.
-    template <typename Load>
-    __device__ __forceinline__ void stageHalo(const Dev& d, uint32_t blk, uint32_t hc, Load&& load)
+    // two records of a halo neighbor
+    struct Pair4
     {
-        if (hc <= kHaloMax)
-        {
-            const uint32_t* idx = d.haloIdx + static_cast<size_t>(blk) * kHaloMax;
-            for (uint32_t q = threadIdx.x; q < hc; q += blockDim.x) { load(q, idx[q]); }
-        }
-        __syncthreads();
-    }
+        float4 a, b;
+    };
+
+    struct BoundaryRec
+    {
+        float4 p;
+        float vol;
+    };
 
     template <bool kFast>
     __global__ void __launch_bounds__(kBlock) kDensity(Dev d)
@@ -39,42 +45,44 @@ namespace tsp
         if (stopped(d)) { return; }
         __shared__ float4 hp[kHaloMax];
         const uint32_t blk = xcdBlock();
-        const uint32_t p = blk * kBlock + threadIdx.x;   // list position; i its particle
-        const uint32_t i = particleAt(d, p);
-        const uint32_t sc = d.blockScene[blk];
-        const Consts& k = d.consts[sc];
-        const uint32_t hc = d.haloCount[blk];
-        stageHalo(d, blk, hc, [&](uint32_t q, uint32_t j) { hp[q] = d.pos[j]; });
-        if (i - d.scenes[sc].offF >= d.scenes[sc].nF) { return; }
+        const Lists l = listsAt(d, blk);
+        const SlotList slots = slotsOf(d, l);
+        const Halo h = haloOf(d, blk);
+        const uint32_t sc = uniformLoad(&d.blockScene[blk]);
+        const Consts k = uniformLoad(&d.consts[sc]);
+        const Scene S = uniformLoad(&d.scenes[sc]);
+        const uint32_t i = l.i;
         const float4 pi = d.pos[i];
+        stageHalo(h, [&](uint32_t j) { return d.pos[j]; }, [&](uint32_t q, const float4& r) { hp[q] = r; });
+        __syncthreads();
+        if (i - S.offF >= S.nF) { return; }
         const float xi = pi.x, yi = pi.y, zi = pi.z;
-        const List ff = listAt(d, REL_FF, p, i);
         float dF;
-        if (ff.n <= kDictMax)
+        const auto sumFF = [&](auto&& ffTerm)
+        {
+            if (h.any) { visitSlots(slots, [&](uint32_t q, uint32_t) { ffTerm(recAt(hp, q)); }); }
+            else { visit(l.list(d, REL_FF), [&](uint32_t j) { ffTerm(d.pos[j]); }); }
+        };
+        if (slots.n <= kDictMax)
         {
             // dict chunk: unscaled weights, scaled once (sph_solver.cpp:797-810)
             float wsum = 0.0f;
-            const auto ffTerm = [&](const float4& pj) { wsum += kwUnscaled<kFast>(dist2(xi - pj.x, yi - pj.y, zi - pj.z), k); };
-            visitFF(ff, hc <= kHaloMax, [&](uint32_t q, uint32_t) { ffTerm(recAt(hp, q)); }, [&](uint32_t j, uint32_t) { ffTerm(d.pos[j]); });
+            sumFF([&](const float4& pj) { wsum += kwUnscaled<kFast>(dist2(xi - pj.x, yi - pj.y, zi - pj.z), k); });
             dF = wsum * k.weightScale;
         }
         else
         {
             // normal chunk: the alpha-scaled weight per neighbor (sph_solver.cpp:826-831)
             float s = 0.0f;
-            const auto ffTerm = [&](const float4& pj) { s = __builtin_fmaf(k.mass, kwNormal<kFast>(xi - pj.x, yi - pj.y, zi - pj.z, k), s); };
-            visitFF(ff, hc <= kHaloMax, [&](uint32_t q, uint32_t) { ffTerm(recAt(hp, q)); }, [&](uint32_t j, uint32_t) { ffTerm(d.pos[j]); });
+            sumFF([&](const float4& pj) { s = __builtin_fmaf(k.mass, kwNormal<kFast>(xi - pj.x, yi - pj.y, zi - pj.z, k), s); });
             dF = s;
         }
         float dB = 0.0f, dR = 0.0f;
-        const List fb = listAt(d, REL_FB, p, i);
-        visit(fb, [&](uint32_t j, uint32_t)
+        visitGather(d, l, REL_FB, [&](uint32_t j) { return d.bpos[j]; }, [&](const float4& bj)
         {
-            const float4 bj = d.bpos[j];
             dB = __builtin_fmaf(bj.w, kwNormal<kFast>(xi - bj.x, yi - bj.y, zi - bj.z, k), dB);
         });
-        const List fr = listAt(d, REL_FR, p, i);
-        visit(fr, [&](uint32_t j, uint32_t)
+        visit(l.list(d, REL_FR), [&](uint32_t j)
         {
             const float4 rj = d.rpos[j];
             dR = __builtin_fmaf(rj.w, kwNormal(xi - rj.x, yi - rj.y, zi - rj.z, k), dR);
@@ -88,19 +96,21 @@ namespace tsp
         if (stopped(d)) { return; }
         __shared__ float4 hp[kHaloMax], hv[kHaloMax];
         const uint32_t blk = xcdBlock();
-        const uint32_t p = blk * kBlock + threadIdx.x;   // list position; i its particle
-        const uint32_t i = particleAt(d, p);
-        const uint32_t sc = d.blockScene[blk];
-        const Consts& k = d.consts[sc];
-        const uint32_t hc = d.haloCount[blk];
-        stageHalo(d, blk, hc, [&](uint32_t q, uint32_t j) { hp[q] = d.pos[j]; hv[q] = d.vel[j]; });
-        if (i - d.scenes[sc].offF >= d.scenes[sc].nF) { return; }
+        const Lists l = listsAt(d, blk);
+        const SlotList slots = slotsOf(d, l);
+        const Halo h = haloOf(d, blk);
+        const uint32_t sc = uniformLoad(&d.blockScene[blk]);
+        const Consts k = uniformLoad(&d.consts[sc]);
+        const Scene S = uniformLoad(&d.scenes[sc]);
+        const uint32_t i = l.i;
         const float4 pi = d.pos[i], vi = d.vel[i];
+        stageHalo(h, [&](uint32_t j) { return Pair4{ d.pos[j], d.vel[j] }; }, [&](uint32_t q, const Pair4& r) { hp[q] = r.a; hv[q] = r.b; });
+        __syncthreads();
+        if (i - S.offF >= S.nF) { return; }
         const float xi = pi.x, yi = pi.y, zi = pi.z, vxi = vi.x, vyi = vi.y, vzi = vi.z;
         float aFx = 0.0f, aFy = 0.0f, aFz = 0.0f;
-        const List ff = listAt(d, REL_FF, p, i);
         // dict chunks scale by the mass after the sum, normal chunks per neighbor (sph_solver.cpp:974-1049)
-        const bool dict = ff.n <= kDictMax;
+        const bool dict = slots.n <= kDictMax;
         // the two forms as two loops (a wave runs the normal one only for a list longer than kDictMax)
         const auto sumFF = [&](auto dictFlag)
         {
@@ -118,30 +128,28 @@ namespace tsp
                 aFy = __builtin_fmaf(coeff, dy, aFy);
                 aFz = __builtin_fmaf(coeff, dz, aFz);
             };
-            visitFF(ff, hc <= kHaloMax, [&](uint32_t q, uint32_t) { ffTerm(recAt(hp, q), recAt(hv, q)); },
-                    [&](uint32_t j, uint32_t) { ffTerm(d.pos[j], d.vel[j]); });
+            if (h.any) { visitSlots(slots, [&](uint32_t q, uint32_t) { ffTerm(recAt(hp, q), recAt(hv, q)); }); }
+            else { visit(l.list(d, REL_FF), [&](uint32_t j) { ffTerm(d.pos[j], d.vel[j]); }); }
         };
         if (dict) { sumFF(Flag<true>{}); } else { sumFF(Flag<false>{}); }
         if (dict) { aFx *= k.mass; aFy *= k.mass; aFz *= k.mass; }
         float aBx = 0.0f, aBy = 0.0f, aBz = 0.0f;
-        const List fb = listAt(d, REL_FB, p, i);
-        visit(fb, [&](uint32_t j, uint32_t e)
+        visitGather(d, l, REL_FB, [&](uint32_t j) { return BoundaryRec{ d.bpos[j], d.bvol[j] }; }, [&](const BoundaryRec& r)
         {
-            const float4 bj = d.bpos[j];
+            const float4& bj = r.p;
             const float dx = xi - bj.x, dy = yi - bj.y, dz = zi - bj.z;
             const float d2 = dist2(dx, dy, dz);
             const float f = kgFactor<kFast>(d2, k);
             const float gx = f * dx, gy = f * dy, gz = f * dz;
             const float dvx = vxi - 0.0f, dvy = vyi - 0.0f, dvz = vzi - 0.0f;
             const float dot = __builtin_fmaf(dvx, dx, __builtin_fmaf(dvy, dy, dvz * dz));
-            const float coeff = (d.bvol[j] * dot) / (d2 + k.hsqEps);
+            const float coeff = (r.vol * dot) / (d2 + k.hsqEps);
             aBx = __builtin_fmaf(coeff, gx, aBx);
             aBy = __builtin_fmaf(coeff, gy, aBy);
             aBz = __builtin_fmaf(coeff, gz, aBz);
         });
         float aRx = 0.0f, aRy = 0.0f, aRz = 0.0f;
-        const List fr = listAt(d, REL_FR, p, i);
-        visit(fr, [&](uint32_t j, uint32_t e)
+        visit(l.list(d, REL_FR), [&](uint32_t j)
         {
             const float4 rj = d.rpos[j], uj = d.rvel[j];
             const float dx = xi - rj.x, dy = yi - rj.y, dz = zi - rj.z;
@@ -167,17 +175,20 @@ namespace tsp
         if (stopped(d)) { return; }
         __shared__ float4 hp[kHaloMax], hv[kHaloMax];
         const uint32_t blk = xcdBlock();
-        const uint32_t p = blk * kBlock + threadIdx.x;   // list position; i its particle
-        const uint32_t i = particleAt(d, p);
-        const uint32_t sc = d.blockScene[blk];
-        const Consts& k = d.consts[sc];
-        const uint32_t hc = d.haloCount[blk];
-        stageHalo(d, blk, hc, [&](uint32_t q, uint32_t j) { hp[q] = d.pos[j]; hv[q] = d.vp[j]; });
-        if (i - d.scenes[sc].offF >= d.scenes[sc].nF) { return; }
+        const Lists l = listsAt(d, blk);
+        const SlotList slots = slotsOf(d, l);
+        const Halo h = haloOf(d, blk);
+        const uint32_t sc = uniformLoad(&d.blockScene[blk]);
+        const Consts k = uniformLoad(&d.consts[sc]);
+        const Scene S = uniformLoad(&d.scenes[sc]);
+        const uint32_t i = l.i;
         const float4 pi = d.pos[i], vi = d.vp[i];
+        const float rho = d.vel[i].w;
+        stageHalo(h, [&](uint32_t j) { return Pair4{ d.pos[j], d.vp[j] }; }, [&](uint32_t q, const Pair4& r) { hp[q] = r.a; hv[q] = r.b; });
+        __syncthreads();
+        if (i - S.offF >= S.nF) { return; }
         const float xi = pi.x, yi = pi.y, zi = pi.z, vxi = vi.x, vyi = vi.y, vzi = vi.z;
         float sF = 0.0f, cFx = 0.0f, cFy = 0.0f, cFz = 0.0f, g2 = 0.0f;
-        const List ff = listAt(d, REL_FF, p, i);
         const auto ffSum = [&](float dx, float dy, float dz, float d2, float kg, const float4& vj)
         {
             const float dvx = vxi - vj.x, dvy = vyi - vj.y, dvz = vzi - vj.z;
@@ -189,34 +200,38 @@ namespace tsp
             g2 = __builtin_fmaf(kg, kg * d2, g2);
         };
         uint32_t far = 0;   // a correction of this list does not fit its four bits
-        visitFF(ff, hc <= kHaloMax, [&](uint32_t q, uint32_t e)
-                {
-                    const float4& pj = recAt(hp, q);
-                    const float dx = xi - pj.x, dy = yi - pj.y, dz = zi - pj.z;
-                    const float d2 = dist2(dx, dy, dz);
-                    const float kg = kgFactor<kFast>(d2, k);
-                    if (kFast)
-                    {
-                        // the pair's kgShort correction for this step's sweeps
-                        const uint32_t ulps = static_cast<uint32_t>(__float_as_int(kg) - __float_as_int(kgShort(d2, k)));
-                        far |= (ulps + 8u) & ~15u;
-                        d.pool[REL_FF][e] = static_cast<uint16_t>(q | (ulps & 15u));
-                    }
-                    ffSum(dx, dy, dz, d2, kg, recAt(hv, q));
-                },
-                [&](uint32_t j, uint32_t)
-                {
-                    const float4 pj = d.pos[j];
-                    const float dx = xi - pj.x, dy = yi - pj.y, dz = zi - pj.z;
-                    const float d2 = dist2(dx, dy, dz);
-                    ffSum(dx, dy, dz, d2, kgFactor<kFast>(d2, k), d.vp[j]);
-                });
-        if (far) { d.haloUlps[blk] = 0u; }
-        float sB = 0.0f, cBx = 0.0f, cBy = 0.0f, cBz = 0.0f;
-        const List fb = listAt(d, REL_FB, p, i);
-        visit(fb, [&](uint32_t j, uint32_t)
+        if (h.any)
         {
-            const float4 bj = d.bpos[j];
+            visitSlots(slots, [&](uint32_t q, uint32_t row)
+            {
+                const float4& pj = recAt(hp, q);
+                const float dx = xi - pj.x, dy = yi - pj.y, dz = zi - pj.z;
+                const float d2 = dist2(dx, dy, dz);
+                const float kg = kgFactor<kFast>(d2, k);
+                if (kFast)
+                {
+                    // the pair's kgShort correction for this step's sweeps
+                    const uint32_t ulps = static_cast<uint32_t>(__float_as_int(kg) - __float_as_int(kgShort(d2, k)));
+                    far |= (ulps + 8u) & ~15u;
+                    slots.p[row * kSlice] = static_cast<uint16_t>(q | (ulps & 15u));
+                }
+                ffSum(dx, dy, dz, d2, kg, recAt(hv, q));
+            });
+        }
+        else
+        {
+            visit(l.list(d, REL_FF), [&](uint32_t j)
+            {
+                const float4 pj = d.pos[j];
+                const float dx = xi - pj.x, dy = yi - pj.y, dz = zi - pj.z;
+                const float d2 = dist2(dx, dy, dz);
+                ffSum(dx, dy, dz, d2, kgFactor<kFast>(d2, k), d.vp[j]);
+            });
+        }
+        if (far) { d.haloInfo[blk].ulps = 0u; }
+        float sB = 0.0f, cBx = 0.0f, cBy = 0.0f, cBz = 0.0f;
+        visitGather(d, l, REL_FB, [&](uint32_t j) { return d.bpos[j]; }, [&](const float4& bj)
+        {
             const float dx = xi - bj.x, dy = yi - bj.y, dz = zi - bj.z;
             const float f = kgFactor<kFast>(dist2(dx, dy, dz), k);
             const float gx = f * dx, gy = f * dy, gz = f * dz;
@@ -229,8 +244,7 @@ namespace tsp
             cBz = __builtin_fmaf(psi, gz, cBz);
         });
         float sR = 0.0f, cRx = 0.0f, cRy = 0.0f, cRz = 0.0f;
-        const List fr = listAt(d, REL_FR, p, i);
-        visit(fr, [&](uint32_t j, uint32_t)
+        visit(l.list(d, REL_FR), [&](uint32_t j)
         {
             const float4 rj = d.rpos[j], uj = d.rvp[j];
             const float dx = xi - rj.x, dy = yi - rj.y, dz = zi - rj.z;
@@ -245,7 +259,7 @@ namespace tsp
             cRz = __builtin_fmaf(psi, gz, cRz);
         });
         sF *= k.mass;
-        const float src = k.rho0 - d.vel[i].w - k.dt * (sF + sB + sR);
+        const float src = k.rho0 - rho - k.dt * (sF + sB + sR);
         const float ctx = cFx * k.cFacF + (cBx + cRx) * k.cFacB;
         const float cty = cFy * k.cFacF + (cBy + cRy) * k.cFacB;
         const float ctz = cFz * k.cFacF + (cBz + cRz) * k.cFacB;
@@ -310,8 +324,7 @@ namespace tsp
     }
 
     // threads of a solver sweep block (one 256-particle tile per block)
-    constexpr uint32_t kSweepThreads = TSP_TUNE_SWEEP_THREADS;
-    static_assert(kBlock % kSweepThreads == 0 && kSweepThreads % 64 == 0, "sweep block size");
+    constexpr uint32_t kSweepThreads = kBlock;
 
     // the bookkeeping of one scene after a Jacobi sweep (sph_solver.cpp:207-261): the scene's block
     // partials summed in a fixed order, the averages, TerminationConditionSatisfied and the error
@@ -387,53 +400,18 @@ namespace tsp
     // a sweep's pressure accelerations; block 0 of a sweep launch first finishes the bookkeeping of
     // the previous Jacobi sweep, which the next Jacobi launch reads. Blocks that see the solve
     // converged skip their particles: the final launch (sweep = false) recomputes every a^p.
-    // The sweeps walk the 256-particle tiles of all scenes. One block per tile, in the XCD-aware
-    // order of xcdBlock(); or (TSP_TUNE_PERSISTENT) a grid of at most kSweepGrid resident blocks,
-    // each walking its XCD's contiguous range of tiles with a stride of the blocks per XCD.
-    constexpr uint32_t kSweepGrid = 256u * 6u;
-
-    template <typename Fn>
-    __device__ __forceinline__ void forTiles(uint32_t nTiles, Fn tile)
-    {
-#if TSP_TUNE_PERSISTENT
-        if (gridDim.x >= nTiles)
-        {
-            tile(xcdBlock());
-            return;
-        }
-        const uint32_t b = blockIdx.x, xcd = b & 7u, stride = gridDim.x >> 3;
-        const uint32_t per = nTiles >> 3, rem = nTiles & 7u;
-        const uint32_t start = xcd < rem ? xcd * (per + 1u) : rem * (per + 1u) + (xcd - rem) * per;
-        const uint32_t end = start + per + (xcd < rem ? 1u : 0u);
-        for (uint32_t t = start + (b >> 3); t < end; t += stride)
-        {
-            tile(t);
-            // the next tile restages the LDS records and flags this one has read
-            __syncthreads();
-        }
-#else
-        (void)nTiles;
-        tile(xcdBlock());
-#endif
-    }
-
-    static inline uint32_t sweepGrid(uint32_t nTiles)
-    {
-#if TSP_TUNE_PERSISTENT
-        return nTiles < kSweepGrid ? nTiles : kSweepGrid;
-#else
-        return nTiles;
-#endif
-    }
-
     // one tile of a sweep's pressure accelerations
     template <bool kFast>
     __device__ __forceinline__ void pressureAccTile(const Dev& d, uint32_t blk, bool sweep)
     {
         __shared__ float4 hp[kHaloMax];
         __shared__ uint32_t skip;
-        const uint32_t sc = d.blockScene[blk];
-        const Consts& k = d.consts[sc];
+        const Lists l = listsAt(d, blk);
+        const SlotList slots = slotsOf(d, l);
+        const Halo h = haloOf(d, blk);
+        const uint32_t sc = uniformLoad(&d.blockScene[blk]);
+        const Consts k = uniformLoad(&d.consts[sc]);
+        const Scene S = uniformLoad(&d.scenes[sc]);
         if (sweep)
         {
             // one read per block, so the whole block leaves together
@@ -441,21 +419,16 @@ namespace tsp
             __syncthreads();
             if (skip) { return; }
         }
-        const uint32_t hc = d.haloCount[blk];
-        const bool ulps = hc <= kHaloMax && d.haloUlps[blk] != 0u;
-        stageHalo(d, blk, hc, [&](uint32_t q, uint32_t j) { hp[q] = d.pos[j]; });
-        for (uint32_t r = 0; r < kBlock / kSweepThreads; r++)
-        {
-        const uint32_t p = blk * kBlock + r * kSweepThreads + threadIdx.x;   // list position; i its particle
-        const uint32_t i = particleAt(d, p);
-        if (i - d.scenes[sc].offF >= d.scenes[sc].nF) { continue; }
+        const uint32_t i = l.i;
         const float4 p4 = d.pos[i];
+        stageHalo(h, [&](uint32_t j) { return d.pos[j]; }, [&](uint32_t q, const float4& r) { hp[q] = r; });
+        __syncthreads();
+        if (i - S.offF >= S.nF) { return; }
         const float xi = p4.x, yi = p4.y, zi = p4.z, pi = p4.w;
         float sx = 0.0f, sy = 0.0f, sz = 0.0f;
-        const List ff = listAt(d, REL_FF, p, i);
         // dict chunks sum (p_i + p_j) kg and scale once; normal chunks scale each neighbor's
         // pressure term (sph_solver.cpp:1573-1640)
-        const bool dict = ff.n <= kDictMax;
+        const bool dict = slots.n <= kDictMax;
         const float outerF = k.mass * pi * k.presDis;
         // the two forms as two loops (a wave runs the normal one only for a list longer than kDictMax)
         const auto sumFF = [&](auto dictFlag)
@@ -473,23 +446,14 @@ namespace tsp
                 sy = __builtin_fmaf(coeff, dy, sy);
                 sz = __builtin_fmaf(coeff, dz, sz);
             };
-            if (kFast && ulps)
-            {
-                visitSlots(ff, [&](uint32_t q) { return recAt(hp, q & kSlotMask); },
-                           [&](const float4& pj, uint32_t q) { ffTerm(pj, q, Flag<true>{}); });
-            }
-            else
-            {
-                visitFF(ff, hc <= kHaloMax, [&](uint32_t q, uint32_t) { ffTerm(recAt(hp, q & kSlotMask), q, Flag<false>{}); },
-                        [&](uint32_t j, uint32_t) { ffTerm(d.pos[j], 0u, Flag<false>{}); });
-            }
+            if (kFast && h.ulps) { visitSlots(slots, [&](uint32_t q, uint32_t) { ffTerm(recAt(hp, q & kSlotMask), q, Flag<true>{}); }); }
+            else if (h.any) { visitSlots(slots, [&](uint32_t q, uint32_t) { ffTerm(recAt(hp, q & kSlotMask), q, Flag<false>{}); }); }
+            else { visit(l.list(d, REL_FF), [&](uint32_t j) { ffTerm(d.pos[j], 0u, Flag<false>{}); }); }
         };
         if (dict) { sumFF(Flag<true>{}); } else { sumFF(Flag<false>{}); }
         float ax = dict ? sx * k.presOuterFF : sx, ay = dict ? sy * k.presOuterFF : sy, az = dict ? sz * k.presOuterFF : sz;
-        const List fb = listAt(d, REL_FB, p, i);
-        visit(fb, [&](uint32_t j, uint32_t)
+        visitGather(d, l, REL_FB, [&](uint32_t j) { return d.bpos[j]; }, [&](const float4& bj)
         {
-            const float4 bj = d.bpos[j];
             const float dx = xi - bj.x, dy = yi - bj.y, dz = zi - bj.z;
             const float f = kgFactor<kFast>(dist2(dx, dy, dz), k);
             const float coeff = k.presOuterB * bj.w * pi;
@@ -497,8 +461,7 @@ namespace tsp
             ay = __builtin_fmaf(coeff, f * dy, ay);
             az = __builtin_fmaf(coeff, f * dz, az);
         });
-        const List fr = listAt(d, REL_FR, p, i);
-        visit(fr, [&](uint32_t j, uint32_t)
+        visit(l.list(d, REL_FR), [&](uint32_t j)
         {
             const float4 rj = d.rpos[j];
             const float dx = xi - rj.x, dy = yi - rj.y, dz = zi - rj.z;
@@ -509,7 +472,6 @@ namespace tsp
             az = __builtin_fmaf(coeff, f * dz, az);
         });
         d.ap[i] = make_float4(0.0f - ax, 0.0f - ay, 0.0f - az, 0.0f);
-        }
     }
 
     template <bool kFast>
@@ -521,7 +483,7 @@ namespace tsp
         {
             for (uint32_t q = blockIdx.x; q < d.nScenes; q += gridDim.x) { finalizeSweep(d, q, nTiles); }
         }
-        forTiles(nTiles, [&](uint32_t blk) { pressureAccTile<kFast>(d, blk, sweep); });
+        pressureAccTile<kFast>(d, xcdBlock(), sweep);
     }
 
 
@@ -537,37 +499,34 @@ namespace tsp
 #else
         __shared__ float4 hp[kHaloMax], ha[kHaloMax];
 #endif
-        const uint32_t sc = d.blockScene[blk];
-        const Consts& k = d.consts[sc];
-        const Scene& S = d.scenes[sc];
+        const Lists l = listsAt(d, blk);
+        const SlotList slots = slotsOf(d, l);
+        const Halo h = haloOf(d, blk);
+        const uint32_t sc = uniformLoad(&d.blockScene[blk]);
+        const Consts k = uniformLoad(&d.consts[sc]);
+        const Scene S = uniformLoad(&d.scenes[sc]);
         // the scene's flags were written by an earlier launch: every thread reads the same values
         if (d.solve[sc].converged) { return; }
         const bool compute = d.solve[sc].compute != 0u;
-        if (blk == S.blk0 && threadIdx.x == 0) { d.solve[sc].pending = 1u; }
-        const uint32_t hc = d.haloCount[blk];
-        const bool ulps = hc <= kHaloMax && d.haloUlps[blk] != 0u;
         // (positions only: the pressures this launch writes into pos.w are not read here)
+        const uint32_t i = l.i;
+        const float4 pi = d.pos[i], ai = d.ap[i];
+        const float src = d.source[i], diag = d.diag[i];
 #if TSP_TUNE_JACOBI_REC24
-        stageHalo(d, blk, hc, [&](uint32_t q, uint32_t j)
+        stageHalo(h, [&](uint32_t j) { return Pair4{ d.pos[j], d.ap[j] }; }, [&](uint32_t q, const Pair4& r)
         {
-            const float4 pj = d.pos[j], aj = d.ap[j];
-            hp[q] = make_float4(pj.x, pj.y, pj.z, aj.x);
-            ha[q] = make_float2(aj.y, aj.z);
+            hp[q] = make_float4(r.a.x, r.a.y, r.a.z, r.b.x);
+            ha[q] = make_float2(r.b.y, r.b.z);
         });
 #else
-        stageHalo(d, blk, hc, [&](uint32_t q, uint32_t j) { hp[q] = d.pos[j]; ha[q] = d.ap[j]; });
+        stageHalo(h, [&](uint32_t j) { return Pair4{ d.pos[j], d.ap[j] }; }, [&](uint32_t q, const Pair4& r) { hp[q] = r.a; ha[q] = r.b; });
 #endif
+        __syncthreads();
         double eRaw = 0.0, ePos = 0.0, eAbs = 0.0;
-        for (uint32_t r = 0; r < kBlock / kSweepThreads; r++)
-        {
-        const uint32_t p = blk * kBlock + r * kSweepThreads + threadIdx.x;   // list position; i its particle
-        const uint32_t i = particleAt(d, p);
         if (i - S.offF < S.nF)
         {
-            const float4 pi = d.pos[i], ai = d.ap[i];
             const float xi = pi.x, yi = pi.y, zi = pi.z, axi = ai.x, ayi = ai.y, azi = ai.z;
             float sf = 0.0f;
-            const List ff = listAt(d, REL_FF, p, i);
             const auto ffTerm = [&](float xj, float yj, float zj, float axj, float ayj, float azj, uint32_t q, auto shortFlag)
             {
                 constexpr bool kShort = decltype(shortFlag)::value;
@@ -596,38 +555,31 @@ namespace tsp
                 return Rec{ pj.x, pj.y, pj.z, aj.x, aj.y, aj.z };
             };
 #endif
-            if (kFast && ulps)
+            const auto fromHalo = [&](uint32_t q, auto shortFlag)
             {
-                visitSlots(ff, [&](uint32_t q) { return haloLoad(q & kSlotMask); },
-                           [&](const Rec& r, uint32_t q) { ffTerm(r.x, r.y, r.z, r.ax, r.ay, r.az, q, Flag<true>{}); });
-            }
+                const Rec r = haloLoad(q & kSlotMask);
+                ffTerm(r.x, r.y, r.z, r.ax, r.ay, r.az, q, shortFlag);
+            };
+            if (kFast && h.ulps) { visitSlots(slots, [&](uint32_t q, uint32_t) { fromHalo(q, Flag<true>{}); }); }
+            else if (h.any) { visitSlots(slots, [&](uint32_t q, uint32_t) { fromHalo(q, Flag<false>{}); }); }
             else
             {
-                visitFF(ff, hc <= kHaloMax,
-                        [&](uint32_t q, uint32_t)
-                        {
-                            const Rec r = haloLoad(q & kSlotMask);
-                            ffTerm(r.x, r.y, r.z, r.ax, r.ay, r.az, 0u, Flag<false>{});
-                        },
-                        [&](uint32_t j, uint32_t)
-                        {
-                            const float4 pj = d.pos[j], aj = d.ap[j];
-                            ffTerm(pj.x, pj.y, pj.z, aj.x, aj.y, aj.z, 0u, Flag<false>{});
-                        });
+                visit(l.list(d, REL_FF), [&](uint32_t j)
+                {
+                    const float4 pj = d.pos[j], aj = d.ap[j];
+                    ffTerm(pj.x, pj.y, pj.z, aj.x, aj.y, aj.z, 0u, Flag<false>{});
+                });
             }
             sf *= k.mass;
             float sb = 0.0f;
-            const List fb = listAt(d, REL_FB, p, i);
-            visit(fb, [&](uint32_t j, uint32_t)
+            visitGather(d, l, REL_FB, [&](uint32_t j) { return d.bpos[j]; }, [&](const float4& bj)
             {
-                const float4 bj = d.bpos[j];
                 const float dx = xi - bj.x, dy = yi - bj.y, dz = zi - bj.z;
                 const float f = kgFactor<kFast>(dist2(dx, dy, dz), k);
                 const float sv = __builtin_fmaf(axi, f * dx, __builtin_fmaf(ayi, f * dy, azi * (f * dz)));
                 sb += bj.w * sv;
             });
-            const List fr = listAt(d, REL_FR, p, i);
-            visit(fr, [&](uint32_t j, uint32_t)
+            visit(l.list(d, REL_FR), [&](uint32_t j)
             {
                 const float4 rj = d.rpos[j];
                 const float dx = xi - rj.x, dy = yi - rj.y, dz = zi - rj.z;
@@ -636,7 +588,6 @@ namespace tsp
                 sb += rj.w * sv;
             });
             const float sys = k.dtsq * (sf + sb);
-            const float src = d.source[i], diag = d.diag[i];
             const float resid = src - sys;
             const float pred = sys - src;
             const bool valid = __builtin_fabsf(diag) > 1e-7f;
@@ -649,7 +600,7 @@ namespace tsp
                 eAbs += __builtin_fabs(e);
             }
         }
-        }
+        if (blk == S.blk0 && threadIdx.x == 0) { d.solve[sc].pending = 1u; }
         if (!compute) { return; }
         eRaw = waveSum(eRaw);
         ePos = waveSum(ePos);
@@ -672,7 +623,7 @@ namespace tsp
     __global__ void __launch_bounds__(kSweepThreads) TSP_WAVES_ATTR(TSP_TUNE_JACOBI_WAVES) kJacobi(Dev d, uint32_t nTiles)
     {
         if (stopped(d)) { return; }
-        forTiles(nTiles, [&](uint32_t blk) { jacobiTile<kFast>(d, blk, nTiles); });
+        jacobiTile<kFast>(d, xcdBlock(), nTiles);
     }
 
     // the bookkeeping of the last sweep of a group, one block per scene, before the host reads
@@ -921,15 +872,15 @@ namespace tsp
     {
         if (!d.nF) { return; }
         const uint32_t n = blocksOf(d.nF);
-        if (d.fastPairs) { kPressureAcc<true><<<sweepGrid(n), kSweepThreads, 0, s>>>(d, sweep, n); }
-        else { kPressureAcc<false><<<sweepGrid(n), kSweepThreads, 0, s>>>(d, sweep, n); }
+        if (d.fastPairs) { kPressureAcc<true><<<n, kSweepThreads, 0, s>>>(d, sweep, n); }
+        else { kPressureAcc<false><<<n, kSweepThreads, 0, s>>>(d, sweep, n); }
     }
     void launchJacobi(hipStream_t s, const Dev& d)
     {
         if (!d.nF) { return; }
         const uint32_t n = blocksOf(d.nF);
-        if (d.fastPairs) { kJacobi<true><<<sweepGrid(n), kSweepThreads, 0, s>>>(d, n); }
-        else { kJacobi<false><<<sweepGrid(n), kSweepThreads, 0, s>>>(d, n); }
+        if (d.fastPairs) { kJacobi<true><<<n, kSweepThreads, 0, s>>>(d, n); }
+        else { kJacobi<false><<<n, kSweepThreads, 0, s>>>(d, n); }
     }
     void launchFinalize(hipStream_t s, const Dev& d)
     {

@@ -461,7 +461,7 @@ struct tsp_ctx
         for (int r = 0; r < 3; r++)
         {
             d.poolCap[r] = cap[r];
-            d.pool[r] = alloc<uint16_t>(cap[r], poolAllocs, MEM_LF);
+            d.pool[r] = alloc<uint16_t>(cap[r] + kPoolPad, poolAllocs, MEM_LF);
         }
         d.rfCap = rfCap;
         d.rfIdx = alloc<uint32_t>(rfCap, poolAllocs, MEM_LR);
@@ -855,15 +855,14 @@ struct tsp_ctx
         d.ffMin = alloc<uint32_t>(nF, work, MEM_LF);
         d.wideList = alloc<uint32_t>(nF, work, MEM_LF);
         d.laneRank = alloc<uint8_t>(nF, work, MEM_LF);
-        d.rankWho = alloc<uint8_t>(nF, work, MEM_LF);
+        d.head = alloc<uint2>(nF, work, MEM_LF);
         d.ffMask = alloc<uint32_t>(static_cast<size_t>(kMaskWords) * nF, work, MEM_SF);
         {
             const uint64_t nBlocks = nF / kBlock;
             d.haloIdx = alloc<uint32_t>(nBlocks * kHaloMax, work, MEM_LF);
-            d.haloCount = alloc<uint32_t>(nBlocks, work, MEM_LF);
-            d.haloUlps = alloc<uint32_t>(nBlocks, work, MEM_LF);
+            d.haloInfo = alloc<HaloInfo>(nBlocks, work, MEM_LF);
             // no block has a halo until the first search builds one
-            hipCheck(hipMemsetAsync(d.haloCount, 0xff, sizeof(uint32_t) * std::max<uint64_t>(nBlocks, 1), stream), "memset");
+            hipCheck(hipMemsetAsync(d.haloInfo, 0xff, sizeof(HaloInfo) * std::max<uint64_t>(nBlocks, 1), stream), "memset");
         }
         d.rfCnt = alloc<uint32_t>(nR, work, MEM_LR);
         d.rbCnt = alloc<uint32_t>(nR, work, MEM_LR);
@@ -2278,11 +2277,7 @@ int tsp_get_neighbors(tsp_ctx* ctx, int rel, uint32_t* counts, uint32_t* idx, ui
         {
             hipCheck(hipMemcpy(cnt.data(), d.cnt[rel] + h.offF, sizeof(uint16_t) * n, hipMemcpyDeviceToHost), "D2H");
             hipCheck(hipMemcpy(meta.data(), d.meta[rel] + s0, sizeof(SliceMeta) * nSlices, hipMemcpyDeviceToHost), "D2H");
-#if TSP_TUNE_LANE_SORT
             hipCheck(hipMemcpy(laneRank.data(), d.laneRank + h.offF, n, hipMemcpyDeviceToHost), "D2H");
-#else
-            for (uint32_t i = 0; i < n; i++) { laneRank[i] = static_cast<uint8_t>(i % kBlock); }
-#endif
         }
         const uint32_t mask = 0xffffu;
         uint64_t tot = 0;
@@ -2294,12 +2289,13 @@ int tsp_get_neighbors(tsp_ctx* ctx, int rel, uint32_t* counts, uint32_t* idx, ui
         if (units) { hipCheck(hipMemcpy(pool.data(), d.pool[rel], sizeof(uint16_t) * units, hipMemcpyDeviceToHost), "D2H"); }
         // FF entries of blocks with a halo are halo slots
         const uint32_t b0 = h.blk0, nBlocks = h.nBlk;
-        std::vector<uint32_t> haloCount, haloIdx;
+        std::vector<HaloInfo> haloInfo;
+        std::vector<uint32_t> haloIdx;
         if (rel == REL_FF && nBlocks)
         {
-            haloCount.resize(nBlocks);
+            haloInfo.resize(nBlocks);
             haloIdx.resize(static_cast<size_t>(nBlocks) * kHaloMax);
-            hipCheck(hipMemcpy(haloCount.data(), d.haloCount + b0, sizeof(uint32_t) * nBlocks, hipMemcpyDeviceToHost), "D2H");
+            hipCheck(hipMemcpy(haloInfo.data(), d.haloInfo + b0, sizeof(HaloInfo) * nBlocks, hipMemcpyDeviceToHost), "D2H");
             hipCheck(hipMemcpy(haloIdx.data(), d.haloIdx + static_cast<size_t>(b0) * kHaloMax, sizeof(uint32_t) * haloIdx.size(),
                                hipMemcpyDeviceToHost), "D2H");
         }
@@ -2312,7 +2308,7 @@ int tsp_get_neighbors(tsp_ctx* ctx, int rel, uint32_t* counts, uint32_t* idx, ui
             const SliceMeta& m = meta[p / kSlice];
             const uint32_t lane = p % kSlice;
             const uint32_t blk = i / kBlock;
-            const bool slots = rel == REL_FF && haloCount[blk] <= kHaloMax;
+            const bool slots = rel == REL_FF && haloInfo[blk].count <= kHaloMax;
             for (uint32_t k = 0; k < (cnt[i] & mask); k++)
             {
                 uint32_t j;

@@ -11,13 +11,12 @@
 //              body-frame offsets, body (u32), id (u64), reaction force (f32); per-body state
 //              field-major (f32) with FP64 force/torque sums
 //   cell grid  dense over the cell frame, one uint2 {begin, end} per cell and particle class
-//   SELL-32    per slice of 32 fluid list positions and relation (FF, FB, FR): one
+//   SELL       per slice of 64 fluid list positions and relation (FF, FB, FR): one
 //              SliceMeta {offset in u16 units, base, pitch, format}; entry k of lane l at
-//              offset + k*32 + l, as u16 (j - base) or u32 j. FF entries of a block with a halo
-//              hold the slot of j in the block's halo instead (same u16/u32 storage, no base).
-//              List position p holds the lists of one particle of p's 256-particle block: p
-//              itself, or, with lane sorting, the block's particles by list length (laneRank,
-//              rankWho)
+//              offset + k*64 + l, as u16 (j - base) or u32 j. FF entries of a block with a halo
+//              hold the slot of j in the block's halo instead (u16, no base).
+//              List position p holds the lists of one particle of p's 256-particle block, the
+//              longest FF lists first (laneRank, head)
 //   halo       per 256-particle block: up to kHaloMax (1064 tuned) distinct FF neighbor indices,
 //              ascending
 #pragma once
@@ -26,8 +25,6 @@
 #include <stdint.h>
 
 // build-time variants of the solver sweeps (all give the same bits; the build picks one):
-//   TSP_TUNE_PREFETCH      the next four list entries load while the current four are summed
-//   TSP_TUNE_GATHER4       the sweeps read the LDS halo records of four entries before summing them
 //   TSP_TUNE_SWEEP_AHEAD   the first sweep group of a step: the previous step's sweeps plus this
 //   TSP_TUNE_BOX_CELLS     the fill stages the fluid cell ranges of its block's stencil box in LDS
 //                          when the box has at most this many cells (0: off)
@@ -44,15 +41,7 @@
 //   TSP_TUNE_GRAPHS        each group of solver sweeps runs as one instantiated HIP graph
 //   TSP_TUNE_PA_WAVES, TSP_TUNE_JACOBI_WAVES   waves per SIMD the compiler must leave room for
 //                          (register budget of the sweep kernels); 0 leaves the choice to it
-//   TSP_TUNE_PERSISTENT    the solver sweeps run as persistent kernels: a resident grid whose
-//                          blocks walk the 256-particle tiles, instead of one block per tile
-//   TSP_TUNE_SLICE         SELL slice height: 32 (a wave covers two slices) or 64 (one slice per wave)
 //   TSP_TUNE_RADIX_BITS    digit width of the LSD radix sorts (8: 256 buckets, 6, 4)
-//   TSP_TUNE_SWEEP_THREADS threads per 256-particle tile of the solver sweeps (256, or 128: two
-//                          particles per thread)
-//   TSP_TUNE_LANE_SORT     the lists of each 256-particle block take its list positions longest
-//                          first, so a wave's lanes walk lists of similar length (1: by FF count,
-//                          2: by FB count, then FF count; 0: positions in particle order)
 //   TSP_TUNE_SEARCH_FLAT   the count pass folds its hits in through selects, its row streams loading
 //                          past their end (1) or branching around those loads (2); or it branches
 //                          on each candidate (0)
@@ -81,12 +70,6 @@
 #ifndef TSP_TUNE_SWEEP_AHEAD
 #define TSP_TUNE_SWEEP_AHEAD -1
 #endif
-#ifndef TSP_TUNE_GATHER4
-#define TSP_TUNE_GATHER4 0
-#endif
-#ifndef TSP_TUNE_PREFETCH
-#define TSP_TUNE_PREFETCH 1
-#endif
 #ifndef TSP_TUNE_JACOBI_REC24
 #define TSP_TUNE_JACOBI_REC24 1
 #endif
@@ -105,26 +88,14 @@
 #ifndef TSP_TUNE_SEARCH_ROW
 #define TSP_TUNE_SEARCH_ROW 1
 #endif
-#ifndef TSP_TUNE_PERSISTENT
-#define TSP_TUNE_PERSISTENT 0
-#endif
 #ifndef TSP_TUNE_SEARCH_FLAT
 #define TSP_TUNE_SEARCH_FLAT 0
-#endif
-#ifndef TSP_TUNE_LANE_SORT
-#define TSP_TUNE_LANE_SORT 1
 #endif
 #ifndef TSP_TUNE_SEARCH_BATCH
 #define TSP_TUNE_SEARCH_BATCH 4
 #endif
-#ifndef TSP_TUNE_SLICE
-#define TSP_TUNE_SLICE 32
-#endif
 #ifndef TSP_TUNE_RADIX_BITS
 #define TSP_TUNE_RADIX_BITS 8
-#endif
-#ifndef TSP_TUNE_SWEEP_THREADS
-#define TSP_TUNE_SWEEP_THREADS 256
 #endif
 #define TSP_WAVES_ATTR_0
 #define TSP_WAVES_ATTR_1 __attribute__((amdgpu_waves_per_eu(1)))
@@ -141,8 +112,7 @@
 namespace tsp
 {
     constexpr int kBlock = 256;          // threads per block: 4 waves of 64
-    constexpr uint32_t kSlice = TSP_TUNE_SLICE;   // SELL slice height (32: a wave covers two slices)
-    static_assert(kSlice == 32 || kSlice == 64, "slice height");
+    constexpr uint32_t kSlice = 64;      // SELL slice height: one slice per wave
     constexpr uint32_t kRadixBits = TSP_TUNE_RADIX_BITS;
     constexpr uint32_t kRadixBins = 1u << kRadixBits;
     static_assert(kRadixBits >= 1 && kRadixBits <= 8, "radix digit width");
@@ -179,6 +149,23 @@ namespace tsp
     {
         static constexpr bool value = B;
     };
+
+    // A wave-uniform record that no thread of the running kernel writes, through the scalar cache: read
+    // from the constant address space, because the compiler takes the vector path for a plain load
+    // once the kernel has stored anything.
+    template <typename T>
+    __device__ __forceinline__ T uniformLoad(const T* p)
+    {
+        constexpr uint32_t kWords = sizeof(T) / 4u;
+        static_assert(sizeof(T) % 4u == 0u, "whole words");
+        using Word = const __attribute__((address_space(4))) uint32_t;
+        Word* w = (Word*)p;
+        uint32_t v[kWords];
+        for (uint32_t q = 0; q < kWords; q++) { v[q] = w[q]; }
+        T r;
+        __builtin_memcpy(&r, v, sizeof(T));
+        return r;
+    }
 
     struct SliceMeta
     {
@@ -339,6 +326,13 @@ namespace tsp
     enum { CR_RHO, CR_DIAG, CR_P, CR_SRC, CR_ERR, CR_OM, CR_VX, CR_VY, CR_VZ, CR_FX, CR_FY, CR_FZ, kCR };
     enum { CB_RHO, CB_DIAG, CB_P, CB_SRC, CB_ERR, CB_OM, kCB };
 
+    // the FF halo of a block
+    struct HaloInfo
+    {
+        uint32_t count;          // its size, or kNoHalo
+        uint32_t ulps;           // 1 while every halo entry's low bits correct kgShort exactly
+    };
+
     // device pointers of one context (passed by value to every kernel)
     struct Dev
     {
@@ -383,16 +377,16 @@ namespace tsp
         SliceMeta *meta[3];
         uint16_t *pool[3];
         uint64_t poolCap[3];     // u16 units
-        uint8_t *laneRank;       // per particle: its list position within its block (lane sorting)
-        uint8_t *rankWho;        // per list position: the particle's index within the block (lane sorting)
+        uint8_t *laneRank;       // per particle: its list position within its block
+        uint2 *head;             // per list position: FF count | FB count << 16, FR count | particle << 16
+                                 // (its index within the block): what a kernel thread reads first
         uint32_t *ffMin;         // per particle: smallest FF neighbor index (0 without FF neighbors), with
                                  // kWideBit set when the list spans more than 0xffff
         uint32_t *wideList;      // the particles with kWideBit, in no particular order (status->wideCount)
         uint32_t *ffMask;        // kMaskWords x nF: per stencil row, bit q = the row's q-th fluid candidate
                                  // is an FF neighbor; then the rows the masks do not cover
         uint32_t *haloIdx;       // per block: kHaloMax particle indices, ascending
-        uint32_t *haloCount;     // per block: halo size, or kNoHalo
-        uint32_t *haloUlps;      // per block: 1 while every halo entry's low bits correct kgShort exactly
+        HaloInfo *haloInfo;      // per block
         // rigid-source CSR (RF), counts of RB and RR
         uint32_t *rfCnt, *rfOff, *rfIdx;
         uint32_t *rbCnt, *rrCnt;
@@ -627,7 +621,7 @@ namespace tsp
     // computes the exact factor of every pair anyway, stores the difference in ulps in the four low
     // bits of the pair's halo entry (zero in a byte offset of 16-byte records), and the solver sweeps
     // add it back with one dot-product instruction: the same bits for 8 issue slots less. A block
-    // with a difference outside [-8, 7] keeps the exact form (Dev::haloUlps). Measured with rootRcp
+    // with a difference outside [-8, 7] keeps the exact form (HaloInfo::ulps). Measured with rootRcp
     // on the 1M cube drop: kJacobi 1,529 to 1,247 VALU instructions per wave, 49.2 to 47.4 us;
     // kPressureAcc 40.2 to 38.0 us; kSourceDiag, which stores the corrections, 66.8 to 69.8 us.
     __device__ __forceinline__ float kgShort(float d2, const Consts& k)
@@ -716,25 +710,9 @@ namespace tsp
     };
 
     // the list position of particle i, and the particle at list position p (both in its block)
-    __device__ __forceinline__ uint32_t sellPos(const Dev& d, uint32_t i)
-    {
-#if TSP_TUNE_LANE_SORT
-        return (i & ~(kBlock - 1u)) + d.laneRank[i];
-#else
-        (void)d;
-        return i;
-#endif
-    }
+    __device__ __forceinline__ uint32_t sellPos(const Dev& d, uint32_t i) { return (i & ~(kBlock - 1u)) + d.laneRank[i]; }
 
-    __device__ __forceinline__ uint32_t particleAt(const Dev& d, uint32_t p)
-    {
-#if TSP_TUNE_LANE_SORT
-        return (p & ~(kBlock - 1u)) + d.rankWho[p];
-#else
-        (void)d;
-        return p;
-#endif
-    }
+    __device__ __forceinline__ uint32_t particleAt(const Dev& d, uint32_t p) { return (p & ~(kBlock - 1u)) + (d.head[p].y >> 16); }
 
     // the list of relation rel of particle i, stored at list position p
     __device__ __forceinline__ List listAt(const Dev& d, int rel, uint32_t p, uint32_t i)
@@ -749,101 +727,194 @@ namespace tsp
 
     __device__ __forceinline__ List listOf(const Dev& d, int rel, uint32_t i) { return listAt(d, rel, sellPos(d, i), i); }
 
-    // visits the entries of one list in storage order, as use(load(j), e): j the neighbor (or its
-    // halo slot when kSlots: the stored value without the slice base) and e the entry's position
-    // in u16 units of the pool, which also indexes the per-entry gradient factors. The index loads
-    // of four entries are issued together, then the four gathers (load), then the four sums (use)
-    // in entry order.
-    template <bool kSlots, typename Load, typename Use>
-    __device__ __forceinline__ void visitSplit(const List& l, Load&& load, Use&& use)
+    // visits the entries of one list in storage order, as fn(j): j the neighbor, or its halo entry as
+    // stored when kSlots. The index loads of four entries are issued together.
+    template <bool kSlots, typename Fn>
+    __device__ __forceinline__ void visitEntries(const List& l, Fn&& fn)
     {
-        const auto fn4 = [&](uint32_t j0, uint32_t j1, uint32_t j2, uint32_t j3, uint32_t e, uint32_t step)
-        {
-            const auto r0 = load(j0);
-            const auto r1 = load(j1);
-            const auto r2 = load(j2);
-            const auto r3 = load(j3);
-            use(r0, e); use(r1, e + step); use(r2, e + 2u * step); use(r3, e + 3u * step);
-        };
-        const auto fn = [&](uint32_t j, uint32_t e) { use(load(j), e); };
         uint32_t q = 0;
         if (l.m.format == kFmtDelta16)
         {
-            const uint32_t e0 = l.m.offset + l.lane;
-            const uint16_t* p = l.pool + e0;
+            const uint16_t* p = l.pool + l.m.offset + l.lane;
             const uint32_t base = kSlots ? 0u : l.m.base;
-#if TSP_TUNE_PREFETCH
-            // the next four indices load while the current four are summed
-            uint32_t j0 = 0, j1 = 0, j2 = 0, j3 = 0;
-            if (l.n >= 4) { j0 = p[0]; j1 = p[kSlice]; j2 = p[2 * kSlice]; j3 = p[3 * kSlice]; }
-            for (; q + 4 <= l.n; q += 4)
-            {
-                uint32_t n0 = 0, n1 = 0, n2 = 0, n3 = 0;
-                if (q + 8 <= l.n)
-                {
-                    n0 = p[(q + 4) * kSlice]; n1 = p[(q + 5) * kSlice];
-                    n2 = p[(q + 6) * kSlice]; n3 = p[(q + 7) * kSlice];
-                }
-                fn4(base + j0, base + j1, base + j2, base + j3, e0 + q * kSlice, kSlice);
-                j0 = n0; j1 = n1; j2 = n2; j3 = n3;
-            }
-#else
             for (; q + 4 <= l.n; q += 4)
             {
                 const uint32_t j0 = p[(q + 0) * kSlice], j1 = p[(q + 1) * kSlice];
                 const uint32_t j2 = p[(q + 2) * kSlice], j3 = p[(q + 3) * kSlice];
-                fn4(base + j0, base + j1, base + j2, base + j3, e0 + q * kSlice, kSlice);
+                fn(base + j0); fn(base + j1); fn(base + j2); fn(base + j3);
             }
-#endif
-            for (; q < l.n; q++) { fn(base + p[q * kSlice], e0 + q * kSlice); }
+            for (; q < l.n; q++) { fn(base + p[q * kSlice]); }
         }
         else
         {
-            const uint32_t e0 = l.m.offset + 2u * l.lane;
             const uint32_t* p = reinterpret_cast<const uint32_t*>(l.pool + l.m.offset) + l.lane;
             for (; q + 4 <= l.n; q += 4)
             {
                 const uint32_t j0 = p[(q + 0) * kSlice], j1 = p[(q + 1) * kSlice];
                 const uint32_t j2 = p[(q + 2) * kSlice], j3 = p[(q + 3) * kSlice];
-                fn4(j0, j1, j2, j3, e0 + 2u * q * kSlice, 2u * kSlice);
+                fn(j0); fn(j1); fn(j2); fn(j3);
             }
-            for (; q < l.n; q++) { fn(p[q * kSlice], e0 + 2u * q * kSlice); }
+            for (; q < l.n; q++) { fn(p[q * kSlice]); }
         }
-    }
-
-    // the same with the neighbor passed through: fn(j, e)
-    template <bool kSlots, typename Fn>
-    __device__ __forceinline__ void visitEntries(const List& l, Fn&& fn)
-    {
-        visitSplit<kSlots>(l, [](uint32_t j) { return j; }, fn);
     }
 
     template <typename Fn>
     __device__ __forceinline__ void visit(const List& l, Fn&& fn) { visitEntries<false>(l, fn); }
 
-    // FF neighbors of a particle: from the block's LDS halo when it has one, else from HBM
-    template <typename FromHalo, typename FromGlobal>
-    __device__ __forceinline__ void visitFF(const List& l, bool halo, FromHalo&& fh, FromGlobal&& fg)
+    // --- the per-particle SPH kernels: one thread per list position of a 256-particle block ---
+
+    // The lists at a thread's position. The slices' headers are read once per wave (a wave's 64
+    // positions are one slice), the counts and the particle in one 8-byte word per position.
+    struct Lists
     {
-        if (halo) { visitEntries<true>(l, fh); }
-        else { visitEntries<false>(l, fg); }
+        uint32_t i, lane;        // the particle, and the position's lane in its slice
+        uint32_t n[3];
+        SliceMeta m[3];
+
+        __device__ __forceinline__ List list(const Dev& d, int rel) const { return List{ d.pool[rel], m[rel], lane, n[rel] }; }
+    };
+
+    __device__ __forceinline__ Lists listsAt(const Dev& d, uint32_t blk)
+    {
+        const uint32_t p = blk * kBlock + threadIdx.x;
+        Lists l;
+        const uint2 h = d.head[p];
+        l.i = blk * kBlock + (h.y >> 16);
+        l.lane = p & (kSlice - 1u);
+        l.n[REL_FF] = h.x & 0xffffu;
+        l.n[REL_FB] = h.x >> 16;
+        l.n[REL_FR] = h.y & 0xffffu;
+        const uint32_t slice = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(p / kSlice)));
+        for (int r = 0; r < 3; r++) { l.m[r] = uniformLoad(&d.meta[r][slice]); }
+        return l;
     }
 
-    // the entries of a list in a block with a halo, as use(load(q), q): q the stored halo entry, load
-    // its record. With TSP_TUNE_GATHER4 the four LDS reads of a group issue before its four sums.
-    template <typename Load, typename Use>
-    __device__ __forceinline__ void visitSlots(const List& l, Load&& load, Use&& use)
+    // rows that a pool holds past its last slice: the first rows of a list and the rows after the
+    // current ones load without a look at the lane's own count
+    constexpr uint32_t kPoolPad = 8u * kSlice;
+
+    // The FF list of a block with a halo (u16 entries, in wave-uniform rows). The first four entries
+    // load with the list's head, before the halo is staged; then four entries load while the four
+    // before are summed. use(q, k) sees entry q at row k in list order.
+    struct SlotList
     {
-#if TSP_TUNE_GATHER4
-        struct Got
+        uint16_t* p;             // the lane's entry in row 0
+        uint32_t pitch, n;
+        uint32_t j[4];
+    };
+
+    __device__ __forceinline__ SlotList slotsOf(const Dev& d, const Lists& l)
+    {
+        SlotList s;
+        s.p = d.pool[REL_FF] + l.m[REL_FF].offset + l.lane;
+        s.pitch = l.m[REL_FF].pitch;
+        s.n = l.n[REL_FF];
+        for (uint32_t u = 0; u < 4; u++) { s.j[u] = s.p[u * kSlice]; }
+        return s;
+    }
+
+    template <typename Use>
+    __device__ __forceinline__ void visitSlots(const SlotList& s, Use&& use)
+    {
+        uint32_t j0 = s.j[0], j1 = s.j[1], j2 = s.j[2], j3 = s.j[3];
+        const uint16_t* p = s.p + 4u * kSlice;
+        uint32_t q = 0;
+        for (; q + 4u <= s.n; q += 4u, p += 4u * kSlice)
         {
-            decltype(load(0u)) r;
-            uint32_t q;
+            uint32_t n0 = 0, n1 = 0, n2 = 0, n3 = 0;
+            if (q + 4u < s.pitch) { n0 = p[0]; n1 = p[kSlice]; n2 = p[2u * kSlice]; n3 = p[3u * kSlice]; }
+            use(j0, q); use(j1, q + 1u); use(j2, q + 2u); use(j3, q + 3u);
+            j0 = n0; j1 = n1; j2 = n2; j3 = n3;
+        }
+        if (q < s.n) { use(j0, q); }
+        if (q + 1u < s.n) { use(j1, q + 1u); }
+        if (q + 2u < s.n) { use(j2, q + 2u); }
+    }
+
+    // A list whose neighbors' records are gathered from memory, as use(load(j)) in list order: the
+    // records of four entries and the indices of the four after them load while the four before are
+    // summed (a chain of one load per four entries instead of two). Entries past the lane's list
+    // repeat its last one and are not used.
+    template <bool kWide, typename Load, typename Use>
+    __device__ __forceinline__ void visitGatherAs(const uint16_t* rows, uint32_t base, uint32_t lane, uint32_t n, Load&& load, Use&& use)
+    {
+        const uint16_t* p16 = rows + lane;
+        const uint32_t* p32 = reinterpret_cast<const uint32_t*>(rows) + lane;
+        using R = decltype(load(0u));
+        const auto entry = [&](uint32_t k)
+        {
+            const uint32_t e = min(k, n - 1u) * kSlice;
+            return kWide ? p32[e] : static_cast<uint32_t>(p16[e]);
         };
-        visitSplit<true>(l, [&](uint32_t q) { return Got{ load(q), q }; }, [&](const Got& g, uint32_t) { use(g.r, g.q); });
-#else
-        visitEntries<true>(l, [&](uint32_t q, uint32_t) { use(load(q), q); });
-#endif
+        const uint32_t b = kWide ? 0u : base;
+        uint32_t j0 = entry(0u), j1 = entry(1u), j2 = entry(2u), j3 = entry(3u);
+        R r0 = load(b + j0), r1 = load(b + j1), r2 = load(b + j2), r3 = load(b + j3);
+        j0 = entry(4u); j1 = entry(5u); j2 = entry(6u); j3 = entry(7u);
+        for (uint32_t q = 0; q < n; q += 4u)
+        {
+            const R s0 = r0, s1 = r1, s2 = r2, s3 = r3;
+            r0 = load(b + j0); r1 = load(b + j1); r2 = load(b + j2); r3 = load(b + j3);
+            j0 = entry(q + 8u); j1 = entry(q + 9u); j2 = entry(q + 10u); j3 = entry(q + 11u);
+            use(s0);
+            if (q + 1u < n) { use(s1); }
+            if (q + 2u < n) { use(s2); }
+            if (q + 3u < n) { use(s3); }
+        }
+    }
+
+    template <typename Load, typename Use>
+    __device__ __forceinline__ void visitGather(const Dev& d, const Lists& l, int rel, Load&& load, Use&& use)
+    {
+        const SliceMeta& m = l.m[rel];
+        if (m.pitch == 0u || l.n[rel] == 0u) { return; }
+        const uint16_t* rows = d.pool[rel] + m.offset;
+        if (m.format == kFmtDelta16) { visitGatherAs<false>(rows, m.base, l.lane, l.n[rel], load, use); }
+        else { visitGatherAs<true>(rows, 0u, l.lane, l.n[rel], load, use); }
+    }
+
+    // A block's FF halo: the indices load at once (all that a halo can hold, so that they need not
+    // wait for its size), then all records, then the records go to LDS.
+    struct Halo
+    {
+        static constexpr uint32_t kPer = (kHaloMax + kBlock - 1u) / kBlock;
+        uint32_t count;          // 0 in a block without a halo
+        bool any;                // the block has a halo
+        bool ulps;               // and its entries' low bits are corrections (HaloInfo::ulps)
+        uint32_t j[kPer];
+    };
+
+    __device__ __forceinline__ Halo haloOf(const Dev& d, uint32_t blk)
+    {
+        Halo h;
+        const uint32_t* idx = d.haloIdx + static_cast<size_t>(blk) * kHaloMax;
+        for (uint32_t u = 0; u < Halo::kPer; u++)
+        {
+            const uint32_t q = u * kBlock + threadIdx.x;
+            h.j[u] = (u + 1u < Halo::kPer || q < kHaloMax) ? idx[q] : 0u;
+        }
+        const HaloInfo info = uniformLoad(&d.haloInfo[blk]);
+        h.any = info.count <= kHaloMax;
+        h.ulps = h.any && info.ulps != 0u;
+        h.count = h.any ? info.count : 0u;
+        return h;
+    }
+
+    // every thread of the block calls it; load(j) reads a record, put(q, record) stores it in LDS
+    template <typename Load, typename Put>
+    __device__ __forceinline__ void stageHalo(const Halo& h, Load&& load, Put&& put)
+    {
+        using R = decltype(load(0u));
+        R r[Halo::kPer];
+        for (uint32_t u = 0; u < Halo::kPer; u++)
+        {
+            const uint32_t q = u * kBlock + threadIdx.x;
+            if (u * kBlock < h.count) { r[u] = load(q < h.count ? h.j[u] : 0u); }
+        }
+        for (uint32_t u = 0; u < Halo::kPer; u++)
+        {
+            const uint32_t q = u * kBlock + threadIdx.x;
+            if (u * kBlock < h.count && q < h.count) { put(q, r[u]); }
+        }
     }
 
     // --- rigid bodies, one body or particle (shared by the rigid kernels and the contact solve) ---

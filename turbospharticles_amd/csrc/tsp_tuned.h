@@ -5,9 +5,6 @@
 #ifndef TSP_TUNE_BOX_CELLS
 #define TSP_TUNE_BOX_CELLS 0
 #endif
-#ifndef TSP_TUNE_GATHER4
-#define TSP_TUNE_GATHER4 0
-#endif
 #ifndef TSP_TUNE_GRAPHS
 #define TSP_TUNE_GRAPHS 1
 #endif
@@ -26,12 +23,6 @@
 #ifndef TSP_TUNE_PA_WAVES
 #define TSP_TUNE_PA_WAVES 6
 #endif
-#ifndef TSP_TUNE_PERSISTENT
-#define TSP_TUNE_PERSISTENT 0
-#endif
-#ifndef TSP_TUNE_PREFETCH
-#define TSP_TUNE_PREFETCH 1
-#endif
 #ifndef TSP_TUNE_QUERY_WAVES
 #define TSP_TUNE_QUERY_WAVES 0
 #endif
@@ -47,20 +38,11 @@
 #ifndef TSP_TUNE_SEARCH_ROW
 #define TSP_TUNE_SEARCH_ROW 1
 #endif
-#ifndef TSP_TUNE_SLICE
-#define TSP_TUNE_SLICE 64
-#endif
 #ifndef TSP_TUNE_STEP_GRAPH
 #define TSP_TUNE_STEP_GRAPH 0
 #endif
 #ifndef TSP_TUNE_SWEEP_AHEAD
 #define TSP_TUNE_SWEEP_AHEAD 2
-#endif
-#ifndef TSP_TUNE_SWEEP_THREADS
-#define TSP_TUNE_SWEEP_THREADS 256
-#endif
-#ifndef TSP_TUNE_LANE_SORT
-#define TSP_TUNE_LANE_SORT 1
 #endif
 #ifndef TSP_TUNE_SEARCH_FLAT
 #define TSP_TUNE_SEARCH_FLAT 0

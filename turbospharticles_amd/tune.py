@@ -1,11 +1,10 @@
 """Autotuner of the build-time variants of the step (the TSP_TUNE_* switches in csrc/tsp_device.h).
 
-Every variant gives the same bits; they differ in how the work maps onto the GPU: the SELL slice
-height (32 or 64 particles per slice), the radix sort's digit width (8, 6 or 4 bits: 4 to 8 passes
-over 28-bit keys), the threads of a solver sweep tile (256, or 128 with two particles each), the
-sweeps' LDS reads of four halo records ahead of their sums, the size of a step's first sweep
+Every variant gives the same bits; they differ in how the work maps onto the GPU: the radix sort's
+digit width (8, 6 or 4 bits: 4 to 8 passes over 28-bit keys), the size of a step's first sweep
 group against the previous step's sweep count, the whole step as one graph launch or launch by
-launch, the FF halo built from page bitmaps or a window bitmap and hash set, prefetched list entries, 24- or 32-byte Jacobi halo records, the halo cap (LDS per sweep block), register budgets of the sweep
+launch, the FF halo built from page bitmaps or a window bitmap and hash set, 24- or 32-byte Jacobi
+halo records, the halo cap (LDS per sweep block), register budgets of the sweep
 kernels, sweep groups as HIP graphs, the neighbor query's walk of the stencil (cell by cell, or
 rows of three cells) and its candidate loads in flight. The
 tuner walks the switches one at a time from the current settings (coordinate descent), keeping a
@@ -38,11 +37,7 @@ TUNED_H = os.path.join(HERE, "csrc", "tsp_tuned.h")
 
 # switch -> values tried (the first is the default of tsp_device.h)
 SPACE = {
-    "TSP_TUNE_SLICE": [32, 64],
     "TSP_TUNE_RADIX_BITS": [8, 6, 4],
-    "TSP_TUNE_SWEEP_THREADS": [256, 128],
-    "TSP_TUNE_PREFETCH": [1, 0],
-    "TSP_TUNE_GATHER4": [0, 1],
     "TSP_TUNE_SWEEP_AHEAD": [-1, 0, 1, 2],
     "TSP_TUNE_STEP_GRAPH": [0, 1],
     "TSP_TUNE_QUERY_WAVES": [0, 6, 8],
@@ -54,10 +49,8 @@ SPACE = {
     "TSP_TUNE_PA_WAVES": [0, 6, 8],
     "TSP_TUNE_JACOBI_WAVES": [0, 6],
     "TSP_TUNE_SEARCH_ROW": [1, 0, 2],
-    "TSP_TUNE_LANE_SORT": [1, 0, 2],
     "TSP_TUNE_SEARCH_FLAT": [0, 1, 2],
     "TSP_TUNE_SEARCH_BATCH": [4, 8],
-    "TSP_TUNE_PERSISTENT": [0, 1],
 }
 
 
