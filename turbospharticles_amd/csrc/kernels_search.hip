@@ -10,18 +10,13 @@
 //   permute   one gather of the packed particle records per particle
 //   cells     dense {begin, end} table over the frame, written at the runs of the sorted keys;
 //             the previous step's runs are cleared first, so no global counter is needed
-//   count     per particle: FF/FB/FR counts over the 27-cell stencil (inclusive cutoff,
-//             distance fma(dx,dx,fma(dy,dy,dz*dz)), neighbor_search.cpp:1130-1249); per
-//             32-particle slice: pitch, base and u16/u32 format by width-32 lane reductions
-//   scan      multi-block exclusive scans (slice offsets, radix digit offsets, RF offsets)
+//   count     per particle: FF/FB/FR hit masks and counts over the 27-cell stencil (inclusive
+//             cutoff, distance fma(dx,dx,fma(dy,dy,dz*dz)), neighbor_search.cpp:1130-1249); per
+//             64-position slice: pitch, base, u16/u32 format and storage
+//   scan      multi-block exclusive scans (radix digit offsets, RF offsets)
 //   fill      writes the entries in the reference's iteration order: z-y-x stencil raster,
-//             ascending index within a cell; FF entries are staged in LDS and written as whole
-//             slice rows. FF lists whose indices span more than 0xffff keep the DictDelta16x2
-//             order of the reference's per-particle dict chunks (low group first, high group
-//             reversed, CPU/backend/neighbor_lists.h:171-197)
-//   halo      per 256-particle block: the distinct FF neighbors (LDS hash set, bitonic sort) and
-//             the block's FF entries rewritten as slots of that list, so the solver kernels
-//             stage the neighbor records in LDS once per block
+//             ascending index within a cell (CPU/backend/neighbor_lists.h:171-197 for wide lists),
+//             and builds the FF halo of each 256-particle block
 #include "tsp_device.h"
 
 namespace tsp
@@ -473,96 +468,217 @@ namespace tsp
     }
 
     // ----------------------------------------------------------------------------------------
-    // query: one thread per fluid particle (sorted order), 27-cell stencil in z-y-x raster order
+    // query: the 27-cell stencil in z-y-x raster order, one block of 768 threads per 256 particles.
+    //
+    // A wave takes 64 particles (one per lane) and three of the nine stencil rows (three x-adjacent
+    // cells each), so three waves share a particle and a lane's chain of dependent candidate loads is a
+    // third as long. The fill always runs so. The count pass does for up to kShareBlocks blocks (two per
+    // CU: the chain is what its time consists of); beyond that one wave walks all nine rows, because
+    // what the waves of a particle repeat, and their barriers, cost more than the shorter chain gains.
+    // kQueryCount, against one lane walking all rows candidate by candidate: 16 blocks 66 to 33 us, 250
+    // blocks 65 to 34 (one wave: 50), 432 blocks 82 to 49 (one wave: 67); 3,907 blocks 215 to 206 (three waves: 228),
+    // 31,250 blocks 1,333 to 1,205 (three waves: 1,446). What bounds the large launches is the vector
+    // memory path: 240 scattered 12-byte records per lane, about 20 cycles a wave each. (Candidates
+    // staged in LDS per 64 particles, in cell order: 250 us at 3,907 blocks, more barriers than loads
+    // saved.)
 
-    // the stencil's cell box, and the frame's cell-table layout kept in registers (the walk
-    // stores lists, so the compiler would otherwise reload the frame at every row)
+    constexpr uint32_t kQueryThreads = 768;
+    constexpr uint32_t kQueryShare = 3;          // waves per 64 particles
+    static_assert(kQueryThreads == kBlock * kQueryShare, "three waves per 64 particles");
+    constexpr uint32_t kShareBlocks = 512;       // most blocks that share particles in the count pass
+    // the word after a particle's masks: rows whose fluid (boundary) candidates the masks do not cover;
+    // all ones without masks
+    constexpr uint32_t kOpenF = 0, kOpenB = kMaskRows;
+
+    // the candidates of a stencil row: q -> q + (q < nA ? oA : oB). The cells 2m and 2m + 1 along x
+    // have consecutive Morton keys, so three x-adjacent cells are two runs of the sorted particles,
+    // ascending along the row.
+    struct RowSpan
+    {
+        uint32_t nA, n, oA, oB;
+
+        __device__ __forceinline__ uint32_t at(uint32_t q) const { return q + (q < nA ? oA : oB); }
+    };
+
+    // the row of the cells r[0..2], the first at an odd x or not
+    __device__ __forceinline__ RowSpan rowSpan(const uint2 (&r)[3], bool odd)
+    {
+        const uint32_t n0 = r[0].y - r[0].x, n1 = r[1].y - r[1].x, n2 = r[2].y - r[2].x;
+        RowSpan s;
+        s.n = n0 + n1 + n2;
+        s.nA = odd ? n0 : n0 + n1;
+        s.oA = (odd || n0) ? r[0].x : r[1].x;
+        s.oB = ((odd && n1) ? r[1].x : r[2].x) - s.nA;
+        return s;
+    }
+
+    // the local cell of a particle, from its position as its key was made
+    struct Cell
+    {
+        int l[3];
+    };
+
+    __device__ __forceinline__ Cell cellOf(const Frame& f, const float4& p)
+    {
+        return Cell{ { floorToInt(p.x * f.cellSizeInv) - f.orig[0], floorToInt(p.y * f.cellSizeInv) - f.orig[1],
+                       floorToInt(p.z * f.cellSizeInv) - f.orig[2] } };
+    }
+
+    // the three cells of a row of the stencil, as loaded
+    struct RowCells
+    {
+        uint2 r[3];
+        bool odd;
+
+        __device__ __forceinline__ RowSpan span() const { return rowSpan(r, odd); }
+    };
+
+    // The stencil of one particle: rows of side x side (y, z), each in chunks of three cells. Where the
+    // stencils of the wave's active particles all lie inside a reach-1 frame (`near`: nearly always) a
+    // row is one address; otherwise its cells are clamped to the frame. The loops over rows stay rolled:
+    // a scene of few blocks pays for every instruction fetched, not only for those executed.
     struct Stencil
     {
-        int lo[3], hi[3];
+        Cell at;
         uint32_t off, dx, dxy;   // first cell of the scene's tables, cells per y step, per z step
+        uint32_t dim[3];
+        int reach;
+        uint32_t side, chunks;
+        uint32_t first, last;    // the wave's rows
+        bool near;
 
-        __device__ __forceinline__ uint32_t cell(int x, int y, int z) const
+        // (lanes without `need` read the first cells of the tables and get an empty row)
+        __device__ __forceinline__ RowCells cells(const uint2* __restrict__ table, uint32_t row, bool need) const
         {
-            return off + static_cast<uint32_t>(x) + dx * static_cast<uint32_t>(y) + dxy * static_cast<uint32_t>(z);
+            RowCells c;
+            if (near)
+            {
+                const uint32_t zy = row;   // 3 (dz + 1) + dy + 1
+                const uint32_t y = static_cast<uint32_t>(at.l[1]) + zy % 3u - 1u, z = static_cast<uint32_t>(at.l[2]) + zy / 3u - 1u;
+                const uint32_t i = need ? off + static_cast<uint32_t>(at.l[0]) - 1u + dx * y + dxy * z : 0u;
+#pragma unroll
+                for (uint32_t q = 0; q < 3u; q++) { c.r[q] = table[i + q]; }
+                if (!need) { for (uint32_t q = 0; q < 3u; q++) { c.r[q] = make_uint2(0u, 0u); } }
+                c.odd = (at.l[0] & 1) == 0;
+                return c;
+            }
+            const uint32_t k = row % chunks, zy = row / chunks;
+            const int y = at.l[1] + static_cast<int>(zy % side) - reach, z = at.l[2] + static_cast<int>(zy / side) - reach;
+            const int x0 = at.l[0] - reach + 3 * static_cast<int>(k), x = max(x0, 0);
+            int nx = min(min(x0 + 2, at.l[0] + reach), static_cast<int>(dim[0]) - 1) - x + 1;
+            if (!need || y < 0 || y >= static_cast<int>(dim[1]) || z < 0 || z >= static_cast<int>(dim[2])) { nx = 0; }
+            const uint32_t i = off + static_cast<uint32_t>(x) + dx * static_cast<uint32_t>(y) + dxy * static_cast<uint32_t>(z);
+#pragma unroll
+            for (int q = 0; q < 3; q++) { c.r[q] = q < nx ? table[i + static_cast<uint32_t>(q)] : make_uint2(0u, 0u); }
+            c.odd = (x & 1) != 0;
+            return c;
         }
     };
 
-    __device__ __forceinline__ bool stencilOf(const Frame& f, uint64_t k, Stencil& s)
+    // share: which of the kShare waves of the 64 particles; active: the lane's particle is in the frame
+    template <uint32_t kShare>
+    __device__ __forceinline__ Stencil stencilOf(const Frame& f, const float4& p, bool active, uint32_t share)
     {
-        if (k >= f.emptyKey) { return false; }
-        const uint64_t m = k - f.keyBase;
-        const int l[3] = { static_cast<int>(compact21(m)), static_cast<int>(compact21(m >> 1)),
-                           static_cast<int>(compact21(m >> 2)) };
-        for (int a = 0; a < 3; a++)
-        {
-            s.lo[a] = max(l[a] - f.reach, 0);
-            s.hi[a] = min(l[a] + f.reach, static_cast<int>(f.dim[a]) - 1);
-        }
+        Stencil s;
+        s.at = cellOf(f, p);
         s.off = f.cellOff;
         s.dx = f.dim[0];
         s.dxy = f.dim[0] * f.dim[1];
-        return true;
-    }
-
-    // The fluid cell ranges of a block's stencil box -- the bounding box of the stencils of its
-    // particles, a few hundred cells for a Morton-ordered block -- staged in LDS, so the rows of
-    // the walk read them there instead of from the cell table. F is null when the box is off for
-    // the block (larger than kBoxCells, or TSP_TUNE_BOX_CELLS = 0).
-    constexpr uint32_t kBoxCells = TSP_TUNE_BOX_CELLS;
-    struct CellBox
-    {
-        const uint2* F;
-        int x0, y0, z0;
-        uint32_t w, wh;
-
-        __device__ __forceinline__ uint32_t at(int x, int y, int z) const
+        s.reach = f.reach;
+        s.side = 2u * static_cast<uint32_t>(f.reach) + 1u;
+        s.chunks = (s.side + 2u) / 3u;
+        bool edge = false;
+        for (int a = 0; a < 3; a++)
         {
-            return static_cast<uint32_t>(x - x0) + w * static_cast<uint32_t>(y - y0) + wh * static_cast<uint32_t>(z - z0);
+            s.dim[a] = f.dim[a];
+            edge = edge || s.at.l[a] < 1 || s.at.l[a] + 2 > static_cast<int>(f.dim[a]);
         }
-    };
-
-    // block-wide (every thread calls it): the box of the active stencils, staged into lds
-    // (kBoxCells entries) when it fits
-    __device__ __forceinline__ CellBox stageCellBox(const Dev& d, const Frame& f, const Stencil& s, bool active,
-                                                    uint2* lds, int* red)
-    {
-        CellBox b{};
-        if (kBoxCells == 0) { return b; }
-        if (threadIdx.x < 3) { red[threadIdx.x] = 0x7fffffff; red[threadIdx.x + 3] = -1; }
-        __syncthreads();
-        if (active)
-        {
-            for (int a = 0; a < 3; a++) { atomicMin(&red[a], s.lo[a]); atomicMax(&red[a + 3], s.hi[a]); }
-        }
-        __syncthreads();
-        b.x0 = red[0]; b.y0 = red[1]; b.z0 = red[2];
-        const int ex = red[3] - red[0] + 1, ey = red[4] - red[1] + 1, ez = red[5] - red[2] + 1;
-        __syncthreads();
-        if (ex <= 0) { return b; }   // no active particle
-        const uint64_t vol = static_cast<uint64_t>(ex) * static_cast<uint64_t>(ey) * static_cast<uint64_t>(ez);
-        if (vol > kBoxCells) { return b; }
-        b.w = static_cast<uint32_t>(ex);
-        b.wh = static_cast<uint32_t>(ex) * static_cast<uint32_t>(ey);
-        for (uint32_t q = threadIdx.x; q < vol; q += blockDim.x)
-        {
-            const int x = b.x0 + static_cast<int>(q % b.w), y = b.y0 + static_cast<int>((q / b.w) % static_cast<uint32_t>(ey));
-            const int z = b.z0 + static_cast<int>(q / b.wh);
-            lds[q] = d.cellF[linearCell(f, x, y, z)];
-        }
-        __syncthreads();
-        b.F = lds;
-        return b;
+        s.near = f.reach == 1 && !__any(active && edge);
+        const uint32_t rows = s.side * s.side * s.chunks;
+        s.first = rows * share / kShare;
+        s.last = rows * (share + 1u) / kShare;
+        return s;
     }
 
     __device__ __forceinline__ bool within(float xi, float yi, float zi, const float4& pj, float r2)
     {
-        const float dx = xi - pj.x, dy = yi - pj.y, dz = zi - pj.z;
-        return __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz)) <= r2;
+        return dist2(xi - pj.x, yi - pj.y, zi - pj.z) <= r2;
     }
 
-    // reductions over the lanes of one SELL slice (with 32-lane slices the two halves of a wave64
-    // are separate)
+    // Bit u of the result: candidate q0 + u of the row (u < n <= 32) lies within the support. The
+    // records of kQueryBatch candidates load together; those past the row's end are read (the record
+    // arrays are padded by kRecordPad) and masked. `tiny` is set by hits with 0 < d2 < 2^-96.
+    constexpr uint32_t kQueryBatch = 4;
+    static_assert(kQueryBatch <= kRecordPad && 32u % kQueryBatch == 0u, "loads past the end of a row");
+
+    __device__ __forceinline__ uint32_t hitMask(const float4* __restrict__ recs, const RowSpan& s, uint32_t q0, uint32_t n,
+                                                float xi, float yi, float zi, float r2, bool& tiny)
+    {
+        uint32_t m = 0;
+        for (uint32_t t = 0; t < n; t += kQueryBatch)
+        {
+            float4 p[kQueryBatch];
+#pragma unroll
+            for (uint32_t u = 0; u < kQueryBatch; u++) { p[u] = recs[s.at(q0 + t + u)]; }
+#pragma unroll
+            for (uint32_t u = 0; u < kQueryBatch; u++)
+            {
+                const float d2 = dist2(xi - p[u].x, yi - p[u].y, zi - p[u].z);
+                const bool hit = d2 <= r2 && t + u < n;
+                m |= (hit ? 1u : 0u) << (t + u);
+                tiny = tiny || (hit && tinyDist2(d2));
+            }
+        }
+        return m;
+    }
+
+    // The same for a whole row of at most 32 candidates, without the tiny test: the run's byte offset, the
+    // distance in the reference's order, the compare and the mask are about eleven instructions per
+    // candidate. Record offsets are 32-bit (kNearMax).
+    constexpr uint32_t kNearBatch = 4;
+    static_assert(kNearBatch <= kRecordPad && 32u % kNearBatch == 0u, "loads past the end of a row");
+    constexpr uint32_t kNearMax = 1u << 27;      // most records for 32-bit byte offsets
+
+    __device__ __forceinline__ uint32_t hitMaskNear(const float4* __restrict__ recs, const RowSpan& s, float xi, float yi,
+                                                    float zi, float r2)
+    {
+        // (the second run's offset counts from the row's start and may lie up to 32 records below 0)
+        const char* p = reinterpret_cast<const char*>(recs) - 32 * sizeof(float4);
+        const uint32_t a = (s.oA + 32u) * static_cast<uint32_t>(sizeof(float4)), b = (s.oB + 32u) * static_cast<uint32_t>(sizeof(float4));
+        uint32_t m = 0, t = 0;
+        for (; t < s.n; t += kNearBatch, p += kNearBatch * sizeof(float4))
+        {
+            float v[kNearBatch][3];
+#pragma unroll
+            for (uint32_t u = 0; u < kNearBatch; u++)
+            {
+                const float* q = reinterpret_cast<const float*>(p + static_cast<size_t>(t + u < s.nA ? a : b) + u * sizeof(float4));
+                v[u][0] = q[0]; v[u][1] = q[1]; v[u][2] = q[2];
+            }
+            __builtin_amdgcn_sched_barrier(0);   // (all loads of the batch before its first test)
+            uint32_t four = 0;
+#pragma unroll
+            for (uint32_t u = 0; u < kNearBatch; u++)
+            {
+                const float d2 = dist2(xi - v[u][0], yi - v[u][1], zi - v[u][2]);
+                four |= (d2 <= r2 ? 8u : 0u) >> u;
+            }
+            m = (m << 4) | four;
+        }
+        if (t == 0u) { return 0u; }
+        m = __brev(m) >> (32u - t);   // candidate 0 came in first
+        return s.n < 32u ? m & ((1u << s.n) - 1u) : m;
+    }
+
+    // A pair can only have 0 < d2 < 2^-96 if all its coordinate differences lie below 2^-48, one of
+    // them nonzero; floats of magnitude 2^-23 and up differ by at least 2^-47. So only particles with a
+    // coordinate nearer to zero than that are tested for such pairs.
+    __device__ __forceinline__ bool mayBeTiny(const float4& p)
+    {
+        return fminf(fminf(__builtin_fabsf(p.x), __builtin_fabsf(p.y)), __builtin_fabsf(p.z)) < 0x1p-23f;
+    }
+
+    // reductions over the lanes of one SELL slice (a wave)
     __device__ __forceinline__ uint32_t sliceMax(uint32_t v)
     {
         for (int o = kSlice / 2; o > 0; o >>= 1) { v = max(v, static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), o, kSlice))); }
@@ -581,947 +697,508 @@ namespace tsp
         return v;
     }
 
-    // the particle index of the q-th fluid candidate of a row stream (the three ranges in order)
-    __device__ __forceinline__ uint32_t rowCandidate(const uint2 (&r)[3], uint32_t q)
+    // the rank of keys[t] (distinct values) among the 256 of the block, the largest first; all threads of
+    // a block of 256 x kShare call it: each share counts a part of the keys. rank[] is zero before and
+    // valid after the next barrier.
+    template <uint32_t kShare>
+    __device__ __forceinline__ void rankDown(const uint32_t* keys, uint32_t* rank)
     {
-        const uint32_t n0 = r[0].y - r[0].x, n01 = n0 + (r[1].y - r[1].x);
-        return q < n0 ? r[0].x + q : (q < n01 ? r[1].x + (q - n0) : r[2].x + (q - n01));
+        const uint32_t t = threadIdx.x & (kBlock - 1u), part = threadIdx.x / kBlock;
+        const uint32_t own = keys[t];
+        const uint32_t lo = part * (kBlock / 4u) / kShare * 4u, hi = (part + 1u) * (kBlock / 4u) / kShare * 4u;
+        uint32_t r = 0;
+        for (uint32_t u = lo; u < hi; u += 4u)
+        {
+            const uint4 v = *reinterpret_cast<const uint4*>(&keys[u]);
+            r += (v.x > own ? 1u : 0u) + (v.y > own ? 1u : 0u) + (v.z > own ? 1u : 0u) + (v.w > own ? 1u : 0u);
+        }
+        atomicAdd(&rank[t], r);
     }
 
-    // The candidates of the stencil, per relation in list order: cells in z-y-x raster order,
-    // ascending index inside a cell. onF(j, pos), onB(j, bpos), onR(j, rpos) see each candidate of
-    // their relation once; the relations are separate lists, so only the order inside each one
-    // matters. withF / withB / withR = false skip a relation's candidates (and its cell ranges);
-    // needF(row) = false skips a row's fluid candidates.
-#if TSP_TUNE_SEARCH_ROW
-    // Row form: the ranges of up to three x-adjacent cells load together, and each relation's
-    // candidates along the row form one stream whose loads issue TSP_TUNE_SEARCH_BATCH at a time
-    // before their tests.
-    template <bool kFlat = false, typename Index, typename Load, typename Fn>
-    __device__ __forceinline__ void rowStream(const uint2 (&r)[3], Index index, Load load, Fn fn)
+    // The count pass (kShare: waves per 64 particles): hit masks, counts and index spans per particle; then the block's list positions,
+    // slice headers and storage. Storage is taken from the pools with one atomic per block (the
+    // blocks' order in the pools does not matter), so no scan over the slices follows.
+    template <uint32_t kShare>
+    __global__ void __launch_bounds__(kBlock * kShare) kQueryCount(Dev d)
     {
-        constexpr uint32_t kW = TSP_TUNE_SEARCH_BATCH;
-#if TSP_TUNE_SEARCH_ROW == 2
-        // cell by cell along the row, kW candidates at a time (a cell's candidates are contiguous)
-        uint32_t q0 = 0;
-#pragma unroll
-        for (int c = 0; c < 3; c++)
-        {
-            const uint32_t b = r[c].x, n = r[c].y - r[c].x;
-            for (uint32_t t = 0; t < n; t += kW)
-            {
-                uint32_t j[kW];
-                float4 p[kW];
-#pragma unroll
-                for (uint32_t u = 0; u < kW; u++)
-                {
-                    j[u] = 0u;
-                    p[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                    if (t + u < n) { j[u] = index(b + t + u); p[u] = load(j[u]); }
-                }
-#pragma unroll
-                for (uint32_t u = 0; u < kW; u++)
-                {
-                    if (t + u < n) { fn(j[u], p[u], q0 + t + u); }
-                }
-            }
-            q0 += n;
-        }
-#else
-        // the row's three ranges as one stream: candidate q is q + the offset of its range
-        const uint32_t n0 = r[0].y - r[0].x, n1 = r[1].y - r[1].x, n2 = r[2].y - r[2].x;
-        const uint32_t n01 = n0 + n1, total = n01 + n2;
-        const uint32_t o0 = r[0].x, o1 = r[1].x - n0, o2 = r[2].x - n01;
-        for (uint32_t t = 0; t < total; t += kW)
-        {
-            uint32_t j[kW];
-            float4 p[kW];
-#pragma unroll
-            for (uint32_t u = 0; u < kW; u++)
-            {
-                if (kFlat)
-                {
-                    // past the stream's end the last candidate loads again (fn does not see it):
-                    // the loads need no branch
-                    const uint32_t q = min(t + u, total - 1u);
-                    const uint32_t e = q + (q < n0 ? o0 : (q < n01 ? o1 : o2));
-                    j[u] = index(e);
-                    p[u] = load(j[u]);
-                }
-                else
-                {
-                    const uint32_t q = t + u;
-                    const uint32_t e = q + (q < n0 ? o0 : (q < n01 ? o1 : o2));
-                    j[u] = 0u;
-                    p[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                    if (q < total) { j[u] = index(e); p[u] = load(j[u]); }
-                }
-            }
-#pragma unroll
-            for (uint32_t u = 0; u < kW; u++)
-            {
-                if (t + u < total) { fn(j[u], p[u], t + u); }
-            }
-        }
-#endif
-    }
-
-    // preF(row, rf) may take a row's fluid candidates itself (returns true) instead of the stream;
-    // postF(row) follows the row's fluid part. row counts the rows of three cells in stencil order.
-    template <bool kFlat = false, typename OnF, typename OnB, typename OnR, typename NeedF, typename PreF, typename PostF>
-    __device__ __forceinline__ void forStencil(const Dev& d, const Frame& f, const Stencil& s, const CellBox& box, bool withF,
-                                               bool withB, bool withR, OnF onF, OnB onB, OnR onR, NeedF needF, PreF preF,
-                                               PostF postF)
-    {
-        const auto same = [](uint32_t e) { return e; };
-        uint32_t row = 0;
-        for (int cz = s.lo[2]; cz <= s.hi[2]; cz++)
-        {
-            for (int cy = s.lo[1]; cy <= s.hi[1]; cy++)
-            {
-                for (int cx = s.lo[0]; cx <= s.hi[0]; cx += 3, row++)
-                {
-                    const int nx = min(3, s.hi[0] - cx + 1);
-                    const uint32_t lin = s.cell(cx, cy, cz);
-                    const bool rowF = withF && needF(row);
-                    uint2 rf[3], rb[3], rr[3];
-#if TSP_TUNE_RANGE_LOADS
-                    // every lane loads the row's nine ranges (cells past the row's end load its
-                    // last cell) and then selects: no predicated loads into zeroed registers, so
-                    // nothing waits on loads still in flight from the previous row
-#pragma unroll
-                    for (int c = 0; c < 3; c++)
-                    {
-                        const bool in = c < nx;
-                        const uint32_t cc = lin + static_cast<uint32_t>(min(c, nx - 1));
-                        const uint2 vf = box.F ? box.F[box.at(cx, cy, cz) + static_cast<uint32_t>(min(c, nx - 1))] : d.cellF[cc];
-                        const uint2 vb = d.cellB[cc], vr = d.cellR[cc];
-                        rf[c] = (in && rowF) ? vf : make_uint2(0u, 0u);
-                        rb[c] = (in && withB) ? vb : make_uint2(0u, 0u);
-                        rr[c] = (in && withR && d.nR) ? vr : make_uint2(0u, 0u);
-                    }
-#else
-#pragma unroll
-                    for (int c = 0; c < 3; c++)
-                    {
-                        const bool in = c < nx;
-                        rf[c] = (in && rowF) ? (box.F ? box.F[box.at(cx, cy, cz) + c] : d.cellF[lin + c]) : make_uint2(0u, 0u);
-                        rb[c] = (in && withB) ? d.cellB[lin + c] : make_uint2(0u, 0u);
-                        rr[c] = (in && withR && d.nR) ? d.cellR[lin + c] : make_uint2(0u, 0u);
-                    }
-#endif
-                    if (rowF)
-                    {
-                        if (!preF(row, rf))
-                        {
-                            rowStream<kFlat>(rf, same, [&](uint32_t j) { return d.pos[j]; },
-                                             [&](uint32_t j, const float4& p, uint32_t q) { onF(j, p, row, q); });
-                        }
-                        postF(row);
-                    }
-                    if (withB)
-                    {
-                        rowStream<kFlat>(rb, same, [&](uint32_t j) { return d.bpos[j]; },
-                                         [&](uint32_t j, const float4& p, uint32_t) { onB(j, p); });
-                    }
-                    if (withR)
-                    {
-                        rowStream<kFlat>(rr, [&](uint32_t e) { return d.idxR[e]; }, [&](uint32_t j) { return d.rpos[j]; },
-                                         [&](uint32_t j, const float4& p, uint32_t) { onR(j, p); });
-                    }
-                }
-            }
-        }
-    }
-#else
-    // Cell form: one cell at a time, its candidates one at a time (no hit masks: every row is
-    // tested, row numbers are not passed)
-    template <bool kFlat = false, typename OnF, typename OnB, typename OnR, typename NeedF, typename PreF, typename PostF>
-    __device__ __forceinline__ void forStencil(const Dev& d, const Frame& f, const Stencil& s, const CellBox&, bool withF,
-                                               bool withB, bool withR, OnF onF, OnB onB, OnR onR, NeedF, PreF, PostF)
-    {
-        for (int cz = s.lo[2]; cz <= s.hi[2]; cz++)
-        {
-            for (int cy = s.lo[1]; cy <= s.hi[1]; cy++)
-            {
-                for (int cx = s.lo[0]; cx <= s.hi[0]; cx++)
-                {
-                    const uint32_t lin = s.cell(cx, cy, cz);
-                    if (withF)
-                    {
-                        const uint2 rf = d.cellF[lin];
-                        for (uint32_t j = rf.x; j < rf.y; j++) { onF(j, d.pos[j], kMaskRows, 0u); }
-                    }
-                    if (withB)
-                    {
-                        const uint2 rb = d.cellB[lin];
-                        for (uint32_t j = rb.x; j < rb.y; j++) { onB(j, d.bpos[j]); }
-                    }
-                    if (withR && d.nR)
-                    {
-                        const uint2 rr = d.cellR[lin];
-                        for (uint32_t q = rr.x; q < rr.y; q++)
-                        {
-                            const uint32_t j = d.idxR[q];
-                            onR(j, d.rpos[j]);
-                        }
-                    }
-                }
-            }
-        }
-    }
-#endif
-
-    __global__ void __launch_bounds__(kBlock) TSP_WAVES_ATTR(TSP_TUNE_QUERY_WAVES) kQueryCount(Dev d, uint32_t nSlices)
-    {
+        __shared__ uint32_t cntS[3][kBlock], minS[3][kBlock], maxS[3][kBlock];
+        __shared__ uint32_t openS[kBlock];       // kOpenF, kOpenB
+        __shared__ __align__(16) uint32_t keyS[kBlock];
+        __shared__ uint32_t rankS[kBlock];
+        __shared__ uint32_t unitsS[3][kBlock / kSlice], entriesS[3][kBlock / kSlice];
+        __shared__ uint32_t baseS[3];
+        __shared__ uint8_t whoS[kBlock];
         const uint32_t blk = xcdBlock();
-        const uint32_t i = blk * kBlock + threadIdx.x;
-        const uint32_t sc = d.blockScene[blk];
-        const Frame& f = d.frames[sc];
-        const float r2 = d.consts[sc].r2;
-        uint32_t cnt[3] = { 0, 0, 0 };
+        const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+        const uint32_t local = (wave / kShare) * 64u + lane, share = wave % kShare;
+        const uint32_t i = blk * kBlock + local;
+        const uint32_t sc = uniformLoad(&d.blockScene[blk]);
+        const Frame f = uniformLoad(&d.frames[sc]);
+        const float r2 = uniformLoad(&d.consts[sc]).r2;
+        if (threadIdx.x < kBlock)
+        {
+            for (int r = 0; r < 3; r++) { cntS[r][threadIdx.x] = 0u; minS[r][threadIdx.x] = kEmpty32; maxS[r][threadIdx.x] = 0u; }
+            openS[threadIdx.x] = 0u;
+            rankS[threadIdx.x] = 0u;
+        }
+        const bool active = keyAt(d, d.keyF, i) < f.emptyKey;
+        const float4 pi = d.pos[i];
+        __syncthreads();
+        const bool masks = f.reach == 1;
+        const Stencil s = stencilOf<kShare>(f, pi, active, share);
+        const bool quick = !__any(active && mayBeTiny(pi)) && max(d.nF, d.nB) < kNearMax;
+        uint32_t cnt[2] = { 0, 0 }, mn[2] = { kEmpty32, kEmpty32 }, mx[2] = { 0, 0 };
+        uint32_t open = 0;
         bool tiny = false;
-        uint32_t mn[3] = { kEmpty32, kEmpty32, kEmpty32 };
-        uint32_t mx[3] = { 0, 0, 0 };
-        Stencil s;
-        // rows the masks do not cover (all of them unless the row form walks a reach-1 stencil)
-        uint32_t uncovered = (1u << kMaskRows) - 1u, rowMask = 0;
-        if (i < d.nF && stencilOf(f, keyAt(d, d.keyF, i), s))
+        // the wave's rows, fluid then boundary; the next row's cells load while the current one is tested
+        RowCells next = s.cells(d.cellF, s.first, active);
+#pragma unroll 1
+        for (uint32_t row = s.first, rel = 0; row < s.last;)
         {
-            const float4 pi = d.pos[i];
-            const bool masks = TSP_TUNE_SEARCH_ROW == 1 && f.reach == 1;
-            if (masks) { uncovered = 0; }
-#if TSP_TUNE_SEARCH_FLAT
-            // a hit updates the counts, spans, tiny flag and masks through selects, without a branch
-            // (nearly every candidate step of a wave has a hit in some lane)
-            const auto hitOf = [&](const float4& pj, float& d2)
+            const RowSpan w = next.span();
+            const uint32_t nextRel = rel ^ 1u, nextRow = row + rel;
+            if (nextRow < s.last) { next = s.cells(nextRel ? d.cellB : d.cellF, nextRow, active); }
+            const float4* recs = rel ? d.bpos : d.pos;
+            uint32_t m = 0, n = 0, lo = kEmpty32, hi = 0;
+            for (uint32_t q0 = 0; q0 < w.n; q0 += 32u)
             {
-                d2 = dist2(pi.x - pj.x, pi.y - pj.y, pi.z - pj.z);
-                return d2 <= r2;
-            };
-            forStencil<TSP_TUNE_SEARCH_FLAT == 1>(d, f, s, CellBox{}, true, true, true,
-                [&](uint32_t j, const float4& pj, uint32_t row, uint32_t q)
+                m = (quick && w.n <= 32u) ? hitMaskNear(recs, w, pi.x, pi.y, pi.z, r2)
+                                          : hitMask(recs, w, q0, min(32u, w.n - q0), pi.x, pi.y, pi.z, r2, tiny);
+                if (m)
                 {
-                    float d2;
-                    const bool hit = hitOf(pj, d2);
-                    cnt[0] += hit ? 1u : 0u;
-                    mn[0] = min(mn[0], hit ? j : kEmpty32);
-                    mx[0] = max(mx[0], hit ? j : 0u);
-                    tiny = tiny || (hit && tinyDist2(d2));
-                    const uint32_t bit = hit ? 1u : 0u;
-                    rowMask |= q < 32u ? bit << q : 0u;
-                    uncovered |= (q >= 32u && row < kMaskRows) ? bit << row : 0u;
-                },
-                [&](uint32_t j, const float4& pj)
-                {
-                    float d2;
-                    const bool hit = hitOf(pj, d2);
-                    cnt[1] += hit ? 1u : 0u;
-                    mn[1] = min(mn[1], hit ? j : kEmpty32);
-                    mx[1] = max(mx[1], hit ? j : 0u);
-                    tiny = tiny || (hit && tinyDist2(d2));
-                },
-                [&](uint32_t j, const float4& pj)
-                {
-                    float d2;
-                    const bool hit = hitOf(pj, d2);
-                    cnt[2] += hit ? 1u : 0u;
-                    mn[2] = min(mn[2], hit ? j : kEmpty32);
-                    mx[2] = max(mx[2], hit ? j : 0u);
-                },
-#else
-            forStencil(d, f, s, CellBox{}, true, true, true,
-                [&](uint32_t j, const float4& pj, uint32_t row, uint32_t q)
-                {
-                    if (within(pi.x, pi.y, pi.z, pj, r2))
-                    {
-                        cnt[0]++; mn[0] = min(mn[0], j); mx[0] = max(mx[0], j);
-                        tiny = tiny || tinyDist2(dist2(pi.x - pj.x, pi.y - pj.y, pi.z - pj.z));
-                        if (q < 32u) { rowMask |= 1u << q; } else if (row < kMaskRows) { uncovered |= 1u << row; }
-                    }
-                },
-                [&](uint32_t j, const float4& pj)
-                {
-                    if (within(pi.x, pi.y, pi.z, pj, r2))
-                    {
-                        cnt[1]++; mn[1] = min(mn[1], j); mx[1] = max(mx[1], j);
-                        tiny = tiny || tinyDist2(dist2(pi.x - pj.x, pi.y - pj.y, pi.z - pj.z));
-                    }
-                },
-                [&](uint32_t j, const float4& pj)
-                {
-                    if (within(pi.x, pi.y, pi.z, pj, r2)) { cnt[2]++; mn[2] = min(mn[2], j); mx[2] = max(mx[2], j); }
-                },
-#endif
-                [&](uint32_t) { return true; },
-                [&](uint32_t, const uint2 (&)[3]) { return false; },
-                [&](uint32_t row)
-                {
-                    if (masks && row < kMaskRows) { d.ffMask[static_cast<size_t>(row) * d.nF + i] = rowMask; }
-                    rowMask = 0;
-                });
+                    n += static_cast<uint32_t>(__popc(m));
+                    lo = min(lo, w.at(q0 + static_cast<uint32_t>(__ffs(static_cast<int>(m))) - 1u));
+                    hi = max(hi, w.at(q0 + 31u - static_cast<uint32_t>(__clz(static_cast<int>(m)))));
+                }
+            }
+            if (masks)
+            {
+                if (w.n > 32u) { open |= 1u << (row + (rel ? kOpenB : kOpenF)); }
+                if (rel == 0u) { d.ffMask[static_cast<size_t>(row) * d.nF + i] = m; }
+                else if (w.n) { d.fbMask[static_cast<size_t>(row) * d.nF + i] = m; }
+            }
+            const uint32_t r = rel;
+            cnt[0] += r ? 0u : n; cnt[1] += r ? n : 0u;
+            mn[0] = r ? mn[0] : min(mn[0], lo); mn[1] = r ? min(mn[1], lo) : mn[1];
+            mx[0] = r ? mx[0] : max(mx[0], hi); mx[1] = r ? max(mx[1], hi) : mx[1];
+            rel = nextRel; row = nextRow;
         }
-        if (i < d.nF)
+        if (d.nR)
         {
-            d.ffMask[static_cast<size_t>(kMaskRows) * d.nF + i] = uncovered;
-            const bool wide = cnt[0] > 0 && mx[0] - mn[0] > 0xffffu;
-            d.cnt[REL_FF][i] = static_cast<uint16_t>(cnt[0]);
-            d.cnt[REL_FB][i] = static_cast<uint16_t>(cnt[1]);
-            d.cnt[REL_FR][i] = static_cast<uint16_t>(cnt[2]);
-            d.ffMin[i] = (cnt[0] > 0 ? mn[0] : 0u) | (wide ? kWideBit : 0u);
+#pragma unroll 1
+            for (uint32_t row = s.first; row < s.last; row++)
+            {
+                const RowSpan w = s.cells(d.cellR, row, active).span();
+                for (uint32_t q = 0; q < w.n; q++)
+                {
+                    const uint32_t j = d.idxR[w.at(q)];
+                    if (within(pi.x, pi.y, pi.z, d.rpos[j], r2))
+                    {
+                        atomicAdd(&cntS[2][local], 1u); atomicMin(&minS[2][local], j); atomicMax(&maxS[2][local], j);
+                    }
+                }
+            }
+        }
+        if (tiny) { atomicOr(&d.status->pairTiny, 1u); }
+        for (int r = 0; r < 2; r++)
+        {
+            if (cnt[r]) { atomicAdd(&cntS[r][local], cnt[r]); atomicMin(&minS[r][local], mn[r]); atomicMax(&maxS[r][local], mx[r]); }
+        }
+        if (open) { atomicOr(&openS[local], open); }
+        __syncthreads();
+        // thread t < 256: particle t of the block
+        const uint32_t t = threadIdx.x, me = blk * kBlock + t;
+        uint32_t c[3] = { 0, 0, 0 }, lo[3] = { kEmpty32, kEmpty32, kEmpty32 }, hi[3] = { 0, 0, 0 };
+        if (t < kBlock)
+        {
+            for (int r = 0; r < 3; r++) { c[r] = cntS[r][t]; lo[r] = minS[r][t]; hi[r] = maxS[r][t]; }
+            const bool wide = c[0] > 0 && hi[0] - lo[0] > 0xffffu;
+            d.ffMask[static_cast<size_t>(kMaskRows) * d.nF + me] = masks ? openS[t] : 0xffffffffu;
+            d.cnt[REL_FF][me] = static_cast<uint16_t>(c[0]);
+            d.cnt[REL_FB][me] = static_cast<uint16_t>(c[1]);
+            d.cnt[REL_FR][me] = static_cast<uint16_t>(c[2]);
+            d.ffMin[me] = (c[0] > 0 ? lo[0] : 0u) | (wide ? kWideBit : 0u);
             // u16 counts, as the reference's (neighbor_lists.h:43)
-            if (cnt[0] > 0xffffu || cnt[1] > 0xffffu || cnt[2] > 0xffffu) { atomicOr(&d.status->overflow, 2u); }
-            if (tiny) { atomicOr(&d.status->pairTiny, 1u); }
+            if (c[0] > 0xffffu || c[1] > 0xffffu || c[2] > 0xffffu) { atomicOr(&d.status->overflow, 2u); }
+            // the block's list positions, longest lists first (ties in particle order): the keys are
+            // made distinct by the thread index in their low byte
+            keyS[t] = (min(c[0], 255u) << 8) | (kBlock - 1u - t);
         }
-        // the particles whose FF list spans more than 0xffff join the list the wide fill walks
-        // (one counter update per wave)
+        __syncthreads();
+        rankDown<kShare>(keyS, rankS);
+        __syncthreads();
+        if (t < kBlock)
         {
-            const bool wideHere = i < d.nF && cnt[0] > 0 && mx[0] - mn[0] > 0xffffu;
-            const uint64_t ballot = __ballot(wideHere);
-            if (ballot != 0ull)
-            {
-                const uint32_t lane64 = threadIdx.x & 63u;
-                const int first = __ffsll(static_cast<unsigned long long>(ballot)) - 1;
-                uint32_t base = 0;
-                if (static_cast<int>(lane64) == first) { base = atomicAdd(&d.status->wideCount, static_cast<uint32_t>(__popcll(ballot))); }
-                base = static_cast<uint32_t>(__shfl(static_cast<int>(base), first, 64));
-                if (wideHere) { d.wideList[base + static_cast<uint32_t>(__popcll(ballot & ((1ull << lane64) - 1ull)))] = i; }
-            }
+            const uint32_t rank = rankS[t];
+            d.laneRank[me] = static_cast<uint8_t>(rank);
+            whoS[rank] = static_cast<uint8_t>(t);
+            for (int r = 0; r < 3; r++) { cntS[r][rank] = c[r]; minS[r][rank] = lo[r]; maxS[r][rank] = hi[r]; }
         }
-        // the block's list positions, longest lists first (ties in particle order): a thread's
-        // rank is the number of the block's sort keys above its own, the keys made distinct by
-        // the thread index in their low byte. The slice statistics below then run over positions.
+        __syncthreads();
+        SliceMeta m[3];
+        if (t < kBlock)
         {
-            __shared__ uint32_t sortKey[kBlock];
-            __shared__ uint32_t byPos[9][kBlock];
-            __shared__ uint8_t who[kBlock];
-            const uint32_t t = threadIdx.x;
-            const uint32_t own = (min(cnt[0], 255u) << 8) | (kBlock - 1u - t);
-            sortKey[t] = own;
-            __syncthreads();
-            uint32_t rank = 0;
-            for (uint32_t u = 0; u < kBlock; u += 4)
+            for (int r = 0; r < 3; r++) { c[r] = cntS[r][t]; lo[r] = minS[r][t]; hi[r] = maxS[r][t]; }
+            d.head[me] = make_uint2((c[0] & 0xffffu) | (c[1] << 16), (c[2] & 0xffffu) | (static_cast<uint32_t>(whoS[t]) << 16));
+            // per slice (a wave's 64 list positions): pitch, base (min index), format, entries
+            for (int r = 0; r < 3; r++)
             {
-                const uint4 v = *reinterpret_cast<const uint4*>(&sortKey[u]);
-                rank += (v.x > own ? 1u : 0u) + (v.y > own ? 1u : 0u) + (v.z > own ? 1u : 0u) + (v.w > own ? 1u : 0u);
-            }
-            if (i < d.nF) { d.laneRank[i] = static_cast<uint8_t>(rank); }
-            who[rank] = static_cast<uint8_t>(t);
-            for (int r = 0; r < 3; r++) { byPos[r][rank] = cnt[r]; byPos[3 + r][rank] = mn[r]; byPos[6 + r][rank] = mx[r]; }
-            __syncthreads();
-            for (int r = 0; r < 3; r++) { cnt[r] = byPos[r][t]; mn[r] = byPos[3 + r][t]; mx[r] = byPos[6 + r][t]; }
-            if (i < d.nF) { d.head[i] = make_uint2((cnt[0] & 0xffffu) | (cnt[1] << 16), (cnt[2] & 0xffffu) | (static_cast<uint32_t>(who[t]) << 16)); }
-        }
-        // per slice (list positions i of the block): pitch, base (min index), format, entries
-        const uint32_t slice = i / kSlice;
-        for (int r = 0; r < 3; r++)
-        {
-            const uint32_t pitch = sliceMax(cnt[r]);
-            const uint32_t smin = sliceMin(mn[r]);
-            const uint32_t smax = sliceMax(mx[r]);
-            const uint32_t sum = sliceSum(cnt[r]);
-            if ((threadIdx.x & (kSlice - 1)) == 0 && slice < nSlices)
-            {
-                SliceMeta m;
-                m.pitch = static_cast<uint16_t>(pitch);
+                const uint32_t pitch = sliceMax(c[r]);
+                const uint32_t smin = sliceMin(lo[r]);
+                const uint32_t smax = sliceMax(hi[r]);
+                const uint32_t sum = sliceSum(c[r]);
                 const bool delta = pitch == 0 || smax - smin <= 0xffffu;
-                m.format = delta ? kFmtDelta16 : kFmtAbs32;
-                m.base = (pitch == 0 || !delta) ? 0u : smin;
-                m.offset = pitch * kSlice * (delta ? 1u : 2u);
-                m.entries = sum;
-                d.meta[r][slice] = m;
+                m[r].pitch = static_cast<uint16_t>(pitch);
+                m[r].format = delta ? kFmtDelta16 : kFmtAbs32;
+                m[r].base = (pitch == 0 || !delta) ? 0u : smin;
+                m[r].offset = pitch * kSlice * (delta ? 1u : 2u);
+                m[r].entries = sum;
+                if (lane == 0u) { unitsS[r][wave] = m[r].offset; entriesS[r][wave] = sum; }
+            }
+        }
+        __syncthreads();
+        if (t < 6u)
+        {
+            // storage of the block's slices and their entries, counted in 64 bits (the host refuses a
+            // pool beyond 2^32 units and regrows one that is too small, before any list is written)
+            static_assert(offsetof(Status, entries) == offsetof(Status, poolUnits) + 3 * sizeof(uint64_t), "one row of counters");
+            const uint32_t r = t % 3u;
+            const uint32_t* v = t < 3u ? unitsS[r] : entriesS[r];
+            unsigned long long sum = 0;
+            for (uint32_t q = 0; q < kBlock / kSlice; q++) { sum += v[q]; }
+            const unsigned long long at = atomicAdd(reinterpret_cast<unsigned long long*>(d.status->poolUnits) + t, sum);
+            if (t < 3u) { baseS[r] = static_cast<uint32_t>(at); }
+        }
+        __syncthreads();
+        if (t < kBlock && lane == 0u)
+        {
+            for (int r = 0; r < 3; r++)
+            {
+                uint32_t o = baseS[r];
+                for (uint32_t q = 0; q < wave; q++) { o += unitsS[r][q]; }
+                m[r].offset = o;
+                d.meta[r][me / kSlice] = m[r];
             }
         }
     }
 
-    // storage units of every slice into a scan buffer of nSlices + 1 entries per relation, and
-    // their total in 64 bits (the u32 scan of the offsets wraps beyond 2^32 units; the host
-    // refuses such a pool before any list is written)
-    __global__ void __launch_bounds__(kBlock) kSliceUnits(Dev d, uint32_t nSlices, uint32_t* __restrict__ units)
-    {
-        __shared__ unsigned long long red[kBlock];
-        const uint32_t q = blockIdx.x * kBlock + threadIdx.x;
-        const uint32_t rel = blockIdx.y;
-        const uint32_t u = q < nSlices ? d.meta[rel][q].offset : 0u;
-        if (q <= nSlices) { units[rel * (nSlices + 1) + q] = u; }
-        red[threadIdx.x] = u;
-        __syncthreads();
-        for (uint32_t o = kBlock / 2; o > 0; o >>= 1)
-        {
-            if (threadIdx.x < o) { red[threadIdx.x] += red[threadIdx.x + o]; }
-            __syncthreads();
-        }
-        if (threadIdx.x == 0 && red[0]) { atomicAdd(reinterpret_cast<unsigned long long*>(&d.status->poolUnits[rel]), red[0]); }
-    }
+    // The fill pass: the lists of a block from the count pass's hit masks (rows they do not cover are
+    // tested again), and the block's FF halo: the distinct FF neighbors of its particles, ascending.
+    // With a halo (at most kHaloMax particles) the FF entries are slots of it, so the solver kernels
+    // stage the neighbor records in LDS once per block; otherwise they are particle indices.
+    //
+    // The halo is a bitmap in LDS over pages of 256 particles, found through a small hash table: a
+    // block's neighbors are runs of the sorted particles in at most about 40 pages. Each run's hit mask
+    // goes into the bitmap whole (two words at most). Ranking the pages orders it, and the bitmap is
+    // then spread into a table of halo slots, one per particle of the pages in page order, so that an
+    // entry is one LDS read at its run's base plus its candidate number. The entries are staged in LDS
+    // by list position and leave as whole slice rows.
+    //
+    // FF lists that span more than 0xffff indices keep the DictDelta16x2 order of the reference's
+    // per-particle dict chunks (neighbor_lists.cpp:838-858): the neighbors within 0xffff of the
+    // smallest form the low group, the rest the high group, which is stored from the back when it fits
+    // 0xffff itself, else the candidate order stays; a list of more than kDictMax entries is no dict
+    // (candidate order).
+    // One kernel in place of the fill, the wide lists' fill and a halo kernel that read all entries back
+    // twice (hash set and sort in LDS): 1M cube drop 352 to 205 us, 8M dam break 2,551 to 1,439 us, 64k
+    // dam break 80 to 37 us, 4k 78 to 36 us. It is bound by its chain of phases (two blocks per CU for
+    // the 66 KB of LDS) and the divergence of the loops over hits.
+    constexpr uint32_t kStage = 40;          // FF entries per list staged in LDS; the rest are stored directly
+    constexpr uint32_t kPages = 64;          // pages of a halo
+    constexpr uint32_t kPageSlots = 128;     // slots of their hash table
+    constexpr uint32_t kPageBits = 8;
+    constexpr uint32_t kPageWords = (1u << kPageBits) / 32u;
 
-    // writes the scanned offsets back, sums the entries and checks the pool capacity
-    __global__ void __launch_bounds__(kBlock) kSliceApply(Dev d, uint32_t nSlices, const uint32_t* __restrict__ offs)
-    {
-        __shared__ uint32_t red[kBlock];
-        const uint32_t q = blockIdx.x * kBlock + threadIdx.x;
-        const uint32_t rel = blockIdx.y;
-        uint32_t e = 0;
-        if (q < nSlices)
-        {
-            SliceMeta& m = d.meta[rel][q];
-            e = m.entries;
-            m.offset = offs[rel * (nSlices + 1) + q];
-        }
-        red[threadIdx.x] = e;
-        __syncthreads();
-        for (uint32_t o = kBlock / 2; o > 0; o >>= 1)
-        {
-            if (threadIdx.x < o) { red[threadIdx.x] += red[threadIdx.x + o]; }
-            __syncthreads();
-        }
-        if (threadIdx.x == 0)
-        {
-            atomicAdd(reinterpret_cast<unsigned long long*>(&d.status->entries[rel]), static_cast<unsigned long long>(red[0]));
-        }
-        if (q == 0)
-        {
-            const uint64_t total = d.status->poolUnits[rel];   // summed in 64 bits by kSliceUnits
-            if (total > d.poolCap[rel]) { atomicOr(&d.status->overflow, 1u); }
-        }
-    }
+    __device__ __forceinline__ uint32_t pageHash(uint32_t page) { return (page * 2654435761u) >> 25; }
+    static_assert(kPageSlots == 1u << 7, "pageHash gives seven bits");
 
-    constexpr uint32_t kStage = 40; // FF entries per thread staged in LDS by the fill (u16 slices)
-
-    __global__ void __launch_bounds__(kBlock) TSP_WAVES_ATTR(TSP_TUNE_QUERY_WAVES) kQueryFill(Dev d)
+    __global__ void __launch_bounds__(kQueryThreads) __attribute__((amdgpu_waves_per_eu(6))) kQueryFill(Dev d)
     {
         if (stopped(d)) { return; }
         __shared__ uint16_t stage[kStage][kBlock];
+        __shared__ __align__(16) uint16_t slotOf[kPages << kPageBits];   // halo entry of each particle of the pages
+        __shared__ uint32_t bits[kPageSlots * kPageWords];
+        __shared__ __align__(16) uint32_t pageKey[kPageSlots];     // page number + 1, 0: free
+        __shared__ uint32_t pageRank[kPageSlots], pageBase[kPages];
+        __shared__ uint32_t partF[kQueryShare][kBlock], partB[kQueryShare][kBlock];
+        __shared__ uint32_t base2S[kBlock], maxRefS[kBlock];
+        __shared__ uint32_t failS, pagesS, countS;
         const uint32_t blk = xcdBlock();
-        const uint32_t t = threadIdx.x;
-        const uint32_t i = blk * kBlock + t;
-        const uint32_t sc = d.blockScene[blk];
-        const Frame& f = d.frames[sc];
-        const float r2 = d.consts[sc].r2;
-        // this particle's list position (its lane and slice), from the count pass; col is its
-        // column of the staging array
-        const uint32_t pos = i < d.nF ? sellPos(d, i) : i;
-        const uint32_t col = pos & (kBlock - 1u);
-        const uint32_t lane = pos & (kSlice - 1), slice = pos / kSlice;
-        Stencil s;
-        const bool active = i < d.nF && stencilOf(f, keyAt(d, d.keyF, i), s);
-        __shared__ uint2 boxF[kBoxCells > 0 ? kBoxCells : 1];
-        __shared__ int boxRed[6];
-        const CellBox box = stageCellBox(d, f, s, active, boxF, boxRed);
-        const uint32_t cF = i < d.nF ? d.cnt[REL_FF][i] : 0u;
-        const uint32_t fMin = i < d.nF ? d.ffMin[i] : 0u;
-        const bool wide = (fMin & kWideBit) != 0u;
-        SliceMeta mF{}, mB{}, mR{};
-        if (i < d.nF) { mF = d.meta[REL_FF][slice]; mB = d.meta[REL_FB][slice]; mR = d.meta[REL_FR][slice]; }
-        // the FF entries stage in LDS as u16 offsets from mF.base: the slice base in a u16 slice,
-        // the particle's smallest neighbor in a u32 slice, whose stores ignore the base (the list
-        // spans at most 0xffff unless wide)
-        if (mF.format != kFmtDelta16) { mF.base = fMin; }
-        const bool staged = !wide;
-        if (active)
-        {
-            const float4 pi = d.pos[i];
-            uint32_t kF = 0, kB = 0, kR = 0;
-            const uint32_t uncovered = d.ffMask[static_cast<size_t>(kMaskRows) * d.nF + i];
-            // the row's hit mask, read before its cell ranges (and the next row's a row ahead): a
-            // covered row without hits loads no range; relations without entries are not walked
-            uint32_t rowMask = 0, nextMask = d.ffMask[i];
-            const auto ffHit = [&](uint32_t j)
-            {
-                if (staged && kF < kStage) { stage[kF][col] = static_cast<uint16_t>(j - mF.base); }
-                else { sellWrite(d.pool[REL_FF], mF, lane, kF, j); }
-                kF++;
-            };
-            forStencil(d, f, s, box, !wide, d.cnt[REL_FB][i] != 0, d.cnt[REL_FR][i] != 0,
-                [&](uint32_t j, const float4& pj, uint32_t, uint32_t)
-                {
-                    if (within(pi.x, pi.y, pi.z, pj, r2)) { ffHit(j); }
-                },
-                [&](uint32_t j, const float4& pj)
-                {
-                    if (within(pi.x, pi.y, pi.z, pj, r2)) { sellWrite(d.pool[REL_FB], mB, lane, kB++, j); }
-                },
-                [&](uint32_t j, const float4& pj)
-                {
-                    if (within(pi.x, pi.y, pi.z, pj, r2)) { sellWrite(d.pool[REL_FR], mR, lane, kR++, j); }
-                },
-                [&](uint32_t row)
-                {
-                    const uint32_t cur = nextMask;
-#if TSP_TUNE_RANGE_LOADS
-                    // unconditional (the last row's word again past the rows): the load stays in flight
-                    nextMask = d.ffMask[static_cast<size_t>(min(row + 1u, kMaskRows - 1u)) * d.nF + i];
-#else
-                    if (row + 1u < kMaskRows) { nextMask = d.ffMask[static_cast<size_t>(row + 1u) * d.nF + i]; }
-#endif
-                    if (row >= kMaskRows || ((uncovered >> row) & 1u)) { return true; }
-                    rowMask = cur;
-                    return rowMask != 0u;
-                },
-                // a row the count pass covered: its hits, in stream order, without loading a position
-                [&](uint32_t row, const uint2 (&rf)[3])
-                {
-                    if (row >= kMaskRows || ((uncovered >> row) & 1u)) { return false; }
-                    uint32_t m = rowMask;
-                    while (m)
-                    {
-                        const uint32_t q = static_cast<uint32_t>(__ffs(static_cast<int>(m))) - 1u;
-                        m &= m - 1u;
-                        ffHit(rowCandidate(rf, q));
-                    }
-                    return true;
-                },
-                [&](uint32_t) {});
-            // (the FF lists of wide particles: kQueryFillWide)
-        }
-        // the staged FF entries leave as whole slice rows: column k of the slice's lanes per store
-        // (thread t writes list position t of the block: the staged entries of the particle there,
-        // whose count and base it reads back; a particle outside the frame has no FF entries)
-        __syncthreads();
-        const uint32_t p = blk * kBlock + t;
-        const uint32_t w = particleAt(d, p);
-        const uint32_t wMin = d.ffMin[w];
-        const uint32_t own = (wMin & kWideBit) ? 0u : min(static_cast<uint32_t>(d.cnt[REL_FF][w]), kStage);
-        SliceMeta mw{};
-        if (own) { mw = d.meta[REL_FF][p / kSlice]; }
-        const uint32_t base = mw.format == kFmtDelta16 ? mw.base : wMin;
-        const uint32_t lw = p & (kSlice - 1);
-        const uint32_t rows = sliceMax(own);
-        if (mw.format == kFmtDelta16)
-        {
-            uint16_t* row = d.pool[REL_FF] + mw.offset + lw;
-            for (uint32_t k = 0; k < rows; k++)
-            {
-                if (k < own) { row[k * kSlice] = stage[k][t]; }
-            }
-        }
-        else
-        {
-            uint32_t* row = reinterpret_cast<uint32_t*>(d.pool[REL_FF] + mw.offset) + lw;
-            for (uint32_t k = 0; k < rows; k++)
-            {
-                if (k < own) { row[k * kSlice] = base + stage[k][t]; }
-            }
-        }
-    }
-
-    // The FF lists of the particles whose list spans more than 0xffff (the count pass lists them):
-    // the DictDelta16x2 split of a per-particle dict (neighbor_lists.cpp:838-858) -- the neighbors
-    // within 0xffff of the smallest form the low group, the rest the high group, which is stored
-    // from the back when it fits 0xffff itself, else the candidate order stays; a list of more than
-    // kDictMax entries is no dict (candidate order). One thread per listed particle walks its
-    // stencil with the count pass's hit masks, twice for a dict: the high group's smallest and the
-    // largest neighbor, then the entries. Such a particle's slice stores u32 entries.
-    __global__ void __launch_bounds__(kBlock) TSP_WAVES_ATTR(TSP_TUNE_QUERY_WAVES) kQueryFillWide(Dev d)
-    {
-        if (stopped(d)) { return; }
-        const uint32_t q = blockIdx.x * kBlock + threadIdx.x;
-        if (q >= d.status->wideCount) { return; }
-        const uint32_t i = d.wideList[q];
-        const uint32_t sc = d.blockScene[i / kBlock];
-        const Frame& f = d.frames[sc];
-        const float r2 = d.consts[sc].r2;
-        Stencil s;
-        if (!stencilOf(f, keyAt(d, d.keyF, i), s)) { return; }
-        const uint32_t pos = sellPos(d, i);
-        const uint32_t lane = pos & (kSlice - 1);
-        const SliceMeta mF = d.meta[REL_FF][pos / kSlice];
+        const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
+        const uint32_t local = (wave / kQueryShare) * 64u + lane, share = wave % kQueryShare;
+        const uint32_t i = blk * kBlock + local;
+        const uint32_t sc = uniformLoad(&d.blockScene[blk]);
+        const Frame f = uniformLoad(&d.frames[sc]);
+        const float r2 = uniformLoad(&d.consts[sc]).r2;
+        for (uint32_t q = t; q < kPageSlots * kPageWords; q += kQueryThreads) { bits[q] = 0u; }
+        if (t < kPageSlots) { pageKey[t] = 0u; pageRank[t] = 0u; }
+        if (t < kPages) { pageBase[t] = 0u; }
+        if (t < kBlock) { base2S[t] = kEmpty32; maxRefS[t] = 0u; }
+        if (t == 0) { failS = 0u; pagesS = 0u; }
+        const bool active = keyAt(d, d.keyF, i) < f.emptyKey;
         const float4 pi = d.pos[i];
-        const uint32_t n = d.cnt[REL_FF][i];
-        const uint32_t minRef = d.ffMin[i] & ~kWideBit;
-        const uint32_t uncovered = d.ffMask[static_cast<size_t>(kMaskRows) * d.nF + i];
-        const auto walk = [&](auto&& onHit)
+        const uint32_t nF = active ? d.cnt[REL_FF][i] : 0u, nB = active ? d.cnt[REL_FB][i] : 0u, nR = active ? d.cnt[REL_FR][i] : 0u;
+        const uint32_t fMin = d.ffMin[i];
+        const uint32_t open = d.ffMask[static_cast<size_t>(kMaskRows) * d.nF + i];
+        const uint32_t pos = blk * kBlock + d.laneRank[i];
+        const uint32_t col = pos & (kBlock - 1u), lw = pos & (kSlice - 1u);
+        const bool masks = f.reach == 1;
+        const Stencil s = stencilOf<kQueryShare>(f, pi, active, share);
+        bool ignored = false;
+        // fn(row span, first candidate, hits) for up to 32 candidates at a time of the wave's rows, in list
+        // order. Three rows inside the frame load their cells and masks at once.
+        const auto each = [&](int rel, bool need, auto&& fn)
         {
-            uint32_t rowMask = 0, nextMask = d.ffMask[i];
-            forStencil(d, f, s, CellBox{}, true, false, false,
-                [&](uint32_t j, const float4& pj, uint32_t, uint32_t)
+            const uint2* table = rel == 0 ? d.cellF : d.cellB;
+            const uint32_t* mask = rel == 0 ? d.ffMask : d.fbMask;
+            const uint32_t opens = masks ? open >> (rel == 0 ? kOpenF : kOpenB) : 0xffffffffu;
+            const auto take = [&](const RowSpan& w, uint32_t row, uint32_t m)
+            {
+                const bool covered = masks && ((opens >> row) & 1u) == 0u;
+                for (uint32_t q0 = 0; q0 < w.n; q0 += 32u)
                 {
-                    if (within(pi.x, pi.y, pi.z, pj, r2)) { onHit(j); }
-                },
-                [&](uint32_t, const float4&) {},
-                [&](uint32_t, const float4&) {},
-                [&](uint32_t row)
-                {
-                    const uint32_t cur = nextMask;
-                    if (row + 1u < kMaskRows) { nextMask = d.ffMask[static_cast<size_t>(row + 1u) * d.nF + i]; }
-                    if (row >= kMaskRows || ((uncovered >> row) & 1u)) { return true; }
-                    rowMask = cur;
-                    return rowMask != 0u;
-                },
-                [&](uint32_t row, const uint2 (&rf)[3])
-                {
-                    if (row >= kMaskRows || ((uncovered >> row) & 1u)) { return false; }
-                    uint32_t m = rowMask;
-                    while (m)
-                    {
-                        const uint32_t b = static_cast<uint32_t>(__ffs(static_cast<int>(m))) - 1u;
-                        m &= m - 1u;
-                        onHit(rowCandidate(rf, b));
-                    }
-                    return true;
-                },
-                [&](uint32_t) {});
-        };
-        const bool dict = n <= kDictMax;
-        uint32_t base2 = kEmpty32, maxRef = 0;
-        if (dict)
-        {
-            walk([&](uint32_t j)
-            {
-                maxRef = max(maxRef, j);
-                if (j - minRef > 0xffffu) { base2 = min(base2, j); }
-            });
-        }
-        const bool split = dict && maxRef - base2 <= 0xffffu;
-        uint32_t kLow = 0, kHigh = n;
-        walk([&](uint32_t j)
-        {
-            if (!split || j - minRef <= 0xffffu) { sellWrite(d.pool[REL_FF], mF, lane, kLow++, j); }
-            else { sellWrite(d.pool[REL_FF], mF, lane, --kHigh, j); }
-        });
-    }
-
-    // ----------------------------------------------------------------------------------------
-    // FF halo of each 256-particle block: the distinct neighbors of the block's particles,
-    // ascending, and the block's FF entries rewritten as slots of that list. One block per
-    // particle block; a halo larger than kHaloMax leaves the block's entries as particle indices.
-
-    constexpr uint32_t kHashSlots = 2048;   // > kHaloMax + kBlock: probes always end
-
-    // The halo slots of a u32 slice are stored as u16 in the first half of
-    // its storage (entry k of lane l at u16 position k * kSlice + l, which the lanes reach only
-    // after reading the u32 entries there), and the slice turns u16 once its entries are written.
-    __device__ __forceinline__ void slotsToU16(const Dev& d, uint32_t i, const SliceMeta& m)
-    {
-        if (i < d.nF && (i & (kSlice - 1)) == 0 && m.format != kFmtDelta16)
-        {
-            SliceMeta& w = d.meta[REL_FF][i / kSlice];
-            w.format = kFmtDelta16;
-            w.base = 0;
-        }
-    }
-    constexpr uint32_t kSortKeys = kHaloMax <= 1024 ? 1024 : 2048;    // power of two >= kHaloMax
-
-    __device__ __forceinline__ uint32_t haloHash(uint32_t j) { return (j * 2654435761u) >> (32 - 11); }
-
-    // slot of j in the hash table (j must be present)
-    __device__ __forceinline__ uint32_t haloFind(const uint32_t* table, uint32_t j)
-    {
-        uint32_t h = haloHash(j);
-        for (uint32_t probe = 0; probe < kHashSlots && table[h] != j; probe++) { h = (h + 1) & (kHashSlots - 1); }
-        return h;
-    }
-
-#if TSP_TUNE_HALO_PAGES
-#error "TSP_TUNE_HALO_PAGES=1 stopped responding in a timing run after the lists were ordered by length within each block; it stays disabled until the cause is found"
-    // The block's FF neighbors by pages of 4096 indices: one LDS bitmap per page (at most
-    // kHaloPages pages, taken in order of arrival), the pages ranked by their number, so the set
-    // bits in page order are the halo in ascending order and an entry's slot is the count of set
-    // bits before it. No hash table and no sort; a block whose neighbors span more pages keeps
-    // particle indices.
-    constexpr uint32_t kPageBits = 12;
-    constexpr uint32_t kPageWords = (1u << kPageBits) / 32;
-    constexpr uint32_t kHaloPages = 32;
-    static_assert(kHaloPages <= kBlock && (kHaloPages * kPageWords) % kBlock == 0, "page table sizes");
-
-    // the slot of page pg in the table (pages arrive in any order; slots fill from 0), or
-    // kHaloPages when the table is full
-    __device__ __forceinline__ uint32_t haloPageSlot(uint32_t* pageId, uint32_t pg)
-    {
-        for (uint32_t s = 0; s < kHaloPages; s++)
-        {
-            uint32_t v = *static_cast<volatile uint32_t*>(&pageId[s]);
-            if (v == kEmpty32) { v = atomicCAS(&pageId[s], kEmpty32, pg); if (v == kEmpty32) { return s; } }
-            if (v == pg) { return s; }
-        }
-        return kHaloPages;
-    }
-
-    __global__ void __launch_bounds__(kBlock) TSP_WAVES_ATTR(TSP_TUNE_QUERY_WAVES) kHaloBuild(Dev d)
-    {
-        if (stopped(d)) { return; }
-        __shared__ uint32_t bits[kHaloPages * kPageWords];
-        __shared__ uint16_t wrank[kHaloPages * kPageWords];
-        __shared__ uint32_t pageId[kHaloPages], slotOfRank[kHaloPages];
-        __shared__ uint32_t full;
-        __shared__ uint32_t waveSum[kBlock / 64];
-        const uint32_t blk = blockIdx.x;
-        const uint32_t t = threadIdx.x;
-        const uint32_t i = blk * kBlock + t;
-        for (uint32_t q = t; q < kHaloPages * kPageWords; q += kBlock) { bits[q] = 0u; }
-        if (t < kHaloPages) { pageId[t] = kEmpty32; }
-        if (t == 0) { full = 0u; }
-        __syncthreads();
-        uint32_t n = 0;
-        SliceMeta m{};
-        if (i < d.nF)
-        {
-            // thread t walks the lists at list position i
-            n = d.cnt[REL_FF][particleAt(d, i)];
-            m = d.meta[REL_FF][i / kSlice];
-        }
-        const uint32_t lane = i & (kSlice - 1);
-        // the entries into their pages' bitmaps (consecutive entries mostly share a page)
-        uint32_t lastPage = kEmpty32, lastSlot = 0;
-        for (uint32_t k = 0; k < n; k++)
-        {
-            const uint32_t j = sellRead(d.pool[REL_FF], m, lane, k);
-            const uint32_t pg = j >> kPageBits;
-            if (pg != lastPage)
-            {
-                lastSlot = haloPageSlot(pageId, pg);
-                if (lastSlot == kHaloPages) { atomicOr(&full, 1u); break; }
-                lastPage = pg;
-            }
-            atomicOr(&bits[lastSlot * kPageWords + ((j >> 5) & (kPageWords - 1u))], 1u << (j & 31u));
-        }
-        __syncthreads();
-        if (full)
-        {
-            if (t == 0) { d.haloInfo[blk].count = kNoHalo; }
-            return;
-        }
-        // the pages in ascending order: slotOfRank[r] is the slot of the r-th smallest page
-        if (t < kHaloPages && pageId[t] != kEmpty32)
-        {
-            const uint32_t pg = pageId[t];
-            uint32_t r = 0;
-            for (uint32_t s = 0; s < kHaloPages; s++) { r += (pageId[s] != kEmpty32 && pageId[s] < pg) ? 1u : 0u; }
-            slotOfRank[r] = t;
-        }
-        __syncthreads();
-        uint32_t np = 0;
-        for (uint32_t s = 0; s < kHaloPages; s++) { np += pageId[s] != kEmpty32 ? 1u : 0u; }
-        // set bits before each word in page order: thread t takes kPer consecutive words of that order
-        constexpr uint32_t kPer = kHaloPages * kPageWords / kBlock;
-        uint32_t pc[kPer], sum = 0;
-#pragma unroll
-        for (uint32_t u = 0; u < kPer; u++)
-        {
-            const uint32_t v = kPer * t + u, r = v / kPageWords;
-            pc[u] = r < np ? static_cast<uint32_t>(__popc(bits[slotOfRank[r] * kPageWords + v % kPageWords])) : 0u;
-            sum += pc[u];
-        }
-        uint32_t incl = sum;
-        for (int o = 1; o < 64; o <<= 1)
-        {
-            const uint32_t v = static_cast<uint32_t>(__shfl_up(static_cast<int>(incl), o, 64));
-            if ((t & 63u) >= static_cast<uint32_t>(o)) { incl += v; }
-        }
-        if ((t & 63u) == 63u) { waveSum[t >> 6] = incl; }
-        __syncthreads();
-        uint32_t count = 0, before = 0;
-        for (uint32_t w = 0; w < kBlock / 64; w++) { before += w < (t >> 6) ? waveSum[w] : 0u; count += waveSum[w]; }
-        if (count > kHaloMax)
-        {
-            if (t == 0) { d.haloInfo[blk].count = kNoHalo; }
-            return;
-        }
-        uint32_t* out = d.haloIdx + static_cast<size_t>(blk) * kHaloMax;
-        uint32_t r = before + incl - sum;
-#pragma unroll
-        for (uint32_t u = 0; u < kPer; u++)
-        {
-            const uint32_t v = kPer * t + u, pr = v / kPageWords;
-            if (pr >= np) { break; }
-            const uint32_t slot = slotOfRank[pr], w = v % kPageWords;
-            wrank[slot * kPageWords + w] = static_cast<uint16_t>(r);
-            uint32_t b = bits[slot * kPageWords + w];
-            const uint32_t base = (pageId[slot] << kPageBits) + 32u * w;
-            while (b)
-            {
-                out[r++] = base + static_cast<uint32_t>(__ffs(static_cast<int>(b))) - 1u;
-                b &= b - 1u;
-            }
-        }
-        if (t == 0) { d.haloInfo[blk].count = count; }
-        __syncthreads();
-        // entries become the byte offsets of their slots, in their storage format
-        lastPage = kEmpty32;
-        for (uint32_t k = 0; k < n; k++)
-        {
-            const uint32_t j = sellRead(d.pool[REL_FF], m, lane, k);
-            const uint32_t pg = j >> kPageBits;
-            if (pg != lastPage)
-            {
-                lastSlot = 0;
-                while (pageId[lastSlot] != pg) { lastSlot++; }
-                lastPage = pg;
-            }
-            const uint32_t q = lastSlot * kPageWords + ((j >> 5) & (kPageWords - 1u));
-            const uint32_t slot = (wrank[q] + static_cast<uint32_t>(__popc(bits[q] & ((1u << (j & 31u)) - 1u)))) << kSlotShift;
-            d.pool[REL_FF][m.offset + k * kSlice + lane] = static_cast<uint16_t>(slot);
-        }
-        slotsToU16(d, i, m);
-    }
-#else
-    __global__ void __launch_bounds__(kBlock) TSP_WAVES_ATTR(TSP_TUNE_QUERY_WAVES) kHaloBuild(Dev d)
-    {
-        if (stopped(d)) { return; }
-        __shared__ uint32_t table[kHashSlots];
-        __shared__ uint16_t rank[kHashSlots];
-        __shared__ uint32_t keys[kSortKeys];
-        __shared__ uint32_t unique, filled, bmin, notDelta, outOfSpan;
-        __shared__ uint32_t waveSum[kBlock / 64];
-        const uint32_t blk = blockIdx.x;
-        const uint32_t t = threadIdx.x;
-        const uint32_t i = blk * kBlock + t;
-        if (t == 0) { unique = 0; filled = 0; bmin = kEmpty32; notDelta = 0; outOfSpan = 0; d.haloInfo[blk].ulps = 1u; }
-        __syncthreads();
-        uint32_t n = 0;
-        SliceMeta m{};
-        if (i < d.nF)
-        {
-            // thread t walks the lists at list position i
-            n = d.cnt[REL_FF][particleAt(d, i)];
-            m = d.meta[REL_FF][i / kSlice];
-        }
-        const uint32_t lane = i & (kSlice - 1);
-        uint32_t* out = d.haloIdx + static_cast<size_t>(blk) * kHaloMax;
-        // When every FF entry of the block lies within 0xffff of the block's smallest (u16 delta
-        // slices whose bases are close), the halo is a bitmap over that window: the set bits in
-        // ascending order are the halo, and an entry's slot is the count of set bits below it.
-        if (n > 0)
-        {
-            if (m.format != kFmtDelta16) { atomicOr(&notDelta, 1u); }
-            else { atomicMin(&bmin, m.base); }
-        }
-        __syncthreads();
-        if (!notDelta)
-        {
-            constexpr uint32_t kWords = kHashSlots;   // 2048 x 32 bits: a window of 0x10000 indices
-            for (uint32_t q = t; q < kWords; q += kBlock) { table[q] = 0u; }
-            __syncthreads();
-            const uint32_t b0 = bmin;
-            for (uint32_t k = 0; k < n; k++)
-            {
-                const uint32_t off = sellRead(d.pool[REL_FF], m, lane, k) - b0;
-                if (off > 0xffffu) { atomicOr(&outOfSpan, 1u); break; }
-                atomicOr(&table[off >> 5], 1u << (off & 31u));
-            }
-            __syncthreads();
-            if (!outOfSpan)
-            {
-                // ranks of the words (eight consecutive words per thread), as u16 in rank[]
-                constexpr uint32_t kPer = kWords / kBlock;
-                uint32_t pc[kPer], sum = 0;
-#pragma unroll
-                for (uint32_t u = 0; u < kPer; u++) { pc[u] = static_cast<uint32_t>(__popc(table[kPer * t + u])); sum += pc[u]; }
-                uint32_t incl = sum;
-                for (int o = 1; o < 64; o <<= 1)
-                {
-                    const uint32_t v = static_cast<uint32_t>(__shfl_up(static_cast<int>(incl), o, 64));
-                    if ((t & 63u) >= static_cast<uint32_t>(o)) { incl += v; }
+                    if (!covered) { m = hitMask(rel == 0 ? d.pos : d.bpos, w, q0, min(32u, w.n - q0), pi.x, pi.y, pi.z, r2, ignored); }
+                    if (m) { fn(w, q0, m); }
                 }
-                if ((t & 63u) == 63u) { waveSum[t >> 6] = incl; }
-                __syncthreads();
-                uint32_t count = 0, before = 0;
-                for (uint32_t w = 0; w < kBlock / 64; w++) { before += w < (t >> 6) ? waveSum[w] : 0u; count += waveSum[w]; }
-                if (count > kHaloMax)
-                {
-                    if (t == 0) { d.haloInfo[blk].count = kNoHalo; }
-                    return;
-                }
-                uint32_t r = before + incl - sum;
+            };
+            if (s.near)
+            {
+                RowCells c[kMaskRows / kQueryShare];
+                uint32_t m[kMaskRows / kQueryShare];
 #pragma unroll
-                for (uint32_t u = 0; u < kPer; u++)
+                for (uint32_t u = 0; u < kMaskRows / kQueryShare; u++)
                 {
-                    const uint32_t w = kPer * t + u;
-                    rank[w] = static_cast<uint16_t>(r);
-                    uint32_t bits = table[w];
-                    while (bits)
-                    {
-                        const uint32_t b = static_cast<uint32_t>(__ffs(static_cast<int>(bits))) - 1u;
-                        out[r++] = b0 + 32u * w + b;
-                        bits &= bits - 1u;
-                    }
+                    c[u] = s.cells(table, s.first + u, need);
+                    m[u] = mask[static_cast<size_t>(s.first + u) * d.nF + i];
                 }
-                if (t == 0) { d.haloInfo[blk].count = count; }
-                __syncthreads();
-                for (uint32_t k = 0; k < n; k++)
-                {
-                    const uint32_t off = sellRead(d.pool[REL_FF], m, lane, k) - b0;
-                    const uint32_t w = off >> 5;
-                    const uint32_t slot = rank[w] + static_cast<uint32_t>(__popc(table[w] & ((1u << (off & 31u)) - 1u)));
-                    d.pool[REL_FF][m.offset + k * kSlice + lane] = static_cast<uint16_t>(slot << kSlotShift);
-                }
+#pragma unroll
+                for (uint32_t u = 0; u < kMaskRows / kQueryShare; u++) { take(c[u].span(), s.first + u, m[u]); }
                 return;
             }
-        }
-        // otherwise a hash set of the block's entries, sorted
-        for (uint32_t q = t; q < kHashSlots; q += kBlock) { table[q] = kEmpty32; }
-        __syncthreads();
-        // insert: open addressing, a relaxed LDS read before the compare-and-swap (most entries
-        // are already present); a thread stops once the halo is known to be too large, so at most
-        // kHaloMax + kBlock values enter the kHashSlots slots and a probe always ends
-        for (uint32_t k = 0; k < n; k++)
-        {
-            if (__hip_atomic_load(&unique, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) > kHaloMax) { break; }
-            const uint32_t j = sellRead(d.pool[REL_FF], m, lane, k);
-            uint32_t h = haloHash(j);
-            for (uint32_t probe = 0; probe < kHashSlots; probe++)
+#pragma unroll 1
+            for (uint32_t row = s.first; row < s.last; row++)
             {
-                uint32_t v = __hip_atomic_load(&table[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                if (v == kEmpty32)
-                {
-                    v = atomicCAS(&table[h], kEmpty32, j);
-                    if (v == kEmpty32) { atomicAdd(&unique, 1u); break; }
-                }
-                if (v == j) { break; }
-                h = (h + 1) & (kHashSlots - 1);
+                take(s.cells(table, row, need).span(), row, masks ? mask[static_cast<size_t>(row) * d.nF + i] : 0u);
             }
-        }
-        __syncthreads();
-        static_assert(kHaloMax + kBlock < kHashSlots && kHaloMax <= kSortKeys, "halo table sizes");
-        const uint32_t count = unique;
-        if (count > kHaloMax)
+        };
+        // the hits of the two runs of a row: fn(first particle of the run's hits, hits from it, its candidate)
+        const auto runs = [&](const RowSpan& w, uint32_t q0, uint32_t m, auto&& fn)
         {
-            if (t == 0) { d.haloInfo[blk].count = kNoHalo; }
-            return;
-        }
-        // compact, pad, sort ascending (bitonic over the power of two at or above the count)
-        const uint32_t nk = 1u << (32 - __clz(static_cast<int>(max(count, 2u) - 1u)));
-        for (uint32_t q = t; q < nk; q += kBlock) { keys[q] = kEmpty32; }
-        __syncthreads();
-        for (uint32_t q = t; q < kHashSlots; q += kBlock)
-        {
-            const uint32_t v = table[q];
-            if (v != kEmpty32) { keys[atomicAdd(&filled, 1u)] = v; }
-        }
-        __syncthreads();
-        for (uint32_t size = 2; size <= nk; size <<= 1)
-        {
-            for (uint32_t stride = size >> 1; stride > 0; stride >>= 1)
+            const uint32_t nA = w.nA > q0 ? min(w.nA - q0, 32u) : 0u;
+            const uint32_t mA = nA < 32u ? m & ((1u << nA) - 1u) : m;
+#pragma unroll
+            for (uint32_t part = 0; part < 2u; part++)
             {
-                for (uint32_t q = t; q < nk; q += kBlock)
+                const uint32_t h = part ? m ^ mA : mA;
+                if (h) { const uint32_t q = static_cast<uint32_t>(__ffs(static_cast<int>(h))) - 1u; fn(q0 + q + (part ? w.oB : w.oA), h >> q, q); }
+            }
+        };
+        const bool wide = (fMin & kWideBit) != 0u;
+        const uint32_t minRef = fMin & ~kWideBit;
+        const bool dict = wide && nF <= kDictMax;
+        // the hash slot of a page; a table that is full gives up on the halo (failS)
+        const auto pageSlot = [&](uint32_t page)
+        {
+            uint32_t h = pageHash(page);
+            for (uint32_t probes = 0; probes < kPageSlots; probes++)
+            {
+                uint32_t v = __hip_atomic_load(&pageKey[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                if (v == 0u)
                 {
-                    const uint32_t r = q ^ stride;
-                    if (r > q)
+                    v = atomicCAS(&pageKey[h], 0u, page + 1u);
+                    if (v == 0u) { atomicAdd(&pagesS, 1u); return h; }
+                }
+                if (v == page + 1u) { return h; }
+                h = (h + 1u) & (kPageSlots - 1u);
+            }
+            failS = 1u;
+            return h;
+        };
+        __syncthreads();
+        // the wave's neighbors: into the bitmap, and counted (a dict list's high group apart), so that
+        // the next waves know where their part of each list starts
+        {
+            uint32_t n = 0, high = 0;
+            each(0, nF != 0u, [&](const RowSpan& w, uint32_t q0, uint32_t m)
+            {
+                n += static_cast<uint32_t>(__popc(m));
+                runs(w, q0, m, [&](uint32_t j, uint32_t h, uint32_t)
+                {
+                    if (dict)
                     {
-                        const uint32_t a = keys[q], b = keys[r];
-                        const bool up = (q & size) == 0;
-                        if ((a > b) == up) { keys[q] = b; keys[r] = a; }
+                        const uint32_t jMax = j + 31u - static_cast<uint32_t>(__clz(static_cast<int>(h)));
+                        atomicMax(&maxRefS[local], jMax);
+                        if (jMax - minRef > 0xffffu)
+                        {
+                            // the first hit of the run beyond the low group
+                            const uint32_t skip = j - minRef > 0xffffu ? 0u : minRef + 0x10000u - j;
+                            const uint32_t hh = h >> skip;
+                            high += static_cast<uint32_t>(__popc(hh));
+                            atomicMin(&base2S[local], j + skip + static_cast<uint32_t>(__ffs(static_cast<int>(hh))) - 1u);
+                        }
                     }
-                }
-                __syncthreads();
+                    const uint32_t word = (j >> 5) & (kPageWords - 1u), sh = j & 31u;
+                    const uint32_t slot = pageSlot(j >> kPageBits);
+                    atomicOr(&bits[slot * kPageWords + word], h << sh);
+                    const uint32_t rest = sh ? h >> (32u - sh) : 0u;
+                    if (rest)
+                    {
+                        const uint32_t next = word + 1u < kPageWords ? slot * kPageWords + word + 1u : pageSlot((j >> kPageBits) + 1u) * kPageWords;
+                        atomicOr(&bits[next], rest);
+                    }
+                });
+            });
+            partF[share][local] = (n - high) | (high << 16);
+            uint32_t nb = 0;
+            if (__any(nB != 0u)) { each(1, nB != 0u, [&](const RowSpan&, uint32_t, uint32_t m) { nb += static_cast<uint32_t>(__popc(m)); }); }
+            partB[share][local] = nb;
+        }
+        __syncthreads();
+        // pages in ascending order: their ranks, then the halo slots where they start
+        const bool fits = !failS && pagesS <= kPages;
+        if (fits && t < 4u * kPageSlots)
+        {
+            const uint32_t p = t & (kPageSlots - 1u), part = t / kPageSlots;
+            const uint32_t own = pageKey[p];
+            uint32_t r = 0;
+            for (uint32_t u = part * (kPageSlots / 4u); u < (part + 1u) * (kPageSlots / 4u); u += 4u)
+            {
+                // (free slots hold 0 and sort last: 0 - 1 is the largest)
+                const uint4 v = *reinterpret_cast<const uint4*>(&pageKey[u]);
+                r += (v.x - 1u < own - 1u ? 1u : 0u) + (v.y - 1u < own - 1u ? 1u : 0u) + (v.z - 1u < own - 1u ? 1u : 0u)
+                     + (v.w - 1u < own - 1u ? 1u : 0u);
+            }
+            if (own) { atomicAdd(&pageRank[p], r); }
+        }
+        __syncthreads();
+        if (fits && t < kPageSlots && pageKey[t])
+        {
+            uint32_t n = 0;
+            for (uint32_t w = 0; w < kPageWords; w++) { n += static_cast<uint32_t>(__popc(bits[t * kPageWords + w])); }
+            pageBase[pageRank[t]] = n;
+        }
+        __syncthreads();
+        if (t < kPages)
+        {
+            const uint32_t own = pageBase[t];
+            uint32_t incl = own;
+            for (int o = 1; o < 64; o <<= 1)
+            {
+                const uint32_t v = static_cast<uint32_t>(__shfl_up(static_cast<int>(incl), o, 64));
+                if (lane >= static_cast<uint32_t>(o)) { incl += v; }
+            }
+            pageBase[t] = incl - own;
+            if (t == kPages - 1u)
+            {
+                countS = (!fits || incl > kHaloMax) ? kNoHalo : incl;
+                d.haloInfo[blk] = HaloInfo{ countS, 1u };
             }
         }
-        for (uint32_t q = t; q < count; q += kBlock)
-        {
-            out[q] = keys[q];
-            rank[haloFind(table, keys[q])] = static_cast<uint16_t>(q);
-        }
-        if (t == 0) { d.haloInfo[blk].count = count; }
+        static_assert(kPages == 64, "the page counts are scanned by one wave");
         __syncthreads();
-        // entries become their rank in the sorted halo, in their storage format
-        for (uint32_t k = 0; k < n; k++)
+        const bool halo = countS != kNoHalo;
+        if (halo)
         {
-            const uint32_t j = sellRead(d.pool[REL_FF], m, lane, k);
-            const uint32_t slot = rank[haloFind(table, j)] << kSlotShift;
-            d.pool[REL_FF][m.offset + k * kSlice + lane] = static_cast<uint16_t>(slot);
+            // one word of the bitmap per thread: its particles into the halo, its slots into the table
+            uint32_t* out = d.haloIdx + static_cast<size_t>(blk) * kHaloMax;
+            for (uint32_t q = t; q < kPageSlots * kPageWords; q += kQueryThreads)
+            {
+                uint32_t b = bits[q];
+                if (b == 0u) { continue; }
+                const uint32_t p = q / kPageWords, w = q & (kPageWords - 1u);
+                const uint32_t rank = pageRank[p];
+                uint32_t r = pageBase[rank];
+                for (uint32_t v = 0; v < w; v++) { r += static_cast<uint32_t>(__popc(bits[p * kPageWords + v])); }
+                const uint32_t j0 = ((pageKey[p] - 1u) << kPageBits) + 32u * w;
+                uint16_t* table = slotOf + (rank << kPageBits) + 32u * w;
+                while (b)
+                {
+                    const uint32_t u = static_cast<uint32_t>(__ffs(static_cast<int>(b))) - 1u;
+                    out[r] = j0 + u;
+                    table[u] = static_cast<uint16_t>(r << kSlotShift);
+                    r++;
+                    b &= b - 1u;
+                }
+            }
+            __syncthreads();
         }
-        slotsToU16(d, i, m);
+        // the entries: FF by slot or index, FB and FR by index
+        uint32_t low = 0, high = 0, kB = 0;
+        for (uint32_t q = 0; q < share; q++) { const uint32_t v = partF[q][local]; low += v & 0xffffu; high += v >> 16; kB += partB[q][local]; }
+        const bool split = dict && maxRefS[local] - base2S[local] <= 0xffffu;
+        if (!split) { low += high; }
+        {
+            const SliceMeta mF = d.meta[REL_FF][pos / kSlice];
+            uint16_t* rows = d.pool[REL_FF] + mF.offset + lw;
+            each(0, nF != 0u, [&](const RowSpan& w, uint32_t q0, uint32_t m)
+            {
+                // table positions of the runs' candidates: the run's first hit is in the table, and the
+                // page after its own, when the run has hits there, is the next in the table
+                uint32_t tA = 0, tB = 0;
+                if (halo)
+                {
+                    runs(w, q0, m, [&](uint32_t j, uint32_t, uint32_t q)
+                    {
+                        uint32_t h = pageHash(j >> kPageBits);
+                        for (uint32_t probes = 0; probes < kPageSlots && pageKey[h] != (j >> kPageBits) + 1u; probes++) { h = (h + 1u) & (kPageSlots - 1u); }
+                        const uint32_t at = (pageRank[h] << kPageBits) + (j & ((1u << kPageBits) - 1u)) - q;
+                        if (q0 + q < w.nA) { tA = at; } else { tB = at; }
+                    });
+                }
+                while (m)
+                {
+                    const uint32_t q = static_cast<uint32_t>(__ffs(static_cast<int>(m))) - 1u;
+                    m &= m - 1u;
+                    const uint32_t j = w.at(q0 + q);
+                    const uint32_t k = (split && j - minRef > 0xffffu) ? nF - ++high : low++;
+                    if (halo)
+                    {
+                        const uint16_t e = slotOf[q + (q0 + q < w.nA ? tA : tB)];
+                        if (k < kStage) { stage[k][col] = e; } else { rows[k * kSlice] = e; }
+                    }
+                    else { sellWrite(d.pool[REL_FF], mF, lw, k, j); }
+                }
+            });
+        }
+        if (__any(nB != 0u))
+        {
+            const SliceMeta mB = d.meta[REL_FB][pos / kSlice];
+            each(1, nB != 0u, [&](const RowSpan& w, uint32_t q0, uint32_t m)
+            {
+                while (m)
+                {
+                    const uint32_t q = static_cast<uint32_t>(__ffs(static_cast<int>(m))) - 1u;
+                    m &= m - 1u;
+                    sellWrite(d.pool[REL_FB], mB, lw, kB++, w.at(q0 + q));
+                }
+            });
+        }
+        if (nR && share == 0u)
+        {
+            // few particles have rigid neighbors: one wave walks their rows
+            const SliceMeta mR = d.meta[REL_FR][pos / kSlice];
+            uint32_t kR = 0;
+#pragma unroll 1
+            for (uint32_t r = 0; r < s.side * s.side * s.chunks; r++)
+            {
+                const RowSpan w = s.cells(d.cellR, r, true).span();
+                for (uint32_t q = 0; q < w.n; q++)
+                {
+                    const uint32_t j = d.idxR[w.at(q)];
+                    if (within(pi.x, pi.y, pi.z, d.rpos[j], r2)) { sellWrite(d.pool[REL_FR], mR, lw, kR++, j); }
+                }
+            }
+        }
+        if (!halo) { return; }
+        __syncthreads();
+        // the staged entries leave as whole slice rows; the slices of a block with a halo are u16 slices
+        const uint32_t p = t & (kBlock - 1u);
+        SliceMeta& m = d.meta[REL_FF][(blk * kBlock + p) / kSlice];
+        const uint32_t n = min(static_cast<uint32_t>(d.head[blk * kBlock + p].x & 0xffffu), kStage);
+        uint16_t* row = d.pool[REL_FF] + m.offset + (p & (kSlice - 1u));
+        for (uint32_t k = t / kBlock; k < n; k += kQueryShare) { row[k * kSlice] = stage[k][p]; }
+        if (t < kBlock && (t & (kSlice - 1u)) == 0u) { m.format = kFmtDelta16; }
     }
-#endif
 
     // ----------------------------------------------------------------------------------------
     // rigid-source lists, one wave per rigid particle: mode 0 counts RF, RB and RR; mode 1 fills
@@ -1673,7 +1350,9 @@ namespace tsp
     {
         if (threadIdx.x != 0) { return; }
         const Status& st = *d.status;
-        const bool refuse = st.abort != 0u || st.overflow != 0u || st.rbTotal != 0ull || st.rrTotal != 0ull
+        bool grow = false;
+        for (int r = 0; r < 3; r++) { grow = grow || st.poolUnits[r] > d.poolCap[r]; }
+        const bool refuse = st.abort != 0u || st.overflow != 0u || grow || st.rbTotal != 0ull || st.rrTotal != 0ull
                             || (st.pairTiny != 0u && d.fastPairs != 0u);
         if (refuse) { d.status->stop |= 1u; }
     }
@@ -1862,32 +1541,15 @@ namespace tsp
 
     void launchQueryCount(hipStream_t s, const Dev& d)
     {
-        const uint32_t nSlices = (d.nF + kSlice - 1) / kSlice;
-        if (d.nF) { kQueryCount<<<blocksFor(d.nF), kBlock, 0, s>>>(d, nSlices); }
-    }
-
-    // units is 3 x (nSlices + 1) u32
-    void launchScanSlices(hipStream_t s, const Dev& d, uint32_t* units, uint32_t* tmp)
-    {
-        const uint32_t nSlices = (d.nF + kSlice - 1) / kSlice;
-        const dim3 g(blocksFor(nSlices + 1ull), 3);
-        kSliceUnits<<<g, kBlock, 0, s>>>(d, nSlices, units);
-        for (uint32_t r = 0; r < 3; r++) { launchScan(s, units + r * (nSlices + 1), nSlices + 1, tmp, &d.status->scanFail); }
-        kSliceApply<<<g, kBlock, 0, s>>>(d, nSlices, units);
+        const uint32_t n = blocksFor(d.nF);
+        if (n == 0u) { return; }
+        if (n <= kShareBlocks) { kQueryCount<kQueryShare><<<n, kQueryThreads, 0, s>>>(d); }
+        else { kQueryCount<1u><<<n, kBlock, 0, s>>>(d); }
     }
 
     void launchQueryFill(hipStream_t s, const Dev& d)
     {
-        if (d.nF)
-        {
-            kQueryFill<<<blocksFor(d.nF), kBlock, 0, s>>>(d);
-            kQueryFillWide<<<blocksFor(d.nF), kBlock, 0, s>>>(d);
-        }
-    }
-
-    void launchHaloBuild(hipStream_t s, const Dev& d)
-    {
-        if (d.nF) { kHaloBuild<<<blocksFor(d.nF), kBlock, 0, s>>>(d); }
+        if (d.nF) { kQueryFill<<<blocksFor(d.nF), kQueryThreads, 0, s>>>(d); }
     }
 
     void launchQueryRigid(hipStream_t s, const Dev& d, int mode, uint32_t* tmp)

@@ -39,7 +39,6 @@ namespace tsp
     void launchClearAll(hipStream_t, uint2*, uint64_t);
     void launchBuildCells(hipStream_t, const Dev&, const uint32_t*, uint32_t, uint2*);
     void launchQueryCount(hipStream_t, const Dev&);
-    void launchScanSlices(hipStream_t, const Dev&, uint32_t*, uint32_t*);
     void launchQueryFill(hipStream_t, const Dev&);
     void launchQueryRigid(hipStream_t, const Dev&, int, uint32_t*);
     void launchStepGate(hipStream_t, const Dev&);
@@ -51,7 +50,6 @@ namespace tsp
     void launchBuildFluid(hipStream_t, const Dev&, uint32_t, uint32_t, const BuildFluid&);
     void launchBuildBoundary(hipStream_t, const BuildBoundary&, uint32_t, float4*, float*, uint64_t*, float*, uint32_t*,
                              uint32_t*, uint32_t*, uint32_t*, uint32_t*, uint32_t*);
-    void launchHaloBuild(hipStream_t, const Dev&);
     void launchAabb(hipStream_t, const Dev&, int, const float4*, uint32_t, uint32_t*);
     void launchDensity(hipStream_t, const Dev&);
     void launchNonPressure(hipStream_t, const Dev&);
@@ -302,7 +300,6 @@ struct tsp_ctx
     uint64_t *idB = nullptr, *idB2 = nullptr;
     uint64_t* idR = nullptr;
     uint32_t* radixHist = nullptr;
-    uint32_t* sliceUnits = nullptr; // 3 x (slices + 1) scan buffer
     uint32_t* aabb = nullptr;       // 6 per scene
     std::vector<void*> arena;       // particle and body arrays (replaced by a relayout)
     std::vector<void*> work;        // search and scene-table buffers sized by the layout
@@ -627,7 +624,7 @@ struct tsp_ctx
         try
         {
             n.nF = nF; n.nB = nB; n.nR = nR; n.nRB = nRB; n.nScenes = S;
-            n.pos = alloc<float4>(nF, A, MEM_PF); npos2 = alloc<float4>(nF, A, MEM_PF);
+            n.pos = alloc<float4>(nF + kRecordPad, A, MEM_PF); npos2 = alloc<float4>(nF + kRecordPad, A, MEM_PF);
             n.vel = alloc<float4>(nF, A, MEM_PF); nvel2 = alloc<float4>(nF, A, MEM_PF);
             n.vp = alloc<float4>(nF, A, MEM_PF); nvp2 = alloc<float4>(nF, A, MEM_PF);
             n.ap = alloc<float4>(nF, A, MEM_PF); nap2 = alloc<float4>(nF, A, MEM_PF);
@@ -639,7 +636,7 @@ struct tsp_ctx
             zero(n.vp, sizeof(float4) * nF); zero(n.ap, sizeof(float4) * nF);
             zero(n.source, sizeof(float) * nF); zero(n.diag, sizeof(float) * nF);
             zero(n.id, sizeof(uint64_t) * nF);
-            n.bpos = alloc<float4>(nB, A, MEM_PB); nbpos2 = alloc<float4>(nB, A, MEM_PB);
+            n.bpos = alloc<float4>(nB + kRecordPad, A, MEM_PB); nbpos2 = alloc<float4>(nB + kRecordPad, A, MEM_PB);
             n.bvol = alloc<float>(nB, A, MEM_PB); nbvol2 = alloc<float>(nB, A, MEM_PB);
             nidB = alloc<uint64_t>(nB, A, MEM_PB); nidB2 = alloc<uint64_t>(nB, A, MEM_PB);
             n.rxrel = alloc<float>(nR, A, MEM_PR); n.ryrel = alloc<float>(nR, A, MEM_PR); n.rzrel = alloc<float>(nR, A, MEM_PR);
@@ -845,18 +842,17 @@ struct tsp_ctx
             d.meta[r] = alloc<SliceMeta>(nSlices, work, MEM_LF);
             zero(d.cnt[r], sizeof(uint16_t) * nF);
         }
-        sliceUnits = alloc<uint32_t>(3ull * (nSlices + 1), work);
         {
-            // block sums of the scans: radix digit offsets, slice units, RF offsets
-            const uint64_t m = std::max<uint64_t>(256ull * nTiles, std::max<uint64_t>(nSlices + 1ull, nR + 1ull));
+            // block sums of the scans: radix digit offsets, RF offsets
+            const uint64_t m = std::max<uint64_t>(256ull * nTiles, nR + 1ull);
             d.scanTmp = alloc<uint32_t>(scanTmpWords(m), work);
             zero(d.scanTmp, sizeof(uint32_t) * scanTmpWords(m));
         }
         d.ffMin = alloc<uint32_t>(nF, work, MEM_LF);
-        d.wideList = alloc<uint32_t>(nF, work, MEM_LF);
         d.laneRank = alloc<uint8_t>(nF, work, MEM_LF);
         d.head = alloc<uint2>(nF, work, MEM_LF);
         d.ffMask = alloc<uint32_t>(static_cast<size_t>(kMaskWords) * nF, work, MEM_SF);
+        d.fbMask = alloc<uint32_t>(static_cast<size_t>(kMaskRows) * nF, work, MEM_SF);
         {
             const uint64_t nBlocks = nF / kBlock;
             d.haloIdx = alloc<uint32_t>(nBlocks * kHaloMax, work, MEM_LF);
@@ -1238,10 +1234,6 @@ struct tsp_ctx
             launchQueryCount(stream, d);
             launchQueryRigid(stream, d, 0, d.scanTmp);
         }
-        {
-            Scope sc(prof, stream, "scan");
-            launchScanSlices(stream, d, sliceUnits, d.scanTmp);
-        }
     }
 
     void neighborSearch(bool allFields)
@@ -1281,7 +1273,9 @@ struct tsp_ctx
                 // slice offsets are u32 in u16 units
                 if (last.poolUnits[r] > 0xffffffffull) { refuse("SELL pool exceeds 2^32 u16 units"); }
             }
-            if (last.overflow & 5u)
+            bool grow = (last.overflow & 4u) != 0u;
+            for (int r = 0; r < 3; r++) { grow = grow || last.poolUnits[r] > d.poolCap[r]; }
+            if (grow)
             {
                 uint64_t cap[3];
                 for (int r = 0; r < 3; r++)
@@ -1307,10 +1301,6 @@ struct tsp_ctx
                 launchQueryRigid(stream, d, contactLists ? 2 : 1, d.scanTmp);
             }
             listsValid = true;
-            {
-                Scope sc(prof, stream, "halo");
-                launchHaloBuild(stream, d);
-            }
             return;
         }
         throw Error{ TSP_ERR_STATE, "cell frame rebuild did not converge" };
@@ -1534,7 +1524,7 @@ struct tsp_ctx
     {
         std::string key(reinterpret_cast<const char*>(&id), sizeof(id));
         key.append(reinterpret_cast<const char*>(&d), sizeof(Dev));
-        const void* extra[5] = { pos2, vel2, idF2, sliceUnits, radixHist };
+        const void* extra[4] = { pos2, vel2, idF2, radixHist };
         key.append(reinterpret_cast<const char*>(extra), sizeof(extra));
         key.append(reinterpret_cast<const char*>(&keyBits), sizeof(keyBits));
         auto it = stepGraphs.find(key);
@@ -1583,7 +1573,6 @@ struct tsp_ctx
             d.stopMask = 1u;
             launchQueryFill(stream, d);
             launchQueryRigid(stream, d, 1, d.scanTmp);
-            launchHaloBuild(stream, d);
             predictLaunches();
         });
         // d.stopMask is 1 here (the state the piece leaves)
@@ -2623,11 +2612,11 @@ uint64_t tsp_batch_footprint(uint32_t n_fluid, uint32_t n_boundary, uint32_t n_r
 {
     // device bytes a scene holds while resident: per fluid slot (segment rounded to 256) about
     // 190 B of records and second buffers, 16 B of sort keys, 160 B of SELL-32 lists at the
-    // initial pool sizes, 26 B of halo, counts, list positions and the wide-list index, and up to
+    // initial pool sizes, 66 B of halo, counts, list heads and boundary hit masks, and up to
     // 24 B of cell tables; per boundary particle 64 B; per rigid particle about 400 B (records,
     // keys, the RF list); per body 256 B
     const uint64_t f = static_cast<uint64_t>(roundUp(n_fluid, kBlock));
-    return f * 416ull + static_cast<uint64_t>(n_boundary) * 64ull + static_cast<uint64_t>(n_rigid) * 400ull
+    return f * 456ull + static_cast<uint64_t>(n_boundary) * 64ull + static_cast<uint64_t>(n_rigid) * 400ull
          + static_cast<uint64_t>(n_bodies) * 256ull + (64ull << 10);
 }
 

@@ -26,14 +26,6 @@
 
 // build-time variants of the solver sweeps (all give the same bits; the build picks one):
 //   TSP_TUNE_SWEEP_AHEAD   the first sweep group of a step: the previous step's sweeps plus this
-//   TSP_TUNE_BOX_CELLS     the fill stages the fluid cell ranges of its block's stencil box in LDS
-//                          when the box has at most this many cells (0: off)
-//   TSP_TUNE_RANGE_LOADS   the stencil walk loads a row's nine cell ranges in every lane and selects
-//                          (1), or loads only the ranges a lane walks (0)
-//   TSP_TUNE_QUERY_WAVES   register budget of the neighbor query and halo kernels: waves per SIMD
-//                          (0: the compiler's choice)
-//   TSP_TUNE_HALO_PAGES    the FF halo of a block from bitmaps over pages of 4096 indices (1), or
-//                          from one 64 Ki-index window bitmap, else a sorted hash set (0)
 //   TSP_TUNE_STEP_GRAPH    a step runs as one captured graph launch with one status read (1), or
 //                          launch by launch with the host reading the status between phases (0)
 //   TSP_TUNE_JACOBI_REC24  kJacobi's halo records take 24 bytes instead of 32 (six blocks per CU)
@@ -42,27 +34,9 @@
 //   TSP_TUNE_PA_WAVES, TSP_TUNE_JACOBI_WAVES   waves per SIMD the compiler must leave room for
 //                          (register budget of the sweep kernels); 0 leaves the choice to it
 //   TSP_TUNE_RADIX_BITS    digit width of the LSD radix sorts (8: 256 buckets, 6, 4)
-//   TSP_TUNE_SEARCH_FLAT   the count pass folds its hits in through selects, its row streams loading
-//                          past their end (1) or branching around those loads (2); or it branches
-//                          on each candidate (0)
-//   TSP_TUNE_SEARCH_ROW    the neighbor query walks the stencil by rows of three cells, loading
-//                          the rows' ranges together and TSP_TUNE_SEARCH_BATCH candidates at a time
-//                          (1: the row's candidates as one stream, 2: cell by cell; 0: the cell walk)
 // the settings chosen by turbospharticles_amd/tune.py, when present, come first
 #if __has_include("tsp_tuned.h")
 #include "tsp_tuned.h"
-#endif
-#ifndef TSP_TUNE_BOX_CELLS
-#define TSP_TUNE_BOX_CELLS 0
-#endif
-#ifndef TSP_TUNE_RANGE_LOADS
-#define TSP_TUNE_RANGE_LOADS 0
-#endif
-#ifndef TSP_TUNE_QUERY_WAVES
-#define TSP_TUNE_QUERY_WAVES 0
-#endif
-#ifndef TSP_TUNE_HALO_PAGES
-#define TSP_TUNE_HALO_PAGES 0
 #endif
 #ifndef TSP_TUNE_STEP_GRAPH
 #define TSP_TUNE_STEP_GRAPH 1
@@ -84,15 +58,6 @@
 #endif
 #ifndef TSP_TUNE_JACOBI_WAVES
 #define TSP_TUNE_JACOBI_WAVES 0
-#endif
-#ifndef TSP_TUNE_SEARCH_ROW
-#define TSP_TUNE_SEARCH_ROW 1
-#endif
-#ifndef TSP_TUNE_SEARCH_FLAT
-#define TSP_TUNE_SEARCH_FLAT 0
-#endif
-#ifndef TSP_TUNE_SEARCH_BATCH
-#define TSP_TUNE_SEARCH_BATCH 4
 #endif
 #ifndef TSP_TUNE_RADIX_BITS
 #define TSP_TUNE_RADIX_BITS 8
@@ -129,11 +94,13 @@ namespace tsp
     constexpr uint32_t kScanHeaderWords = 4;
     inline constexpr uint64_t scanTmpWords(uint64_t m) { return kScanHeaderWords + 2ull * ((m + 2047ull) / 2048ull); }
 
-    // FF hit masks of the count pass (one word per stencil row of three cells, reach 1): the fill
-    // takes the hits from them and loads no candidate position. A row with more than 32 fluid
-    // candidates is marked in the last word and tested again by the fill.
+    // Hit masks of the count pass (one word per stencil row of three cells, reach 1): the fill takes the
+    // hits from them and loads no candidate position. A row with more than 32 candidates is marked in
+    // the last word and tested again by the fill.
     constexpr uint32_t kMaskRows = 9;
     constexpr uint32_t kMaskWords = kMaskRows + 1;
+    // records past the end of the position arrays that the query may read (and does not use)
+    constexpr uint32_t kRecordPad = 8;
     // FF neighbor halo of a 256-particle block: the distinct FF neighbors of its particles,
     // ascending; the FF entries of the block then hold halo slots instead of particle indices
     constexpr uint32_t kHaloMax = TSP_TUNE_HALO_MAX; // 24 B x 1064 records in kJacobi: six blocks per CU
@@ -180,11 +147,11 @@ namespace tsp
     struct Status
     {
         uint32_t abort;          // some scene's particle left its inner cell frame: restart the search
-        uint32_t overflow;       // a SELL pool is too small
+        uint32_t overflow;       // 2: a count exceeds its u16 storage; 4: the RF list is too small
         uint32_t bUnsorted;      // boundary ids are not non-decreasing under the frames
         uint32_t pairTiny;       // some FF or FB pair has 0 < d2 < 2^-96: the kernels take the general sqrt
         uint32_t scanFail;       // sticky: a one-pass scan gave up waiting (kResetSearch keeps it)
-        uint32_t wideCount;      // particles in wideList (FF lists spanning more than 0xffff)
+        uint32_t pad0;
         uint32_t stop;           // a captured step stops early: 1 = its search needs the host, 2 = its
                                  // solve needs more sweeps (kernels launched with stopMask skip)
         uint64_t poolUnits[3];   // u16 units used by FF, FB, FR
@@ -382,9 +349,9 @@ namespace tsp
                                  // (its index within the block): what a kernel thread reads first
         uint32_t *ffMin;         // per particle: smallest FF neighbor index (0 without FF neighbors), with
                                  // kWideBit set when the list spans more than 0xffff
-        uint32_t *wideList;      // the particles with kWideBit, in no particular order (status->wideCount)
         uint32_t *ffMask;        // kMaskWords x nF: per stencil row, bit q = the row's q-th fluid candidate
-                                 // is an FF neighbor; then the rows the masks do not cover
+                                 // is an FF neighbor; then a word about the rows (kOpenF and on, kernels_search.hip)
+        uint32_t *fbMask;        // kMaskRows x nF: the same for the boundary candidates (rows that have any)
         uint32_t *haloIdx;       // per block: kHaloMax particle indices, ascending
         HaloInfo *haloInfo;      // per block
         // rigid-source CSR (RF), counts of RB and RR

@@ -3,10 +3,8 @@
 Every variant gives the same bits; they differ in how the work maps onto the GPU: the radix sort's
 digit width (8, 6 or 4 bits: 4 to 8 passes over 28-bit keys), the size of a step's first sweep
 group against the previous step's sweep count, the whole step as one graph launch or launch by
-launch, the FF halo built from page bitmaps or a window bitmap and hash set, 24- or 32-byte Jacobi
-halo records, the halo cap (LDS per sweep block), register budgets of the sweep
-kernels, sweep groups as HIP graphs, the neighbor query's walk of the stencil (cell by cell, or
-rows of three cells) and its candidate loads in flight. The
+launch, 24- or 32-byte Jacobi halo records, the halo cap (LDS per sweep block), register budgets of the sweep
+kernels, sweep groups as HIP graphs. The
 tuner walks the switches one at a time from the current settings (coordinate descent), keeping a
 change when it shortens the measured step.
 
@@ -40,17 +38,11 @@ SPACE = {
     "TSP_TUNE_RADIX_BITS": [8, 6, 4],
     "TSP_TUNE_SWEEP_AHEAD": [-1, 0, 1, 2],
     "TSP_TUNE_STEP_GRAPH": [0, 1],
-    "TSP_TUNE_QUERY_WAVES": [0, 6, 8],
-    "TSP_TUNE_RANGE_LOADS": [0, 1],
-    "TSP_TUNE_BOX_CELLS": [0, 512, 768, 1024],
     "TSP_TUNE_JACOBI_REC24": [1, 0],
     "TSP_TUNE_HALO_MAX": [1000, 960, 1024, 1064],
     "TSP_TUNE_GRAPHS": [1, 0],
     "TSP_TUNE_PA_WAVES": [0, 6, 8],
     "TSP_TUNE_JACOBI_WAVES": [0, 6],
-    "TSP_TUNE_SEARCH_ROW": [1, 0, 2],
-    "TSP_TUNE_SEARCH_FLAT": [0, 1, 2],
-    "TSP_TUNE_SEARCH_BATCH": [4, 8],
 }
 
 
