@@ -10,73 +10,124 @@
 namespace tsp
 {
     constexpr uint32_t kHistBins = 65536;   // neighbor counts are stored in 16 bits
+    constexpr uint32_t kRelations = 6;      // FF, FB, FR (u16 counts), RF, RB, RR (u32)
 
-    // counts of one relation of one scene: u16 (FF, FB, FR) or u32 (RF, RB, RR)
-    __global__ void __launch_bounds__(kBlock) kStatsHist(const uint16_t* __restrict__ c16, const uint32_t* __restrict__ c32,
-        uint32_t mask, uint32_t n, uint32_t* __restrict__ hist)
+    // the counts of one scene
+    struct StatsCounts
     {
-        const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-        if (i >= n) { return; }
-        const uint32_t v = c16 ? (static_cast<uint32_t>(c16[i]) & mask) : c32[i];
-        atomicAdd(&hist[v < kHistBins ? v : kHistBins - 1u], 1u);
+        const uint16_t* c16[3];
+        const uint32_t* c32[3];
+        uint32_t nF, nR;
+    };
+
+    // Histograms of all six relations' counts. Nearly all counts fall into a few dozen bins, so a global
+    // atomic per particle runs at the rate of one address (4.7 ms per relation at 1M particles); each
+    // block counts the low bins in LDS first and adds its nonzero ones (1M: all six in 20 us).
+    constexpr uint32_t kLowBins = 512;
+
+    __global__ void __launch_bounds__(kBlock) kStatsHist(StatsCounts c, uint32_t* __restrict__ hist)
+    {
+        __shared__ uint32_t low[kRelations][kLowBins];
+        for (uint32_t q = threadIdx.x; q < kRelations * kLowBins; q += kBlock) { low[q / kLowBins][q % kLowBins] = 0u; }
+        __syncthreads();
+        const uint32_t stride = gridDim.x * kBlock;
+        const auto count = [&](uint32_t r, uint32_t v)
+        {
+            if (v < kLowBins) { atomicAdd(&low[r][v], 1u); }
+            else { atomicAdd(&hist[r * kHistBins + min(v, kHistBins - 1u)], 1u); }
+        };
+        for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < c.nF; i += stride)
+        {
+            for (uint32_t r = 0; r < 3u; r++) { count(r, c.c16[r][i]); }
+        }
+        for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < c.nR; i += stride)
+        {
+            for (uint32_t r = 0; r < 3u; r++) { count(3u + r, c.c32[r][i]); }
+        }
+        __syncthreads();
+        for (uint32_t q = threadIdx.x; q < kRelations * kLowBins; q += kBlock)
+        {
+            const uint32_t v = low[q / kLowBins][q % kLowBins];
+            if (v) { atomicAdd(&hist[(q / kLowBins) * kHistBins + q % kLowBins], v); }
+        }
     }
 
-    // minimum, maximum and the value at sorted position (99 (n - 1)) / 100 of a histogram of n
-    // values (ComputeStatsFromHistogram, statistics_kernels.cu:82-127), and their sum; one block
-    __global__ void __launch_bounds__(kBlock) kStatsHistScan(const uint32_t* __restrict__ hist, uint32_t n,
-        uint64_t* __restrict__ out)
+    // Block r < 6: minimum, maximum and the value at sorted position (99 (n - 1)) / 100 of relation r's
+    // histogram (ComputeStatsFromHistogram, statistics_kernels.cu:82-127), and the sum of its values.
+    // Block 6: the fluid sums of kStatsFluid's partials. Chunks of 1024 bins: a wave sums four of them,
+    // one wave scans the 64 chunk counts, then the chunk that holds the percentile (all in 13 us at 1M
+    // particles; one thread scanning bins and partials took 6 x 46 + 843 us).
+    constexpr uint32_t kScanThreads = 1024;
+    constexpr uint32_t kChunk = 1024;
+    constexpr uint32_t kChunks = kHistBins / kChunk;
+    static_assert(kChunks == 64, "one wave scans the chunks");
+
+    __device__ __forceinline__ uint32_t waveScan(uint32_t v)
     {
-        constexpr uint32_t kPer = kHistBins / kBlock;
-        __shared__ uint32_t chunk[kBlock];
-        __shared__ uint64_t wsum[kBlock];
-        const uint32_t t = threadIdx.x;
-        uint32_t s = 0;
-        uint64_t ws = 0;
-        for (uint32_t b = 0; b < kPer; b++)
+        for (int o = 1; o < 64; o <<= 1)
         {
-            const uint32_t h = hist[t * kPer + b];
-            s += h;
-            ws += static_cast<uint64_t>(h) * (t * kPer + b);
+            const uint32_t u = static_cast<uint32_t>(__shfl_up(static_cast<int>(v), o, 64));
+            if ((threadIdx.x & 63u) >= static_cast<uint32_t>(o)) { v += u; }
         }
-        chunk[t] = s;
-        wsum[t] = ws;
+        return v;
+    }
+
+    __device__ void histogramStats(const uint32_t* __restrict__ hist, uint32_t n, uint64_t* __restrict__ out)
+    {
+        __shared__ uint32_t chunk[kChunks];
+        __shared__ unsigned long long total;
+        __shared__ uint32_t mn, mx;
+        const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+        if (threadIdx.x == 0) { total = 0ull; mn = kHistBins; mx = 0u; }
         __syncthreads();
-        if (t != 0) { return; }
-        uint64_t total = 0;
-        for (uint32_t c = 0; c < kBlock; c++) { total += wsum[c]; }
-        uint32_t mn = 0, mx = 0, p99 = 0;
+        unsigned long long sum = 0;
+        uint32_t lo = kHistBins, hi = 0;
+        for (uint32_t c = wave; c < kChunks; c += kScanThreads / 64u)
+        {
+            uint32_t s = 0;
+            for (uint32_t q = 0; q < kChunk / 64u; q++)
+            {
+                const uint32_t v = c * kChunk + q * 64u + lane, h = hist[v];
+                s += h;
+                sum += static_cast<unsigned long long>(h) * v;
+                if (h) { lo = min(lo, v); hi = max(hi, v); }
+            }
+            for (int o = 32; o > 0; o >>= 1) { s += static_cast<uint32_t>(__shfl_xor(static_cast<int>(s), o, 64)); }
+            if (lane == 0u) { chunk[c] = s; }
+        }
+        if (hi || lo < kHistBins) { atomicAdd(&total, sum); atomicMin(&mn, lo); atomicMax(&mx, hi); }
+        __syncthreads();
+        if (wave != 0u) { return; }
+        uint32_t p99 = 0;
         if (n > 0)
         {
-            const uint64_t i99 = (99ull * static_cast<uint64_t>(n - 1u)) / 100ull;
-            uint64_t before = 0;
-            bool haveMin = false, haveP99 = false;
-            uint32_t lastChunk = 0;
-            for (uint32_t c = 0; c < kBlock; c++)
+            const uint32_t i99 = static_cast<uint32_t>((99ull * static_cast<uint64_t>(n - 1u)) / 100ull);
+            const uint32_t incl = waveScan(chunk[lane]);
+            const uint32_t c = static_cast<uint32_t>(__ffsll(static_cast<unsigned long long>(__ballot(incl > i99)))) - 1u;
+            uint32_t before = c ? static_cast<uint32_t>(__shfl(static_cast<int>(incl), static_cast<int>(c) - 1, 64)) : 0u;
+            for (uint32_t q = 0; q < kChunk / 64u; q++)
             {
-                if (chunk[c] == 0u) { continue; }
-                const uint32_t lo = c * kPer;
-                if (!haveMin)
-                {
-                    for (uint32_t v = lo; v < lo + kPer; v++) { if (hist[v]) { mn = v; break; } }
-                    haveMin = true;
-                }
-                lastChunk = c;
-                const uint64_t after = before + chunk[c];
-                if (!haveP99 && i99 < after)
-                {
-                    uint64_t b = before;
-                    for (uint32_t v = lo; v < lo + kPer; v++)
-                    {
-                        b += hist[v];
-                        if (i99 < b) { p99 = v; break; }
-                    }
-                    haveP99 = true;
-                }
-                before = after;
+                const uint32_t v = c * kChunk + q * 64u;
+                const uint32_t in = before + waveScan(hist[v + lane]);
+                const unsigned long long past = __ballot(in > i99);
+                if (past) { p99 = v + static_cast<uint32_t>(__ffsll(past)) - 1u; break; }
+                before = static_cast<uint32_t>(__shfl(static_cast<int>(in), 63, 64));
             }
-            for (uint32_t v = lastChunk * kPer + kPer; v > lastChunk * kPer; v--) { if (hist[v - 1]) { mx = v - 1; break; } }
         }
-        out[0] = mn; out[1] = mx; out[2] = p99; out[3] = total;
+        if (lane == 0u)
+        {
+            out[0] = n ? mn : 0u; out[1] = mx; out[2] = p99; out[3] = total;
+        }
+    }
+
+    __device__ void fluidStats(const double* __restrict__ partial, uint32_t nBlocks, double* __restrict__ out);
+
+    __global__ void __launch_bounds__(kScanThreads) kStatsScan(StatsCounts c, const uint32_t* __restrict__ hist,
+        const double* __restrict__ partial, uint32_t nBlocks, uint64_t* __restrict__ counts, double* __restrict__ fluid)
+    {
+        const uint32_t r = blockIdx.x;
+        if (r < kRelations) { histogramStats(hist + static_cast<size_t>(r) * kHistBins, r < 3u ? c.nF : c.nR, counts + 4u * r); }
+        else { fluidStats(partial, nBlocks, fluid); }
     }
 
     // per block of the scene's fluid: FP64 sums of the density error terms and of |v|, min and max |v|
@@ -119,55 +170,69 @@ namespace tsp
         }
     }
 
-    __global__ void __launch_bounds__(kBlock) kStatsFluidSum(const double* __restrict__ partial, uint32_t nBlocks,
-        double* __restrict__ out)
+    // the block partials summed in a fixed order: 1,024 threads stride over them, then a tree
+    __device__ void fluidStats(const double* __restrict__ partial, uint32_t nBlocks, double* __restrict__ out)
     {
-        if (threadIdx.x != 0) { return; }
+        __shared__ double red[6][kScanThreads / 64];
         double a[4] = { 0, 0, 0, 0 };
-        double lo = nBlocks ? 3.4e38 : 0.0, hi = 0.0;
-        for (uint32_t b = 0; b < nBlocks; b++)
+        double lo = 3.4e38, hi = 0.0;
+        for (uint32_t b = threadIdx.x; b < nBlocks; b += kScanThreads)
         {
             for (int r = 0; r < 4; r++) { a[r] += partial[6ull * b + r]; }
-            lo = partial[6ull * b + 4] < lo ? partial[6ull * b + 4] : lo;
-            hi = partial[6ull * b + 5] > hi ? partial[6ull * b + 5] : hi;
+            lo = fmin(lo, partial[6ull * b + 4]);
+            hi = fmax(hi, partial[6ull * b + 5]);
+        }
+        for (int o = 32; o > 0; o >>= 1)
+        {
+            for (int r = 0; r < 4; r++) { a[r] += __shfl_xor(a[r], o, 64); }
+            lo = fmin(lo, __shfl_xor(lo, o, 64));
+            hi = fmax(hi, __shfl_xor(hi, o, 64));
+        }
+        const uint32_t w = threadIdx.x >> 6;
+        if ((threadIdx.x & 63u) == 0u) { for (int r = 0; r < 4; r++) { red[r][w] = a[r]; } red[4][w] = lo; red[5][w] = hi; }
+        __syncthreads();
+        if (threadIdx.x != 0) { return; }
+        for (uint32_t q = 1; q < kScanThreads / 64u; q++)
+        {
+            for (int r = 0; r < 4; r++) { a[r] += red[r][q]; }
+            lo = fmin(lo, red[4][q]);
+            hi = fmax(hi, red[5][q]);
         }
         for (int r = 0; r < 4; r++) { out[r] = a[r]; }
-        out[4] = lo; out[5] = hi;
+        out[4] = nBlocks ? lo : 0.0;
+        out[5] = hi;
     }
 
-    __global__ void __launch_bounds__(kBlock) kStatsClear(uint32_t* __restrict__ hist)
+    __global__ void __launch_bounds__(kBlock) kStatsClear(uint4* __restrict__ hist)
     {
-        hist[blockIdx.x * kBlock + threadIdx.x] = 0u;
+        hist[blockIdx.x * kBlock + threadIdx.x] = make_uint4(0u, 0u, 0u, 0u);
     }
 
     static inline uint32_t blocksN(uint64_t n) { return static_cast<uint32_t>((n + kBlock - 1) / kBlock); }
 
-    // hist: kHistBins words (cleared by a kernel, not a memset node, so the sequence can be
-    // captured); out4: min, max, p99, sum
-    void launchStatsCounts(hipStream_t s, const uint16_t* c16, const uint32_t* c32, uint32_t mask, uint32_t n,
-                           uint32_t* hist, uint64_t* out4)
+    // hist: kRelations x kHistBins words (cleared by a kernel, not a memset node, so the sequence can be
+    // captured); partial: 6 doubles per block of nF; counts: per relation min, max, p99, sum; fluid: sums
+    // of raw, positive, absolute error and |v|, min and max |v|
+    void launchStats(hipStream_t s, const uint16_t* const (&c16)[3], const uint32_t* const (&c32)[3], uint32_t nF, uint32_t nR,
+                     const float4* vel, uint32_t off, float rho0, uint32_t* hist, double* partial, uint64_t* counts, double* fluid)
     {
-        kStatsClear<<<kHistBins / kBlock, kBlock, 0, s>>>(hist);
-        if (n) { kStatsHist<<<blocksN(n), kBlock, 0, s>>>(c16, c32, mask, n, hist); }
-        kStatsHistScan<<<1, kBlock, 0, s>>>(hist, n, out4);
-    }
-
-    // partial: 6 doubles per block of n; out6: sums of raw, positive, absolute error and |v|, min and max |v|
-    void launchStatsFluid(hipStream_t s, const float4* vel, uint32_t off, uint32_t n, float rho0, double* partial, double* out6)
-    {
-        if (n) { kStatsFluid<<<blocksN(n), kBlock, 0, s>>>(vel, off, n, rho0, partial); }
-        kStatsFluidSum<<<1, kBlock, 0, s>>>(partial, blocksN(n), out6);
+        StatsCounts c{ { c16[0], c16[1], c16[2] }, { c32[0], c32[1], c32[2] }, nF, nR };
+        kStatsClear<<<kRelations * kHistBins / (4u * kBlock), kBlock, 0, s>>>(reinterpret_cast<uint4*>(hist));
+        const uint32_t n = nF > nR ? nF : nR;
+        if (n) { kStatsHist<<<min(256u, blocksN(n)), kBlock, 0, s>>>(c, hist); }
+        if (nF) { kStatsFluid<<<blocksN(nF), kBlock, 0, s>>>(vel, off, nF, rho0, partial); }
+        kStatsScan<<<kRelations + 1u, kScanThreads, 0, s>>>(c, hist, partial, blocksN(nF), counts, fluid);
     }
 
     // --- the statistics scratch of the allocation-free entry point (tsp_get_statistics_noalloc):
     //     one static array per GPU, for callers that cannot allocate device memory. Layout: the
-    //     count histogram, the relations' (min, max, p99, sum), the fluid sums, then 6 FP64 block
+    //     count histograms, the relations' (min, max, p99, sum), the fluid sums, then 6 FP64 block
     //     partials per 256 fluid particles of a scene of at most kStatsMaxFluid particles.
     //     Every call on one GPU shares that GPU's array: calls that overlap on one GPU (contexts
     //     on different streams) race, and each call leaves its values in it. ---
     constexpr uint32_t kStatsMaxFluid = 1u << 24;
     constexpr size_t kStatsHistOff = 0;
-    constexpr size_t kStatsCountsOff = kStatsHistOff + sizeof(uint32_t) * kHistBins;
+    constexpr size_t kStatsCountsOff = kStatsHistOff + sizeof(uint32_t) * kRelations * kHistBins;
     constexpr size_t kStatsFluidOff = kStatsCountsOff + 256;
     constexpr size_t kStatsPartialOff = kStatsFluidOff + 256;
     constexpr size_t kStatsScratchBytes = kStatsPartialOff + sizeof(double) * 6 * (kStatsMaxFluid / kBlock);

@@ -64,8 +64,8 @@ namespace tsp
     void launchRigidReduce(hipStream_t, const Dev&);
     void launchRigidPredict(hipStream_t, const Dev&);
     void launchRigidIntegrate(hipStream_t, const Dev&);
-    void launchStatsCounts(hipStream_t, const uint16_t*, const uint32_t*, uint32_t, uint32_t, uint32_t*, uint64_t*);
-    void launchStatsFluid(hipStream_t, const float4*, uint32_t, uint32_t, float, double*, double*);
+    void launchStats(hipStream_t, const uint16_t* const (&)[3], const uint32_t* const (&)[3], uint32_t, uint32_t, const float4*,
+                     uint32_t, float, uint32_t*, double*, uint64_t*, double*);
     hipError_t statsScratchInit(int);
     bool statsScratch(int, uint32_t**, uint64_t**, double**, double**, uint32_t*);
 }
@@ -1784,6 +1784,7 @@ struct tsp_ctx
     std::vector<void*> statAllocs;
     uint32_t* statHist = nullptr;
     uint64_t* statCounts = nullptr;   // 6 relations x (min, max, p99, sum)
+    static constexpr size_t kStatsFluidAt = 256;   // bytes from the counts to the fluid sums, as in the static scratch
     double* statFluid = nullptr;      // sums of raw, positive, absolute error and |v|, min and max |v|
     double* statPartial = nullptr;
     uint64_t statPartialCap = 0;
@@ -1814,25 +1815,22 @@ struct tsp_ctx
         {
             sync();
             releaseList(statAllocs);
-            statHist = this->statHist = alloc<uint32_t>(65536, statAllocs);
-            statCounts = this->statCounts = alloc<uint64_t>(24, statAllocs);
-            statFluid = this->statFluid = alloc<double>(6, statAllocs);
+            statHist = this->statHist = alloc<uint32_t>(6ull * 65536ull, statAllocs);
+            // the counts, and the fluid sums at kStatsFluidAt behind them (one copy reads both)
+            statCounts = this->statCounts = alloc<uint64_t>(2ull * kStatsFluidAt / sizeof(uint64_t), statAllocs);
+            statFluid = this->statFluid = reinterpret_cast<double*>(statCounts + kStatsFluidAt / sizeof(uint64_t));
             statPartialCap = std::max<uint64_t>(nb, 1024);
             statPartial = this->statPartial = alloc<double>(6 * statPartialCap, statAllocs);
         }
         const uint16_t* c16[3] = { d.cnt[REL_FF] + h.offF, d.cnt[REL_FB] + h.offF, d.cnt[REL_FR] + h.offF };
-        for (int r = 0; r < 3; r++)
-        {
-            launchStatsCounts(stream, c16[r], nullptr, 0xffffu, h.nF, statHist, statCounts + 4 * r);
-        }
         const uint32_t* c32[3] = { d.rfCnt + h.offR, d.rbCnt + h.offR, d.rrCnt + h.offR };
-        for (int r = 0; r < 3; r++) { launchStatsCounts(stream, nullptr, c32[r], 0u, h.nR, statHist, statCounts + 4 * (3 + r)); }
-        launchStatsFluid(stream, d.vel, h.offF, h.nF, h.params.rest_density, statPartial, statFluid);
-        uint64_t cnt[24];
-        double fl[6];
-        hipCheck(hipMemcpyAsync(cnt, statCounts, sizeof(cnt), hipMemcpyDeviceToHost, stream), "D2H");
-        hipCheck(hipMemcpyAsync(fl, statFluid, sizeof(fl), hipMemcpyDeviceToHost, stream), "D2H");
+        launchStats(stream, c16, c32, h.nF, h.nR, d.vel, h.offF, h.params.rest_density, statHist, statPartial, statCounts, statFluid);
+        uint64_t got[(kStatsFluidAt + 64) / sizeof(uint64_t)];
+        hipCheck(hipMemcpyAsync(got, statCounts, sizeof(got), hipMemcpyDeviceToHost, stream), "D2H");
         sync();
+        const uint64_t* cnt = got;
+        double fl[6];
+        std::memcpy(fl, got + kStatsFluidAt / sizeof(uint64_t), sizeof(fl));
         std::memset(out, 0, sizeof(*out));
         out->n_fluid = h.nF; out->n_boundary = h.nB; out->n_rigid = h.nR;
         out->solver_iters = h.nF ? h.last.iters : 0;
