@@ -218,7 +218,9 @@ int tsp_get_statistics(tsp_ctx *ctx, tsp_statistics *out);
 int tsp_get_statistics_noalloc(tsp_ctx *ctx, tsp_statistics *out);
 
 /* Device memory a context holds, by what it stores, in bytes (I_SimBackend::FillMemoryRecord,
-   core/backend_sim.h:239, with the buckets of eval/memory/categories.h:59-78). */
+   core/backend_sim.h:239, with the buckets of eval/memory/categories.h:59-78). Blocks of at most
+   2 GiB that a context keeps for its next layout after it replaced one are not counted; they go
+   when the device runs out of other memory and with the context. */
 typedef struct tsp_memory {
     uint64_t particles[3];      /* fluid, boundary, rigid particle (and body) arrays */
     uint64_t search[3];         /* sort keys and indices, cell tables: fluid, boundary, rigid */

@@ -17,6 +17,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <deque>
 #include <map>
 #include <unordered_map>
 #include <string>
@@ -25,6 +26,7 @@
 #include "scene_plan.h"
 #include "tsp_device.h"
 #include "tsp_hip.h"
+#include "tsp_transfer.h"
 
 namespace tsp
 {
@@ -67,6 +69,9 @@ namespace tsp
     void launchStats(hipStream_t, const uint16_t* const (&)[3], const uint32_t* const (&)[3], uint32_t, uint32_t, const float4*,
                      uint32_t, float, uint32_t*, double*, uint64_t*, double*);
     hipError_t statsScratchInit(int);
+    void launchTransfer(hipStream_t, bool, const XferBatch&, uint32_t*);
+    void launchLocalKeys(hipStream_t, const Dev&, const uint32_t*, uint32_t, uint32_t, uint64_t, uint64_t, uint64_t*);
+    void launchLocalOrder(hipStream_t, const uint32_t*, uint32_t, uint32_t, uint32_t*);
     bool statsScratch(int, uint32_t**, uint64_t**, double**, double**, uint32_t*);
 }
 
@@ -350,7 +355,10 @@ struct tsp_ctx
         releaseList(frameAllocs);
         releaseList(work);
         releaseList(arena);
+        dropSpare();
         if (hostBlock) { (void)hipHostFree(hostBlock); }
+        if (stage) { (void)hipHostFree(stage); }
+        for (hipEvent_t e : stageEv) { if (e) { (void)hipEventDestroy(e); } }
         if (forkEv) { (void)hipEventDestroy(forkEv); }
         if (joinEv) { (void)hipEventDestroy(joinEv); }
         if (side) { (void)hipStreamDestroy(side); }
@@ -359,18 +367,59 @@ struct tsp_ctx
 
     // device memory the context holds, by what it stores (tsp_memory)
     enum MemCat : uint8_t { MEM_PF, MEM_PB, MEM_PR, MEM_SF, MEM_SB, MEM_SR, MEM_LF, MEM_LR, MEM_MISC, kMemCats };
-    std::unordered_map<void*, std::pair<uint64_t, uint8_t>> allocated;
+    struct Held
+    {
+        uint64_t bytes;     // asked for
+        uint64_t size;      // of the block
+        uint8_t cat;
+    };
+    std::unordered_map<void*, Held> allocated;
     uint64_t memBytes[kMemCats] = {};
     uint64_t memTotal = 0, memPeak = 0;
+
+    // Released blocks wait here for the next layout, which mostly asks for the same sizes: a scene pulled
+    // anew freed and allocated 83 blocks, 9.4 of the 11.7 ms of a pull at 1M particles (hipFree unmaps).
+    // At most kSpareMost bytes stay (under 1% of the device); they go when the device has no other memory
+    // left, and with the context. Blocks come back in the order of the context's streams, whose work on
+    // them was waited for or precedes their next use.
+    static constexpr uint64_t kSpareMost = 2ull << 30;
+    std::multimap<uint64_t, void*> spare;
+    uint64_t spareBytes = 0;
+
+    void dropSpare()
+    {
+        for (const auto& s : spare) { (void)hipFree(s.second); }
+        spare.clear();
+        spareBytes = 0;
+    }
 
     template <typename T>
     T* alloc(size_t n, std::vector<void*>& list, MemCat cat = MEM_MISC)
     {
         void* p = nullptr;
         const uint64_t bytes = std::max<size_t>(n, 1) * sizeof(T);
-        hipCheck(hipMalloc(&p, bytes), "hipMalloc");
+        uint64_t size = bytes;
+        const auto it = spare.lower_bound(bytes);
+        if (it != spare.end() && it->first <= bytes + bytes / 8u + 256u)
+        {
+            size = it->first;
+            p = it->second;
+            spareBytes -= size;
+            spare.erase(it);
+        }
+        else
+        {
+            hipError_t e = hipMalloc(&p, bytes);
+            if (e == hipErrorOutOfMemory && !spare.empty())
+            {
+                (void)hipGetLastError();
+                dropSpare();
+                e = hipMalloc(&p, bytes);
+            }
+            hipCheck(e, "hipMalloc");
+        }
         list.push_back(p);
-        allocated[p] = { bytes, static_cast<uint8_t>(cat) };
+        allocated[p] = Held{ bytes, size, static_cast<uint8_t>(cat) };
         memBytes[cat] += bytes;
         memTotal += bytes;
         memPeak = std::max(memPeak, memTotal);
@@ -382,13 +431,13 @@ struct tsp_ctx
         for (void* p : list)
         {
             const auto it = allocated.find(p);
-            if (it != allocated.end())
-            {
-                memBytes[it->second.second] -= it->second.first;
-                memTotal -= it->second.first;
-                allocated.erase(it);
-            }
-            (void)hipFree(p);
+            const Held h = it->second;
+            memBytes[h.cat] -= h.bytes;
+            memTotal -= h.bytes;
+            allocated.erase(it);
+            if (spareBytes + h.size > kSpareMost) { (void)hipFree(p); continue; }
+            spare.emplace(h.size, p);
+            spareBytes += h.size;
         }
         list.clear();
     }
@@ -414,6 +463,97 @@ struct tsp_ctx
     void zero(void* dst, size_t bytes)
     {
         if (bytes) { hipCheck(hipMemsetAsync(dst, 0, bytes, stream), "hipMemsetAsync"); }
+    }
+
+    // --- fields between the caller and the device, through pinned memory (kernels_transfer.hip) ---
+    // two buffers of up to kStageMost bytes (one when everything fits in it), kept with the context
+    static constexpr size_t kStageMost = 8u << 20;
+    char* stage = nullptr;
+    size_t stageBytes = 0;            // of one buffer
+    int stageBufs = 0;
+    hipEvent_t stageEv[2] = { nullptr, nullptr };
+
+    void ensureStage(size_t bytes, int bufs)
+    {
+        if (stage && stageBytes >= bytes && stageBufs >= bufs) { return; }
+        bytes = std::max(bytes, stageBytes);
+        bufs = std::max(bufs, stageBufs);
+        if (stage) { sync(); (void)hipHostFree(stage); stage = nullptr; stageBytes = 0; stageBufs = 0; }
+        for (hipEvent_t& e : stageEv)
+        {
+            if (!e) { hipCheck(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate"); }
+        }
+        hipCheck(hipHostMalloc(reinterpret_cast<void**>(&stage), bytes * static_cast<size_t>(bufs)), "hipHostMalloc");
+        stageBytes = bytes;
+        stageBufs = bufs;
+    }
+
+    // moves every field out to the caller, or in; returns when the caller's memory is no longer needed
+    // and, out, is filled (the stream's earlier work is waited for; in, later work on it sees the data).
+    // While one buffer is on the device the other is copied on the host.
+    void transfer(const std::vector<XferField>& fields, bool out)
+    {
+        uint64_t total = 0;
+        for (const XferField& f : fields) { total += (f.n + 3ull) / 4ull * 16ull; }
+        if (!total) { return; }
+        const bool one = total <= kStageMost;
+        ensureStage(one ? std::max<size_t>(static_cast<size_t>(total), 64u << 10) : kStageMost, one ? 1 : 2);
+        const uint64_t words = stageBytes / 4u;
+        std::vector<StageCopy> copies[2];
+        bool busy[2] = { false, false };
+        const auto finish = [&](int k)
+        {
+            if (!busy[k]) { return; }
+            hipCheck(hipEventSynchronize(stageEv[k]), "hipEventSynchronize");
+            if (out) { copyStage(copies[k], stage + stageBytes * static_cast<size_t>(k), true); }
+            busy[k] = false;
+        };
+        size_t fi = 0;
+        uint64_t done = 0;            // words of fields[fi] already moved
+        int k = 0;
+        while (fi < fields.size())
+        {
+            finish(k);
+            copies[k].clear();
+            XferBatch b{};
+            uint64_t at = 0;
+            while (fi < fields.size() && b.count < kXferPieces && at < words)
+            {
+                const XferField& f = fields[fi];
+                const uint64_t n = std::min(f.n - done, words - at);
+                if (n)
+                {
+                    const uint32_t q = b.count++;
+                    b.piece[q] = XferPiece{ f.dev, f.stride, f.comps, static_cast<uint32_t>(done), static_cast<uint32_t>(n),
+                                            static_cast<uint32_t>(at), 0u };
+                    b.block[q + 1u] = b.block[q] + static_cast<uint32_t>((n + kXferBlock - 1u) / kXferBlock);
+                    copies[k].push_back(StageCopy{ f.host + done * 4u, static_cast<size_t>(at) * 4u, static_cast<size_t>(n) * 4u });
+                    at += (n + 3ull) & ~3ull;
+                    done += n;
+                }
+                if (done == f.n) { fi++; done = 0; }
+            }
+            char* s = stage + stageBytes * static_cast<size_t>(k);
+            if (!out) { copyStage(copies[k], s, false); }
+            launchTransfer(stream, out, b, reinterpret_cast<uint32_t*>(s));
+            hipCheck(hipGetLastError(), "transfer launch");
+            hipCheck(hipEventRecord(stageEv[k], stream), "hipEventRecord");
+            busy[k] = true;
+            if (stageBufs > 1) { k ^= 1; }
+        }
+        finish(k);
+        finish(k ^ 1);
+    }
+
+    // n elements of a contiguous array, or the first comps words of n records of `stride` bytes
+    template <typename T>
+    static void addField(std::vector<XferField>& fields, const void* host, const T* dev, uint64_t n, uint32_t stride = 0,
+                         uint32_t comps = 1)
+    {
+        if (!host || !n) { return; }
+        const uint64_t wordsEach = stride ? comps : sizeof(T) / 4ull;
+        fields.push_back(XferField{ static_cast<char*>(const_cast<void*>(host)), reinterpret_cast<char*>(const_cast<T*>(dev)),
+                                    stride ? stride : 4u, comps, n * wordsEach });
     }
 
     uint32_t nScenes() const { return static_cast<uint32_t>(scenes.size()); }
@@ -462,6 +602,23 @@ struct tsp_ctx
         }
         d.rfCap = rfCap;
         d.rfIdx = alloc<uint32_t>(rfCap, poolAllocs, MEM_LR);
+    }
+
+    // the fluid fields of a scene in the records of n (missing fields are left out)
+    static void fluidFields(std::vector<XferField>& fields, const Dev& n, const SceneHost& h, float* const* f)
+    {
+        const int comp[4][4] = { { TSP_F_X, TSP_F_Y, TSP_F_Z, TSP_F_PRESSURE }, { TSP_F_VX, TSP_F_VY, TSP_F_VZ, TSP_F_DENSITY },
+                                 { TSP_F_VPX, TSP_F_VPY, TSP_F_VPZ, -1 }, { TSP_F_APX, TSP_F_APY, TSP_F_APZ, -1 } };
+        const float4* rec[4] = { n.pos, n.vel, n.vp, n.ap };
+        for (int r = 0; r < 4; r++)
+        {
+            for (int c = 0; c < 4; c++)
+            {
+                if (comp[r][c] >= 0) { addField(fields, f[comp[r][c]], &rec[r][h.offF].x + c, h.nF, sizeof(float4)); }
+            }
+        }
+        addField(fields, f[TSP_F_SOURCE], n.source + h.offF, h.nF);
+        addField(fields, f[TSP_F_DIAG], n.diag + h.offF, h.nF);
     }
 
     // --- a planned scene's fluid and boundary generated in the new arena (n) at h's offsets ---
@@ -644,6 +801,8 @@ struct tsp_ctx
             n.rfx = alloc<float>(nR, A, MEM_PR); n.rfy = alloc<float>(nR, A, MEM_PR); n.rfz = alloc<float>(nR, A, MEM_PR);
             n.rbody = alloc<uint32_t>(nR, A, MEM_PR);
             nidR = alloc<uint64_t>(nR, A, MEM_PR);
+            zero(n.rxrel, sizeof(float) * nR); zero(n.ryrel, sizeof(float) * nR); zero(n.rzrel, sizeof(float) * nR);
+            zero(n.rpos, sizeof(float4) * nR); zero(n.rvel, sizeof(float4) * nR); zero(n.rvp, sizeof(float4) * nR);
             n.rb = alloc<float>(static_cast<size_t>(TSP_RB_COUNT) * nRB1, A, MEM_PR);
             n.rbPred = alloc<float>(9 * nRB1, A, MEM_PR);
             n.rbForce = alloc<float>(6 * nRB1, A, MEM_PR);
@@ -653,15 +812,22 @@ struct tsp_ctx
             n.byBodyIdx = alloc<uint32_t>(nR, A, MEM_PR);
             n.blockScene = alloc<uint32_t>(nF / kBlock, A, MEM_PF);
             n.bodyScene = alloc<uint32_t>(nRB, A, MEM_PR);
-            n.sceneB = alloc<uint16_t>(nB, A, MEM_PB);
+            n.sceneB = alloc<uint16_t>(nB + 1ull, A, MEM_PB);   // (moved in whole words)
 
-            const auto field = [](const float* f, uint32_t i, float dflt) { return f ? f[i] : dflt; };
-            std::vector<uint64_t> seq;
-            const auto ids = [&](const uint64_t* given, uint32_t cnt) -> const uint64_t* {
-                if (given) { return given; }
-                seq.resize(cnt);
-                for (uint32_t i = 0; i < cnt; i++) { seq[i] = i; }
-                return seq.data();
+            // the new scenes' fields, moved in one transfer; values the views leave out live here meanwhile
+            std::vector<XferField> fields;
+            std::deque<std::vector<float>> given;
+            std::deque<std::vector<uint64_t>> givenIds;
+            const auto ids = [&](const uint64_t* have, uint32_t cnt) -> const uint64_t* {
+                if (have || !cnt) { return have; }
+                givenIds.emplace_back(cnt);
+                for (uint32_t i = 0; i < cnt; i++) { givenIds.back()[i] = i; }
+                return givenIds.back().data();
+            };
+            const auto orConst = [&](const float* have, uint32_t cnt, float value) -> const float* {
+                if (have || !cnt) { return have; }
+                given.emplace_back(cnt, value);
+                return given.back().data();
             };
             for (size_t q = 0; q < src.size(); q++)
             {
@@ -702,86 +868,42 @@ struct tsp_ctx
                 }
                 const tsp_state_view* s = src[q].view;
                 if (src[q].plan) { buildOnDevice(n, h, *src[q].plan, nidB); }
-                // fluid: the SoA fields of the view packed into the float4 records
+                // fluid (missing fields stay zero) and boundary (ensureBoundaryCoefficientsPresent
+                // defaults: psi = massB, V = psi / rho0)
                 if (!src[q].plan)
                 {
-                    std::vector<float4> r[4];
-                    for (auto& v : r) { v.resize(h.nF); }
-                    std::vector<float> src1(h.nF), diag1(h.nF);
-                    float* const* f = s->fluid;
-                    for (uint32_t i = 0; i < h.nF; i++)
-                    {
-                        r[0][i] = make_float4(field(f[TSP_F_X], i, 0), field(f[TSP_F_Y], i, 0), field(f[TSP_F_Z], i, 0),
-                                              field(f[TSP_F_PRESSURE], i, 0));
-                        r[1][i] = make_float4(field(f[TSP_F_VX], i, 0), field(f[TSP_F_VY], i, 0), field(f[TSP_F_VZ], i, 0),
-                                              field(f[TSP_F_DENSITY], i, 0));
-                        r[2][i] = make_float4(field(f[TSP_F_VPX], i, 0), field(f[TSP_F_VPY], i, 0), field(f[TSP_F_VPZ], i, 0), 0.0f);
-                        r[3][i] = make_float4(field(f[TSP_F_APX], i, 0), field(f[TSP_F_APY], i, 0), field(f[TSP_F_APZ], i, 0), 0.0f);
-                        src1[i] = field(f[TSP_F_SOURCE], i, 0);
-                        diag1[i] = field(f[TSP_F_DIAG], i, 0);
-                    }
-                    float4* dst[4] = { n.pos, n.vel, n.vp, n.ap };
-                    for (int k = 0; k < 4; k++) { h2d(dst[k] + h.offF, r[k].data(), sizeof(float4) * h.nF); }
-                    h2d(n.source + h.offF, src1.data(), sizeof(float) * h.nF);
-                    h2d(n.diag + h.offF, diag1.data(), sizeof(float) * h.nF);
-                    h2d(n.id + h.offF, ids(s->fluid_id, h.nF), sizeof(uint64_t) * h.nF);
-                }
-                // boundary (ensureBoundaryCoefficientsPresent defaults: psi = massB, V = psi / rho0)
-                if (!src[q].plan)
-                {
+                    const Dev& dn = n;
+                    fluidFields(fields, dn, h, s->fluid);
+                    addField(fields, ids(s->fluid_id, h.nF), n.id + h.offF, h.nF);
                     const float hh = h.params.particle_size, rho0 = h.params.rest_density;
                     const float massB = rho0 * hh * hh * hh;
                     const float volB = rho0 > 0.0f ? massB / rho0 : 0.0f;
-                    std::vector<float4> r(h.nB);
-                    std::vector<float> vol(h.nB);
-                    float* const* f = s->boundary;
-                    for (uint32_t i = 0; i < h.nB; i++)
-                    {
-                        r[i] = make_float4(field(f[TSP_B_X], i, 0), field(f[TSP_B_Y], i, 0), field(f[TSP_B_Z], i, 0),
-                                           field(f[TSP_B_PSI], i, massB));
-                        vol[i] = field(f[TSP_B_VOL], i, volB);
-                    }
-                    h2d(n.bpos + h.offB, r.data(), sizeof(float4) * h.nB);
-                    h2d(n.bvol + h.offB, vol.data(), sizeof(float) * h.nB);
-                    h2d(nidB + h.offB, ids(s->boundary_id, h.nB), sizeof(uint64_t) * h.nB);
+                    const float* xyz[3];
+                    for (int a = 0; a < 3; a++) { xyz[a] = orConst(s->boundary[TSP_B_X + a], h.nB, 0.0f); }
+                    for (int a = 0; a < 3; a++) { addField(fields, xyz[a], &n.bpos[h.offB].x + a, h.nB, sizeof(float4)); }
+                    addField(fields, orConst(s->boundary[TSP_B_PSI], h.nB, massB), &n.bpos[h.offB].w, h.nB, sizeof(float4));
+                    addField(fields, orConst(s->boundary[TSP_B_VOL], h.nB, volB), n.bvol + h.offB, h.nB);
+                    addField(fields, ids(s->boundary_id, h.nB), nidB + h.offB, h.nB);
                 }
                 // rigid particles: body-frame offsets; the world records follow from the body state
-                {
-                    float* const* f = s->rigid;
-                    std::vector<float> rel[3];
-                    std::vector<float4> wp(h.nR), wv(h.nR), wvp(h.nR);
-                    for (int a = 0; a < 3; a++) { rel[a].resize(h.nR); }
-                    for (uint32_t i = 0; i < h.nR; i++)
-                    {
-                        rel[0][i] = field(f[TSP_R_XREL], i, 0);
-                        rel[1][i] = field(f[TSP_R_YREL], i, 0);
-                        rel[2][i] = field(f[TSP_R_ZREL], i, 0);
-                        wp[i] = make_float4(0.0f, 0.0f, 0.0f, field(f[TSP_R_PSI], i, 0));
-                        wv[i] = make_float4(0.0f, 0.0f, 0.0f, field(f[TSP_R_VOL], i, 0));
-                        wvp[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                    }
-                    h2d(n.rxrel + h.offR, rel[0].data(), sizeof(float) * h.nR);
-                    h2d(n.ryrel + h.offR, rel[1].data(), sizeof(float) * h.nR);
-                    h2d(n.rzrel + h.offR, rel[2].data(), sizeof(float) * h.nR);
-                    h2d(n.rpos + h.offR, wp.data(), sizeof(float4) * h.nR);
-                    h2d(n.rvel + h.offR, wv.data(), sizeof(float4) * h.nR);
-                    h2d(n.rvp + h.offR, wvp.data(), sizeof(float4) * h.nR);
-                    h2d(nidR + h.offR, ids(s->rigid_id, h.nR), sizeof(uint64_t) * h.nR);
-                }
+                addField(fields, s->rigid[TSP_R_XREL], n.rxrel + h.offR, h.nR);
+                addField(fields, s->rigid[TSP_R_YREL], n.ryrel + h.offR, h.nR);
+                addField(fields, s->rigid[TSP_R_ZREL], n.rzrel + h.offR, h.nR);
+                addField(fields, s->rigid[TSP_R_PSI], &n.rpos[h.offR].w, h.nR, sizeof(float4));
+                addField(fields, s->rigid[TSP_R_VOL], &n.rvel[h.offR].w, h.nR, sizeof(float4));
+                addField(fields, ids(s->rigid_id, h.nR), nidR + h.offR, h.nR);
                 // bodies (a missing orientation field is the identity)
                 for (size_t f = 0; f < TSP_RB_COUNT; f++)
                 {
-                    std::vector<float> v(h.nRB);
                     const bool diagonal = f == TSP_RB_A00 || f == TSP_RB_A11 || f == TSP_RB_A22;
-                    for (uint32_t b = 0; b < h.nRB; b++) { v[b] = s->body[f] ? s->body[f][b] : (diagonal ? 1.0f : 0.0f); }
-                    h2d(n.rb + f * nRB1 + h.offRB, v.data(), sizeof(float) * h.nRB);
+                    addField(fields, orConst(s->body[f], h.nRB, diagonal ? 1.0f : 0.0f), n.rb + f * nRB1 + h.offRB, h.nRB);
                 }
             }
             // tables rebuilt from the host records: body of each rigid particle, the particles of
             // each body (BuildRigidParticleIndicesByBody, sync/state_sim.h:609-631), scene maps
             std::vector<uint32_t> rbody(nR), off(nRB + 1ull, 0), idx(nR);
             std::vector<uint32_t> blockScene(nF / kBlock), bodyScene(nRB);
-            std::vector<uint16_t> sceneB(nB);
+            std::vector<uint16_t> sceneB(nB + 1ull);
             for (uint32_t s = 0; s < S; s++)
             {
                 const SceneHost& h = ns[s];
@@ -794,12 +916,13 @@ struct tsp_ctx
             for (uint32_t b = 0; b < nRB; b++) { off[b + 1] += off[b]; }
             std::vector<uint32_t> w(off);
             for (uint32_t i = 0; i < nR; i++) { idx[w[rbody[i]]++] = i; }
-            h2d(n.rbody, rbody.data(), sizeof(uint32_t) * nR);
-            h2d(n.byBodyOff, off.data(), sizeof(uint32_t) * (nRB + 1ull));
-            h2d(n.byBodyIdx, idx.data(), sizeof(uint32_t) * nR);
-            h2d(n.blockScene, blockScene.data(), sizeof(uint32_t) * blockScene.size());
-            h2d(n.bodyScene, bodyScene.data(), sizeof(uint32_t) * nRB);
-            h2d(n.sceneB, sceneB.data(), sizeof(uint16_t) * nB);
+            addField(fields, rbody.data(), n.rbody, nR);
+            addField(fields, off.data(), n.byBodyOff, nRB + 1ull);
+            addField(fields, idx.data(), n.byBodyIdx, nR);
+            addField(fields, blockScene.data(), n.blockScene, blockScene.size());
+            addField(fields, bodyScene.data(), n.bodyScene, nRB);
+            if (nB) { addField(fields, sceneB.data(), reinterpret_cast<uint32_t*>(n.sceneB), (nB + 1ull) / 2ull); }
+            transfer(fields, false);
             sync();
         }
         catch (...)
@@ -1670,72 +1793,23 @@ struct tsp_ctx
             throw Error{ TSP_ERR_INVALID, "state view counts differ from the backend" };
         }
         const size_t nRB1 = std::max<uint32_t>(d.nRB, 1);
+        std::vector<XferField> fields;
+        fluidFields(fields, d, h, s->fluid);
+        addField(fields, s->fluid_id, d.id + h.offF, h.nF);
+        for (int a = 0; a < 3; a++) { addField(fields, s->boundary[TSP_B_X + a], &d.bpos[h.offB].x + a, h.nB, sizeof(float4)); }
+        addField(fields, s->boundary[TSP_B_PSI], &d.bpos[h.offB].w, h.nB, sizeof(float4));
+        addField(fields, s->boundary[TSP_B_VOL], d.bvol + h.offB, h.nB);
+        addField(fields, s->boundary_id, idB + h.offB, h.nB);
+        addField(fields, s->rigid[TSP_R_XREL], d.rxrel + h.offR, h.nR);
+        addField(fields, s->rigid[TSP_R_YREL], d.ryrel + h.offR, h.nR);
+        addField(fields, s->rigid[TSP_R_ZREL], d.rzrel + h.offR, h.nR);
+        addField(fields, s->rigid[TSP_R_PSI], &d.rpos[h.offR].w, h.nR, sizeof(float4));
+        addField(fields, s->rigid[TSP_R_VOL], &d.rvel[h.offR].w, h.nR, sizeof(float4));
+        addField(fields, s->rigid_id, idR + h.offR, h.nR);
+        for (size_t f = 0; f < TSP_RB_COUNT; f++) { addField(fields, s->body[f], d.rb + f * nRB1 + h.offRB, h.nRB); }
+        transfer(fields, true);
         sync();
-        const auto d2h = [&](void* dst, const void* src, size_t bytes) {
-            if (dst && bytes) { hipCheck(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream), "D2H"); }
-        };
-        // fluid records unpacked into the SoA fields of the view
-        {
-            const uint32_t n = h.nF;
-            std::vector<float4> q[4];
-            const float4* srcs[4] = { d.pos, d.vel, d.vp, d.ap };
-            for (int r = 0; r < 4; r++)
-            {
-                q[r].resize(n);
-                d2h(q[r].data(), srcs[r] + h.offF, sizeof(float4) * n);
-            }
-            sync();
-            float* const* f = s->fluid;
-            const int comp[4][4] = { { TSP_F_X, TSP_F_Y, TSP_F_Z, TSP_F_PRESSURE }, { TSP_F_VX, TSP_F_VY, TSP_F_VZ, TSP_F_DENSITY },
-                                     { TSP_F_VPX, TSP_F_VPY, TSP_F_VPZ, -1 }, { TSP_F_APX, TSP_F_APY, TSP_F_APZ, -1 } };
-            for (int r = 0; r < 4; r++)
-            {
-                for (int c = 0; c < 4; c++)
-                {
-                    float* out = comp[r][c] >= 0 ? f[comp[r][c]] : nullptr;
-                    if (!out) { continue; }
-                    for (uint32_t i = 0; i < n; i++) { out[i] = reinterpret_cast<const float*>(&q[r][i])[c]; }
-                }
-            }
-            d2h(f[TSP_F_SOURCE], d.source + h.offF, sizeof(float) * n);
-            d2h(f[TSP_F_DIAG], d.diag + h.offF, sizeof(float) * n);
-        }
-        d2h(s->fluid_id, d.id + h.offF, sizeof(uint64_t) * h.nF);
-        {
-            const uint32_t n = h.nB;
-            std::vector<float4> q(n);
-            d2h(q.data(), d.bpos + h.offB, sizeof(float4) * n);
-            sync();
-            float* const* f = s->boundary;
-            const int comp[4] = { TSP_B_X, TSP_B_Y, TSP_B_Z, TSP_B_PSI };
-            for (int c = 0; c < 4; c++)
-            {
-                if (!f[comp[c]]) { continue; }
-                for (uint32_t i = 0; i < n; i++) { f[comp[c]][i] = reinterpret_cast<const float*>(&q[i])[c]; }
-            }
-            d2h(f[TSP_B_VOL], d.bvol + h.offB, sizeof(float) * n);
-        }
-        d2h(s->boundary_id, idB + h.offB, sizeof(uint64_t) * h.nB);
-        {
-            const uint32_t n = h.nR;
-            float* const* f = s->rigid;
-            d2h(f[TSP_R_XREL], d.rxrel + h.offR, sizeof(float) * n);
-            d2h(f[TSP_R_YREL], d.ryrel + h.offR, sizeof(float) * n);
-            d2h(f[TSP_R_ZREL], d.rzrel + h.offR, sizeof(float) * n);
-            std::vector<float4> wp(n), wv(n);
-            d2h(wp.data(), d.rpos + h.offR, sizeof(float4) * n);
-            d2h(wv.data(), d.rvel + h.offR, sizeof(float4) * n);
-            sync();
-            for (uint32_t i = 0; i < n; i++)
-            {
-                if (f[TSP_R_PSI]) { f[TSP_R_PSI][i] = wp[i].w; }
-                if (f[TSP_R_VOL]) { f[TSP_R_VOL][i] = wv[i].w; }
-                if (s->rigid_body) { s->rigid_body[i] = h.rbodyLocal[i]; }
-            }
-        }
-        d2h(s->rigid_id, idR + h.offR, sizeof(uint64_t) * h.nR);
-        for (size_t f = 0; f < TSP_RB_COUNT; f++) { d2h(s->body[f], d.rb + f * nRB1 + h.offRB, sizeof(float) * h.nRB); }
-        sync();
+        if (s->rigid_body) { for (uint32_t i = 0; i < h.nR; i++) { s->rigid_body[i] = h.rbodyLocal[i]; } }
         for (uint32_t b = 0; b < h.nRB; b++)
         {
             if (s->body_id) { s->body_id[b] = h.bodyId[b]; }
@@ -1886,46 +1960,22 @@ struct tsp_ctx
         if (scanFailed) { throw Error{ TSP_ERR_STATE, "a one-pass scan gave up waiting for a predecessor tile" }; }
         v->n_fluid = count;
         if (count > v->cap_fluid) { throw Error{ TSP_ERR_CAPACITY, "the fluid export arrays hold fewer particles than the surface set" }; }
-        if (count && v->fluid_xyz) { d2h(v->fluid_xyz, expXyz, sizeof(float) * 3ull * count); }
-        if (count && v->fluid_vel_mag) { d2h(v->fluid_vel_mag, expSpeed, sizeof(float) * count); }
-        if (v->boundary_xyz && h.nB)
+        std::vector<XferField> fields;
+        addField(fields, v->fluid_xyz, expXyz, 3ull * count);
+        addField(fields, v->fluid_vel_mag, expSpeed, count);
+        std::vector<uint64_t> ids(v->boundary_xyz && v->boundary_is_mesh ? h.nB : 0);
+        if (v->boundary_xyz)
         {
-            std::vector<float4> b(h.nB);
-            d2h(b.data(), d.bpos + h.offB, sizeof(float4) * h.nB);
-            for (uint32_t i = 0; i < h.nB; i++)
-            {
-                v->boundary_xyz[3ull * i] = b[i].x; v->boundary_xyz[3ull * i + 1] = b[i].y; v->boundary_xyz[3ull * i + 2] = b[i].z;
-            }
-            if (v->boundary_vol) { d2h(v->boundary_vol, d.bvol + h.offB, sizeof(float) * h.nB); }
-            if (v->boundary_is_mesh)
-            {
-                std::vector<uint64_t> ids(h.nB);
-                d2h(ids.data(), idB + h.offB, sizeof(uint64_t) * h.nB);
-                for (uint32_t i = 0; i < h.nB; i++) { v->boundary_is_mesh[i] = ids[i] >= meshIdBegin ? 1u : 0u; }
-            }
+            addField(fields, v->boundary_xyz, d.bpos + h.offB, h.nB, sizeof(float4), 3);
+            addField(fields, v->boundary_vol, d.bvol + h.offB, h.nB);
+            addField(fields, ids.data(), idB + h.offB, ids.size());
         }
-        if (h.nR)
-        {
-            std::vector<float4> r(h.nR);
-            if (v->rigid_xyz)
-            {
-                d2h(r.data(), d.rpos + h.offR, sizeof(float4) * h.nR);
-                for (uint32_t i = 0; i < h.nR; i++)
-                {
-                    v->rigid_xyz[3ull * i] = r[i].x; v->rigid_xyz[3ull * i + 1] = r[i].y; v->rigid_xyz[3ull * i + 2] = r[i].z;
-                }
-            }
-            if (v->rigid_vol)
-            {
-                d2h(r.data(), d.rvel + h.offR, sizeof(float4) * h.nR);
-                for (uint32_t i = 0; i < h.nR; i++) { v->rigid_vol[i] = r[i].w; }
-            }
-            if (v->rigid_body)
-            {
-                d2h(v->rigid_body, d.rbody + h.offR, sizeof(uint32_t) * h.nR);
-                for (uint32_t i = 0; i < h.nR; i++) { v->rigid_body[i] -= h.offRB; }
-            }
-        }
+        addField(fields, v->rigid_xyz, d.rpos + h.offR, h.nR, sizeof(float4), 3);
+        if (h.nR) { addField(fields, v->rigid_vol, &d.rvel[h.offR].w, h.nR, sizeof(float4)); }
+        addField(fields, v->rigid_body, d.rbody + h.offR, h.nR);
+        transfer(fields, true);
+        for (size_t i = 0; i < ids.size(); i++) { v->boundary_is_mesh[i] = ids[i] >= meshIdBegin ? 1u : 0u; }
+        if (v->rigid_body) { for (uint32_t i = 0; i < h.nR; i++) { v->rigid_body[i] -= h.offRB; } }
     }
 
     // one relayout: the listed scenes leave, new scenes join at the end
@@ -2316,42 +2366,32 @@ int tsp_get_sort(tsp_ctx* ctx, uint32_t* orderF, uint64_t* keysF, uint32_t* orde
         const Dev& d = ctx->d;
         const SceneHost& h = ctx->scenes[0];
         ctx->sync();
-        // scene-local Morton ids; out-of-frame ids as all ones
-        // key i of a key array (u32, or u64 in two words)
-        const auto widen = [&](uint64_t* dst, const uint32_t* src, uint32_t off, uint32_t n) {
-            std::vector<uint64_t> k(n);
-            if (n && d.key64)
-            {
-                hipCheck(hipMemcpy(k.data(), reinterpret_cast<const uint64_t*>(src) + off, sizeof(uint64_t) * n,
-                                   hipMemcpyDeviceToHost), "D2H");
-            }
-            else if (n)
-            {
-                std::vector<uint32_t> k32(n);
-                hipCheck(hipMemcpy(k32.data(), src + off, sizeof(uint32_t) * n, hipMemcpyDeviceToHost), "D2H");
-                for (uint32_t i = 0; i < n; i++) { k[i] = k32[i]; }
-            }
-            for (uint32_t i = 0; i < n; i++) { dst[i] = k[i] >= h.frame.emptyKey ? ~0ull : k[i] - h.frame.keyBase; }
-        };
+        // scene-local Morton ids (out-of-frame ids as all ones) and order, laid out for the copy in
+        // buffers that are free between calls: the second buffers of the re-order
+        std::vector<XferField> fields;
+        const uint64_t base = h.frame.keyBase, empty = h.frame.emptyKey;
         if (orderF && h.nF)
         {
-            hipCheck(hipMemcpy(orderF, d.idxF + h.offF, sizeof(uint32_t) * h.nF, hipMemcpyDeviceToHost), "D2H");
-            for (uint32_t i = 0; i < h.nF; i++) { orderF[i] -= h.offF; }
+            uint32_t* o = reinterpret_cast<uint32_t*>(ctx->vel2);
+            launchLocalOrder(ctx->stream, d.idxF, h.offF, h.nF, o);
+            ctx->addField(fields, orderF, o, h.nF);
         }
-        if (keysF) { widen(keysF, d.keyF, h.offF, h.nF); }
+        if (keysF && h.nF)
+        {
+            uint64_t* k = reinterpret_cast<uint64_t*>(ctx->pos2);
+            launchLocalKeys(ctx->stream, d, d.keyF, h.offF, h.nF, base, empty, k);
+            ctx->addField(fields, keysF, k, h.nF);
+        }
         if ((orderB || keysB) && h.nB)
         {
             // the boundary order relative to the pulled order, from the ids (sequence ids on pull)
             launchKeys(ctx->stream, d, kPopB, d.bpos, d.nB, false, d.keyF2, d.idxF2);
-            ctx->sync();
-            if (keysB) { widen(keysB, d.keyF2, h.offB, h.nB); }
-            if (orderB)
-            {
-                std::vector<uint64_t> idb(h.nB);
-                hipCheck(hipMemcpy(idb.data(), ctx->idB + h.offB, sizeof(uint64_t) * h.nB, hipMemcpyDeviceToHost), "D2H");
-                for (uint32_t i = 0; i < h.nB; i++) { orderB[i] = static_cast<uint32_t>(idb[i]); }
-            }
+            uint64_t* k = reinterpret_cast<uint64_t*>(ctx->bpos2);
+            launchLocalKeys(ctx->stream, d, d.keyF2, h.offB, h.nB, base, empty, k);
+            ctx->addField(fields, keysB, k, h.nB);
+            ctx->addField(fields, orderB, ctx->idB + h.offB, h.nB, sizeof(uint64_t));
         }
+        ctx->transfer(fields, true);
         return TSP_OK;
     });
 }
