@@ -174,22 +174,21 @@ namespace tsp
     }
 
     bool launchRadixSort(hipStream_t, bool, uint32_t*, uint32_t*, uint32_t*, uint32_t*, uint32_t, uint32_t, uint32_t*, uint32_t*,
-                         uint32_t*, bool);
+                         bool, bool);
 
     void launchBuildFluid(hipStream_t s, const Dev& d, uint32_t off, uint32_t n, const BuildFluid& b)
     {
         if (n) { kBuildFluid<<<blocksN(n), kBlock, 0, s>>>(d, off, n, b); }
     }
 
-    // scratch: xyz 3n floats; key, idx, key2, idx2 n words each; hist 256 per 2048-key tile;
-    // tmp a zeroed scan state for the digit counts (its word 2 is set if a scan gave up)
+    // scratch: xyz 3n floats; key, idx, key2, idx2 n words each; sort a zeroed sort state (its spare
+    // word 3 is set if a look-back gave up)
     void launchBuildBoundary(hipStream_t s, const BuildBoundary& c, uint32_t n, float4* bpos, float* bvol, uint64_t* ids,
-                             float* xyz, uint32_t* key, uint32_t* idx, uint32_t* key2, uint32_t* idx2, uint32_t* hist,
-                             uint32_t* tmp)
+                             float* xyz, uint32_t* key, uint32_t* idx, uint32_t* key2, uint32_t* idx2, uint32_t* sort)
     {
         if (!n) { return; }
         kBuildBoundaryPos<<<blocksN(n), kBlock, 0, s>>>(c, n, xyz, ids, key, idx);
-        launchRadixSort(s, false, key, idx, key2, idx2, n, c.bits[0] + c.bits[1] + c.bits[2], hist, tmp, tmp + 2, true);
+        launchRadixSort(s, false, key, idx, key2, idx2, n, c.bits[0] + c.bits[1] + c.bits[2], sort, sort + 3, false, true);
         kBuildBoundaryCoeff<<<blocksN(n), kBlock, 0, s>>>(c, n, xyz, key, idx, bpos, bvol);
     }
 }

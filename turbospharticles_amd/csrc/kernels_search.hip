@@ -26,35 +26,103 @@ namespace tsp
 
     constexpr uint32_t kScanTile = 2048;
 
+    // exclusive scan over the lanes of a wave; sum: the wave's total in every lane
+    __device__ __forceinline__ uint32_t waveExclusiveScan(uint32_t v, uint32_t& sum)
+    {
+        const uint32_t lane = threadIdx.x & 63u;
+        uint32_t incl = v;
+        for (int o = 1; o < 64; o <<= 1)
+        {
+            const uint32_t u = static_cast<uint32_t>(__shfl_up(static_cast<int>(incl), o, 64));
+            if (lane >= static_cast<uint32_t>(o)) { incl += u; }
+        }
+        sum = static_cast<uint32_t>(__shfl(static_cast<int>(incl), 63, 64));
+        return incl - v;
+    }
+
+    // exclusive scan over the first kBlock threads of a block (the others pass and get anything)
     __device__ __forceinline__ uint32_t blockExclusiveScan(uint32_t v, uint32_t& total)
     {
-        __shared__ uint32_t s[kBlock];
-        s[threadIdx.x] = v;
+        __shared__ uint32_t tot[kBlock / 64];
+        uint32_t sum;
+        uint32_t r = waveExclusiveScan(v, sum);
+        const uint32_t wave = threadIdx.x >> 6;
+        if (wave < kBlock / 64 && (threadIdx.x & 63u) == 0u) { tot[wave] = sum; }
         __syncthreads();
-        for (uint32_t off = 1; off < kBlock; off <<= 1)
+        total = 0;
+        for (uint32_t w = 0; w < kBlock / 64; w++)
         {
-            const uint32_t a = threadIdx.x >= off ? s[threadIdx.x - off] : 0u;
-            __syncthreads();
-            s[threadIdx.x] += a;
-            __syncthreads();
+            if (w < wave) { r += tot[w]; }
+            total += tot[w];
         }
-        total = s[kBlock - 1];
-        const uint32_t r = s[threadIdx.x] - v;
-        __syncthreads();
         return r;
     }
 
-    // One-pass exclusive scan (decoupled look-back, Merrill & Garland 2016): each block takes the
-    // next tile number from a counter, so a tile waits only on tiles whose blocks started before
+    // Decoupled look-back (Merrill & Garland 2016), for the scan and the sort passes: each block takes
+    // the next tile number from a counter, so a tile waits only on tiles whose blocks started before
     // it; it publishes its sum, adds its predecessors' sums walking back to the first inclusive
-    // prefix, publishes that prefix and writes its values. Status words carry the scan's epoch
-    // (bit 33 up), a prefix flag (bit 32) and the value, so no clearing pass is needed: the block
-    // of the last tile resets the counter and counts the scan in the epoch word. A scan's epoch is
-    // 1 + (scans before it mod 2^31 - 1), never 0, so the zeroed state of a new buffer matches no
-    // scan. A wait longer than kScanSpins polls gives up and sets the fail word (never expected;
-    // the host reports it).
+    // prefix, publishes that prefix and writes its values. Status words carry the launch's epoch
+    // (bit 33 up), a prefix flag (bit 32) and the value in one 64-bit word, so the polls need no
+    // ordering and no clearing pass is needed: the last block resets the counter and counts the
+    // launch in the epoch word. A launch's epoch is 1 + (launches before it mod 2^31 - 1), never 0,
+    // so the zeroed state of a new buffer matches no launch. A wait longer than kScanSpins polls
+    // gives up and sets the fail word (never expected; the host reports it).
+    // A walk reads many predecessors at a time: a poll is a round trip to memory (the XCDs share no
+    // L2).
     constexpr uint32_t kScanSpins = 1u << 20;
+    constexpr unsigned long long kScanPrefix = 1ull << 32;
 
+    __device__ __forceinline__ unsigned long long scanTag(uint32_t epoch)
+    {
+        return static_cast<unsigned long long>(epoch % 0x7fffffffu + 1u) << 33;
+    }
+
+    __device__ __forceinline__ unsigned long long pollStatus(const unsigned long long* w)
+    {
+        return __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+
+    __device__ __forceinline__ void publishStatus(unsigned long long* w, unsigned long long v)
+    {
+        __hip_atomic_store(w, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+
+    // the sum of the tiles before `tile` (> 0), by one whole wave: 64 predecessors at a time
+    __device__ __forceinline__ uint32_t lookBackWave(const unsigned long long* status, uint32_t tile, unsigned long long tag,
+        uint32_t* fail)
+    {
+        const uint32_t lane = threadIdx.x & 63u;
+        uint32_t prefix = 0, spins = 0;
+        uint32_t left = tile;   // tiles not added yet: 0 .. left - 1
+        for (;;)
+        {
+            const unsigned long long w = lane < left ? pollStatus(&status[left - 1u - lane]) : 0ull;
+            const bool ready = (w >> 33) == (tag >> 33);
+            const uint64_t readyMask = __ballot(ready);
+            const uint64_t prefMask = __ballot(ready && (w & kScanPrefix) != 0ull);
+            // lanes of the unbroken run of ready tiles, up to the first prefix
+            uint32_t run = readyMask == ~0ull ? 64u : static_cast<uint32_t>(__ffsll(static_cast<unsigned long long>(~readyMask))) - 1u;
+            const uint32_t pre = prefMask == 0ull ? 64u : static_cast<uint32_t>(__ffsll(static_cast<unsigned long long>(prefMask))) - 1u;
+            const bool done = pre < run;
+            if (done) { run = pre + 1u; }
+            uint32_t v = lane < run ? static_cast<uint32_t>(w) : 0u;
+            for (int o = 32; o > 0; o >>= 1) { v += static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), o, 64)); }
+            prefix += v;
+            left -= run;
+            if (done || left == 0u) { return prefix; }
+            if (run == 0u)
+            {
+                if (++spins > kScanSpins)
+                {
+                    if (lane == 0u) { atomicOr(fail, 1u); }
+                    return prefix;
+                }
+                __builtin_amdgcn_s_sleep(1);
+            }
+        }
+    }
+
+    // One-pass exclusive scan. 8 M values (3,907 tiles): 178 us, 2,070 with one thread walking back tile by tile.
     __global__ void __launch_bounds__(kBlock) kScanOnePass(uint32_t* __restrict__ v, uint32_t m, uint32_t* __restrict__ tmp,
         uint32_t* __restrict__ fail)
     {
@@ -70,42 +138,31 @@ namespace tsp
         }
         __syncthreads();
         const uint32_t tile = sTile;
-        const unsigned long long tag = static_cast<unsigned long long>(sEpoch % 0x7fffffffu + 1u) << 33;
+        const unsigned long long tag = scanTag(sEpoch);
         const uint32_t base = tile * kScanTile + threadIdx.x * 8u;
         uint32_t loc[8];
         uint32_t sum = 0;
         for (uint32_t q = 0; q < 8; q++) { loc[q] = base + q < m ? v[base + q] : 0u; sum += loc[q]; }
         uint32_t total;
         const uint32_t r = blockExclusiveScan(sum, total);
-        if (threadIdx.x == 0)
+        if (threadIdx.x < 64u)
         {
-            constexpr unsigned long long kPrefix = 1ull << 32;
             uint32_t prefix = 0;
             if (tile > 0)
             {
-                __hip_atomic_store(&status[tile], tag | total, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-                uint32_t j = tile - 1, spins = 0;
-                for (;;)
-                {
-                    const unsigned long long w = __hip_atomic_load(&status[j], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
-                    if ((w >> 33) != (tag >> 33))
-                    {
-                        if (++spins > kScanSpins) { atomicOr(fail, 1u); break; }
-                        __builtin_amdgcn_s_sleep(2);
-                        continue;
-                    }
-                    prefix += static_cast<uint32_t>(w);
-                    if ((w & kPrefix) || j == 0) { break; }
-                    j--;
-                }
+                if (threadIdx.x == 0) { publishStatus(&status[tile], tag | total); }
+                prefix = lookBackWave(status, tile, tag, fail);
             }
-            __hip_atomic_store(&status[tile], tag | kPrefix | (prefix + total), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-            sPrefix = prefix;
-            if (tile == nb - 1)
+            if (threadIdx.x == 0)
             {
-                // every block has drawn its tile: ready the counter and epoch for the next scan
-                __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(epochWord, sEpoch + 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+                publishStatus(&status[tile], tag | kScanPrefix | (prefix + total));
+                sPrefix = prefix;
+                if (tile == nb - 1)
+                {
+                    // every block has drawn its tile: ready the counter and epoch for the next scan
+                    __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    __hip_atomic_store(epochWord, sEpoch + 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+                }
             }
         }
         __syncthreads();
@@ -196,14 +253,66 @@ namespace tsp
         return cellKey(f, q.x, q.y, q.z, check, d.status, &d.solve[s]);
     }
 
+    // the digits of a key counted in LDS, cnt[pass][digit]
+    template <typename K>
+    __device__ __forceinline__ void countDigits(uint32_t (&cnt)[kRadixPasses<K>][kRadixBins], K k, uint32_t passes)
+    {
+#pragma unroll
+        for (uint32_t q = 0; q < kRadixPasses<K>; q++)
+        {
+            if (q < passes) { atomicAdd(&cnt[q][static_cast<uint32_t>(k >> (q * kRadixBits)) & (kRadixBins - 1u)], 1u); }
+        }
+    }
+
+    template <typename K>
+    __device__ __forceinline__ void clearDigits(uint32_t (&cnt)[kRadixPasses<K>][kRadixBins], uint32_t passes)
+    {
+        for (uint32_t q = 0; q < passes; q++) { cnt[q][threadIdx.x] = 0u; }
+        __syncthreads();
+    }
+
+    template <typename K>
+    __device__ __forceinline__ void addDigits(const uint32_t (&cnt)[kRadixPasses<K>][kRadixBins], uint32_t passes,
+        uint32_t* __restrict__ state)
+    {
+        __syncthreads();
+        for (uint32_t q = 0; q < passes; q++)
+        {
+            const uint32_t c = cnt[q][threadIdx.x];
+            if (c) { atomicAdd(&state[kRadixHeaderWords + q * kRadixBins + threadIdx.x], c); }
+        }
+    }
+
+    // keys and indices of a population; passes > 0 adds
+    // the digit counts of all sort passes to the sort state (particles in motion are nearly in
+    // order, so a block meets few digits and adds few words)
     template <typename K>
     __global__ void __launch_bounds__(kBlock) kKeys(Dev d, int pop, const float4* __restrict__ p, uint32_t n, bool check,
-        K* __restrict__ key, uint32_t* __restrict__ idx)
+        K* __restrict__ key, uint32_t* __restrict__ idx, uint32_t* __restrict__ state, uint32_t passes)
     {
+        __shared__ uint32_t cnt[kRadixPasses<K>][kRadixBins];
+        if (passes) { clearDigits<K>(cnt, passes); }
         const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-        if (i >= n) { return; }
-        key[i] = static_cast<K>(particleKey(d, pop, p, i, check));
-        idx[i] = i;
+        if (i < n)
+        {
+            const K k = static_cast<K>(particleKey(d, pop, p, i, check));
+            key[i] = k;
+            idx[i] = i;
+            countDigits<K>(cnt, k, passes);
+        }
+        if (passes) { addDigits<K>(cnt, passes, state); }
+    }
+
+    // the digit counts of keys that another kernel wrote
+    template <typename K>
+    __global__ void __launch_bounds__(kBlock) kRadixCount(const K* __restrict__ key, uint32_t n, uint32_t* __restrict__ state,
+        uint32_t passes)
+    {
+        __shared__ uint32_t cnt[kRadixPasses<K>][kRadixBins];
+        clearDigits<K>(cnt, passes);
+        const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+        if (i < n) { countDigits<K>(cnt, key[i], passes); }
+        addDigits<K>(cnt, passes, state);
     }
 
     // boundary keys; flags a descent so the host knows whether the order needs a sort
@@ -220,193 +329,347 @@ namespace tsp
     }
 
     // ----------------------------------------------------------------------------------------
-    // stable LSD radix sort, kRadixBits-bit digits (kRadixBins <= 256 buckets), tiles of 2048 keys
+    // stable LSD radix sort, 8-bit digits, in three forms by the number of keys.
+    //   up to 2^14   one launch of one block (kSortSmall)
+    //   up to 2^18   one launch per digit (kRadixPass): the counts of all digits come first, with the keys
+    //                (they do not depend on the order); a tile ranks its keys, publishes its digit counts,
+    //                adds up those of the tiles before it by decoupled look-back (one digit per thread)
+    //                and writes its keys
+    //   more         three launches per digit (kRadixHist, kRadixDigitScan, kRadixScatter)
+    // Look-back saves six of ten launches, which is most of a small sort's time (64,000 particles: 66 us of
+    // kernels in ten launches to 39 us in four), but every poll passes the L2s by: with 489 tiles a pass
+    // took 48 us, with 3,907 tiles 333 to 505, against 19 and 75 to 100 in three launches. With the scan
+    // of all counts by one look-back between them, in place of one block per digit, those three took 34 and 242.
 
-    constexpr uint32_t kTile = 2048;
-    constexpr uint32_t kRounds = kTile / kBlock;
+    // ranks of one wave's keys among those of the same digit, in key order (round r, then lane);
+    // cnt: the wave's digit counts, zeroed before and complete after. The counter is read by all lanes
+    // of a digit and then advanced by the lowest one: LDS serves a wave's accesses in order, the fences
+    // keep the compiler to it.
+    template <typename K, uint32_t kPer>
+    __device__ __forceinline__ void rankWave(uint32_t* cnt, const K (&k)[kPer], uint32_t first, uint32_t n, uint32_t shift,
+        uint32_t bits, uint32_t (&rank)[kPer])
+    {
+        const uint32_t digitBits = min(kRadixBits, bits - shift);   // the key's bits end here
+        const uint32_t lane = threadIdx.x & 63u;
+        const uint64_t lanesBelow = (lane == 0) ? 0ull : (~0ull >> (64u - lane));
+#pragma unroll
+        for (uint32_t r = 0; r < kPer; r++)
+        {
+            rank[r] = 0u;
+            if (first + r * 64u >= n) { continue; }
+            const bool valid = first + r * 64u + lane < n;
+            const uint32_t dg = static_cast<uint32_t>(k[r] >> shift) & (kRadixBins - 1u);
+            uint64_t match = __ballot(valid);
+#pragma unroll
+            for (uint32_t bit = 0; bit < kRadixBits; bit++)
+            {
+                if (bit >= digitBits) { break; }
+                const bool set = (dg >> bit) & 1u;
+                const uint64_t bs = __ballot(set);
+                match &= set ? bs : ~bs;
+            }
+            const uint32_t below = __popcll(match & lanesBelow);
+            if (valid)
+            {
+                const uint32_t before = cnt[dg];
+                rank[r] = before + below;
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                if (below == 0u) { cnt[dg] = before + __popcll(match); }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        }
+    }
+
+    // the sum of one digit's counts in the tiles before `tile` (> 0), by one thread per digit: eight
+    // predecessors at a time
+    __device__ __forceinline__ uint32_t lookBackDigit(const unsigned long long* status, uint32_t tile, uint32_t digit,
+        unsigned long long tag, uint32_t* fail)
+    {
+        constexpr uint32_t kAhead = 8;
+        uint32_t prefix = 0, spins = 0;
+        uint32_t left = tile;
+        for (;;)
+        {
+            unsigned long long w[kAhead];
+#pragma unroll
+            for (uint32_t q = 0; q < kAhead; q++)
+            {
+                w[q] = q < left ? pollStatus(&status[static_cast<uint64_t>(left - 1u - q) * kRadixBins + digit]) : 0ull;
+            }
+            uint32_t run = 0;
+            bool open = true, done = false;
+#pragma unroll
+            for (uint32_t q = 0; q < kAhead; q++)
+            {
+                open = open && !done && (w[q] >> 33) == (tag >> 33);
+                if (open)
+                {
+                    prefix += static_cast<uint32_t>(w[q]);
+                    run++;
+                    done = (w[q] & kScanPrefix) != 0ull;
+                }
+            }
+            left -= run;
+            if (done || left == 0u) { return prefix; }
+            if (run == 0u)
+            {
+                if (++spins > kScanSpins)
+                {
+                    atomicOr(fail, 1u);
+                    return prefix;
+                }
+                __builtin_amdgcn_s_sleep(1);
+            }
+        }
+    }
+
+    // what a sort pass's two forms share: a tile's keys in registers, ranked wave by wave; then, with the
+    // place of the tile's first key of digit t known to thread t, every key's place
+    template <typename K, uint32_t kPer>
+    struct TileKeys
+    {
+        static constexpr uint32_t kWaves = kBlock / 64;
+        K k[kPer];
+        uint32_t ix[kPer], rank[kPer], c[kWaves];
+        uint32_t first;
+
+        // cnt: zeroed; the tile's count of digit t comes back in thread t
+        __device__ __forceinline__ uint32_t load(uint32_t (&cnt)[kWaves][kRadixBins], const K* __restrict__ keyIn,
+            const uint32_t* __restrict__ idxIn, uint32_t tile, uint32_t n, uint32_t shift, uint32_t bits)
+        {
+            const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+            first = tile * (kBlock * kPer) + wave * (64u * kPer);
+#pragma unroll
+            for (uint32_t r = 0; r < kPer; r++)
+            {
+                const uint32_t i = first + r * 64u + lane;
+                k[r] = i < n ? keyIn[i] : K(0);
+                ix[r] = i < n ? idxIn[i] : 0u;
+            }
+            rankWave<K, kPer>(cnt[wave], k, first, n, shift, bits, rank);
+            __syncthreads();
+            uint32_t total = 0;
+            for (uint32_t w = 0; w < kWaves; w++) { c[w] = cnt[w][threadIdx.x]; total += c[w]; }
+            return total;
+        }
+
+        __device__ __forceinline__ void store(uint32_t (&cnt)[kWaves][kRadixBins], K* __restrict__ keyOut,
+            uint32_t* __restrict__ idxOut, uint32_t at, uint32_t n, uint32_t shift)
+        {
+            const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+            for (uint32_t w = 0; w < kWaves; w++) { cnt[w][threadIdx.x] = at; at += c[w]; }
+            __syncthreads();
+#pragma unroll
+            for (uint32_t r = 0; r < kPer; r++)
+            {
+                if (first + r * 64u + lane < n)
+                {
+                    const uint32_t o = cnt[wave][static_cast<uint32_t>(k[r] >> shift) & (kRadixBins - 1u)] + rank[r];
+                    // (out of range only after a look-back gave up)
+                    if (o < n) { keyOut[o] = k[r]; idxOut[o] = ix[r]; }
+                }
+            }
+        }
+    };
+
+    // one digit of a sort with few tiles. state: the header (tile counter, epoch, blocks that have read),
+    // the digit counts of all passes and the tiles' status words. The block that reads them last clears
+    // what this pass used.
+    template <typename K, uint32_t kPer>
+    __global__ void __launch_bounds__(kBlock) kRadixPass(const K* __restrict__ keyIn, const uint32_t* __restrict__ idxIn,
+        K* __restrict__ keyOut, uint32_t* __restrict__ idxOut, uint32_t n, uint32_t pass, uint32_t bits,
+        uint32_t* __restrict__ state, uint32_t* __restrict__ fail)
+    {
+        constexpr uint32_t kWaves = kBlock / 64;
+        static_assert(kRadixBins == kBlock, "one digit per thread");
+        __shared__ uint32_t cnt[kWaves][kRadixBins];
+        __shared__ uint32_t sHist[kRadixBins];
+        __shared__ uint32_t sTile, sEpoch, sLast;
+        uint32_t* hist = state + kRadixHeaderWords + pass * kRadixBins;
+        unsigned long long* status = reinterpret_cast<unsigned long long*>(state + kRadixStatusAt);
+        const uint32_t t = threadIdx.x;
+        if (t == 0)
+        {
+            sEpoch = __hip_atomic_load(&state[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            sTile = __hip_atomic_fetch_add(&state[0], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        sHist[t] = hist[t];
+        for (uint32_t w = 0; w < kWaves; w++) { cnt[w][t] = 0u; }
+        __syncthreads();
+        // this block has what it reads of the state (the counts are in LDS); its turn among the blocks
+        // comes back while the keys load, and is looked at when they are placed
+        uint32_t readers = 0;
+        if (t == 0) { readers = __hip_atomic_fetch_add(&state[2], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+        const uint32_t tile = sTile;
+        const unsigned long long tag = scanTag(sEpoch);
+        TileKeys<K, kPer> keys;
+        const uint32_t total = keys.load(cnt, keyIn, idxIn, tile, n, pass * kRadixBits, bits);
+        unsigned long long* mine = &status[static_cast<uint64_t>(tile) * kRadixBins + t];
+        publishStatus(mine, tag | (tile == 0u ? kScanPrefix : 0ull) | total);
+        uint32_t all;
+        uint32_t at = blockExclusiveScan(sHist[t], all);
+        if (tile > 0u)
+        {
+            const uint32_t prefix = lookBackDigit(status, tile, t, tag, fail);
+            publishStatus(mine, tag | kScanPrefix | (prefix + total));
+            at += prefix;
+        }
+        if (t == 0) { sLast = readers == gridDim.x - 1u; }
+        keys.store(cnt, keyOut, idxOut, at, n, pass * kRadixBits);   // (a barrier after sLast is written)
+        if (sLast)
+        {
+            hist[t] = 0u;
+            if (t == 0)
+            {
+                __hip_atomic_store(&state[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(&state[2], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(&state[1], sEpoch + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+    }
+
+    // one digit of a sort with many tiles, in three launches: the tiles' digit counts (hist[digit][tile]),
+    // their exclusive scan along the tiles of each digit (a block per digit: no block waits for another),
+    // and the scatter, which adds the digits before.
+    constexpr uint32_t kManyPer = kRadixManyTile / kBlock;
 
     template <typename K>
     __global__ void __launch_bounds__(kBlock) kRadixHist(const K* __restrict__ key, uint32_t n, uint32_t shift,
         uint32_t nTiles, uint32_t* __restrict__ hist)
     {
         __shared__ uint32_t cnt[kRadixBins];
-        if (threadIdx.x < kRadixBins) { cnt[threadIdx.x] = 0; }
+        cnt[threadIdx.x] = 0;
         __syncthreads();
-        const uint32_t base = blockIdx.x * kTile;
-        for (uint32_t r = 0; r < kRounds; r++)
+        const uint32_t base = blockIdx.x * kRadixManyTile + threadIdx.x;
+#pragma unroll
+        for (uint32_t r = 0; r < kManyPer; r++)
         {
-            const uint32_t i = base + r * kBlock + threadIdx.x;
+            const uint32_t i = base + r * kBlock;
             if (i < n) { atomicAdd(&cnt[static_cast<uint32_t>(key[i] >> shift) & (kRadixBins - 1u)], 1u); }
         }
         __syncthreads();
-        if (threadIdx.x < kRadixBins) { hist[threadIdx.x * nTiles + blockIdx.x] = cnt[threadIdx.x]; }
+        hist[threadIdx.x * nTiles + blockIdx.x] = cnt[threadIdx.x];
     }
 
-    template <typename K>
-    __global__ void __launch_bounds__(kBlock) kRadixScatter(const K* __restrict__ keyIn,
-        const uint32_t* __restrict__ idxIn, K* __restrict__ keyOut, uint32_t* __restrict__ idxOut, uint32_t n,
-        uint32_t shift, uint32_t nTiles, const uint32_t* __restrict__ offsets)
+    __global__ void __launch_bounds__(kBlock) kRadixDigitScan(uint32_t* __restrict__ hist, uint32_t nTiles,
+        uint32_t* __restrict__ totals)
     {
-        __shared__ uint32_t run[kRadixBins];
-        __shared__ uint32_t waveCnt[kBlock / 64][kRadixBins];
-        const uint32_t t = threadIdx.x;
-        const uint32_t wave = t >> 6, lane = t & 63u;
-        if (t < kRadixBins)
+        uint32_t* row = hist + static_cast<uint64_t>(blockIdx.x) * nTiles;
+        uint32_t before = 0;
+        for (uint32_t b = 0; b < nTiles; b += kRadixManyTile)
         {
-            run[t] = offsets[t * nTiles + blockIdx.x];
-            for (uint32_t w = 0; w < kBlock / 64; w++) { waveCnt[w][t] = 0; }
+            const uint32_t base = b + threadIdx.x * kManyPer;
+            uint32_t loc[kManyPer], sum = 0;
+#pragma unroll
+            for (uint32_t q = 0; q < kManyPer; q++) { loc[q] = base + q < nTiles ? row[base + q] : 0u; sum += loc[q]; }
+            uint32_t total;
+            uint32_t run = before + blockExclusiveScan(sum, total);
+            __syncthreads();
+#pragma unroll
+            for (uint32_t q = 0; q < kManyPer; q++)
+            {
+                if (base + q < nTiles) { row[base + q] = run; }
+                run += loc[q];
+            }
+            before += total;
         }
-        __syncthreads();
-        const uint64_t lanesBelow = (lane == 0) ? 0ull : (~0ull >> (64u - lane));
-        const uint32_t base = blockIdx.x * kTile;
-        for (uint32_t r = 0; r < kRounds; r++)
-        {
-            const uint32_t i = base + r * kBlock + t;
-            const bool valid = i < n;
-            const K k = valid ? keyIn[i] : K(0);
-            const uint32_t d = static_cast<uint32_t>(k >> shift) & (kRadixBins - 1u);
-            // lanes of this wave holding the same digit
-            uint64_t match = __ballot(valid);
-            for (uint32_t bit = 0; bit < kRadixBits; bit++)
-            {
-                const bool set = (d >> bit) & 1u;
-                const uint64_t bs = __ballot(set);
-                match &= set ? bs : ~bs;
-            }
-            const uint32_t rankInWave = __popcll(match & lanesBelow);
-            if (valid && rankInWave == 0) { waveCnt[wave][d] = __popcll(match); }
-            __syncthreads();
-            uint32_t rank = 0;
-            if (valid)
-            {
-                rank = run[d] + rankInWave;
-                for (uint32_t w = 0; w < wave; w++) { rank += waveCnt[w][d]; }
-            }
-            __syncthreads();
-            if (t < kRadixBins)
-            {
-                uint32_t tot = 0;
-                for (uint32_t w = 0; w < kBlock / 64; w++) { tot += waveCnt[w][t]; waveCnt[w][t] = 0; }
-                run[t] += tot;
-            }
-            __syncthreads();
-            if (valid)
-            {
-                keyOut[rank] = k;
-                idxOut[rank] = idxIn[i];
-            }
-        }
+        if (threadIdx.x == 0) { totals[blockIdx.x] = before; }
     }
 
-    // the whole stable LSD sort of up to kSmallSort keys in one block of 1024 threads (one launch
-    // instead of five per digit). Per digit: each thread loads its 16 elements (i = c*1024 + t) at
-    // once; the digit counts are scanned by the first 256 threads with wave shuffles; then the
-    // elements are ranked chunk by chunk in element order: wave ballots give the rank inside a
-    // wave, 256 digit threads turn the per-wave counts into per-wave offsets, and the elements
-    // scatter. The passes alternate between the two buffers in global memory, and an odd pass
-    // count copies back at the end.
-    constexpr uint32_t kSmallThreads = 1024;
-    constexpr uint32_t kSmallPer = 16;
-    constexpr uint32_t kSmallSort = kSmallThreads * kSmallPer;
-
     template <typename K>
-    __global__ void __launch_bounds__(kSmallThreads) kSortSmall(K* __restrict__ key, uint32_t* __restrict__ idx,
-        K* __restrict__ key2, uint32_t* __restrict__ idx2, uint32_t n, uint32_t bits)
+    __global__ void __launch_bounds__(kBlock) kRadixScatter(const K* __restrict__ keyIn, const uint32_t* __restrict__ idxIn,
+        K* __restrict__ keyOut, uint32_t* __restrict__ idxOut, uint32_t n, uint32_t shift, uint32_t bits, uint32_t nTiles,
+        const uint32_t* __restrict__ hist, const uint32_t* __restrict__ totals)
+    {
+        __shared__ uint32_t cnt[kBlock / 64][kRadixBins];
+        const uint32_t t = threadIdx.x;
+        const uint32_t before = hist[t * nTiles + blockIdx.x];
+        const uint32_t total = totals[t];
+        for (uint32_t w = 0; w < kBlock / 64; w++) { cnt[w][t] = 0u; }
+        __syncthreads();
+        TileKeys<K, kManyPer> keys;
+        keys.load(cnt, keyIn, idxIn, blockIdx.x, n, shift, bits);
+        uint32_t all;
+        const uint32_t at = blockExclusiveScan(total, all) + before;
+        keys.store(cnt, keyOut, idxOut, at, n, shift);
+    }
+
+    // the whole sort of up to kSmallSort keys in one block of 1024 threads (one launch). A wave holds
+    // 64 x kPer consecutive keys in registers and ranks them by itself; the 256 digits then add up the
+    // waves' counts, and the keys and indices change places through LDS, a word at a time (64 KB for the
+    // most keys, whatever their width).
+    constexpr uint32_t kSmallThreads = 1024;
+    constexpr uint32_t kSmallSort = kSmallThreads * 16;
+
+    template <typename K, uint32_t kPer>
+    __global__ void __launch_bounds__(kSmallThreads) kSortSmall(K* __restrict__ key, uint32_t* __restrict__ idx, uint32_t n,
+        uint32_t bits)
     {
         constexpr uint32_t kWaves = kSmallThreads / 64;
-        __shared__ uint32_t run[kRadixBins];
-        __shared__ uint32_t waveTot[4];
         __shared__ uint32_t cnt[kWaves][kRadixBins];
-        __shared__ uint32_t pre[kWaves][kRadixBins];
+        __shared__ uint32_t word[kSmallThreads * kPer];
         const uint32_t t = threadIdx.x;
         const uint32_t wave = t >> 6, lane = t & 63u;
-        const uint64_t lanesBelow = (lane == 0) ? 0ull : (~0ull >> (64u - lane));
-        for (uint32_t w = 0; w < kWaves; w++) { if (t < kRadixBins) { cnt[w][t] = 0; } }
-        K* kIn = key; uint32_t* iIn = idx; K* kOut = key2; uint32_t* iOut = idx2;
+        const uint32_t first = wave * (64u * kPer);
+        K k[kPer];
+        uint32_t ix[kPer], rank[kPer];
+#pragma unroll
+        for (uint32_t r = 0; r < kPer; r++)
+        {
+            const uint32_t i = first + r * 64u + lane;
+            k[r] = i < n ? key[i] : K(0);
+            ix[r] = i < n ? idx[i] : 0u;
+        }
+        const auto exchange = [&](auto&& get, auto&& set)
+        {
+#pragma unroll
+            for (uint32_t r = 0; r < kPer; r++) { if (first + r * 64u + lane < n) { word[rank[r]] = get(r); } }
+            __syncthreads();
+#pragma unroll
+            for (uint32_t r = 0; r < kPer; r++) { if (first + r * 64u + lane < n) { set(r, word[first + r * 64u + lane]); } }
+            __syncthreads();
+        };
         for (uint32_t shift = 0; shift < bits; shift += kRadixBits)
         {
-            K kr[kSmallPer];
-            uint32_t ir[kSmallPer];
-#pragma unroll
-            for (uint32_t c = 0; c < kSmallPer; c++)
-            {
-                const uint32_t i = c * kSmallThreads + t;
-                kr[c] = i < n ? kIn[i] : K(0);
-                ir[c] = i < n ? iIn[i] : 0u;
-            }
-            if (t < kRadixBins) { run[t] = 0; }
+            for (uint32_t w = t / kRadixBins; w < kWaves; w += kSmallThreads / kRadixBins) { cnt[w][t & (kRadixBins - 1u)] = 0u; }
             __syncthreads();
-#pragma unroll
-            for (uint32_t c = 0; c < kSmallPer; c++)
-            {
-                if (c * kSmallThreads + t < n) { atomicAdd(&run[static_cast<uint32_t>(kr[c] >> shift) & (kRadixBins - 1u)], 1u); }
-            }
+            rankWave<K, kPer>(cnt[wave], k, first, n, shift, bits, rank);
             __syncthreads();
-            // exclusive scan of the 256 digit counts: inclusive scan per wave, then the wave totals
-            uint32_t v = 0, incl = 0;
+            uint32_t c[kWaves];
+            uint32_t total = 0;
             if (t < kRadixBins)
             {
-                v = run[t];
-                incl = v;
-                for (int o = 1; o < 64; o <<= 1)
-                {
-                    const uint32_t u = static_cast<uint32_t>(__shfl_up(static_cast<int>(incl), o, 64));
-                    if (lane >= static_cast<uint32_t>(o)) { incl += u; }
-                }
-                if (lane == 63) { waveTot[wave] = incl; }
+#pragma unroll
+                for (uint32_t w = 0; w < kWaves; w++) { c[w] = cnt[w][t]; total += c[w]; }
             }
-            __syncthreads();
+            uint32_t all;
+            uint32_t at = blockExclusiveScan(total, all);
             if (t < kRadixBins)
             {
-                uint32_t off = 0;
-                for (uint32_t w = 0; w < wave; w++) { off += waveTot[w]; }
-                run[t] = off + incl - v;
+#pragma unroll
+                for (uint32_t w = 0; w < kWaves; w++) { cnt[w][t] = at; at += c[w]; }
             }
             __syncthreads();
 #pragma unroll
-            for (uint32_t c = 0; c < kSmallPer; c++)
+            for (uint32_t r = 0; r < kPer; r++)
             {
-                if (c * kSmallThreads >= n) { break; }
-                const uint32_t i = c * kSmallThreads + t;
-                const bool valid = i < n;
-                const K k = kr[c];
-                const uint32_t dg = static_cast<uint32_t>(k >> shift) & (kRadixBins - 1u);
-                uint64_t match = __ballot(valid);
-                for (uint32_t bit = 0; bit < kRadixBits; bit++)
-                {
-                    const bool set = (dg >> bit) & 1u;
-                    const uint64_t bs = __ballot(set);
-                    match &= set ? bs : ~bs;
-                }
-                const uint32_t rankInWave = __popcll(match & lanesBelow);
-                if (valid && rankInWave == 0) { cnt[wave][dg] = __popcll(match); }
-                __syncthreads();
-                // per digit: offsets of the waves' runs (and the counts cleared for the next chunk)
-                if (t < kRadixBins)
-                {
-                    uint32_t cw[kWaves];
-#pragma unroll
-                    for (uint32_t w = 0; w < kWaves; w++) { cw[w] = cnt[w][t]; }
-                    uint32_t acc = run[t];
-#pragma unroll
-                    for (uint32_t w = 0; w < kWaves; w++) { pre[w][t] = acc; acc += cw[w]; cnt[w][t] = 0; }
-                    run[t] = acc;
-                }
-                __syncthreads();
-                if (valid)
-                {
-                    const uint32_t rank = pre[wave][dg] + rankInWave;
-                    kOut[rank] = k;
-                    iOut[rank] = ir[c];
-                }
+                if (first + r * 64u + lane < n) { rank[r] += cnt[wave][static_cast<uint32_t>(k[r] >> shift) & (kRadixBins - 1u)]; }
             }
-            __syncthreads();
-            K* tk = kIn; kIn = kOut; kOut = tk;
-            uint32_t* ti = iIn; iIn = iOut; iOut = ti;
+            // the digits of this pass are used up: the key itself moves, then its index
+            if constexpr (sizeof(K) == 8)
+            {
+                exchange([&](uint32_t r) { return static_cast<uint32_t>(k[r] >> 32); },
+                         [&](uint32_t r, uint32_t w) { k[r] = (static_cast<K>(w) << 32) | static_cast<uint32_t>(k[r]); });
+            }
+            exchange([&](uint32_t r) { return static_cast<uint32_t>(k[r]); },
+                     [&](uint32_t r, uint32_t w) { k[r] = static_cast<K>((k[r] & ~static_cast<K>(0xffffffffu)) | w); });
+            exchange([&](uint32_t r) { return ix[r]; }, [&](uint32_t r, uint32_t w) { ix[r] = w; });
         }
-        if (kIn != key)
+#pragma unroll
+        for (uint32_t r = 0; r < kPer; r++)
         {
-            for (uint32_t i = t; i < n; i += kSmallThreads) { key[i] = kIn[i]; idx[i] = iIn[i]; }
+            const uint32_t i = first + r * 64u + lane;
+            if (i < n) { key[i] = k[r]; idx[i] = ix[r]; }
         }
     }
 
@@ -1457,15 +1720,28 @@ namespace tsp
 
     static inline uint32_t blocksFor(uint64_t n) { return static_cast<uint32_t>((n + kBlock - 1) / kBlock); }
 
+    // a sort of n keys runs as one block and uses no sort state
+    bool radixSortSingleBlock(uint32_t n) { return n <= kSmallSort; }
+
+    static uint32_t radixPasses(uint32_t bits) { return (bits + kRadixBits - 1u) / kRadixBits; }
+
+
     void launchResetSearch(hipStream_t s, const Dev& d) { kResetSearch<<<1, kBlock, 0, s>>>(d); }
 
     // key arrays hold u32 keys, or u64 keys (two words each) when d.key64
+    // state: the sort state that takes the digit counts when kRadixPass sorts the keys by `bits` bits
+    // (null: the keys are not sorted)
     void launchKeys(hipStream_t s, const Dev& d, int pop, const float4* p, uint32_t n, bool check, uint32_t* key,
-                    uint32_t* idx)
+                    uint32_t* idx, uint32_t bits, uint32_t* state)
     {
         if (!n) { return; }
-        if (d.key64) { kKeys<<<blocksFor(n), kBlock, 0, s>>>(d, pop, p, n, check, reinterpret_cast<uint64_t*>(key), idx); }
-        else { kKeys<<<blocksFor(n), kBlock, 0, s>>>(d, pop, p, n, check, key, idx); }
+        const uint32_t passes = state && !radixSortSingleBlock(n) && n <= kRadixSmallTiles ? radixPasses(bits) : 0u;
+        const uint32_t nb = blocksFor(n);
+        if (d.key64)
+        {
+            kKeys<<<nb, kBlock, 0, s>>>(d, pop, p, n, check, reinterpret_cast<uint64_t*>(key), idx, state, passes);
+        }
+        else { kKeys<<<nb, kBlock, 0, s>>>(d, pop, p, n, check, key, idx, state, passes); }
     }
 
     void launchKeysSorted(hipStream_t s, const Dev& d, const float4* p, uint32_t n, uint32_t* key, uint32_t* idx)
@@ -1477,20 +1753,32 @@ namespace tsp
 
     template <typename K>
     static bool radixSort(hipStream_t s, K* key, uint32_t* idx, K* key2, uint32_t* idx2, uint32_t n, uint32_t bits,
-                          uint32_t* hist, uint32_t* tmp, uint32_t* fail, bool copyBack)
+                          uint32_t* state, uint32_t* fail, bool counted, bool copyBack)
     {
         if (n <= kSmallSort)
         {
-            kSortSmall<K><<<1, kSmallThreads, 0, s>>>(key, idx, key2, idx2, n, bits);
+            // fewer keys per lane leave fewer waves idle: 4,096 keys fill 16 waves with four each
+            if (n <= kSmallThreads * 4u) { kSortSmall<K, 4><<<1, kSmallThreads, 0, s>>>(key, idx, n, bits); }
+            else if (n <= kSmallThreads * 8u) { kSortSmall<K, 8><<<1, kSmallThreads, 0, s>>>(key, idx, n, bits); }
+            else { kSortSmall<K, 16><<<1, kSmallThreads, 0, s>>>(key, idx, n, bits); }
             return false;
         }
-        const uint32_t nTiles = (n + kTile - 1) / kTile;
+        const uint32_t passes = radixPasses(bits);
+        const bool few = n <= kRadixSmallTiles;
+        const uint32_t nTiles = few ? (n + kRadixTileMin - 1) / kRadixTileMin : (n + kRadixManyTile - 1) / kRadixManyTile;
+        if (few && !counted) { kRadixCount<K><<<blocksFor(n), kBlock, 0, s>>>(key, n, state, passes); }
         K* kIn = key; uint32_t* iIn = idx; K* kOut = key2; uint32_t* iOut = idx2;
-        for (uint32_t shift = 0; shift < bits; shift += kRadixBits)
+        for (uint32_t q = 0; q < passes; q++)
         {
-            kRadixHist<K><<<nTiles, kBlock, 0, s>>>(kIn, n, shift, nTiles, hist);
-            launchScan(s, hist, kRadixBins * nTiles, tmp, fail);
-            kRadixScatter<K><<<nTiles, kBlock, 0, s>>>(kIn, iIn, kOut, iOut, n, shift, nTiles, hist);
+            if (few) { kRadixPass<K, kRadixPerMin><<<nTiles, kBlock, 0, s>>>(kIn, iIn, kOut, iOut, n, q, bits, state, fail); }
+            else
+            {
+                uint32_t* totals = state + kRadixManyAt;
+                uint32_t* hist = totals + kRadixBins;
+                kRadixHist<K><<<nTiles, kBlock, 0, s>>>(kIn, n, q * kRadixBits, nTiles, hist);
+                kRadixDigitScan<<<kRadixBins, kBlock, 0, s>>>(hist, nTiles, totals);
+                kRadixScatter<K><<<nTiles, kBlock, 0, s>>>(kIn, iIn, kOut, iOut, n, q * kRadixBits, bits, nTiles, hist, totals);
+            }
             K* t = kIn; kIn = kOut; kOut = t;
             uint32_t* ti = iIn; iIn = iOut; iOut = ti;
         }
@@ -1501,22 +1789,21 @@ namespace tsp
         return false;
     }
 
-    // a sort of n keys runs as one block and uses neither the digit counts nor the scan state
-    bool radixSortSingleBlock(uint32_t n) { return n <= kSmallSort; }
-
-    // sorts (key, idx) stably by the low `bits` bits; tmp is a scan state for 256 x ceil(n / 2048)
-    // values, fail its give-up word. The result ends in (key, idx), or, without copyBack, in
-    // (key2, idx2) after an odd number of passes: the return value says which.
+    // sorts (key, idx) stably by the low `bits` bits; state is a sort state of radixStateWords(n) words,
+    // zeroed when allocated, fail its give-up word; counted: the keys come from launchKeys, which has added the digit
+    // counts where they are needed. The
+    // result ends in (key, idx), or, without copyBack, in (key2, idx2) after an odd number of passes:
+    // the return value says which.
     bool launchRadixSort(hipStream_t s, bool key64, uint32_t* key, uint32_t* idx, uint32_t* key2, uint32_t* idx2,
-                         uint32_t n, uint32_t bits, uint32_t* hist, uint32_t* tmp, uint32_t* fail, bool copyBack)
+                         uint32_t n, uint32_t bits, uint32_t* state, uint32_t* fail, bool counted, bool copyBack)
     {
         if (n < 2) { return false; }
         if (key64)
         {
-            return radixSort(s, reinterpret_cast<uint64_t*>(key), idx, reinterpret_cast<uint64_t*>(key2), idx2, n, bits, hist,
-                             tmp, fail, copyBack);
+            return radixSort(s, reinterpret_cast<uint64_t*>(key), idx, reinterpret_cast<uint64_t*>(key2), idx2, n, bits, state,
+                             fail, counted, copyBack);
         }
-        return radixSort(s, key, idx, key2, idx2, n, bits, hist, tmp, fail, copyBack);
+        return radixSort(s, key, idx, key2, idx2, n, bits, state, fail, counted, copyBack);
     }
 
     void launchPermute(hipStream_t s, const Gather& g, const uint32_t* idx)

@@ -31,10 +31,10 @@
 namespace tsp
 {
     void launchResetSearch(hipStream_t, const Dev&);
-    void launchKeys(hipStream_t, const Dev&, int, const float4*, uint32_t, bool, uint32_t*, uint32_t*);
+    void launchKeys(hipStream_t, const Dev&, int, const float4*, uint32_t, bool, uint32_t*, uint32_t*, uint32_t, uint32_t*);
     void launchKeysSorted(hipStream_t, const Dev&, const float4*, uint32_t, uint32_t*, uint32_t*);
     bool launchRadixSort(hipStream_t, bool, uint32_t*, uint32_t*, uint32_t*, uint32_t*, uint32_t, uint32_t, uint32_t*, uint32_t*,
-                         uint32_t*, bool);
+                         bool, bool);
     bool radixSortSingleBlock(uint32_t n);
     void launchPermute(hipStream_t, const Gather&, const uint32_t*);
     void launchClearCells(hipStream_t, const Dev&, const uint32_t*, uint32_t, uint2*);
@@ -51,7 +51,7 @@ namespace tsp
     void launchExportSurface(hipStream_t, const Dev&, uint32_t, uint32_t, uint32_t, uint32_t*, uint32_t*, float*, float*);
     void launchBuildFluid(hipStream_t, const Dev&, uint32_t, uint32_t, const BuildFluid&);
     void launchBuildBoundary(hipStream_t, const BuildBoundary&, uint32_t, float4*, float*, uint64_t*, float*, uint32_t*,
-                             uint32_t*, uint32_t*, uint32_t*, uint32_t*, uint32_t*);
+                             uint32_t*, uint32_t*, uint32_t*, uint32_t*);
     void launchAabb(hipStream_t, const Dev&, int, const float4*, uint32_t, uint32_t*);
     void launchDensity(hipStream_t, const Dev&);
     void launchNonPressure(hipStream_t, const Dev&);
@@ -304,7 +304,7 @@ struct tsp_ctx
     float* bvol2 = nullptr;
     uint64_t *idB = nullptr, *idB2 = nullptr;
     uint64_t* idR = nullptr;
-    uint32_t* radixHist = nullptr;
+    uint32_t* radixState = nullptr;
     uint32_t* aabb = nullptr;       // 6 per scene
     std::vector<void*> arena;       // particle and body arrays (replaced by a relayout)
     std::vector<void*> work;        // search and scene-table buffers sized by the layout
@@ -677,7 +677,6 @@ struct tsp_ctx
         }
         if (totalBits > 32) { throw Error{ TSP_ERR_CAPACITY, "container too large for the device builder's 32-bit cell keys" }; }
         const uint32_t nB = h.nB;
-        const uint64_t nTiles = (nB + 2047ull) / 2048ull;
         std::vector<void*> tmp;
         try
         {
@@ -686,14 +685,13 @@ struct tsp_ctx
             uint32_t* idx = alloc<uint32_t>(nB, tmp);
             uint32_t* key2 = alloc<uint32_t>(nB, tmp);
             uint32_t* idx2 = alloc<uint32_t>(nB, tmp);
-            uint32_t* hist = alloc<uint32_t>(256ull * nTiles, tmp);
-            uint32_t* sums = alloc<uint32_t>(scanTmpWords(256ull * nTiles), tmp);
-            zero(sums, sizeof(uint32_t) * scanTmpWords(256ull * nTiles));
+            uint32_t* sort = alloc<uint32_t>(radixStateWords(nB), tmp);
+            zero(sort, sizeof(uint32_t) * radixStateWords(nB));
             launchBuildBoundary(stream, bb, nB, n.bpos + h.offB, n.bvol + h.offB, nidB + h.offB, xyz, key, idx, key2, idx2,
-                                hist, sums);
+                                sort);
             hipCheck(hipGetLastError(), "device builder launch");
             uint32_t scanFailed = 0;
-            d2h(&scanFailed, sums + 2, sizeof(uint32_t));
+            d2h(&scanFailed, sort + 3, sizeof(uint32_t));
             if (scanFailed) { throw Error{ TSP_ERR_STATE, "a one-pass scan gave up waiting for a predecessor tile" }; }
         }
         catch (...)
@@ -955,8 +953,8 @@ struct tsp_ctx
         d.keyR2 = alloc<uint32_t>(2ull * nR, work, MEM_SR);
         d.idxR = alloc<uint32_t>(nR, work, MEM_SR);
         d.idxR2 = alloc<uint32_t>(nR, work, MEM_SR);
-        const uint64_t nTiles = (nSort + 2047ull) / 2048ull;
-        radixHist = alloc<uint32_t>(256ull * nTiles, work);
+        radixState = alloc<uint32_t>(radixStateWords(nSort), work);
+        zero(radixState, sizeof(uint32_t) * radixStateWords(nSort));
         aabb = alloc<uint32_t>(6ull * S, work);
         const uint32_t nSlices = (nF + kSlice - 1) / kSlice;
         for (int r = 0; r < 3; r++)
@@ -966,8 +964,8 @@ struct tsp_ctx
             zero(d.cnt[r], sizeof(uint16_t) * nF);
         }
         {
-            // block sums of the scans: radix digit offsets, RF offsets
-            const uint64_t m = std::max<uint64_t>(256ull * nTiles, nR + 1ull);
+            // block sums of the scans over the rigid particles (RF, RB and RR offsets)
+            const uint64_t m = nR + 1ull;
             d.scanTmp = alloc<uint32_t>(scanTmpWords(m), work);
             zero(d.scanTmp, sizeof(uint32_t) * scanTmpWords(m));
         }
@@ -1241,8 +1239,8 @@ struct tsp_ctx
             sync();
             if (unsorted)
             {
-                if (launchRadixSort(stream, d.key64, d.keyF, d.idxF, d.keyF2, d.idxF2, d.nB, keyBits, radixHist, d.scanTmp,
-                                    &d.status->scanFail, false))
+                if (launchRadixSort(stream, d.key64, d.keyF, d.idxF, d.keyF2, d.idxF2, d.nB, keyBits, radixState,
+                                    &d.status->scanFail, false, false))
                 {
                     std::swap(d.keyF, d.keyF2);
                     std::swap(d.idxF, d.idxF2);
@@ -1306,9 +1304,9 @@ struct tsp_ctx
                 hipCheck(hipStreamWaitEvent(side, forkEv, 0), "hipStreamWaitEvent");
                 rs = side;
             }
-            launchKeys(rs, d, kPopR, d.rpos, d.nR, true, d.keyR, d.idxR);
-            if (launchRadixSort(rs, d.key64, d.keyR, d.idxR, d.keyR2, d.idxR2, d.nR, keyBits, radixHist, d.scanTmp,
-                                &d.status->scanFail, false))
+            launchKeys(rs, d, kPopR, d.rpos, d.nR, true, d.keyR, d.idxR, keyBits, radixState);
+            if (launchRadixSort(rs, d.key64, d.keyR, d.idxR, d.keyR2, d.idxR2, d.nR, keyBits, radixState,
+                                &d.status->scanFail, true, false))
             {
                 std::swap(d.keyR, d.keyR2);
                 std::swap(d.idxR, d.idxR2);
@@ -1317,9 +1315,9 @@ struct tsp_ctx
         }
         {
             Scope sc(prof, stream, "keys_sort");
-            launchKeys(stream, d, kPopF, d.pos, d.nF, true, d.keyF, d.idxF);
-            if (launchRadixSort(stream, d.key64, d.keyF, d.idxF, d.keyF2, d.idxF2, d.nF, keyBits, radixHist, d.scanTmp,
-                                &d.status->scanFail, false))
+            launchKeys(stream, d, kPopF, d.pos, d.nF, true, d.keyF, d.idxF, keyBits, radixState);
+            if (launchRadixSort(stream, d.key64, d.keyF, d.idxF, d.keyF2, d.idxF2, d.nF, keyBits, radixState,
+                                &d.status->scanFail, true, false))
             {
                 std::swap(d.keyF, d.keyF2);
                 std::swap(d.idxF, d.idxF2);
@@ -1647,7 +1645,7 @@ struct tsp_ctx
     {
         std::string key(reinterpret_cast<const char*>(&id), sizeof(id));
         key.append(reinterpret_cast<const char*>(&d), sizeof(Dev));
-        const void* extra[4] = { pos2, vel2, idF2, radixHist };
+        const void* extra[4] = { pos2, vel2, idF2, radixState };
         key.append(reinterpret_cast<const char*>(extra), sizeof(extra));
         key.append(reinterpret_cast<const char*>(&keyBits), sizeof(keyBits));
         auto it = stepGraphs.find(key);
@@ -2385,7 +2383,7 @@ int tsp_get_sort(tsp_ctx* ctx, uint32_t* orderF, uint64_t* keysF, uint32_t* orde
         if ((orderB || keysB) && h.nB)
         {
             // the boundary order relative to the pulled order, from the ids (sequence ids on pull)
-            launchKeys(ctx->stream, d, kPopB, d.bpos, d.nB, false, d.keyF2, d.idxF2);
+            launchKeys(ctx->stream, d, kPopB, d.bpos, d.nB, false, d.keyF2, d.idxF2, 0u, nullptr);
             uint64_t* k = reinterpret_cast<uint64_t*>(ctx->bpos2);
             launchLocalKeys(ctx->stream, d, d.keyF2, h.offB, h.nB, base, empty, k);
             ctx->addField(fields, keysB, k, h.nB);

@@ -33,7 +33,6 @@
 //   TSP_TUNE_GRAPHS        each group of solver sweeps runs as one instantiated HIP graph
 //   TSP_TUNE_PA_WAVES, TSP_TUNE_JACOBI_WAVES   waves per SIMD the compiler must leave room for
 //                          (register budget of the sweep kernels); 0 leaves the choice to it
-//   TSP_TUNE_RADIX_BITS    digit width of the LSD radix sorts (8: 256 buckets, 6, 4)
 // the settings chosen by turbospharticles_amd/tune.py, when present, come first
 #if __has_include("tsp_tuned.h")
 #include "tsp_tuned.h"
@@ -59,9 +58,6 @@
 #ifndef TSP_TUNE_JACOBI_WAVES
 #define TSP_TUNE_JACOBI_WAVES 0
 #endif
-#ifndef TSP_TUNE_RADIX_BITS
-#define TSP_TUNE_RADIX_BITS 8
-#endif
 #define TSP_WAVES_ATTR_0
 #define TSP_WAVES_ATTR_1 __attribute__((amdgpu_waves_per_eu(1)))
 #define TSP_WAVES_ATTR_2 __attribute__((amdgpu_waves_per_eu(2)))
@@ -78,9 +74,9 @@ namespace tsp
 {
     constexpr int kBlock = 256;          // threads per block: 4 waves of 64
     constexpr uint32_t kSlice = 64;      // SELL slice height: one slice per wave
-    constexpr uint32_t kRadixBits = TSP_TUNE_RADIX_BITS;
+    constexpr uint32_t kRadixBits = 8;
     constexpr uint32_t kRadixBins = 1u << kRadixBits;
-    static_assert(kRadixBits >= 1 && kRadixBits <= 8, "radix digit width");
+    template <typename K> inline constexpr uint32_t kRadixPasses = 8u * sizeof(K) / kRadixBits;
     constexpr uint32_t kEmpty32 = 0xffffffffu;
     constexpr uint32_t kFmtDelta16 = 0;
     constexpr uint32_t kFmtAbs32 = 1;
@@ -93,6 +89,23 @@ namespace tsp
     // word per 2048-value tile; zeroed when allocated
     constexpr uint32_t kScanHeaderWords = 4;
     inline constexpr uint64_t scanTmpWords(uint64_t m) { return kScanHeaderWords + 2ull * ((m + 2047ull) / 2048ull); }
+
+    // state of the sorts of up to n keys, zeroed when allocated: tile counter, epoch, readers and a spare
+    // word, the digit counts of up to eight passes and 256 u64 status words per tile of kRadixTileMin keys;
+    // for sorts of more than kRadixSmallTiles keys then the totals and tile counts of one pass (a place
+    // of their own: stale counts must not be taken for status words)
+    constexpr uint32_t kRadixHeaderWords = 4;
+    constexpr uint32_t kRadixStatusAt = kRadixHeaderWords + kRadixPasses<uint64_t> * kRadixBins;
+    constexpr uint32_t kRadixPerMin = 4;
+    constexpr uint32_t kRadixTileMin = kBlock * kRadixPerMin;
+    constexpr uint32_t kRadixSmallTiles = 1u << 18;
+    constexpr uint32_t kRadixManyAt = kRadixStatusAt + 2u * kRadixBins * (kRadixSmallTiles / kRadixTileMin);
+    constexpr uint32_t kRadixManyTile = 2048;
+    inline constexpr uint64_t radixStateWords(uint64_t n)
+    {
+        return n > kRadixSmallTiles ? kRadixManyAt + kRadixBins * (1ull + (n + kRadixManyTile - 1u) / kRadixManyTile)
+                                    : kRadixStatusAt + 2ull * kRadixBins * ((n + kRadixTileMin - 1u) / kRadixTileMin);
+    }
 
     // Hit masks of the count pass (one word per stencil row of three cells, reach 1): the fill takes the
     // hits from them and loads no candidate position. A row with more than 32 candidates is marked in

@@ -17,9 +17,6 @@
 #ifndef TSP_TUNE_PA_WAVES
 #define TSP_TUNE_PA_WAVES 6
 #endif
-#ifndef TSP_TUNE_RADIX_BITS
-#define TSP_TUNE_RADIX_BITS 8
-#endif
 #ifndef TSP_TUNE_STEP_GRAPH
 #define TSP_TUNE_STEP_GRAPH 0
 #endif

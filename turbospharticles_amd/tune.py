@@ -35,7 +35,6 @@ TUNED_H = os.path.join(HERE, "csrc", "tsp_tuned.h")
 
 # switch -> values tried (the first is the default of tsp_device.h)
 SPACE = {
-    "TSP_TUNE_RADIX_BITS": [8, 6, 4],
     "TSP_TUNE_SWEEP_AHEAD": [-1, 0, 1, 2],
     "TSP_TUNE_STEP_GRAPH": [0, 1],
     "TSP_TUNE_JACOBI_REC24": [1, 0],
