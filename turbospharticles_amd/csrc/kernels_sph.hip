@@ -313,13 +313,32 @@ namespace tsp
             s.pending = 0;
             s.iters++;
             s.compute = (s.iters >= k.minIters && (k.termCond != 0 || terminated(s, k))) ? 1u : 0u;
+            for (uint32_t q = 0; q < kBarWords; q += kBarLine) { d.solveBar[static_cast<size_t>(sc) * kBarWords + q] = 0u; }
         }
+        for (uint32_t q = threadIdx.x; q < kFlagCopies * kSolveBlocksMost; q += kBlock) { d.solveFlag[q] = 0u; }
     }
 
-    // sum over the 64 lanes of a wave (a fixed xor tree: the same order on every run)
+    // the value of the lane `kRot` further in the lane's row of 16 (rotating)
+    template <int kRot>
+    __device__ __forceinline__ double rowRotate(double v)
+    {
+        const long long u = __double_as_longlong(v);
+        const int lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(u), 0x120 + kRot, 0xf, 0xf, true);
+        const int hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(u >> 32), 0x120 + kRot, 0xf, 0xf, true);
+        return __longlong_as_double(static_cast<long long>(hi) << 32 | static_cast<uint32_t>(lo));
+    }
+
+    // sum over the 64 lanes of a wave (a fixed xor tree: the same order on every run). After the steps of
+    // 32, 16 and 8 lanes a row repeats every 8 lanes, so a rotation by 4 pairs the lanes that an xor of 4
+    // pairs, and so on.
     __device__ __forceinline__ double waveSum(double v)
     {
-        for (int o = 32; o > 0; o >>= 1) { v += __shfl_xor(v, o, 64); }
+        v += __shfl_xor(v, 32, 64);
+        v += __shfl_xor(v, 16, 64);
+        v += rowRotate<8>(v);
+        v += rowRotate<4>(v);
+        v += rowRotate<2>(v);
+        v += rowRotate<1>(v);
         return v;
     }
 
@@ -397,6 +416,68 @@ namespace tsp
         __syncthreads();
     }
 
+    // the FR terms of a pressure acceleration
+    __device__ __forceinline__ void pressureFR(const Dev& d, const Lists& l, const Consts& k, const float4& p4, float& ax, float& ay, float& az)
+    {
+        visit(l.list(d, REL_FR), [&](uint32_t j)
+        {
+            const float4 rj = d.rpos[j];
+            const float dx = p4.x - rj.x, dy = p4.y - rj.y, dz = p4.z - rj.z;
+            const float f = kgFactor(dist2(dx, dy, dz), k);
+            const float coeff = k.presOuterB * rj.w * p4.w;
+            ax = __builtin_fmaf(coeff, f * dx, ax);
+            ay = __builtin_fmaf(coeff, f * dy, ay);
+            az = __builtin_fmaf(coeff, f * dz, az);
+        });
+    }
+
+    // the pressure acceleration of a particle at p4 (x, y, z, pressure): its FF sum over the staged halo, or
+    // over posOf(j) in a block without one, and its FB and FR sums
+    template <bool kFast, typename PosOf>
+    __device__ __forceinline__ void pressureAt(const Dev& d, const Lists& l, const SlotList& slots, const Halo& h, const float4* hp,
+        const Consts& k, const float4& p4, PosOf&& posOf, float (&a)[3])
+    {
+        const float xi = p4.x, yi = p4.y, zi = p4.z, pi = p4.w;
+        float sx = 0.0f, sy = 0.0f, sz = 0.0f;
+        // dict chunks sum (p_i + p_j) kg and scale once; normal chunks scale each neighbor's
+        // pressure term (sph_solver.cpp:1573-1640)
+        const bool dict = slots.n <= kDictMax;
+        const float outerF = k.mass * pi * k.presDis;
+        // the two forms as two loops (a wave runs the normal one only for a list longer than kDictMax)
+        const auto sumFF = [&](auto dictFlag)
+        {
+            constexpr bool kDict = decltype(dictFlag)::value;
+            // q: the pair's halo entry where its low bits correct kgShort (kShort)
+            const auto ffTerm = [&](const float4& pj, uint32_t q, auto shortFlag)
+            {
+                constexpr bool kShort = decltype(shortFlag)::value;
+                const float dx = xi - pj.x, dy = yi - pj.y, dz = zi - pj.z;
+                const float d2 = dist2(dx, dy, dz);
+                const float kg = kShort ? addUlps(kgShort(d2, k), q) : kgFactor<kFast>(d2, k);
+                const float coeff = (kDict ? pi + pj.w : outerF + k.mass * pj.w * k.presDis) * kg;
+                sx = __builtin_fmaf(coeff, dx, sx);
+                sy = __builtin_fmaf(coeff, dy, sy);
+                sz = __builtin_fmaf(coeff, dz, sz);
+            };
+            if (kFast && h.ulps) { visitSlots(slots, [&](uint32_t q, uint32_t) { ffTerm(recAt(hp, q & kSlotMask), q, Flag<true>{}); }); }
+            else if (h.any) { visitSlots(slots, [&](uint32_t q, uint32_t) { ffTerm(recAt(hp, q & kSlotMask), q, Flag<false>{}); }); }
+            else { visit(l.list(d, REL_FF), [&](uint32_t j) { ffTerm(posOf(j), 0u, Flag<false>{}); }); }
+        };
+        if (dict) { sumFF(Flag<true>{}); } else { sumFF(Flag<false>{}); }
+        float ax = dict ? sx * k.presOuterFF : sx, ay = dict ? sy * k.presOuterFF : sy, az = dict ? sz * k.presOuterFF : sz;
+        visitGather(d, l, REL_FB, [&](uint32_t j) { return d.bpos[j]; }, [&](const float4& bj)
+        {
+            const float dx = xi - bj.x, dy = yi - bj.y, dz = zi - bj.z;
+            const float f = kgFactor<kFast>(dist2(dx, dy, dz), k);
+            const float coeff = k.presOuterB * bj.w * pi;
+            ax = __builtin_fmaf(coeff, f * dx, ax);
+            ay = __builtin_fmaf(coeff, f * dy, ay);
+            az = __builtin_fmaf(coeff, f * dz, az);
+        });
+        pressureFR(d, l, k, p4, ax, ay, az);
+        a[0] = 0.0f - ax; a[1] = 0.0f - ay; a[2] = 0.0f - az;
+    }
+
     // a sweep's pressure accelerations; block 0 of a sweep launch first finishes the bookkeeping of
     // the previous Jacobi sweep, which the next Jacobi launch reads. Blocks that see the solve
     // converged skip their particles: the final launch (sweep = false) recomputes every a^p.
@@ -424,54 +505,9 @@ namespace tsp
         stageHalo(h, [&](uint32_t j) { return d.pos[j]; }, [&](uint32_t q, const float4& r) { hp[q] = r; });
         __syncthreads();
         if (i - S.offF >= S.nF) { return; }
-        const float xi = p4.x, yi = p4.y, zi = p4.z, pi = p4.w;
-        float sx = 0.0f, sy = 0.0f, sz = 0.0f;
-        // dict chunks sum (p_i + p_j) kg and scale once; normal chunks scale each neighbor's
-        // pressure term (sph_solver.cpp:1573-1640)
-        const bool dict = slots.n <= kDictMax;
-        const float outerF = k.mass * pi * k.presDis;
-        // the two forms as two loops (a wave runs the normal one only for a list longer than kDictMax)
-        const auto sumFF = [&](auto dictFlag)
-        {
-            constexpr bool kDict = decltype(dictFlag)::value;
-            // q: the pair's halo entry where its low bits correct kgShort (kShort)
-            const auto ffTerm = [&](const float4& pj, uint32_t q, auto shortFlag)
-            {
-                constexpr bool kShort = decltype(shortFlag)::value;
-                const float dx = xi - pj.x, dy = yi - pj.y, dz = zi - pj.z;
-                const float d2 = dist2(dx, dy, dz);
-                const float kg = kShort ? addUlps(kgShort(d2, k), q) : kgFactor<kFast>(d2, k);
-                const float coeff = (kDict ? pi + pj.w : outerF + k.mass * pj.w * k.presDis) * kg;
-                sx = __builtin_fmaf(coeff, dx, sx);
-                sy = __builtin_fmaf(coeff, dy, sy);
-                sz = __builtin_fmaf(coeff, dz, sz);
-            };
-            if (kFast && h.ulps) { visitSlots(slots, [&](uint32_t q, uint32_t) { ffTerm(recAt(hp, q & kSlotMask), q, Flag<true>{}); }); }
-            else if (h.any) { visitSlots(slots, [&](uint32_t q, uint32_t) { ffTerm(recAt(hp, q & kSlotMask), q, Flag<false>{}); }); }
-            else { visit(l.list(d, REL_FF), [&](uint32_t j) { ffTerm(d.pos[j], 0u, Flag<false>{}); }); }
-        };
-        if (dict) { sumFF(Flag<true>{}); } else { sumFF(Flag<false>{}); }
-        float ax = dict ? sx * k.presOuterFF : sx, ay = dict ? sy * k.presOuterFF : sy, az = dict ? sz * k.presOuterFF : sz;
-        visitGather(d, l, REL_FB, [&](uint32_t j) { return d.bpos[j]; }, [&](const float4& bj)
-        {
-            const float dx = xi - bj.x, dy = yi - bj.y, dz = zi - bj.z;
-            const float f = kgFactor<kFast>(dist2(dx, dy, dz), k);
-            const float coeff = k.presOuterB * bj.w * pi;
-            ax = __builtin_fmaf(coeff, f * dx, ax);
-            ay = __builtin_fmaf(coeff, f * dy, ay);
-            az = __builtin_fmaf(coeff, f * dz, az);
-        });
-        visit(l.list(d, REL_FR), [&](uint32_t j)
-        {
-            const float4 rj = d.rpos[j];
-            const float dx = xi - rj.x, dy = yi - rj.y, dz = zi - rj.z;
-            const float f = kgFactor(dist2(dx, dy, dz), k);
-            const float coeff = k.presOuterB * rj.w * pi;
-            ax = __builtin_fmaf(coeff, f * dx, ax);
-            ay = __builtin_fmaf(coeff, f * dy, ay);
-            az = __builtin_fmaf(coeff, f * dz, az);
-        });
-        d.ap[i] = make_float4(0.0f - ax, 0.0f - ay, 0.0f - az, 0.0f);
+        float a[3];
+        pressureAt<kFast>(d, l, slots, h, hp, k, p4, [&](uint32_t j) { return d.pos[j]; }, a);
+        d.ap[i] = make_float4(a[0], a[1], a[2], 0.0f);
     }
 
     template <bool kFast>
@@ -487,18 +523,122 @@ namespace tsp
     }
 
 
+    __device__ __forceinline__ void addError(float pred, const Consts& k, double& eRaw, double& ePos, double& eAbs)
+    {
+        const double e = static_cast<double>(pred / k.rho0);
+        eRaw += e;
+        ePos += 0.0 < e ? e : 0.0;
+        eAbs += __builtin_fabs(e);
+    }
+
+    // a block's error sums, in a fixed order; true in the thread that has them
+    __device__ __forceinline__ bool blockSums(double eRaw, double ePos, double eAbs, double (&red)[3][kSweepThreads / 64], double (&sum)[3])
+    {
+        eRaw = waveSum(eRaw);
+        ePos = waveSum(ePos);
+        eAbs = waveSum(eAbs);
+        const uint32_t w = threadIdx.x >> 6;
+        if ((threadIdx.x & 63u) == 0) { red[0][w] = eRaw; red[1][w] = ePos; red[2][w] = eAbs; }
+        __syncthreads();
+        if (threadIdx.x != 0) { return false; }
+        for (int r = 0; r < 3; r++)
+        {
+            sum[r] = 0.0;
+            for (uint32_t q = 0; q < kSweepThreads / 64; q++) { sum[r] += red[r][q]; }
+        }
+        return true;
+    }
+
+    // a neighbor of a Jacobi sweep: position and a^p
+    struct SweepRec
+    {
+        float x, y, z, ax, ay, az;
+    };
+
+    // the FR terms of a Jacobi sweep
+    __device__ __forceinline__ void relaxedFR(const Dev& d, const Lists& l, const Consts& k, const float4& at, float axi, float ayi, float azi,
+        float& sb)
+    {
+        visit(l.list(d, REL_FR), [&](uint32_t j)
+        {
+            const float4 rj = d.rpos[j];
+            const float dx = at.x - rj.x, dy = at.y - rj.y, dz = at.z - rj.z;
+            const float f = kgFactor(dist2(dx, dy, dz), k);
+            const float sv = __builtin_fmaf(axi, f * dx, __builtin_fmaf(ayi, f * dy, azi * (f * dz)));
+            sb += rj.w * sv;
+        });
+    }
+
+    // the relaxed pressure from the sums over fluid and boundary, and the predicted density error
+    __device__ __forceinline__ float relaxedOf(const Consts& k, float sf, float sb, float p, float src, float diag, float& pred)
+    {
+        const float sys = k.dtsq * (sf + sb);
+        const float resid = src - sys;
+        pred = sys - src;
+        const bool valid = __builtin_fabsf(diag) > 1e-7f;
+        return vmax(0.0f, valid ? __builtin_fmaf(k.omega, resid / diag, p) : 0.0f);
+    }
+
+    // the relaxed pressure of a particle at `at` with acceleration ai and pressure p, and its predicted
+    // density error; hp and ha hold the halo as (x, y, z, a^p x | a^p y, a^p z), 24 KB per block: six
+    // blocks per CU; recOf(j) in a block without one
+    template <bool kFast, typename RecOf>
+    __device__ __forceinline__ float relaxedAt(const Dev& d, const Lists& l, const SlotList& slots, const Halo& h, const float4* hp,
+        const float2* ha, const Consts& k, const float4& at, const float4& ai, float p, float src, float diag, RecOf&& recOf,
+        float& pred)
+    {
+        const float xi = at.x, yi = at.y, zi = at.z, axi = ai.x, ayi = ai.y, azi = ai.z;
+        float sf = 0.0f;
+        const auto ffTerm = [&](float xj, float yj, float zj, float axj, float ayj, float azj, uint32_t q, auto shortFlag)
+        {
+            constexpr bool kShort = decltype(shortFlag)::value;
+            const float dx = xi - xj, dy = yi - yj, dz = zi - zj;
+            const float d2 = dist2(dx, dy, dz);
+            const float kg = kShort ? addUlps(kgShort(d2, k), q) : kgFactor<kFast>(d2, k);
+            const float sv = __builtin_fmaf(axi - axj, dx, __builtin_fmaf(ayi - ayj, dy, (azi - azj) * dz));
+            sf = __builtin_fmaf(kg, sv, sf);
+        };
+        const auto haloLoad = [&](uint32_t q)
+        {
+            const float4 pj = recAt(hp, q);
+            const float2 aj = recAt(ha, q);
+            return SweepRec{ pj.x, pj.y, pj.z, pj.w, aj.x, aj.y };
+        };
+        const auto fromHalo = [&](uint32_t q, auto shortFlag)
+        {
+            const SweepRec r = haloLoad(q & kSlotMask);
+            ffTerm(r.x, r.y, r.z, r.ax, r.ay, r.az, q, shortFlag);
+        };
+        if (kFast && h.ulps) { visitSlots(slots, [&](uint32_t q, uint32_t) { fromHalo(q, Flag<true>{}); }); }
+        else if (h.any) { visitSlots(slots, [&](uint32_t q, uint32_t) { fromHalo(q, Flag<false>{}); }); }
+        else
+        {
+            visit(l.list(d, REL_FF), [&](uint32_t j)
+            {
+                const SweepRec r = recOf(j);
+                ffTerm(r.x, r.y, r.z, r.ax, r.ay, r.az, 0u, Flag<false>{});
+            });
+        }
+        sf *= k.mass;
+        float sb = 0.0f;
+        visitGather(d, l, REL_FB, [&](uint32_t j) { return d.bpos[j]; }, [&](const float4& bj)
+        {
+            const float dx = xi - bj.x, dy = yi - bj.y, dz = zi - bj.z;
+            const float f = kgFactor<kFast>(dist2(dx, dy, dz), k);
+            const float sv = __builtin_fmaf(axi, f * dx, __builtin_fmaf(ayi, f * dy, azi * (f * dz)));
+            sb += bj.w * sv;
+        });
+        relaxedFR(d, l, k, at, axi, ayi, azi, sb);
+        return relaxedOf(k, sf, sb, p, src, diag, pred);
+    }
+
     // one tile of a Jacobi sweep; nTot is the number of tiles (the stride of the error partials)
     template <bool kFast>
     __device__ __forceinline__ void jacobiTile(const Dev& d, uint32_t blk, uint32_t nTot)
     {
         __shared__ double red[3][kSweepThreads / 64];
-#if TSP_TUNE_JACOBI_REC24
-        // 24-byte halo records (x, y, z, a^p x | a^p y, a^p z): 24 KB per block, six blocks per CU
         __shared__ float4 hp[kHaloMax];
         __shared__ float2 ha[kHaloMax];
-#else
-        __shared__ float4 hp[kHaloMax], ha[kHaloMax];
-#endif
         const Lists l = listsAt(d, blk);
         const SlotList slots = slotsOf(d, l);
         const Halo h = haloOf(d, blk);
@@ -512,110 +652,30 @@ namespace tsp
         const uint32_t i = l.i;
         const float4 pi = d.pos[i], ai = d.ap[i];
         const float src = d.source[i], diag = d.diag[i];
-#if TSP_TUNE_JACOBI_REC24
         stageHalo(h, [&](uint32_t j) { return Pair4{ d.pos[j], d.ap[j] }; }, [&](uint32_t q, const Pair4& r)
         {
             hp[q] = make_float4(r.a.x, r.a.y, r.a.z, r.b.x);
             ha[q] = make_float2(r.b.y, r.b.z);
         });
-#else
-        stageHalo(h, [&](uint32_t j) { return Pair4{ d.pos[j], d.ap[j] }; }, [&](uint32_t q, const Pair4& r) { hp[q] = r.a; ha[q] = r.b; });
-#endif
         __syncthreads();
         double eRaw = 0.0, ePos = 0.0, eAbs = 0.0;
         if (i - S.offF < S.nF)
         {
-            const float xi = pi.x, yi = pi.y, zi = pi.z, axi = ai.x, ayi = ai.y, azi = ai.z;
-            float sf = 0.0f;
-            const auto ffTerm = [&](float xj, float yj, float zj, float axj, float ayj, float azj, uint32_t q, auto shortFlag)
+            float pred;
+            d.pos[i].w = relaxedAt<kFast>(d, l, slots, h, hp, ha, k, pi, ai, pi.w, src, diag, [&](uint32_t j)
             {
-                constexpr bool kShort = decltype(shortFlag)::value;
-                const float dx = xi - xj, dy = yi - yj, dz = zi - zj;
-                const float d2 = dist2(dx, dy, dz);
-                const float kg = kShort ? addUlps(kgShort(d2, k), q) : kgFactor<kFast>(d2, k);
-                const float sv = __builtin_fmaf(axi - axj, dx, __builtin_fmaf(ayi - ayj, dy, (azi - azj) * dz));
-                sf = __builtin_fmaf(kg, sv, sf);
-            };
-            // a halo record: position and a^p of one neighbor
-            struct Rec
-            {
-                float x, y, z, ax, ay, az;
-            };
-#if TSP_TUNE_JACOBI_REC24
-            const auto haloLoad = [&](uint32_t q)
-            {
-                const float4 pj = recAt(hp, q);
-                const float2 aj = recAt(ha, q);
-                return Rec{ pj.x, pj.y, pj.z, pj.w, aj.x, aj.y };
-            };
-#else
-            const auto haloLoad = [&](uint32_t q)
-            {
-                const float4 pj = recAt(hp, q), aj = recAt(ha, q);
-                return Rec{ pj.x, pj.y, pj.z, aj.x, aj.y, aj.z };
-            };
-#endif
-            const auto fromHalo = [&](uint32_t q, auto shortFlag)
-            {
-                const Rec r = haloLoad(q & kSlotMask);
-                ffTerm(r.x, r.y, r.z, r.ax, r.ay, r.az, q, shortFlag);
-            };
-            if (kFast && h.ulps) { visitSlots(slots, [&](uint32_t q, uint32_t) { fromHalo(q, Flag<true>{}); }); }
-            else if (h.any) { visitSlots(slots, [&](uint32_t q, uint32_t) { fromHalo(q, Flag<false>{}); }); }
-            else
-            {
-                visit(l.list(d, REL_FF), [&](uint32_t j)
-                {
-                    const float4 pj = d.pos[j], aj = d.ap[j];
-                    ffTerm(pj.x, pj.y, pj.z, aj.x, aj.y, aj.z, 0u, Flag<false>{});
-                });
-            }
-            sf *= k.mass;
-            float sb = 0.0f;
-            visitGather(d, l, REL_FB, [&](uint32_t j) { return d.bpos[j]; }, [&](const float4& bj)
-            {
-                const float dx = xi - bj.x, dy = yi - bj.y, dz = zi - bj.z;
-                const float f = kgFactor<kFast>(dist2(dx, dy, dz), k);
-                const float sv = __builtin_fmaf(axi, f * dx, __builtin_fmaf(ayi, f * dy, azi * (f * dz)));
-                sb += bj.w * sv;
-            });
-            visit(l.list(d, REL_FR), [&](uint32_t j)
-            {
-                const float4 rj = d.rpos[j];
-                const float dx = xi - rj.x, dy = yi - rj.y, dz = zi - rj.z;
-                const float f = kgFactor(dist2(dx, dy, dz), k);
-                const float sv = __builtin_fmaf(axi, f * dx, __builtin_fmaf(ayi, f * dy, azi * (f * dz)));
-                sb += rj.w * sv;
-            });
-            const float sys = k.dtsq * (sf + sb);
-            const float resid = src - sys;
-            const float pred = sys - src;
+                const float4 pj = d.pos[j], aj = d.ap[j];
+                return SweepRec{ pj.x, pj.y, pj.z, aj.x, aj.y, aj.z };
+            }, pred);
             const bool valid = __builtin_fabsf(diag) > 1e-7f;
-            d.pos[i].w = vmax(0.0f, valid ? __builtin_fmaf(k.omega, resid / diag, pi.w) : 0.0f);
-            if (compute && valid)
-            {
-                const double e = static_cast<double>(pred / k.rho0);
-                eRaw += e;
-                ePos += 0.0 < e ? e : 0.0;
-                eAbs += __builtin_fabs(e);
-            }
+            if (compute && valid) { addError(pred, k, eRaw, ePos, eAbs); }
         }
         if (blk == S.blk0 && threadIdx.x == 0) { d.solve[sc].pending = 1u; }
         if (!compute) { return; }
-        eRaw = waveSum(eRaw);
-        ePos = waveSum(ePos);
-        eAbs = waveSum(eAbs);
-        const uint32_t w = threadIdx.x >> 6;
-        if ((threadIdx.x & 63u) == 0) { red[0][w] = eRaw; red[1][w] = ePos; red[2][w] = eAbs; }
-        __syncthreads();
-        if (threadIdx.x == 0)
+        double sum[3];
+        if (blockSums(eRaw, ePos, eAbs, red, sum))
         {
-            for (int r = 0; r < 3; r++)
-            {
-                double s = 0.0;
-                for (uint32_t q = 0; q < kSweepThreads / 64; q++) { s += red[r][q]; }
-                d.errPartial[static_cast<size_t>(r) * nTot + blk] = s;
-            }
+            for (int r = 0; r < 3; r++) { d.errPartial[static_cast<size_t>(r) * nTot + blk] = sum[r]; }
         }
     }
 
@@ -624,6 +684,473 @@ namespace tsp
     {
         if (stopped(d)) { return; }
         jacobiTile<kFast>(d, xcdBlock(), nTiles);
+    }
+
+    // --- the whole solve in one launch, for a context of few blocks ---
+    // A sweep of 64,000 particles is two launches of 9 to 10 us with 4 us between them, of which the pair
+    // sums take a third: the rest is launch, drain and the loads that every launch repeats. Here the blocks
+    // stay: positions, list heads and the particle's own values are loaded once, each half sweep
+    // gathers only what the other half wrote, and the blocks of a scene meet at a barrier after it (the
+    // scenes are independent). The bookkeeping of a sweep is done by every block for itself from the
+    // partial sums, in the order of finalizeSweep, beside the next accelerations; those of the sweep that
+    // converged are the final ones. No host read, and the same bits. A sweep of 64,000 particles: 27 us launch
+    // by launch, 11.8 here (a fifth each the two sums, a quarter each the two barriers); 4,096 particles: 17
+    // and 10.5. With two blocks per CU (111,000 particles) it was no faster than the launches.
+    // The blocks must all be resident: the host asks for at most one per CU, and the first barrier, before
+    // anything is written, gives up when other work keeps some block out for kEntrySpins polls: the scene's
+    // blocks then leave together, and the host runs the sweeps launch by launch. Past the first
+    // barrier every block of the scene is running.
+    constexpr uint32_t kEntrySpins = 4000;
+    constexpr uint32_t kBarSpins = 1u << 20;
+    // offsets into a scene's entry words: arrivals, and the outcome
+    constexpr uint32_t kBarArrived = 0, kBarEntry = kBarLine;
+    constexpr uint32_t kEntryOpen = 0, kEntryGo = 1, kEntryGaveUp = 2;
+
+    // What another block reads in the same launch goes past the L2 of the block's XCD both ways: device-scope
+    // words.
+    __device__ __forceinline__ void putWord(float* p, float v)
+    {
+        __hip_atomic_store(reinterpret_cast<uint32_t*>(p), __float_as_uint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ __forceinline__ float getWord(const float* p)
+    {
+        return __uint_as_float(__hip_atomic_load(reinterpret_cast<const uint32_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    }
+    __device__ __forceinline__ void putAcc(float4* p, float x, float y, float z)
+    {
+        unsigned long long* w = reinterpret_cast<unsigned long long*>(p);
+        __hip_atomic_store(w, static_cast<unsigned long long>(__float_as_uint(y)) << 32 | __float_as_uint(x), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(w + 1, static_cast<unsigned long long>(__float_as_uint(z)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ __forceinline__ float4 getAcc(const float4* p)
+    {
+        const unsigned long long* w = reinterpret_cast<const unsigned long long*>(p);
+        const unsigned long long a = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned long long b = __hip_atomic_load(w + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return make_float4(__uint_as_float(static_cast<uint32_t>(a)), __uint_as_float(static_cast<uint32_t>(a >> 32)),
+                           __uint_as_float(static_cast<uint32_t>(b)), 0.0f);
+    }
+
+    // a value that is the same in every lane
+    __device__ __forceinline__ float uniform(float v)
+    {
+        return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+    }
+
+    // The n-th barrier (from 1) of a scene's blocks, in two halves. Arrival, all threads: every store before it
+    // has reached memory (the wait is for the stores themselves: they carry the device scope, no cache
+    // holds them back) before the block raises its flag to n. A flag per block, all read by the waiting
+    // wave at once, in as many copies as there are XCDs (readers of one line queue up): from the last of 250
+    // arrivals on 3,700 cycles at least; 5,000 with one copy, 6,300 with a counter and a word that says go.
+    __device__ __forceinline__ void arriveScene(uint32_t* flags, uint32_t blk, uint32_t n)
+    {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        const uint32_t copy = threadIdx.x - (kSweepThreads - 64u);
+        if (copy < kFlagCopies)
+        {
+            __hip_atomic_store(&flags[copy * kSolveBlocksMost + blk], n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+
+    // The wait for the others, all threads (the last wave polls). False when the block gave up waiting
+    // (never expected).
+    __device__ __forceinline__ bool meetScene(const uint32_t* flags, const Scene& S, uint32_t n, uint32_t* fail)
+    {
+        __shared__ uint32_t met;
+        if (threadIdx.x >= kSweepThreads - 64u)
+        {
+            constexpr uint32_t kPolls = kSolveBlocksMost / 64u;
+            const uint32_t lane = threadIdx.x & 63u;
+            flags += (blockIdx.x & (kFlagCopies - 1u)) * kSolveBlocksMost + S.blk0;
+            uint32_t spins = 0;
+            for (;;)
+            {
+                uint32_t f[kPolls];
+                for (uint32_t q = 0; q < kPolls; q++)
+                {
+                    const uint32_t b = q * 64u + lane;
+                    f[q] = b < S.nBlk ? __hip_atomic_load(&flags[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : n;
+                }
+                bool here = true;
+                for (uint32_t q = 0; q < kPolls; q++) { here = here && f[q] >= n; }
+                if (__ballot(!here) == 0ull) { break; }
+                if (++spins > kBarSpins) { break; }
+            }
+            if (lane == 0u)
+            {
+                met = spins <= kBarSpins;
+                if (spins > kBarSpins) { atomicOr(fail, 1u); }
+            }
+        }
+        __syncthreads();
+        return met != 0u;
+    }
+
+    // the first barrier: true for all blocks of the scene, or false for all
+    __device__ __forceinline__ bool enterScene(uint32_t* bar, uint32_t nBlk)
+    {
+        __shared__ uint32_t outcome;
+        if (threadIdx.x == 0)
+        {
+            uint32_t seen = kEntryOpen;
+            const uint32_t before = __hip_atomic_fetch_add(&bar[kBarArrived], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (before + 1u == nBlk)
+            {
+                // (seen comes back as what was there: gave up, or open)
+                if (__hip_atomic_compare_exchange_strong(&bar[kBarEntry], &seen, kEntryGo, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                         __HIP_MEMORY_SCOPE_AGENT)) { seen = kEntryGo; }
+            }
+            else
+            {
+                for (uint32_t spins = 0; seen == kEntryOpen; spins++)
+                {
+                    seen = __hip_atomic_load(&bar[kBarEntry], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if (seen == kEntryOpen && spins >= kEntrySpins)
+                    {
+                        if (__hip_atomic_compare_exchange_strong(&bar[kBarEntry], &seen, kEntryGaveUp, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                                 __HIP_MEMORY_SCOPE_AGENT)) { seen = kEntryGaveUp; }
+                    }
+                }
+            }
+            outcome = seen;
+        }
+        __syncthreads();
+        return outcome == kEntryGo;
+    }
+
+    // What a thread keeps of its pairs for the whole solve, in a wave whose FF lists have at most kKeepFF
+    // entries: the FF entries' distances, gradient factors and halo slots in registers, and the FB entries'
+    // gradients and psi in LDS (the first kRowsFB entries; further ones in d.fbGrad, each read by the
+    // thread that wrote it). A half sweep then gathers 4 or 12 bytes per pair from LDS instead of 16 or 24, which is what the sums
+    // are bound by (64 records of 16 bytes at random places take the LDS about 25 cycles, three times what
+    // they take in a row), and computes a third.
+    constexpr uint32_t kKeepFF = 40;
+    constexpr uint32_t kRowsFB = 20;
+
+    struct Kept
+    {
+        float dx[kKeepFF], dy[kKeepFF], dz[kKeepFF], kg[kKeepFF];
+        uint32_t slots[kKeepFF / 2];   // two entries each
+        uint32_t n, pitch, nAll;       // of the FF list, of its slice, and of the wave's shortest list
+        uint32_t nB;
+        float4* fb;                    // the lane's FB record in row 0, in LDS; from row kRowsFB on in memory
+        float4* fbMore;
+
+        __device__ __forceinline__ uint32_t slot(uint32_t q) const { return (q & 1u) ? slots[q / 2u] >> 16 : slots[q / 2u] & 0xffffu; }
+
+        template <bool kFast>
+        __device__ __forceinline__ void fill(const Dev& d, const Lists& l, const SlotList& s, const Halo& h, const float4* hp,
+            float4* rows, const Consts& k, const float4& at)
+        {
+            n = s.n;
+            pitch = s.pitch;
+            uint32_t m = n;
+            for (int o = 32; o > 0; o >>= 1) { m = min(m, static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), o, 64))); }
+            nAll = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(m)));
+            const auto put = [&](uint32_t q, uint32_t entry, auto shortFlag)
+            {
+                constexpr bool kShort = decltype(shortFlag)::value;
+                const float4& pj = recAt(hp, entry & kSlotMask);
+                dx[q] = at.x - pj.x; dy[q] = at.y - pj.y; dz[q] = at.z - pj.z;
+                const float d2 = dist2(dx[q], dy[q], dz[q]);
+                kg[q] = kShort ? addUlps(kgShort(d2, k), entry) : kgFactor<kFast>(d2, k);
+            };
+#pragma unroll
+            for (uint32_t q = 0; q < kKeepFF; q += 2u)
+            {
+                // (an entry past the list repeats the first one, or slot 0, and is not used)
+                uint32_t e0 = s.p[(q < n ? q : 0u) * kSlice], e1 = s.p[(q + 1u < n ? q + 1u : 0u) * kSlice];
+                e0 = n ? e0 : 0u;
+                e1 = n ? e1 : 0u;
+                if (kFast && h.ulps) { put(q, e0, Flag<true>{}); put(q + 1u, e1, Flag<true>{}); }
+                else { put(q, e0, Flag<false>{}); put(q + 1u, e1, Flag<false>{}); }
+                slots[q / 2u] = (e0 & kSlotMask) | (e1 & kSlotMask) << 16;
+            }
+            nB = l.n[REL_FB];
+            fb = rows;
+            fbMore = d.fbGrad + l.m[REL_FB].offset + l.lane;
+            uint32_t row = 0;
+            visitGather(d, l, REL_FB, [&](uint32_t j) { return d.bpos[j]; }, [&](const float4& bj)
+            {
+                const float dx = at.x - bj.x, dy = at.y - bj.y, dz = at.z - bj.z;
+                const float f = kgFactor<kFast>(dist2(dx, dy, dz), k);
+                const float4 g = make_float4(f * dx, f * dy, f * dz, bj.w);
+                if (row < kRowsFB) { fb[row * kBlock] = g; } else { fbMore[row * kSlice] = g; }
+                row++;
+            });
+        }
+
+        // visits the FF entries in list order, as use(q, load(slot)); four entries load while the four before
+        // are summed
+        template <typename Load, typename Use>
+        __device__ __forceinline__ void visitFF(Load&& load, Use&& use)
+        {
+            using R = decltype(load(0u));
+            // (opaque here: unpacked ahead of the sweeps' loop they would take twice the registers)
+#pragma unroll
+            for (uint32_t q = 0; q < kKeepFF / 2u; q++) { asm volatile("" : "+v"(slots[q])); }
+            asm volatile("" : "+v"(n));
+            R r0 = load(slot(0u)), r1 = load(slot(1u)), r2 = load(slot(2u)), r3 = load(slot(3u));
+#pragma unroll
+            for (uint32_t q = 0; q < kKeepFF; q += 4u)
+            {
+                if (q < pitch)
+                {
+                    R n0{}, n1{}, n2{}, n3{};
+                    if (q + 4u < kKeepFF)
+                    {
+                        n0 = load(slot(q + 4u)); n1 = load(slot(q + 5u)); n2 = load(slot(q + 6u)); n3 = load(slot(q + 7u));
+                    }
+                    if (q + 4u <= nAll) { use(q, r0); use(q + 1u, r1); use(q + 2u, r2); use(q + 3u, r3); }
+                    else
+                    {
+                        if (q < n) { use(q, r0); }
+                        if (q + 1u < n) { use(q + 1u, r1); }
+                        if (q + 2u < n) { use(q + 2u, r2); }
+                        if (q + 3u < n) { use(q + 3u, r3); }
+                    }
+                    r0 = n0; r1 = n1; r2 = n2; r3 = n3;
+                }
+            }
+        }
+
+        template <typename Use>
+        __device__ __forceinline__ void visitFB(Use&& use) const
+        {
+            uint32_t q = 0;
+            const uint32_t near = min(nB, kRowsFB);
+            for (; q + 4u <= near; q += 4u)
+            {
+                const float4 b0 = fb[q * kBlock], b1 = fb[(q + 1u) * kBlock], b2 = fb[(q + 2u) * kBlock], b3 = fb[(q + 3u) * kBlock];
+                use(b0); use(b1); use(b2); use(b3);
+            }
+            for (; q < near; q++) { use(fb[q * kBlock]); }
+            for (; q < nB; q++) { use(fbMore[q * kSlice]); }
+        }
+
+        // pressureAt and relaxedAt from what is kept
+        __device__ __forceinline__ void pressure(const Dev& d, const Lists& l, const float* hw, const Consts& k, const float4& p4,
+            float (&a)[3])
+        {
+            const float pi = p4.w;
+            float sx = 0.0f, sy = 0.0f, sz = 0.0f;
+            visitFF([&](uint32_t e) { return hw[e >> kSlotShift]; }, [&](uint32_t q, float pj)
+            {
+                const float coeff = (pi + pj) * kg[q];
+                sx = __builtin_fmaf(coeff, dx[q], sx);
+                sy = __builtin_fmaf(coeff, dy[q], sy);
+                sz = __builtin_fmaf(coeff, dz[q], sz);
+            });
+            float ax = sx * k.presOuterFF, ay = sy * k.presOuterFF, az = sz * k.presOuterFF;
+            visitFB([&](const float4& g)
+            {
+                const float coeff = k.presOuterB * g.w * pi;
+                ax = __builtin_fmaf(coeff, g.x, ax);
+                ay = __builtin_fmaf(coeff, g.y, ay);
+                az = __builtin_fmaf(coeff, g.z, az);
+            });
+            pressureFR(d, l, k, p4, ax, ay, az);
+            a[0] = 0.0f - ax; a[1] = 0.0f - ay; a[2] = 0.0f - az;
+        }
+
+        __device__ __forceinline__ float relaxed(const Dev& d, const Lists& l, const float* hw, const float2* ha, const Consts& k,
+            const float4& p4, const float (&a)[3], float src, float diag, float& pred)
+        {
+            struct Acc
+            {
+                float x;
+                float2 yz;
+            };
+            float sf = 0.0f;
+            visitFF([&](uint32_t e) { return Acc{ hw[e >> kSlotShift], recAt(ha, e) }; }, [&](uint32_t q, const Acc& r)
+            {
+                sf = __builtin_fmaf(kg[q], __builtin_fmaf(a[0] - r.x, dx[q],
+                                    __builtin_fmaf(a[1] - r.yz.x, dy[q], (a[2] - r.yz.y) * dz[q])), sf);
+            });
+            sf *= k.mass;
+            float sb = 0.0f;
+            visitFB([&](const float4& g)
+            {
+                sb += g.w * __builtin_fmaf(a[0], g.x, __builtin_fmaf(a[1], g.y, a[2] * g.z));
+            });
+            relaxedFR(d, l, k, p4, a[0], a[1], a[2], sb);
+            return relaxedOf(k, sf, sb, p4.w, src, diag, pred);
+        }
+    };
+
+    template <bool kFast>
+    __global__ void __launch_bounds__(kSweepThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) kSolve(Dev d)
+    {
+        __shared__ double red[3][kSweepThreads / 64];
+        __shared__ double part[3][kSolveBlocksMost];
+        __shared__ double sums[3];
+        __shared__ float4 hp[kHaloMax];
+        __shared__ float2 ha[kHaloMax];
+        __shared__ float hw[kHaloMax];   // hp's last word by itself
+        __shared__ float4 fbRows[kRowsFB * kBlock];
+        const uint32_t nTot = gridDim.x, t = threadIdx.x;
+        const uint32_t blk = xcdBlock();
+        const Lists l = listsAt(d, blk);
+        const SlotList slots = slotsOf(d, l);
+        Halo h = haloOf(d, blk);
+        const uint32_t sc = uniformLoad(&d.blockScene[blk]);
+        const Consts k = uniformLoad(&d.consts[sc]);
+        const Scene S = uniformLoad(&d.scenes[sc]);
+        const uint32_t i = l.i;
+        float4 p4 = d.pos[i];
+        const float src = d.source[i], diag = d.diag[i];
+        const bool active = i - S.offF < S.nF;
+        stageHalo(h, [&](uint32_t j) { return d.pos[j]; }, [&](uint32_t q, const float4& r) { hp[q] = r; hw[q] = r.w; });
+        // the state that kSolverInit left; every thread keeps it (nothing of it is read here again)
+        Solve s = uniformLoad(&d.solve[sc]);
+        uint32_t* bar = d.solveBar + static_cast<size_t>(sc) * kBarWords;
+        if (!enterScene(bar, S.nBlk)) { return; }   // (a barrier: the halo is staged)
+        Kept kept;
+        const bool keep = h.any && __ballot(active && l.n[REL_FF] > kKeepFF) == 0ull;
+        if (keep && active) { kept.fill<kFast>(d, l, slots, h, hp, fbRows + t, k, p4); }
+        const bool valid = __builtin_fabsf(diag) > 1e-7f;
+        uint32_t meet = 0;
+        for (;;)
+        {
+            const bool pending = meet != 0u;
+            // (opaque: the addresses are made in each round)
+            for (uint32_t u = 0; u < Halo::kPer; u++) { asm volatile("" : "+v"(h.j[u])); }
+            if (pending)
+            {
+                // the pressures of the sweep before and, if it took its errors, all blocks' sums of them
+                float w[Halo::kPer];
+                for (uint32_t u = 0; u < Halo::kPer; u++)
+                {
+                    if (u * kBlock < h.count) { w[u] = getWord(&d.pos[u * kBlock + t < h.count ? h.j[u] : 0u].w); }
+                }
+                if (s.compute)
+                {
+                    for (int r = 0; r < 3; r++)
+                    {
+                        const unsigned long long* from = reinterpret_cast<const unsigned long long*>(d.errPartial)
+                                                       + static_cast<size_t>(r) * nTot + S.blk0;
+                        for (uint32_t b = t; b < kSolveBlocksMost; b += kSweepThreads)
+                        {
+                            if (b < S.nBlk)
+                            {
+                                part[r][b] = __longlong_as_double(static_cast<long long>(
+                                    __hip_atomic_load(&from[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)));
+                            }
+                        }
+                    }
+                }
+                for (uint32_t u = 0; u < Halo::kPer; u++) { if (u * kBlock + t < h.count) { hp[u * kBlock + t].w = w[u]; hw[u * kBlock + t] = w[u]; } }
+                __syncthreads();
+            }
+            float a[3] = { 0.0f, 0.0f, 0.0f };
+            if (active)
+            {
+                if (keep) { kept.pressure(d, l, hw, k, p4, a); }
+                else
+                {
+                    pressureAt<kFast>(d, l, slots, h, hp, k, p4, [&](uint32_t j)
+                    {
+                        const float4 q = d.pos[j];
+                        return make_float4(q.x, q.y, q.z, getWord(&d.pos[j].w));
+                    }, a);
+                }
+                putAcc(&d.ap[i], a[0], a[1], a[2]);
+            }
+            arriveScene(d.solveFlag, blk, ++meet);
+            if (pending)
+            {
+                // finalizeSweep's sums, in its order (a wave per sum), and its decision
+                s.sweeps++;
+                if (s.compute)
+                {
+                    const uint32_t r = t >> 6;
+                    if (r < 3u)
+                    {
+                        double v[kSweepThreads / 64];
+                        for (uint32_t w = 0; w < kSweepThreads / 64; w++)
+                        {
+                            v[w] = 0.0;
+                            for (uint32_t b = w * 64u + (t & 63u); b < S.nBlk; b += kSweepThreads) { v[w] += part[r][b]; }
+                        }
+                        for (uint32_t w = 0; w < kSweepThreads / 64; w++) { v[w] = waveSum(v[w]); }
+                        double sum = v[0];
+                        for (uint32_t w = 1; w < kSweepThreads / 64; w++) { sum += v[w]; }
+                        if ((t & 63u) == 0u) { sums[r] = sum; }
+                    }
+                    __syncthreads();
+                    const float n = static_cast<float>(S.nF);
+                    s.avgRaw = uniform(static_cast<float>(sums[0]) / n);
+                    s.avgPos = uniform(static_cast<float>(sums[1]) / n);
+                    s.avgAbs = uniform(static_cast<float>(sums[2]) / n);
+                    if (blk == S.blk0 && t == 0)
+                    {
+                        Solve& out = d.solve[sc];
+                        out.sumRaw = sums[0]; out.sumPos = sums[1]; out.sumAbs = sums[2];
+                        out.avgRaw = s.avgRaw; out.avgPos = s.avgPos; out.avgAbs = s.avgAbs;
+                    }
+                }
+                if (terminated(s, k)) { break; }
+                s.iters++;
+                s.compute = (s.iters >= k.minIters && (k.termCond != 0 || terminated(s, k))) ? 1u : 0u;
+            }
+            if (!meetScene(d.solveFlag, S, meet, &d.status->scanFail)) { return; }
+            {
+                float4 w[Halo::kPer];
+                for (uint32_t u = 0; u < Halo::kPer; u++)
+                {
+                    if (u * kBlock < h.count) { w[u] = getAcc(&d.ap[u * kBlock + t < h.count ? h.j[u] : 0u]); }
+                }
+                for (uint32_t u = 0; u < Halo::kPer; u++)
+                {
+                    if (u * kBlock + t < h.count)
+                    {
+                        hp[u * kBlock + t].w = w[u].x;
+                        hw[u * kBlock + t] = w[u].x;
+                        ha[u * kBlock + t] = make_float2(w[u].y, w[u].z);
+                    }
+                }
+                __syncthreads();
+            }
+            double eRaw = 0.0, ePos = 0.0, eAbs = 0.0;
+            if (active)
+            {
+                float pred;
+                if (keep) { p4.w = kept.relaxed(d, l, hw, ha, k, p4, a, src, diag, pred); }
+                else
+                {
+                    p4.w = relaxedAt<kFast>(d, l, slots, h, hp, ha, k, p4, make_float4(a[0], a[1], a[2], 0.0f), p4.w, src, diag, [&](uint32_t j)
+                    {
+                        const float4 pj = d.pos[j], aj = getAcc(&d.ap[j]);
+                        return SweepRec{ pj.x, pj.y, pj.z, aj.x, aj.y, aj.z };
+                    }, pred);
+                }
+                putWord(&d.pos[i].w, p4.w);
+                if (s.compute && valid) { addError(pred, k, eRaw, ePos, eAbs); }
+            }
+            if (s.compute)
+            {
+                double sum[3];
+                if (blockSums(eRaw, ePos, eAbs, red, sum))
+                {
+                    for (int r = 0; r < 3; r++)
+                    {
+                        __hip_atomic_store(reinterpret_cast<unsigned long long*>(d.errPartial) + static_cast<size_t>(r) * nTot + blk,
+                                           static_cast<unsigned long long>(__double_as_longlong(sum[r])), __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT);
+                    }
+                }
+            }
+            arriveScene(d.solveFlag, blk, ++meet);
+            if (!meetScene(d.solveFlag, S, meet, &d.status->scanFail)) { return; }
+        }
+        if (blk == S.blk0 && t == 0)
+        {
+            Solve& out = d.solve[sc];
+            out.iters = s.iters; out.sweeps = s.sweeps; out.compute = s.compute; out.converged = 1u;
+        }
     }
 
     // the bookkeeping of the last sweep of a group, one block per scene, before the host reads
@@ -881,6 +1408,12 @@ namespace tsp
         const uint32_t n = blocksOf(d.nF);
         if (d.fastPairs) { kJacobi<true><<<n, kSweepThreads, 0, s>>>(d, n); }
         else { kJacobi<false><<<n, kSweepThreads, 0, s>>>(d, n); }
+    }
+    void launchSolve(hipStream_t s, const Dev& d)
+    {
+        if (!d.nF) { return; }
+        if (d.fastPairs) { kSolve<true><<<blocksOf(d.nF), kSweepThreads, 0, s>>>(d); }
+        else { kSolve<false><<<blocksOf(d.nF), kSweepThreads, 0, s>>>(d); }
     }
     void launchFinalize(hipStream_t s, const Dev& d)
     {

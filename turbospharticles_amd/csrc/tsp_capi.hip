@@ -59,6 +59,7 @@ namespace tsp
     void launchPressureAcc(hipStream_t, const Dev&, bool);
     void launchJacobi(hipStream_t, const Dev&);
     void launchFinalize(hipStream_t, const Dev&);
+    void launchSolve(hipStream_t, const Dev&);
     void launchIntegration(hipStream_t, const Dev&);
     void launchRigidUpdate(hipStream_t, const Dev&, bool);
     void launchRigidClearGravity(hipStream_t, const Dev&);
@@ -304,6 +305,9 @@ struct tsp_ctx
     float* bvol2 = nullptr;
     uint64_t *idB = nullptr, *idB2 = nullptr;
     uint64_t* idR = nullptr;
+    uint32_t cuCount = 0;           // of the device
+    uint32_t solveHold = 0;         // steps until a solve in one launch is tried again (one gave up)
+    static constexpr uint32_t kSolveHold = 256;
     uint32_t* radixState = nullptr;
     uint32_t* aabb = nullptr;       // 6 per scene
     std::vector<void*> arena;       // particle and body arrays (replaced by a relayout)
@@ -573,7 +577,7 @@ struct tsp_ctx
         sync();
         prof.resolve();
         last = *hostStatus;
-        if (last.scanFail) { throw Error{ TSP_ERR_STATE, "a one-pass scan gave up waiting for a predecessor tile" }; }
+        if (last.scanFail) { throw Error{ TSP_ERR_STATE, "a kernel gave up waiting for another block" }; }
     }
 
     void uploadConsts()
@@ -602,6 +606,14 @@ struct tsp_ctx
         }
         d.rfCap = rfCap;
         d.rfIdx = alloc<uint32_t>(rfCap, poolAllocs, MEM_LR);
+        d.fbGrad = nullptr;
+    }
+
+    // the FB records of a solve in one launch (contexts of few blocks), for the present pools
+    void allocSolve()
+    {
+        if (d.fbGrad || d.nF / kBlock > kSolveBlocksMost) { return; }
+        d.fbGrad = alloc<float4>(d.poolCap[1], poolAllocs, MEM_LF);
     }
 
     // the fluid fields of a scene in the records of n (missing fields are left out)
@@ -692,7 +704,7 @@ struct tsp_ctx
             hipCheck(hipGetLastError(), "device builder launch");
             uint32_t scanFailed = 0;
             d2h(&scanFailed, sort + 3, sizeof(uint32_t));
-            if (scanFailed) { throw Error{ TSP_ERR_STATE, "a one-pass scan gave up waiting for a predecessor tile" }; }
+            if (scanFailed) { throw Error{ TSP_ERR_STATE, "a kernel gave up waiting for another block" }; }
         }
         catch (...)
         {
@@ -1004,6 +1016,8 @@ struct tsp_ctx
         contactLists = false;
         contactRB = 0;
         d.errPartial = alloc<double>(3ull * (nF / kBlock), work);
+        d.solveFlag = alloc<uint32_t>(kFlagCopies * kSolveBlocksMost, work);
+        d.solveBar = alloc<uint32_t>(static_cast<uint64_t>(kBarWords) * S, work);
         {
             static_assert(sizeof(Status) <= kSolveOff, "status block layout");
             unsigned char* blk = alloc<unsigned char>(kSolveOff + sizeof(Solve) * S, work);
@@ -1050,6 +1064,7 @@ struct tsp_ctx
                 }
                 allocPools(cap, rfCap);
             }
+            allocSolve();
         }
         // world records of the rigid particles from the body state
         launchRigidUpdate(stream, d, false);
@@ -1406,6 +1421,7 @@ struct tsp_ctx
                 }
                 const uint64_t rfCap = std::max<uint64_t>(d.rfCap, last.rfTotal + last.rfTotal / 8 + 64);
                 allocPools(cap, rfCap);
+                allocSolve();
                 for (SceneHost& h : scenes) { h.flags |= TSP_FLAG_LIST_REGROWN; }
             }
             // the contact solve's RB and RR lists are stored when some scene has entries
@@ -1532,6 +1548,14 @@ struct tsp_ctx
         return static_cast<uint32_t>(std::max<int64_t>(1, std::min<int64_t>(guess, maxSweeps)));
     }
 
+    // every scene's solve has converged (by the states read last)
+    bool allSolved() const
+    {
+        bool all = true;
+        for (uint32_t s = 0; s < nScenes(); s++) { all = all && (scenes[s].nF == 0 || hostSolve[s].converged); }
+        return all;
+    }
+
     // relaxed Jacobi sweeps of all scenes until every scene has converged; each group is followed
     // by one read of the solver states. queued sweeps have run already (their states read).
     void solveLoop(uint32_t queued, uint32_t group, uint32_t maxSweeps)
@@ -1540,9 +1564,7 @@ struct tsp_ctx
         {
             if (queued > 0)
             {
-                bool all = true;
-                for (uint32_t s = 0; s < nScenes(); s++) { all = all && (scenes[s].nF == 0 || hostSolve[s].converged); }
-                if (all) { return; }
+                if (allSolved()) { return; }
             }
             const uint32_t n = std::min(group, maxSweeps - queued);
             if (n == 0) { throw Error{ TSP_ERR_STATE, "pressure solve did not stop at max_solver_iters" }; }
@@ -1553,9 +1575,19 @@ struct tsp_ctx
         }
     }
 
-    // final pressure accelerations, rigid coupling, integration and the contact solve
-    void tailLaunches()
+    // the solve of a context of few blocks runs as one launch (kSolve), unless launches are being timed one
+    // by one
+    bool solveInOne() const
     {
+        const uint32_t nBlocks = d.nF / kBlock;
+        return !prof.on && d.fbGrad && !solveHold && nBlocks <= kSolveBlocksMost && nBlocks <= cuCount;
+    }
+
+    // final pressure accelerations (unless the solve left them), rigid coupling, integration and the
+    // contact solve
+    void tailLaunches(bool accDone = false)
+    {
+        if (!accDone)
         {
             Scope sc(prof, stream, "pressure_acc_final");
             launchPressureAcc(stream, d, false);
@@ -1740,9 +1772,18 @@ struct tsp_ctx
         }
         neighborSearch(false);
         predictLaunches();
-        if (anyFluid) { solveLoop(0, group, maxSweeps); }
-        else { readStatus(); }
-        tailLaunches();
+        bool solved = false;
+        if (anyFluid && solveInOne())
+        {
+            launchSolve(stream, d);
+            readStatus();
+            solved = allSolved();
+            if (!solved) { solveHold = kSolveHold; }
+        }
+        else if (solveHold) { solveHold--; }
+        if (!anyFluid) { readStatus(); }
+        else if (!solved) { solveLoop(0, group, maxSweeps); }
+        tailLaunches(solved);
         stepBookkeeping();
     }
 
@@ -1955,7 +1996,7 @@ struct tsp_ctx
         hipCheck(hipMemcpyAsync(&count, expFlags + h.nF, sizeof(uint32_t), hipMemcpyDeviceToHost, stream), "D2H");
         hipCheck(hipMemcpyAsync(&scanFailed, &d.status->scanFail, sizeof(uint32_t), hipMemcpyDeviceToHost, stream), "D2H");
         sync();
-        if (scanFailed) { throw Error{ TSP_ERR_STATE, "a one-pass scan gave up waiting for a predecessor tile" }; }
+        if (scanFailed) { throw Error{ TSP_ERR_STATE, "a kernel gave up waiting for another block" }; }
         v->n_fluid = count;
         if (count > v->cap_fluid) { throw Error{ TSP_ERR_CAPACITY, "the fluid export arrays hold fewer particles than the surface set" }; }
         std::vector<XferField> fields;
@@ -2080,6 +2121,8 @@ int tsp_create(int device, tsp_ctx** out)
     if (hipGetDeviceCount(&n) != hipSuccess || device < 0 || device >= n) { return TSP_ERR_HIP; }
     tsp_ctx* c = new tsp_ctx();
     c->device = device;
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess) { c->cuCount = static_cast<uint32_t>(cus); }
     // statsScratchInit: the device address of this device's statistics scratch, once per device
     if (hipSetDevice(device) != hipSuccess || statsScratchInit(device) != hipSuccess
         || hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess

@@ -28,7 +28,6 @@
 //   TSP_TUNE_SWEEP_AHEAD   the first sweep group of a step: the previous step's sweeps plus this
 //   TSP_TUNE_STEP_GRAPH    a step runs as one captured graph launch with one status read (1), or
 //                          launch by launch with the host reading the status between phases (0)
-//   TSP_TUNE_JACOBI_REC24  kJacobi's halo records take 24 bytes instead of 32 (six blocks per CU)
 //   TSP_TUNE_HALO_MAX      FF halo records per 256-particle block (LDS per sweep block)
 //   TSP_TUNE_GRAPHS        each group of solver sweeps runs as one instantiated HIP graph
 //   TSP_TUNE_PA_WAVES, TSP_TUNE_JACOBI_WAVES   waves per SIMD the compiler must leave room for
@@ -42,9 +41,6 @@
 #endif
 #ifndef TSP_TUNE_SWEEP_AHEAD
 #define TSP_TUNE_SWEEP_AHEAD -1
-#endif
-#ifndef TSP_TUNE_JACOBI_REC24
-#define TSP_TUNE_JACOBI_REC24 1
 #endif
 #ifndef TSP_TUNE_HALO_MAX
 #define TSP_TUNE_HALO_MAX 1000
@@ -106,6 +102,13 @@ namespace tsp
         return n > kRadixSmallTiles ? kRadixManyAt + kRadixBins * (1ull + (n + kRadixManyTile - 1u) / kRadixManyTile)
                                     : kRadixStatusAt + 2ull * kRadixBins * ((n + kRadixTileMin - 1u) / kRadixTileMin);
     }
+
+    // kSolve: the most blocks of its launch (and no more than one per CU), and a scene's entry words, one
+    // to a 128-byte line
+    constexpr uint32_t kSolveBlocksMost = 256;
+    constexpr uint32_t kFlagCopies = 8;
+    constexpr uint32_t kBarLine = 32;
+    constexpr uint32_t kBarWords = 2 * kBarLine;
 
     // Hit masks of the count pass (one word per stencil row of three cells, reach 1): the fill takes the
     // hits from them and loads no candidate position. A row with more than 32 candidates is marked in
@@ -386,6 +389,9 @@ namespace tsp
         float *cIw;                  // 9 x nRB: world inverse inertia
         float *cLoad;                // 6 x nRB: contact force and torque
         uint32_t *cBodyB;            // nRB: boundary contacts of each movable body
+        float4 *fbGrad;          // per FB pool unit: gradient and psi of an entry, kept for a solve in one launch
+        uint32_t *solveFlag;     // per block of such a launch: the barriers that it has come to (zeroed by kSolverInit)
+        uint32_t *solveBar;      // kBarWords per scene: the entry of kSolve (zeroed by kSolverInit)
         // reductions and scans
         double *errPartial;      // Jacobi error partials, [3][blocks of the fluid grid]
         uint32_t *scanTmp;       // block sums of the multi-block scans

@@ -8,9 +8,6 @@
 #ifndef TSP_TUNE_HALO_MAX
 #define TSP_TUNE_HALO_MAX 1064
 #endif
-#ifndef TSP_TUNE_JACOBI_REC24
-#define TSP_TUNE_JACOBI_REC24 1
-#endif
 #ifndef TSP_TUNE_JACOBI_WAVES
 #define TSP_TUNE_JACOBI_WAVES 6
 #endif

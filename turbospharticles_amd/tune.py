@@ -37,7 +37,6 @@ TUNED_H = os.path.join(HERE, "csrc", "tsp_tuned.h")
 SPACE = {
     "TSP_TUNE_SWEEP_AHEAD": [-1, 0, 1, 2],
     "TSP_TUNE_STEP_GRAPH": [0, 1],
-    "TSP_TUNE_JACOBI_REC24": [1, 0],
     "TSP_TUNE_HALO_MAX": [1000, 960, 1024, 1064],
     "TSP_TUNE_GRAPHS": [1, 0],
     "TSP_TUNE_PA_WAVES": [0, 6, 8],
