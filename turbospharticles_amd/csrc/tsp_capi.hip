@@ -50,7 +50,7 @@ namespace tsp
     void launchContactSolve(hipStream_t, const Dev&, uint32_t, uint32_t*);
     void launchExportSurface(hipStream_t, const Dev&, uint32_t, uint32_t, uint32_t, uint32_t*, uint32_t*, float*, float*);
     void launchBuildFluid(hipStream_t, const Dev&, uint32_t, uint32_t, const BuildFluid&);
-    void launchBuildBoundary(hipStream_t, const BuildBoundary&, uint32_t, float4*, float*, uint64_t*, float*, uint32_t*,
+    void launchBuildBoundary(hipStream_t, const BuildBoundary&, uint32_t, float4*, float*, uint64_t*, float*, float4*, uint32_t*,
                              uint32_t*, uint32_t*, uint32_t*, uint32_t*);
     void launchAabb(hipStream_t, const Dev&, int, const float4*, uint32_t, uint32_t*);
     void launchDensity(hipStream_t, const Dev&);
@@ -633,8 +633,31 @@ struct tsp_ctx
         addField(fields, f[TSP_F_DIAG], n.diag + h.offF, h.nF);
     }
 
+    // scratch of the device builder, for the largest boundary of the scenes of a relayout: they are
+    // generated one after the other on the stream
+    struct BuildScratch
+    {
+        float* xyz = nullptr;
+        float4* rec = nullptr;
+        uint32_t *key = nullptr, *idx = nullptr, *key2 = nullptr, *idx2 = nullptr, *sort = nullptr;
+    };
+
+    BuildScratch buildScratch(uint32_t most, std::vector<void*>& list)
+    {
+        BuildScratch b;
+        b.xyz = alloc<float>(3ull * most, list);
+        b.rec = alloc<float4>(most, list);
+        b.key = alloc<uint32_t>(most, list);
+        b.idx = alloc<uint32_t>(most, list);
+        b.key2 = alloc<uint32_t>(most, list);
+        b.idx2 = alloc<uint32_t>(most, list);
+        b.sort = alloc<uint32_t>(radixStateWords(most), list);
+        zero(b.sort, sizeof(uint32_t) * radixStateWords(most));
+        return b;
+    }
+
     // --- a planned scene's fluid and boundary generated in the new arena (n) at h's offsets ---
-    void buildOnDevice(const Dev& n, const SceneHost& h, const tsp::scene::Plan& plan, uint64_t* nidB)
+    void buildOnDevice(const Dev& n, const SceneHost& h, const tsp::scene::Plan& plan, uint64_t* nidB, const BuildScratch& b)
     {
         const tsp::scene::Params& p = plan.p;
         const tsp::scene::FluidBlock& fb = plan.fluid;
@@ -688,31 +711,9 @@ struct tsp_ctx
             totalBits += bits;
         }
         if (totalBits > 32) { throw Error{ TSP_ERR_CAPACITY, "container too large for the device builder's 32-bit cell keys" }; }
-        const uint32_t nB = h.nB;
-        std::vector<void*> tmp;
-        try
-        {
-            float* xyz = alloc<float>(3ull * nB, tmp);
-            uint32_t* key = alloc<uint32_t>(nB, tmp);
-            uint32_t* idx = alloc<uint32_t>(nB, tmp);
-            uint32_t* key2 = alloc<uint32_t>(nB, tmp);
-            uint32_t* idx2 = alloc<uint32_t>(nB, tmp);
-            uint32_t* sort = alloc<uint32_t>(radixStateWords(nB), tmp);
-            zero(sort, sizeof(uint32_t) * radixStateWords(nB));
-            launchBuildBoundary(stream, bb, nB, n.bpos + h.offB, n.bvol + h.offB, nidB + h.offB, xyz, key, idx, key2, idx2,
-                                sort);
-            hipCheck(hipGetLastError(), "device builder launch");
-            uint32_t scanFailed = 0;
-            d2h(&scanFailed, sort + 3, sizeof(uint32_t));
-            if (scanFailed) { throw Error{ TSP_ERR_STATE, "a kernel gave up waiting for another block" }; }
-        }
-        catch (...)
-        {
-            (void)hipStreamSynchronize(stream);
-            releaseList(tmp);
-            throw;
-        }
-        releaseList(tmp);
+        launchBuildBoundary(stream, bb, h.nB, n.bpos + h.offB, n.bvol + h.offB, nidB + h.offB, b.xyz, b.rec, b.key, b.idx, b.key2,
+                            b.idx2, b.sort);
+        hipCheck(hipGetLastError(), "device builder launch");
     }
 
     // --- storage of the contact solve sized by the RB and RR entries of a search ---
@@ -783,7 +784,7 @@ struct tsp_ctx
         const uint32_t S = static_cast<uint32_t>(ns.size());
         const size_t nRB1 = std::max<uint32_t>(nRB, 1), oldRB1 = std::max<uint32_t>(d.nRB, 1);
 
-        std::vector<void*> A;
+        std::vector<void*> A, scratch;
         Dev n = d;
         float4 *npos2, *nvel2, *nvp2, *nap2, *nbpos2;
         float *nsource2, *ndiag2, *nbvol2;
@@ -839,6 +840,10 @@ struct tsp_ctx
                 given.emplace_back(cnt, value);
                 return given.back().data();
             };
+            uint32_t mostB = 0;
+            for (size_t q = 0; q < src.size(); q++) { if (src[q].keep < 0 && src[q].plan) { mostB = std::max(mostB, ns[q].nB); } }
+            BuildScratch build;
+            if (mostB) { build = buildScratch(mostB, scratch); }
             for (size_t q = 0; q < src.size(); q++)
             {
                 const SceneHost& h = ns[q];
@@ -877,7 +882,7 @@ struct tsp_ctx
                     continue;
                 }
                 const tsp_state_view* s = src[q].view;
-                if (src[q].plan) { buildOnDevice(n, h, *src[q].plan, nidB); }
+                if (src[q].plan) { buildOnDevice(n, h, *src[q].plan, nidB, build); }
                 // fluid (missing fields stay zero) and boundary (ensureBoundaryCoefficientsPresent
                 // defaults: psi = massB, V = psi / rho0)
                 if (!src[q].plan)
@@ -933,14 +938,22 @@ struct tsp_ctx
             addField(fields, bodyScene.data(), n.bodyScene, nRB);
             if (nB) { addField(fields, sceneB.data(), reinterpret_cast<uint32_t*>(n.sceneB), (nB + 1ull) / 2ull); }
             transfer(fields, false);
+            if (mostB)
+            {
+                uint32_t scanFailed = 0;
+                d2h(&scanFailed, build.sort + 3, sizeof(uint32_t));
+                if (scanFailed) { throw Error{ TSP_ERR_STATE, "a kernel gave up waiting for another block" }; }
+            }
             sync();
         }
         catch (...)
         {
             (void)hipStreamSynchronize(stream);
+            releaseList(scratch);
             releaseList(A);
             throw;
         }
+        releaseList(scratch);
 
         // install the new arena
         releaseList(arena);
