@@ -183,22 +183,6 @@ namespace tsp
         kScanOnePass<<<nb, kBlock, 0, s>>>(v, m, tmp, fail);
     }
 
-    // clears the search status block and the scenes' frame-abort flags
-    __global__ void __launch_bounds__(kBlock) kResetSearch(Dev d)
-    {
-        constexpr uint32_t words = static_cast<uint32_t>(sizeof(Status) / sizeof(uint32_t));
-        static_assert(words <= kBlock, "the reset covers one block");
-        constexpr uint32_t keep = static_cast<uint32_t>(offsetof(Status, scanFail) / sizeof(uint32_t));
-        if (threadIdx.x < words && threadIdx.x != keep) { reinterpret_cast<uint32_t*>(d.status)[threadIdx.x] = 0u; }
-        for (uint32_t s = threadIdx.x; s < d.nScenes; s += kBlock)
-        {
-            Solve& so = d.solve[s];
-            so.abort = 0u;
-            so.contactActive = 0u; so.contactDone = 0u; so.contactIters = 0u; so.contactConverged = 0u;
-            so.contactAvg = 0.0f; so.contactBoundary = 0u; so.contactBad = 0u; so.contacts = 0ull;
-        }
-    }
-
     // ----------------------------------------------------------------------------------------
     // keys
 
@@ -676,14 +660,18 @@ namespace tsp
     // ----------------------------------------------------------------------------------------
     // permutation (gather into the second buffers)
 
-    __global__ void __launch_bounds__(kBlock) kPermute(Gather g, const uint32_t* __restrict__ idx)
+    __device__ __forceinline__ void gatherOne(const Gather& g, const uint32_t* __restrict__ idx, uint32_t i)
     {
-        const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-        if (i >= g.n) { return; }
         const uint32_t o = idx[i];
         for (uint32_t f = 0; f < g.n4; f++) { g.d4[f][i] = g.s4[f][o]; }
         for (uint32_t f = 0; f < g.n1; f++) { g.d1[f][i] = g.s1[f][o]; }
         if (g.idS) { g.idD[i] = g.idS[o]; }
+    }
+
+    __global__ void __launch_bounds__(kBlock) kPermute(Gather g, const uint32_t* __restrict__ idx)
+    {
+        const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+        if (i < g.n) { gatherOne(g, idx, i); }
     }
 
     // ----------------------------------------------------------------------------------------
@@ -696,16 +684,40 @@ namespace tsp
         return linearCell(f, compact21(m), compact21(m >> 1), compact21(m >> 2));
     }
 
-    // clears the cells of the runs of the previous sorted keys
-    __global__ void __launch_bounds__(kBlock) kClearCells(Dev d, const uint32_t* __restrict__ key, uint32_t n,
+    // the search status block and the scenes' frame-abort flags cleared, by one block
+    __device__ __forceinline__ void resetSearch(const Dev& d)
+    {
+        constexpr uint32_t words = static_cast<uint32_t>(sizeof(Status) / sizeof(uint32_t));
+        static_assert(words <= kBlock, "the reset covers one block");
+        constexpr uint32_t keep = static_cast<uint32_t>(offsetof(Status, scanFail) / sizeof(uint32_t));
+        if (threadIdx.x < words && threadIdx.x != keep) { reinterpret_cast<uint32_t*>(d.status)[threadIdx.x] = 0u; }
+        for (uint32_t s = threadIdx.x; s < d.nScenes; s += kBlock)
+        {
+            Solve& so = d.solve[s];
+            so.abort = 0u;
+            so.contactActive = 0u; so.contactDone = 0u; so.contactIters = 0u; so.contactConverged = 0u;
+            so.contactAvg = 0.0f; so.contactBoundary = 0u; so.contactBad = 0u; so.contacts = 0ull;
+        }
+    }
+
+    // a search's start: the status block reset, and the cells of the runs of the previous sorted keys
+    // (the only ones that are not empty) of the fluid and the rigid particles cleared
+    __device__ __forceinline__ void clearCells(const Dev& d, const uint32_t* __restrict__ key, uint32_t i, uint32_t n,
         uint2* __restrict__ cell)
     {
-        const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
         if (i >= n) { return; }
         const uint64_t k = keyAt(d, key, i);
         const Frame& f = d.frames[sceneOfKey(d, k)];
         if (k >= f.emptyKey) { return; }
         if (i == 0 || keyAt(d, key, i - 1) != k) { cell[linearOfKey(f, k)] = make_uint2(0u, 0u); }
+    }
+
+    __global__ void __launch_bounds__(kBlock) kResetSearch(Dev d, uint32_t blocksF)
+    {
+        if (blockIdx.x == 0u) { resetSearch(d); return; }
+        const uint32_t b = blockIdx.x - 1u;
+        if (b < blocksF) { clearCells(d, d.keyF, b * kBlock + threadIdx.x, d.nF, d.cellF); }
+        else { clearCells(d, d.keyR, (b - blocksF) * kBlock + threadIdx.x, d.nR, d.cellR); }
     }
 
     __global__ void __launch_bounds__(kBlock) kClearAll(uint2* __restrict__ cell, uint64_t n)
@@ -714,11 +726,9 @@ namespace tsp
         if (q < n) { cell[q] = make_uint2(0u, 0u); }
     }
 
-    __global__ void __launch_bounds__(kBlock) kBuildCells(Dev d, const uint32_t* __restrict__ key, uint32_t n,
+    __device__ __forceinline__ void buildCells(const Dev& d, const uint32_t* __restrict__ key, uint32_t i, uint32_t n,
         uint2* __restrict__ cell)
     {
-        const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-        if (i >= n) { return; }
         const uint64_t k = keyAt(d, key, i);
         const Frame& f = d.frames[sceneOfKey(d, k)];
         if (k >= f.emptyKey) { return; }
@@ -728,6 +738,22 @@ namespace tsp
         const uint32_t lin = linearOfKey(f, k);
         if (first) { cell[lin].x = i; }
         if (last) { cell[lin].y = i + 1; }
+    }
+
+    __global__ void __launch_bounds__(kBlock) kBuildCells(Dev d, const uint32_t* __restrict__ key, uint32_t n,
+        uint2* __restrict__ cell)
+    {
+        const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+        if (i < n) { buildCells(d, key, i, n, cell); }
+    }
+
+    // the fluid's re-order and its cells
+    __global__ void __launch_bounds__(kBlock) kPermuteCells(Dev d, Gather g)
+    {
+        const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+        if (i >= g.n) { return; }
+        gatherOne(g, d.idxF, i);
+        buildCells(d, d.keyF, i, g.n, d.cellF);
     }
 
     // ----------------------------------------------------------------------------------------
@@ -1726,7 +1752,12 @@ namespace tsp
     static uint32_t radixPasses(uint32_t bits) { return (bits + kRadixBits - 1u) / kRadixBits; }
 
 
-    void launchResetSearch(hipStream_t s, const Dev& d) { kResetSearch<<<1, kBlock, 0, s>>>(d); }
+    // cells: the cell tables hold the runs of the sorted keys, which are cleared
+    void launchResetSearch(hipStream_t s, const Dev& d, bool cells)
+    {
+        const uint32_t nF = cells ? blocksFor(d.nF) : 0u, nR = cells ? blocksFor(d.nR) : 0u;
+        kResetSearch<<<1u + nF + nR, kBlock, 0, s>>>(d, nF);
+    }
 
     // key arrays hold u32 keys, or u64 keys (two words each) when d.key64
     // state: the sort state that takes the digit counts when kRadixPass sorts the keys by `bits` bits
@@ -1811,9 +1842,9 @@ namespace tsp
         if (g.n) { kPermute<<<blocksFor(g.n), kBlock, 0, s>>>(g, idx); }
     }
 
-    void launchClearCells(hipStream_t s, const Dev& d, const uint32_t* key, uint32_t n, uint2* cell)
+    void launchPermuteCells(hipStream_t s, const Dev& d, const Gather& g)
     {
-        if (n) { kClearCells<<<blocksFor(n), kBlock, 0, s>>>(d, key, n, cell); }
+        if (g.n) { kPermuteCells<<<blocksFor(g.n), kBlock, 0, s>>>(d, g); }
     }
 
     void launchClearAll(hipStream_t s, uint2* cell, uint64_t n)

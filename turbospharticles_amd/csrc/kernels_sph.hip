@@ -169,12 +169,52 @@ namespace tsp
         d.vp[i] = make_float4(__builtin_fmaf(ax, k.dt, vxi), __builtin_fmaf(ay, k.dt, vyi), __builtin_fmaf(az, k.dt, vzi), 0.0f);
     }
 
+    // TerminationConditionSatisfied, sph_solver.cpp:686-732
+    __device__ __forceinline__ bool terminated(const Solve& s, const Consts& k)
+    {
+        if (s.iters < k.minIters) { return false; }
+        if (s.iters >= k.maxIters) { return true; }
+        switch (k.termCond)
+        {
+        case 0: return s.iters >= k.fixedIters;
+        case 1: return s.avgRaw <= k.densityDevTarget;
+        case 2: return s.avgPos <= k.densityDevTarget;
+        case 3: return s.avgAbs <= k.densityDevTarget;
+        default: return s.iters >= 3;
+        }
+    }
+
+    // the solver state before the first sweep: N_solverIters_ = 1, errors 0, then the
+    // increment and error decision of the first sweep (sph_solver.cpp:207-235); by one block
+    __device__ __forceinline__ void solverInit(const Dev& d)
+    {
+        for (uint32_t sc = threadIdx.x; sc < d.nScenes; sc += kBlock)
+        {
+            Solve& s = d.solve[sc];
+            const Consts& k = d.consts[sc];
+            const bool any = d.scenes[sc].nF > 0;
+            s.iters = any ? 1u : 0u;
+            s.avgRaw = s.avgPos = s.avgAbs = 0.0f;
+            s.sumRaw = s.sumPos = s.sumAbs = 0.0;
+            s.converged = any ? 0u : 1u;
+            s.sweeps = 0;
+            s.pending = 0;
+            s.iters++;
+            s.compute = (s.iters >= k.minIters && (k.termCond != 0 || terminated(s, k))) ? 1u : 0u;
+            for (uint32_t q = 0; q < kBarWords; q += kBarLine) { d.solveBar[static_cast<size_t>(sc) * kBarWords + q] = 0u; }
+        }
+        for (uint32_t q = threadIdx.x; q < kFlagCopies * kSolveBlocksMost; q += kBlock) { d.solveFlag[q] = 0u; }
+    }
+
     template <bool kFast>
     __global__ void __launch_bounds__(kBlock) kSourceDiag(Dev d)
     {
         if (stopped(d)) { return; }
+        // the block after the tiles' readies the solver states
+        const uint32_t nTiles = d.nF / kBlock;
+        if (blockIdx.x == nTiles) { solverInit(d); return; }
         __shared__ float4 hp[kHaloMax], hv[kHaloMax];
-        const uint32_t blk = xcdBlock();
+        const uint32_t blk = xcdBlock(nTiles);
         const Lists l = listsAt(d, blk);
         const SlotList slots = slotsOf(d, l);
         const Halo h = haloOf(d, blk);
@@ -278,44 +318,6 @@ namespace tsp
         d.source[i] = src;
         d.diag[i] = diag;
         d.pos[i].w = vmax(0.0f, valid ? init : 0.0f);
-    }
-
-    // TerminationConditionSatisfied, sph_solver.cpp:686-732
-    __device__ __forceinline__ bool terminated(const Solve& s, const Consts& k)
-    {
-        if (s.iters < k.minIters) { return false; }
-        if (s.iters >= k.maxIters) { return true; }
-        switch (k.termCond)
-        {
-        case 0: return s.iters >= k.fixedIters;
-        case 1: return s.avgRaw <= k.densityDevTarget;
-        case 2: return s.avgPos <= k.densityDevTarget;
-        case 3: return s.avgAbs <= k.densityDevTarget;
-        default: return s.iters >= 3;
-        }
-    }
-
-    // the solver state before the first sweep: N_solverIters_ = 1, errors 0, then the
-    // increment and error decision of the first sweep (sph_solver.cpp:207-235)
-    __global__ void __launch_bounds__(kBlock) kSolverInit(Dev d)
-    {
-        if (stopped(d)) { return; }
-        for (uint32_t sc = threadIdx.x; sc < d.nScenes; sc += kBlock)
-        {
-            Solve& s = d.solve[sc];
-            const Consts& k = d.consts[sc];
-            const bool any = d.scenes[sc].nF > 0;
-            s.iters = any ? 1u : 0u;
-            s.avgRaw = s.avgPos = s.avgAbs = 0.0f;
-            s.sumRaw = s.sumPos = s.sumAbs = 0.0;
-            s.converged = any ? 0u : 1u;
-            s.sweeps = 0;
-            s.pending = 0;
-            s.iters++;
-            s.compute = (s.iters >= k.minIters && (k.termCond != 0 || terminated(s, k))) ? 1u : 0u;
-            for (uint32_t q = 0; q < kBarWords; q += kBarLine) { d.solveBar[static_cast<size_t>(sc) * kBarWords + q] = 0u; }
-        }
-        for (uint32_t q = threadIdx.x; q < kFlagCopies * kSolveBlocksMost; q += kBlock) { d.solveFlag[q] = 0u; }
     }
 
     // the value of the lane `kRot` further in the lane's row of 16 (rotating)
@@ -1004,7 +1006,7 @@ namespace tsp
         const float src = d.source[i], diag = d.diag[i];
         const bool active = i - S.offF < S.nF;
         stageHalo(h, [&](uint32_t j) { return d.pos[j]; }, [&](uint32_t q, const float4& r) { hp[q] = r; hw[q] = r.w; });
-        // the state that kSolverInit left; every thread keeps it (nothing of it is read here again)
+        // the state that solverInit left; every thread keeps it (nothing of it is read here again)
         Solve s = uniformLoad(&d.solve[sc]);
         uint32_t* bar = d.solveBar + static_cast<size_t>(sc) * kBarWords;
         if (!enterScene(bar, S.nBlk)) { return; }   // (a barrier: the halo is staged)
@@ -1187,22 +1189,6 @@ namespace tsp
         if (i < d.nR) { rigidUpdateOne(d, i, predicted); }
     }
 
-    // ClearRigidForcesAndAddGravity, cpu_backend.cpp:2065-2087
-    __global__ void kRigidClearGravity(Dev d)
-    {
-        if (stopped(d)) { return; }
-        const uint32_t b = blockIdx.x * kBlock + threadIdx.x;
-        if (b >= d.nRB) { return; }
-        const Consts& k = d.consts[d.bodyScene[b]];
-        const uint32_t nb = d.nRB;
-        for (int f = 0; f < 6; f++) { d.rbForce[f * nb + b] = 0.0f; }
-        const float m = rbv(d, RB_MASS, b), mi = rbv(d, RB_MASS_INV, b);
-        if (m <= 0.0f || mi <= 0.0f) { return; }
-        d.rbForce[0 * nb + b] += m * k.gx;
-        d.rbForce[1 * nb + b] += m * k.gy;
-        d.rbForce[2 * nb + b] += m * k.gz;
-    }
-
     // AccumulateRigidParticleNonPressureForces_ChunkedSELL / ...PressureForces (sph_solver.cpp:1151-1223,
     // :1717-1778): reaction of the fluid neighbors of each rigid particle
     __global__ void __launch_bounds__(kBlock) kRigidForces(Dev d, bool pressure)
@@ -1256,55 +1242,6 @@ namespace tsp
         else { d.rfx[i] = fx; d.rfy[i] = fy; d.rfz[i] = fz; }
     }
 
-    // ReduceRigidParticleForcesToBody, cpu_backend.cpp:2089-2172, with FP64 sums: one block per body
-    // one block of kReduceThreads per body: a body's particles are few blocks' worth, so the
-    // block is wide to keep the chains of dependent loads and sums short
-    constexpr uint32_t kReduceThreads = 1024;
-
-    __global__ void __launch_bounds__(kReduceThreads) kRigidReduce(Dev d)
-    {
-        if (stopped(d)) { return; }
-        __shared__ double red[6][kReduceThreads];
-        const uint32_t b = blockIdx.x;
-        const uint32_t nb = d.nRB;
-        const float a[9] = { rbv(d, RB_A00 + 0, b), rbv(d, RB_A00 + 1, b), rbv(d, RB_A00 + 2, b),
-                             rbv(d, RB_A00 + 3, b), rbv(d, RB_A00 + 4, b), rbv(d, RB_A00 + 5, b),
-                             rbv(d, RB_A00 + 6, b), rbv(d, RB_A00 + 7, b), rbv(d, RB_A00 + 8, b) };
-        double acc[6] = { 0, 0, 0, 0, 0, 0 };
-        for (uint32_t q = d.byBodyOff[b] + threadIdx.x; q < d.byBodyOff[b + 1]; q += kReduceThreads)
-        {
-            const uint32_t i = d.byBodyIdx[q];
-            const float lx = d.rxrel[i], ly = d.ryrel[i], lz = d.rzrel[i];
-            const float rx = __builtin_fmaf(a[0], lx, __builtin_fmaf(a[1], ly, a[2] * lz));
-            const float ry = __builtin_fmaf(a[3], lx, __builtin_fmaf(a[4], ly, a[5] * lz));
-            const float rz = __builtin_fmaf(a[6], lx, __builtin_fmaf(a[7], ly, a[8] * lz));
-            const double fx = d.rfx[i], fy = d.rfy[i], fz = d.rfz[i];
-            acc[0] += fx; acc[1] += fy; acc[2] += fz;
-            acc[3] += static_cast<double>(ry) * fz - static_cast<double>(rz) * fy;
-            acc[4] += static_cast<double>(rz) * fx - static_cast<double>(rx) * fz;
-            acc[5] += static_cast<double>(rx) * fy - static_cast<double>(ry) * fx;
-        }
-        for (int f = 0; f < 6; f++) { red[f][threadIdx.x] = acc[f]; }
-        __syncthreads();
-        for (uint32_t o = kReduceThreads / 2; o > 0; o >>= 1)
-        {
-            if (threadIdx.x < o) { for (int f = 0; f < 6; f++) { red[f][threadIdx.x] += red[f][threadIdx.x + o]; } }
-            __syncthreads();
-        }
-        if (threadIdx.x == 0)
-        {
-            for (int f = 0; f < 6; f++) { d.rbForce[f * nb + b] += static_cast<float>(red[f][0]); }
-        }
-    }
-
-    // PredictRigidBodies, cpu_backend.cpp:2174-2235
-    __global__ void kRigidPredict(Dev d)
-    {
-        if (stopped(d)) { return; }
-        const uint32_t b = blockIdx.x * kBlock + threadIdx.x;
-        if (b < d.nRB) { rigidPredictOne(d, b); }
-    }
-
     __device__ __forceinline__ bool normalize3(float& x, float& y, float& z)
     {
         const float len = __builtin_sqrtf(__builtin_fmaf(x, x, __builtin_fmaf(y, y, z * z)));
@@ -1319,12 +1256,9 @@ namespace tsp
         return __builtin_fmaf(ax, bx, __builtin_fmaf(ay, by, az * bz));
     }
 
-    // IntegrateRigidBodies, cpu_backend.cpp:2237-2303
-    __global__ void kRigidIntegrate(Dev d)
+    // IntegrateRigidBodies, cpu_backend.cpp:2237-2303, one body
+    __device__ __forceinline__ void rigidIntegrateOne(const Dev& d, uint32_t b)
     {
-        if (stopped(d)) { return; }
-        const uint32_t b = blockIdx.x * kBlock + threadIdx.x;
-        if (b >= d.nRB) { return; }
         const Consts& k = d.consts[d.bodyScene[b]];
         const uint32_t nb = d.nRB;
         float* rb = d.rb;
@@ -1369,6 +1303,80 @@ namespace tsp
         for (int q = 0; q < 9; q++) { rb[(RB_A00 + q) * nb + b] = out[q]; }
     }
 
+    // ClearRigidForcesAndAddGravity and ReduceRigidParticleForcesToBody (cpu_backend.cpp:2065-2172) of one
+    // body, with FP64 sums, by its block of kBodyThreads; thread 0 writes the sums
+    constexpr uint32_t kBodyThreads = 1024;
+
+    __device__ __forceinline__ void rigidForceSums(const Dev& d, uint32_t b)
+    {
+        __shared__ double red[6][kBodyThreads];
+        const uint32_t t = threadIdx.x;
+        const uint32_t nb = d.nRB;
+        const float a[9] = { rbv(d, RB_A00 + 0, b), rbv(d, RB_A00 + 1, b), rbv(d, RB_A00 + 2, b),
+                             rbv(d, RB_A00 + 3, b), rbv(d, RB_A00 + 4, b), rbv(d, RB_A00 + 5, b),
+                             rbv(d, RB_A00 + 6, b), rbv(d, RB_A00 + 7, b), rbv(d, RB_A00 + 8, b) };
+        double acc[6] = { 0, 0, 0, 0, 0, 0 };
+        for (uint32_t q = d.byBodyOff[b] + t; q < d.byBodyOff[b + 1]; q += kBodyThreads)
+        {
+            const uint32_t i = d.byBodyIdx[q];
+            const float lx = d.rxrel[i], ly = d.ryrel[i], lz = d.rzrel[i];
+            const float rx = __builtin_fmaf(a[0], lx, __builtin_fmaf(a[1], ly, a[2] * lz));
+            const float ry = __builtin_fmaf(a[3], lx, __builtin_fmaf(a[4], ly, a[5] * lz));
+            const float rz = __builtin_fmaf(a[6], lx, __builtin_fmaf(a[7], ly, a[8] * lz));
+            const double fx = d.rfx[i], fy = d.rfy[i], fz = d.rfz[i];
+            acc[0] += fx; acc[1] += fy; acc[2] += fz;
+            acc[3] += static_cast<double>(ry) * fz - static_cast<double>(rz) * fy;
+            acc[4] += static_cast<double>(rz) * fx - static_cast<double>(rx) * fz;
+            acc[5] += static_cast<double>(rx) * fy - static_cast<double>(ry) * fx;
+        }
+        for (int f = 0; f < 6; f++) { red[f][t] = acc[f]; }
+        __syncthreads();
+        for (uint32_t o = kBodyThreads / 2; o >= 64u; o >>= 1)
+        {
+            if (t < o) { for (int f = 0; f < 6; f++) { red[f][t] += red[f][t + o]; } }
+            __syncthreads();
+        }
+        if (t >= 64u) { return; }
+        for (int f = 0; f < 6; f++)
+        {
+            // the last six halvings in the first wave (lanes past each half hold what is not used)
+            double v = red[f][t];
+            for (int o = 32; o > 0; o >>= 1) { v += __shfl_down(v, o, 64); }
+            acc[f] = v;
+        }
+        if (t != 0u) { return; }
+        const Consts& k = d.consts[d.bodyScene[b]];
+        const float m = rbv(d, RB_MASS, b), mi = rbv(d, RB_MASS_INV, b);
+        float g[6] = { 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f };
+        if (!(m <= 0.0f || mi <= 0.0f)) { g[0] += m * k.gx; g[1] += m * k.gy; g[2] += m * k.gz; }
+        for (int f = 0; f < 6; f++) { d.rbForce[f * nb + b] = g[f] + static_cast<float>(acc[f]); }
+    }
+
+    // A body's part of a step in one block: the force sums, the prediction, the integration and the body's
+    // particles, whichever `parts` asks for, in this order. Each was a launch of 4 to 10 us of which little
+    // more than the launch was needed. More than kBodyParticles in the context are updated by a launch of
+    // their own: one block takes about 2 us per thousand (6,364 particles: 22 us together, 16 apart).
+    constexpr uint32_t kBodyParticles = 2048;
+    enum BodyParts { kBodySums = 1, kBodyPredict = 2, kBodyIntegrate = 4, kBodyUpdate = 8, kBodyUpdatePredicted = 16 };
+
+    __global__ void __launch_bounds__(kBodyThreads) kRigidBody(Dev d, uint32_t parts)
+    {
+        if (stopped(d)) { return; }
+        const uint32_t b = blockIdx.x;
+        if (parts & kBodySums) { rigidForceSums(d, b); }
+        if (threadIdx.x == 0u)
+        {
+            if (parts & kBodyPredict) { rigidPredictOne(d, b); }
+            if (parts & kBodyIntegrate) { rigidIntegrateOne(d, b); }
+        }
+        if ((parts & (kBodyUpdate | kBodyUpdatePredicted)) == 0u) { return; }
+        __syncthreads();   // (the body's new state, written by thread 0, is read by the block)
+        for (uint32_t q = d.byBodyOff[b] + threadIdx.x; q < d.byBodyOff[b + 1]; q += kBodyThreads)
+        {
+            rigidUpdateOne(d, d.byBodyIdx[q], (parts & kBodyUpdatePredicted) != 0u);
+        }
+    }
+
     // ----------------------------------------------------------------------------------------
     // host launchers
 
@@ -1388,12 +1396,9 @@ namespace tsp
     }
     void launchSourceDiag(hipStream_t s, const Dev& d)
     {
-        if (d.nF)
-        {
-            if (d.fastPairs) { kSourceDiag<true><<<blocksOf(d.nF), kBlock, 0, s>>>(d); }
-            else { kSourceDiag<false><<<blocksOf(d.nF), kBlock, 0, s>>>(d); }
-        }
-        if (d.nScenes) { kSolverInit<<<1, kBlock, 0, s>>>(d); }
+        if (!d.nScenes) { return; }
+        if (d.fastPairs) { kSourceDiag<true><<<blocksOf(d.nF) + 1u, kBlock, 0, s>>>(d); }
+        else { kSourceDiag<false><<<blocksOf(d.nF) + 1u, kBlock, 0, s>>>(d); }
     }
     void launchPressureAcc(hipStream_t s, const Dev& d, bool sweep)
     {
@@ -1422,12 +1427,24 @@ namespace tsp
     void launchIntegration(hipStream_t s, const Dev& d) { if (d.nF) { kIntegration<<<blocksOf(d.nF), kBlock, 0, s>>>(d); } }
 
     void launchRigidUpdate(hipStream_t s, const Dev& d, bool predicted) { if (d.nR) { kRigidUpdate<<<blocksOf(d.nR), kBlock, 0, s>>>(d, predicted); } }
-    void launchRigidClearGravity(hipStream_t s, const Dev& d) { if (d.nRB) { kRigidClearGravity<<<blocksOf(d.nRB), kBlock, 0, s>>>(d); } }
     void launchRigidForces(hipStream_t s, const Dev& d, bool pressure)
     {
         if (d.nR) { kRigidForces<<<blocksOf(64ull * d.nR), kBlock, 0, s>>>(d, pressure); }
     }
-    void launchRigidReduce(hipStream_t s, const Dev& d) { if (d.nRB) { kRigidReduce<<<d.nRB, kReduceThreads, 0, s>>>(d); } }
-    void launchRigidPredict(hipStream_t s, const Dev& d) { if (d.nRB) { kRigidPredict<<<blocksOf(d.nRB), kBlock, 0, s>>>(d); } }
-    void launchRigidIntegrate(hipStream_t s, const Dev& d) { if (d.nRB) { kRigidIntegrate<<<blocksOf(d.nRB), kBlock, 0, s>>>(d); } }
+    static void launchRigidBody(hipStream_t s, const Dev& d, uint32_t parts)
+    {
+        if (!d.nRB) { return; }
+        const bool alone = d.nR > kBodyParticles;
+        constexpr uint32_t kUpdates = kBodyUpdate | kBodyUpdatePredicted;
+        kRigidBody<<<d.nRB, kBodyThreads, 0, s>>>(d, alone ? parts & ~kUpdates : parts);
+        if (alone && (parts & kUpdates)) { launchRigidUpdate(s, d, (parts & kBodyUpdatePredicted) != 0u); }
+    }
+    // the bodies after the non-pressure reaction: forces, prediction, predicted particles
+    void launchRigidPredict(hipStream_t s, const Dev& d) { launchRigidBody(s, d, kBodySums | kBodyPredict | kBodyUpdatePredicted); }
+    // after the pressure reaction: forces; then (a contact solve adds its loads between) the bodies' new state
+    void launchRigidSums(hipStream_t s, const Dev& d) { launchRigidBody(s, d, kBodySums); }
+    void launchRigidFinish(hipStream_t s, const Dev& d, bool sums)
+    {
+        launchRigidBody(s, d, (sums ? kBodySums : 0u) | kBodyPredict | kBodyIntegrate | kBodyUpdate);
+    }
 }

@@ -30,14 +30,14 @@
 
 namespace tsp
 {
-    void launchResetSearch(hipStream_t, const Dev&);
+    void launchResetSearch(hipStream_t, const Dev&, bool);
     void launchKeys(hipStream_t, const Dev&, int, const float4*, uint32_t, bool, uint32_t*, uint32_t*, uint32_t, uint32_t*);
     void launchKeysSorted(hipStream_t, const Dev&, const float4*, uint32_t, uint32_t*, uint32_t*);
     bool launchRadixSort(hipStream_t, bool, uint32_t*, uint32_t*, uint32_t*, uint32_t*, uint32_t, uint32_t, uint32_t*, uint32_t*,
                          bool, bool);
     bool radixSortSingleBlock(uint32_t n);
     void launchPermute(hipStream_t, const Gather&, const uint32_t*);
-    void launchClearCells(hipStream_t, const Dev&, const uint32_t*, uint32_t, uint2*);
+    void launchPermuteCells(hipStream_t, const Dev&, const Gather&);
     void launchClearAll(hipStream_t, uint2*, uint64_t);
     void launchBuildCells(hipStream_t, const Dev&, const uint32_t*, uint32_t, uint2*);
     void launchQueryCount(hipStream_t, const Dev&);
@@ -62,11 +62,10 @@ namespace tsp
     void launchSolve(hipStream_t, const Dev&);
     void launchIntegration(hipStream_t, const Dev&);
     void launchRigidUpdate(hipStream_t, const Dev&, bool);
-    void launchRigidClearGravity(hipStream_t, const Dev&);
     void launchRigidForces(hipStream_t, const Dev&, bool);
-    void launchRigidReduce(hipStream_t, const Dev&);
     void launchRigidPredict(hipStream_t, const Dev&);
-    void launchRigidIntegrate(hipStream_t, const Dev&);
+    void launchRigidSums(hipStream_t, const Dev&);
+    void launchRigidFinish(hipStream_t, const Dev&, bool);
     void launchStats(hipStream_t, const uint16_t* const (&)[3], const uint32_t* const (&)[3], uint32_t, uint32_t, const float4*,
                      uint32_t, float, uint32_t*, double*, uint64_t*, double*);
     hipError_t statsScratchInit(int);
@@ -1260,7 +1259,7 @@ struct tsp_ctx
         // boundary: re-sorted only if its ids are not already non-decreasing (neighbor_search.cpp:1755-1811)
         if (d.nB)
         {
-            launchResetSearch(stream, d);
+            launchResetSearch(stream, d, false);
             launchKeysSorted(stream, d, d.bpos, d.nB, d.keyF, d.idxF);
             uint32_t unsorted = 0;
             hipCheck(hipMemcpyAsync(&unsorted, &d.status->bUnsorted, 4, hipMemcpyDeviceToHost, stream), "flag D2H");
@@ -1307,18 +1306,34 @@ struct tsp_ctx
         }
     }
 
+    // the rigid particles' part of a search phase on the side stream, the fluid's beside it (they read the
+    // same sorted particles and write different lists), while the fluid's leaves room on the chip: 432
+    // blocks hide 30 us of rigid launches; with 3,907 the small launches wait behind them, and a step of
+    // 2.8 ms is 1% slower
+    static constexpr uint32_t kBesideBlocks = 1024;
+
+    template <typename Rigid, typename Fluid>
+    void besideRigid(Rigid&& rigid, Fluid&& fluid)
+    {
+        const bool fork = d.nR && !prof.on && d.nF / kBlock <= kBesideBlocks;
+        if (fork)
+        {
+            hipCheck(hipEventRecord(forkEv, stream), "hipEventRecord");
+            hipCheck(hipStreamWaitEvent(side, forkEv, 0), "hipStreamWaitEvent");
+            rigid(side);
+            hipCheck(hipEventRecord(joinEv, side), "hipEventRecord");
+        }
+        fluid();
+        if (fork) { hipCheck(hipStreamWaitEvent(stream, joinEv, 0), "hipStreamWaitEvent"); }
+        else if (d.nR) { rigid(stream); }
+    }
+
     // the search up to its status: keys, sorts, re-order, cell tables, counts, list offsets
     void searchFront(bool allFields)
     {
         {
             Scope sc(prof, stream, "reset");
-            launchResetSearch(stream, d);
-            // the runs of the previous sorted keys are the only non-empty cells
-            if (!cellsClean)
-            {
-                launchClearCells(stream, d, d.keyF, d.nF, d.cellF);
-                launchClearCells(stream, d, d.keyR, d.nR, d.cellR);
-            }
+            launchResetSearch(stream, d, !cellsClean);
         }
         // a single-block rigid sort shares no scratch with the fluid sort: it runs beside it
         const bool fork = d.nR && radixSortSingleBlock(d.nR) && !prof.on;
@@ -1339,6 +1354,7 @@ struct tsp_ctx
                 std::swap(d.keyR, d.keyR2);
                 std::swap(d.idxR, d.idxR2);
             }
+            launchBuildCells(rs, d, d.keyR, d.nR, d.cellR);
             if (fork) { hipCheck(hipEventRecord(joinEv, side), "hipEventRecord"); }
         }
         {
@@ -1368,20 +1384,14 @@ struct tsp_ctx
             }
             g.idS = d.id; g.idD = idF2;
             g.n = d.nF;
-            launchPermute(stream, g, d.idxF);
+            launchPermuteCells(stream, d, g);
         }
         swapFields(allFields);
+        cellsClean = false;
         if (fork) { hipCheck(hipStreamWaitEvent(stream, joinEv, 0), "hipStreamWaitEvent"); }
         {
-            Scope sc(prof, stream, "cells");
-            launchBuildCells(stream, d, d.keyF, d.nF, d.cellF);
-            launchBuildCells(stream, d, d.keyR, d.nR, d.cellR);
-            cellsClean = false;
-        }
-        {
             Scope sc(prof, stream, "query_count");
-            launchQueryCount(stream, d);
-            launchQueryRigid(stream, d, 0, d.scanTmp);
+            besideRigid([&](hipStream_t rs) { launchQueryRigid(rs, d, 0, d.scanTmp); }, [&]() { launchQueryCount(stream, d); });
         }
     }
 
@@ -1447,8 +1457,8 @@ struct tsp_ctx
             }
             {
                 Scope sc(prof, stream, "query_fill");
-                launchQueryFill(stream, d);
-                launchQueryRigid(stream, d, contactLists ? 2 : 1, d.scanTmp);
+                besideRigid([&](hipStream_t rs) { launchQueryRigid(rs, d, contactLists ? 2 : 1, d.scanTmp); },
+                            [&]() { launchQueryFill(stream, d); });
             }
             listsValid = true;
             return;
@@ -1523,7 +1533,6 @@ struct tsp_ctx
             Scope sc(prof, stream, "density");
             launchDensity(stream, d);
         }
-        if (d.nRB) { launchRigidClearGravity(stream, d); }
         {
             Scope sc(prof, stream, "nonpressure");
             launchNonPressure(stream, d);
@@ -1532,9 +1541,7 @@ struct tsp_ctx
         {
             Scope sc(prof, stream, "rigid");
             launchRigidForces(stream, d, false);
-            launchRigidReduce(stream, d);
             launchRigidPredict(stream, d);
-            launchRigidUpdate(stream, d, true);
         }
         {
             Scope sc(prof, stream, "source_diag");
@@ -1605,24 +1612,22 @@ struct tsp_ctx
             Scope sc(prof, stream, "pressure_acc_final");
             launchPressureAcc(stream, d, false);
         }
+        const bool contacts = d.nRB && contactLists;
         if (d.nRB)
         {
             Scope sc(prof, stream, "rigid");
             launchRigidForces(stream, d, true);
-            launchRigidClearGravity(stream, d);
-            launchRigidReduce(stream, d);
+            if (contacts) { launchRigidSums(stream, d); }
         }
         {
             Scope sc(prof, stream, "integration");
             launchIntegration(stream, d);
         }
-        if (d.nRB && contactLists) { solveContacts(); }
+        if (contacts) { solveContacts(); }
         if (d.nRB)
         {
             Scope sc(prof, stream, "rigid");
-            launchRigidPredict(stream, d);
-            launchRigidIntegrate(stream, d);
-            launchRigidUpdate(stream, d, false);
+            launchRigidFinish(stream, d, !contacts);
         }
     }
 
@@ -1737,8 +1742,7 @@ struct tsp_ctx
             searchFront(false);
             launchStepGate(stream, d);
             d.stopMask = 1u;
-            launchQueryFill(stream, d);
-            launchQueryRigid(stream, d, 1, d.scanTmp);
+            besideRigid([&](hipStream_t rs) { launchQueryRigid(rs, d, 1, d.scanTmp); }, [&]() { launchQueryFill(stream, d); });
             predictLaunches();
         });
         // d.stopMask is 1 here (the state the piece leaves)

@@ -390,8 +390,8 @@ namespace tsp
         float *cLoad;                // 6 x nRB: contact force and torque
         uint32_t *cBodyB;            // nRB: boundary contacts of each movable body
         float4 *fbGrad;          // per FB pool unit: gradient and psi of an entry, kept for a solve in one launch
-        uint32_t *solveFlag;     // per block of such a launch: the barriers that it has come to (zeroed by kSolverInit)
-        uint32_t *solveBar;      // kBarWords per scene: the entry of kSolve (zeroed by kSolverInit)
+        uint32_t *solveFlag;     // per block of such a launch: the barriers that it has come to (zeroed by solverInit)
+        uint32_t *solveBar;      // kBarWords per scene: the entry of kSolve (zeroed by solverInit)
         // reductions and scans
         double *errPartial;      // Jacobi error partials, [3][blocks of the fluid grid]
         uint32_t *scanTmp;       // block sums of the multi-block scans
@@ -662,13 +662,15 @@ namespace tsp
 
     // blocks are dispatched round-robin over the 8 XCDs; this maps them so that each XCD walks
     // one contiguous range of particles, which keeps neighbor gathers inside its own L2
-    __device__ __forceinline__ uint32_t xcdBlock()
+    __device__ __forceinline__ uint32_t xcdBlock(uint32_t nb)
     {
-        const uint32_t nb = gridDim.x, b = blockIdx.x;
+        const uint32_t b = blockIdx.x;
         const uint32_t xcd = b & 7u, k = b >> 3;
         const uint32_t per = nb >> 3, rem = nb & 7u;
         return xcd < rem ? xcd * (per + 1u) + k : rem * (per + 1u) + (xcd - rem) * per + k;
     }
+    __device__ __forceinline__ uint32_t xcdBlock() { return xcdBlock(gridDim.x); }
+
     // FF entries of a block with a halo hold the byte offset of the neighbor's 16-byte record in
     // the block's LDS halo (slot << kSlotShift), so a sweep addresses the record without a shift
     // (kSourceDiag puts each pair's kgShort correction into the four low bits: kSlotMask)
