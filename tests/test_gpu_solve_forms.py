@@ -96,3 +96,22 @@ def test_scenes_of_one_context_stop_by_themselves():
             g.step(1)
             same(b.push(i), g.push())
             same_report(b.info(i), g.info())
+
+
+def test_context_that_held_a_larger_scene():
+    print("case: 120,000 particles, then 4,900, then 65,000", flush=True)
+    p = scenes.make_params(H, termination_cond=scenes.TERM_POS)
+    g = HipBackend(0)
+    g.set_params(p)
+    for st in (block(60, 50, 40), block(17, 17, 17), block(65, 40, 25)):
+        fresh = HipBackend(0)
+        fresh.set_params(p)
+        fresh.profile_enable(True)
+        for b in (g, fresh):
+            b.pull(st)
+            b.step(2)
+        same(g.push(), fresh.push())
+        same_report(g.info(), fresh.info())
+        if st.n[0] < 65536:
+            # the solve's records are sized by the scene, not by the pools that the context keeps
+            assert g.memory().alloc_bytes - fresh.memory().alloc_bytes < (1 << 30)

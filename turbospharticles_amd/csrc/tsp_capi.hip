@@ -313,6 +313,8 @@ struct tsp_ctx
     std::vector<void*> work;        // search and scene-table buffers sized by the layout
     std::vector<void*> frameAllocs; // cell tables
     std::vector<void*> poolAllocs;  // SELL-32 pools and the RF list
+    std::vector<void*> solveAllocs; // the FB records of a solve in one launch
+    uint64_t fbCap = 0;
     std::vector<void*> contactAllocs; // RB/RR lists and the contact boundary arrays (grown on demand)
     uint64_t cellCap = 0;
     uint64_t cellLimit = 0xffffffffull;   // most cells of all scenes' frames (tsp_set_cell_limit)
@@ -353,6 +355,7 @@ struct tsp_ctx
         dropStepGraphs();
         releaseList(statAllocs);
         releaseList(poolAllocs);
+        releaseList(solveAllocs);
         releaseList(contactAllocs);
         releaseList(expAllocs);
         releaseList(frameAllocs);
@@ -605,14 +608,28 @@ struct tsp_ctx
         }
         d.rfCap = rfCap;
         d.rfIdx = alloc<uint32_t>(rfCap, poolAllocs, MEM_LR);
-        d.fbGrad = nullptr;
     }
 
-    // the FB records of a solve in one launch (contexts of few blocks), for the present pools
+    // The FB records of a solve in one launch, for contexts of few blocks: as long as the FB pool, but no
+    // more than 64 units per particle (the pool may be a larger scene's that the context held before; a
+    // search that uses more solves launch by launch, and so does a context without the memory).
     void allocSolve()
     {
-        if (d.fbGrad || d.nF / kBlock > kSolveBlocksMost) { return; }
-        d.fbGrad = alloc<float4>(d.poolCap[1], poolAllocs, MEM_LF);
+        const bool few = d.nF != 0u && d.nF / kBlock <= kSolveBlocksMost;
+        const uint64_t want = few ? std::min<uint64_t>(d.poolCap[1], 64ull * d.nF + 1024u) : 0u;
+        if (want == 0u || want > fbCap)
+        {
+            releaseList(solveAllocs);
+            d.fbGrad = nullptr;
+            fbCap = 0;
+        }
+        if (want == 0u || d.fbGrad) { return; }
+        try
+        {
+            d.fbGrad = alloc<float4>(want, solveAllocs, MEM_LF);
+            fbCap = want;
+        }
+        catch (const Error&) { (void)hipGetLastError(); }
     }
 
     // the fluid fields of a scene in the records of n (missing fields are left out)
@@ -1600,7 +1617,7 @@ struct tsp_ctx
     bool solveInOne() const
     {
         const uint32_t nBlocks = d.nF / kBlock;
-        return !prof.on && d.fbGrad && !solveHold && nBlocks <= kSolveBlocksMost && nBlocks <= cuCount;
+        return !prof.on && d.fbGrad && last.poolUnits[1] <= fbCap && !solveHold && nBlocks <= kSolveBlocksMost && nBlocks <= cuCount;
     }
 
     // final pressure accelerations (unless the solve left them), rigid coupling, integration and the
