@@ -218,19 +218,30 @@ int tsp_get_statistics(tsp_ctx *ctx, tsp_statistics *out);
 int tsp_get_statistics_noalloc(tsp_ctx *ctx, tsp_statistics *out);
 
 /* Device memory a context holds, by what it stores, in bytes (I_SimBackend::FillMemoryRecord,
-   core/backend_sim.h:239, with the buckets of eval/memory/categories.h:59-78). Blocks of at most
-   2 GiB that a context keeps for its next layout after it replaced one are not counted; they go
-   when the device runs out of other memory and with the context. */
+   core/backend_sim.h:239, with the buckets of eval/memory/categories.h:59-78). misc includes the
+   blocks that a context keeps for its next layout after it replaced one: at most 2 GiB, and 8 GiB
+   over all contexts on a GPU. An allocation of any context of the process that finds no other memory takes
+   them back; for other users of the GPU, tsp_trim gives them back. */
 typedef struct tsp_memory {
     uint64_t particles[3];      /* fluid, boundary, rigid particle (and body) arrays */
     uint64_t search[3];         /* sort keys and indices, cell tables: fluid, boundary, rigid */
     uint64_t lists[3];          /* fluid-source lists (SELL-32 pools, counts, slice metadata,
                                    halos); none for boundary sources; rigid-source lists */
-    uint64_t misc;              /* scans, reductions, solver state, statistics and export scratch */
+    uint64_t misc;              /* scans, reductions, solver state, statistics and export scratch,
+                                   kept blocks */
     uint64_t alloc_bytes;       /* all of the above */
     uint64_t peak_alloc_bytes;  /* the largest alloc_bytes since tsp_create */
 } tsp_memory;
 int tsp_get_memory(tsp_ctx *ctx, tsp_memory *out);
+
+/* gives back the blocks that the context keeps for its next layout (a program calls it before it
+   hands the GPU's memory to something else). No reference counterpart: the reference frees. */
+int tsp_trim(tsp_ctx *ctx);
+
+/* the most device memory that the contexts of the process on this GPU may hold together when this
+   one allocates (no limit by default). An allocation beyond it fails as one that the GPU has no
+   memory for: the blocks kept by all contexts are given back first. No reference counterpart. */
+int tsp_set_memory_limit(tsp_ctx *ctx, uint64_t max_bytes);
 
 /* Sync::ExportSnapshot (sync/snapshots.h:37-66) as the caller's arrays. The fluid arrays hold
    the exported particles: those near the surface (IsNearSurfaceFluidParticle, core/backend_sim.h:

@@ -174,6 +174,8 @@ def _declare_hip(lib):
         "tsp_get_statistics": (i, [vp, ctypes.POINTER(TspStatistics)]),
         "tsp_get_statistics_noalloc": (i, [vp, ctypes.POINTER(TspStatistics)]),
         "tsp_get_memory": (i, [vp, ctypes.POINTER(TspMemory)]),
+        "tsp_trim": (i, [vp]),
+        "tsp_set_memory_limit": (i, [vp, ctypes.c_uint64]),
         "tsp_batch_scene_statistics": (i, [vp, ctypes.c_uint32, ctypes.POINTER(TspStatistics)]),
         "tsp_export_snapshot": (i, [vp, ctypes.c_uint32, ctypes.c_uint64, ctypes.POINTER(TspExportView)]),
         "tsp_batch_export_snapshot": (i, [vp, ctypes.c_uint32, ctypes.c_uint32, ctypes.c_uint64,

@@ -175,6 +175,14 @@ class HipBackend:
         self._check(self.lib.tsp_get_memory(self.h, ctypes.byref(m)), "tsp_get_memory")
         return m
 
+    def trim(self):
+        """Gives back the device blocks kept for the next layout (tsp_trim)."""
+        self._check(self.lib.tsp_trim(self.h), "tsp_trim")
+
+    def set_memory_limit(self, max_bytes):
+        """The most device memory of all contexts on this GPU when this one allocates (tsp_set_memory_limit)."""
+        self._check(self.lib.tsp_set_memory_limit(self.h, int(max_bytes)), "tsp_set_memory_limit")
+
     # I_SimBackend::FillStatisticsRecord
     def statistics(self):
         st = _capi.TspStatistics()
@@ -349,6 +357,11 @@ class HipBatch:
 
     # the per-launch-group times (HipBackend.profile_read)
     profile_read = HipBackend.profile_read
+
+    # the context's device memory (HipBackend.memory, trim, set_memory_limit)
+    memory = HipBackend.memory
+    trim = HipBackend.trim
+    set_memory_limit = HipBackend.set_memory_limit
 
     @staticmethod
     def footprint(n):

@@ -24,6 +24,7 @@
 #include <vector>
 
 #include "scene_plan.h"
+#include "tsp_blocks.h"
 #include "tsp_device.h"
 #include "tsp_hip.h"
 #include "tsp_transfer.h"
@@ -361,7 +362,7 @@ struct tsp_ctx
         releaseList(frameAllocs);
         releaseList(work);
         releaseList(arena);
-        dropSpare();
+        blocks.trim();
         if (hostBlock) { (void)hipHostFree(hostBlock); }
         if (stage) { (void)hipHostFree(stage); }
         for (hipEvent_t e : stageEv) { if (e) { (void)hipEventDestroy(e); } }
@@ -371,64 +372,35 @@ struct tsp_ctx
         if (stream) { (void)hipStreamDestroy(stream); }
     }
 
-    // device memory the context holds, by what it stores (tsp_memory)
+    // device memory the context uses, by what it stores (tsp_memory)
     enum MemCat : uint8_t { MEM_PF, MEM_PB, MEM_PR, MEM_SF, MEM_SB, MEM_SR, MEM_LF, MEM_LR, MEM_MISC, kMemCats };
     struct Held
     {
-        uint64_t bytes;     // asked for
         uint64_t size;      // of the block
         uint8_t cat;
     };
+    Blocks blocks;          // and the released blocks that it keeps
     std::unordered_map<void*, Held> allocated;
     uint64_t memBytes[kMemCats] = {};
-    uint64_t memTotal = 0, memPeak = 0;
-
-    // Released blocks wait here for the next layout, which mostly asks for the same sizes: a scene pulled
-    // anew freed and allocated 83 blocks, 9.4 of the 11.7 ms of a pull at 1M particles (hipFree unmaps).
-    // At most kSpareMost bytes stay (under 1% of the device); they go when the device has no other memory
-    // left, and with the context. Blocks come back in the order of the context's streams, whose work on
-    // them was waited for or precedes their next use.
-    static constexpr uint64_t kSpareMost = 2ull << 30;
-    std::multimap<uint64_t, void*> spare;
-    uint64_t spareBytes = 0;
-
-    void dropSpare()
-    {
-        for (const auto& s : spare) { (void)hipFree(s.second); }
-        spare.clear();
-        spareBytes = 0;
-    }
 
     template <typename T>
     T* alloc(size_t n, std::vector<void*>& list, MemCat cat = MEM_MISC)
     {
         void* p = nullptr;
-        const uint64_t bytes = std::max<size_t>(n, 1) * sizeof(T);
-        uint64_t size = bytes;
-        const auto it = spare.lower_bound(bytes);
-        if (it != spare.end() && it->first <= bytes + bytes / 8u + 256u)
+        uint64_t size = 0;
+        list.reserve(list.size() + 1u);
+        hipCheck(blocks.take(std::max<size_t>(n, 1) * sizeof(T), &p, &size), "hipMalloc");
+        try
         {
-            size = it->first;
-            p = it->second;
-            spareBytes -= size;
-            spare.erase(it);
+            allocated[p] = Held{ size, static_cast<uint8_t>(cat) };
         }
-        else
+        catch (...)
         {
-            hipError_t e = hipMalloc(&p, bytes);
-            if (e == hipErrorOutOfMemory && !spare.empty())
-            {
-                (void)hipGetLastError();
-                dropSpare();
-                e = hipMalloc(&p, bytes);
-            }
-            hipCheck(e, "hipMalloc");
+            blocks.release(p, size);
+            throw;
         }
         list.push_back(p);
-        allocated[p] = Held{ bytes, size, static_cast<uint8_t>(cat) };
-        memBytes[cat] += bytes;
-        memTotal += bytes;
-        memPeak = std::max(memPeak, memTotal);
+        memBytes[cat] += size;
         return static_cast<T*>(p);
     }
 
@@ -438,14 +410,26 @@ struct tsp_ctx
         {
             const auto it = allocated.find(p);
             const Held h = it->second;
-            memBytes[h.cat] -= h.bytes;
-            memTotal -= h.bytes;
+            memBytes[h.cat] -= h.size;
             allocated.erase(it);
-            if (spareBytes + h.size > kSpareMost) { (void)hipFree(p); continue; }
-            spare.emplace(h.size, p);
-            spareBytes += h.size;
+            blocks.release(p, h.size);
         }
         list.clear();
+    }
+
+    // a graph made ready to run; the kept blocks go when the device has no other memory for it
+    hipGraphExec_t instantiate(hipGraph_t g)
+    {
+        hipGraphExec_t e = nullptr;
+        hipError_t rc = hipGraphInstantiate(&e, g, nullptr, nullptr, 0);
+        if (rc == hipErrorOutOfMemory && blocks.trimDevice())
+        {
+            (void)hipGetLastError();
+            rc = hipGraphInstantiate(&e, g, nullptr, nullptr, 0);
+        }
+        (void)hipGraphDestroy(g);
+        hipCheck(rc, "hipGraphInstantiate");
+        return e;
     }
 
     void sync() { hipCheck(hipStreamSynchronize(stream), "hipStreamSynchronize"); }
@@ -1532,11 +1516,7 @@ struct tsp_ctx
                 throw;
             }
             hipCheck(hipStreamEndCapture(stream, &g), "hipStreamEndCapture");
-            hipGraphExec_t e = nullptr;
-            const hipError_t rc = hipGraphInstantiate(&e, g, nullptr, nullptr, 0);
-            (void)hipGraphDestroy(g);
-            hipCheck(rc, "hipGraphInstantiate");
-            it = graphs.emplace(std::move(key), e).first;
+            it = graphs.emplace(std::move(key), instantiate(g)).first;
         }
         hipCheck(hipGraphLaunch(it->second, stream), "hipGraphLaunch");
     }
@@ -1738,11 +1718,9 @@ struct tsp_ctx
             }
             hipCheck(hipStreamEndCapture(stream, &g), "hipStreamEndCapture");
             StepGraph sg;
-            const hipError_t rc = hipGraphInstantiate(&sg.exec, g, nullptr, nullptr, 0);
-            (void)hipGraphDestroy(g);
             sg.after = d; sg.pos2 = pos2; sg.vel2 = vel2; sg.idF2 = idF2;
             d = before; pos2 = p2; vel2 = v2; idF2 = i2;
-            hipCheck(rc, "hipGraphInstantiate");
+            sg.exec = instantiate(g);
             it = stepGraphs.emplace(std::move(key), sg).first;
         }
         hipCheck(hipGraphLaunch(it->second.exec, stream), "hipGraphLaunch");
@@ -2155,6 +2133,7 @@ int tsp_create(int device, tsp_ctx** out)
     if (hipGetDeviceCount(&n) != hipSuccess || device < 0 || device >= n) { return TSP_ERR_HIP; }
     tsp_ctx* c = new tsp_ctx();
     c->device = device;
+    c->blocks.join(device);
     int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess) { c->cuCount = static_cast<uint32_t>(cus); }
     // statsScratchInit: the device address of this device's statistics scratch, once per device
@@ -2549,9 +2528,26 @@ int tsp_get_memory(tsp_ctx* ctx, tsp_memory* out)
         }
         out->lists[0] = ctx->memBytes[tsp_ctx::MEM_LF];
         out->lists[2] = ctx->memBytes[tsp_ctx::MEM_LR];
-        out->misc = ctx->memBytes[tsp_ctx::MEM_MISC];
-        out->alloc_bytes = ctx->memTotal;
-        out->peak_alloc_bytes = ctx->memPeak;
+        uint64_t kept = 0;
+        ctx->blocks.bytes(&kept, &out->alloc_bytes, &out->peak_alloc_bytes);
+        out->misc = ctx->memBytes[tsp_ctx::MEM_MISC] + kept;
+        return TSP_OK;
+    });
+}
+
+int tsp_trim(tsp_ctx* ctx)
+{
+    return guarded(ctx, [&]() {
+        ctx->blocks.trim();
+        return TSP_OK;
+    });
+}
+
+int tsp_set_memory_limit(tsp_ctx* ctx, uint64_t max_bytes)
+{
+    return guarded(ctx, [&]() {
+        if (max_bytes == 0) { throw Error{ TSP_ERR_INVALID, "memory limit of 0 bytes" }; }
+        ctx->blocks.setLimit(max_bytes);
         return TSP_OK;
     });
 }
