@@ -325,6 +325,8 @@ struct tsp_ctx
     uint64_t contactRB = 0;         // RB entries (bounds the contact boundary particles)
     uint32_t* contactScanTmp = nullptr;
 
+    bool workReady = false;         // the buffers of the layout are all there (an allocation may fail between)
+    uint32_t layouts = 0;           // arenas installed
     bool layoutDirty = true;        // key bases and cell offsets must be assigned again
     bool listsValid = false;        // a neighbor search ran since the last layout
     bool cellsClean = false;        // fluid and rigid cell tables hold no runs
@@ -585,13 +587,17 @@ struct tsp_ctx
     void allocPools(const uint64_t cap[3], uint64_t rfCap)
     {
         releaseList(poolAllocs);
+        // (a pool counts as long as it says only once it is there, here and below: an allocation that
+        // fails leaves sizes of 0, and the next search or layout asks again)
+        for (int r = 0; r < 3; r++) { d.poolCap[r] = 0; }
+        d.rfCap = 0;
         for (int r = 0; r < 3; r++)
         {
-            d.poolCap[r] = cap[r];
             d.pool[r] = alloc<uint16_t>(cap[r] + kPoolPad, poolAllocs, MEM_LF);
+            d.poolCap[r] = cap[r];
         }
-        d.rfCap = rfCap;
         d.rfIdx = alloc<uint32_t>(rfCap, poolAllocs, MEM_LR);
+        d.rfCap = rfCap;
     }
 
     // The FB records of a solve in one launch, for contexts of few blocks: as long as the FB pool, but no
@@ -719,7 +725,7 @@ struct tsp_ctx
     // --- storage of the contact solve sized by the RB and RR entries of a search ---
     void ensureContactCapacity(uint64_t rbTotal, uint64_t rrTotal)
     {
-        if (rbTotal <= d.rbCap && rrTotal <= d.rrCap && !contactAllocs.empty()) { return; }
+        if (rbTotal <= d.rbCap && rrTotal <= d.rrCap && d.rbCap) { return; }
         if (rbTotal > 0x7fffffffull || rrTotal > 0x7fffffffull)
         {
             throw Error{ TSP_ERR_CAPACITY, "rigid contact lists exceed 2^31 entries" };
@@ -728,8 +734,7 @@ struct tsp_ctx
         const uint64_t rrCap = std::max<uint64_t>(d.rrCap, rrTotal + rrTotal / 4 + 256);
         sync();
         releaseList(contactAllocs);
-        d.rbCap = rbCap;
-        d.rrCap = rrCap;
+        d.rbCap = d.rrCap = 0;
         d.rbIdx = alloc<uint32_t>(rbCap, contactAllocs, MEM_LR);
         d.rrIdx = alloc<uint32_t>(rrCap, contactAllocs, MEM_LR);
         d.cbLocal = alloc<uint32_t>(rbCap, contactAllocs, MEM_LR);
@@ -742,6 +747,8 @@ struct tsp_ctx
         const uint64_t m = std::max<uint64_t>(d.nB + 1ull, rbCap + 1);
         contactScanTmp = alloc<uint32_t>(scanTmpWords(m), contactAllocs);
         zero(contactScanTmp, sizeof(uint32_t) * scanTmpWords(m));
+        d.rbCap = rbCap;
+        d.rrCap = rrCap;
     }
 
     // SolveRigidContacts (CPU/backend/rigid_solver.cpp:602-799) for every scene whose rigid
@@ -956,6 +963,8 @@ struct tsp_ctx
         releaseList(scratch);
 
         // install the new arena
+        workReady = false;
+        layouts++;
         releaseList(arena);
         arena = std::move(A);
         d = n;
@@ -1082,6 +1091,7 @@ struct tsp_ctx
         // world records of the rigid particles from the body state
         launchRigidUpdate(stream, d, false);
         sync();
+        workReady = true;
     }
 
     // a scene record for a new scene from a host state (validates it)
@@ -1121,6 +1131,7 @@ struct tsp_ctx
     //     tables and the boundary order ---
     void layoutFrames()
     {
+        layoutDirty = true;   // (until the end: a refusal or a failed allocation leaves it so)
         const uint32_t S = nScenes();
         bool rebuild = false;
         for (const SceneHost& h : scenes) { rebuild = rebuild || !h.frameValid; }
@@ -1244,13 +1255,15 @@ struct tsp_ctx
         d.key64 = keyBits > 32 ? 1u : 0u;
         h2d(d.frames, frames.data(), sizeof(Frame) * S);
         h2d(d.sceneKey0, key0.data(), sizeof(uint64_t) * key0.size());
-        if (cells > cellCap || frameAllocs.empty())
+        if (cells > cellCap || cellCap == 0)
         {
             releaseList(frameAllocs);
-            cellCap = std::max<uint64_t>(cells, 1);
-            d.cellF = alloc<uint2>(cellCap, frameAllocs, MEM_SF);
-            d.cellB = alloc<uint2>(cellCap, frameAllocs, MEM_SB);
-            d.cellR = alloc<uint2>(cellCap, frameAllocs, MEM_SR);
+            cellCap = 0;
+            const uint64_t cap = std::max<uint64_t>(cells, 1);
+            d.cellF = alloc<uint2>(cap, frameAllocs, MEM_SF);
+            d.cellB = alloc<uint2>(cap, frameAllocs, MEM_SB);
+            d.cellR = alloc<uint2>(cap, frameAllocs, MEM_SR);
+            cellCap = cap;
         }
         launchClearAll(stream, d.cellF, cells);
         launchClearAll(stream, d.cellB, cells);
@@ -1403,6 +1416,7 @@ struct tsp_ctx
         if (rebuild) { layoutFrames(); }
         for (int attempt = 0; attempt < 4; attempt++)
         {
+            listsValid = false;   // (their counts and headers are overwritten)
             searchFront(allFields);
             readStatus();
             if (last.abort)
@@ -1424,7 +1438,6 @@ struct tsp_ctx
             const auto refuse = [&](const char* why)
             {
                 swapFields(allFields);
-                listsValid = false;
                 throw Error{ TSP_ERR_CAPACITY, why };
             };
             if (last.overflow & 2u) { refuse("neighbor count exceeds the u16 count storage"); }
@@ -1918,6 +1931,7 @@ struct tsp_ctx
     // context's buffers, and nothing is allocated
     void statistics(uint32_t si, tsp_statistics* out, bool noAlloc = false)
     {
+        requireWork();
         const SceneHost& h = scenes[si];
         const uint64_t nb = (static_cast<uint64_t>(h.nF) + kBlock - 1) / kBlock;
         uint32_t* statHist = this->statHist;
@@ -1936,16 +1950,18 @@ struct tsp_ctx
                 throw Error{ TSP_ERR_CAPACITY, "the allocation-free statistics take scenes of at most 2^24 fluid particles" };
             }
         }
-        else if (!statHist || statPartialCap < nb)
+        else if (statPartialCap == 0 || statPartialCap < nb)
         {
             sync();
             releaseList(statAllocs);
+            statPartialCap = 0;
             statHist = this->statHist = alloc<uint32_t>(6ull * 65536ull, statAllocs);
             // the counts, and the fluid sums at kStatsFluidAt behind them (one copy reads both)
             statCounts = this->statCounts = alloc<uint64_t>(2ull * kStatsFluidAt / sizeof(uint64_t), statAllocs);
             statFluid = this->statFluid = reinterpret_cast<double*>(statCounts + kStatsFluidAt / sizeof(uint64_t));
-            statPartialCap = std::max<uint64_t>(nb, 1024);
-            statPartial = this->statPartial = alloc<double>(6 * statPartialCap, statAllocs);
+            const uint64_t cap = std::max<uint64_t>(nb, 1024);
+            statPartial = this->statPartial = alloc<double>(6 * cap, statAllocs);
+            statPartialCap = cap;
         }
         const uint16_t* c16[3] = { d.cnt[REL_FF] + h.offF, d.cnt[REL_FB] + h.offF, d.cnt[REL_FR] + h.offF };
         const uint32_t* c32[3] = { d.rfCnt + h.offR, d.rbCnt + h.offR, d.rrCnt + h.offR };
@@ -1996,12 +2012,14 @@ struct tsp_ctx
         {
             sync();
             releaseList(expAllocs);
-            expCap = std::max<uint64_t>(h.nF + 1ull, 1024);
-            expFlags = alloc<uint32_t>(expCap, expAllocs);
-            expTmp = alloc<uint32_t>(scanTmpWords(expCap), expAllocs);
-            zero(expTmp, sizeof(uint32_t) * scanTmpWords(expCap));
-            expXyz = alloc<float>(3 * expCap, expAllocs);
-            expSpeed = alloc<float>(expCap, expAllocs);
+            expCap = 0;
+            const uint64_t cap = std::max<uint64_t>(h.nF + 1ull, 1024);
+            expFlags = alloc<uint32_t>(cap, expAllocs);
+            expTmp = alloc<uint32_t>(scanTmpWords(cap), expAllocs);
+            zero(expTmp, sizeof(uint32_t) * scanTmpWords(cap));
+            expXyz = alloc<float>(3 * cap, expAllocs);
+            expSpeed = alloc<float>(cap, expAllocs);
+            expCap = cap;
         }
         launchExportSurface(stream, d, h.offF, h.nF, threshold, expFlags, expTmp, expXyz, expSpeed);
         uint32_t count = 0, scanFailed = 0;
@@ -2027,6 +2045,18 @@ struct tsp_ctx
         transfer(fields, true);
         for (size_t i = 0; i < ids.size(); i++) { v->boundary_is_mesh[i] = ids[i] >= meshIdBegin ? 1u : 0u; }
         if (v->rigid_body) { for (uint32_t i = 0; i < h.nR; i++) { v->rigid_body[i] -= h.offRB; } }
+    }
+
+    // for what reads or writes more than the scenes' state: a layout whose buffers could not all be
+    // allocated has kept the state only, and is made again
+    void requireWork()
+    {
+        if (workReady) { return; }
+        sync();
+        releaseList(work);
+        std::vector<Source> all(nScenes());
+        for (uint32_t q = 0; q < nScenes(); q++) { all[q].keep = static_cast<int>(q); }
+        relayout(all);
     }
 
     // one relayout: the listed scenes leave, new scenes join at the end
@@ -2065,19 +2095,28 @@ struct tsp_ctx
             if (x.keep < 0) { x.host.id = nextId++; ids.push_back(x.host.id); }
         }
         const uint32_t nKept = static_cast<uint32_t>(src.size()) - nAdd;
-        relayout(src);
         // the new scenes' frames and key ranges are laid out now, so a context that cannot hold
         // them refuses them here rather than at the next step
+        const uint32_t before = layouts;
         try
         {
+            relayout(src);
             layoutFrames();
         }
-        catch (const Error& e)
+        catch (const Error&)
         {
-            if (e.code != TSP_ERR_CAPACITY || nAdd == 0) { throw; }
-            std::vector<Source> back(nKept);
-            for (uint32_t q = 0; q < nKept; q++) { back[q].keep = static_cast<int>(q); }
-            relayout(back);
+            // the new scenes leave again; those that stay lie before them in the arena, whatever failed after it
+            if (layouts == before || nAdd == 0) { throw; }
+            scenes.resize(nKept);
+            workReady = false;
+            try
+            {
+                requireWork();
+            }
+            catch (const Error&)
+            {
+                // no memory for that either: the next call that needs the buffers tries again
+            }
             throw;
         }
         if (outIds) { for (uint32_t q = 0; q < nAdd; q++) { outIds[q] = ids[q]; } }
@@ -2094,6 +2133,7 @@ struct tsp_ctx
     {
         if (scenes.empty()) { throw Error{ TSP_ERR_STATE, "no state" }; }
     }
+
 };
 
 namespace
@@ -2184,7 +2224,7 @@ int tsp_set_params(tsp_ctx* ctx, const tsp_params* p)
             h.params = *p;
             changed = true;
         }
-        if (changed) { ctx->uploadConsts(); }
+        if (changed && ctx->workReady) { ctx->uploadConsts(); }
         return TSP_OK;
     });
 }
@@ -2285,6 +2325,7 @@ int tsp_neighbor_search(tsp_ctx* ctx)
 {
     return guarded(ctx, [&]() {
         if (ctx->scenes.empty() || !ctx->paramsSet) { throw Error{ TSP_ERR_STATE, "neighbor search before pull/params" }; }
+        ctx->requireWork();
         for (SceneHost& h : ctx->scenes) { h.flags = 0; }
         if (ctx->d.nF == 0 && ctx->d.nB == 0 && ctx->d.nR == 0) { return TSP_OK; }
         ctx->neighborSearch(true);
@@ -2298,6 +2339,7 @@ int tsp_step(tsp_ctx* ctx, uint32_t n)
 {
     return guarded(ctx, [&]() {
         if (ctx->scenes.empty() || !ctx->paramsSet) { throw Error{ TSP_ERR_STATE, "step before pull/params" }; }
+        ctx->requireWork();
         ctx->steps(n);
         return TSP_OK;
     });
@@ -2329,6 +2371,7 @@ int tsp_get_neighbors(tsp_ctx* ctx, int rel, uint32_t* counts, uint32_t* idx, ui
     return guarded(ctx, [&]() {
         if (rel < 0 || rel > 5) { throw Error{ TSP_ERR_INVALID, "relation must be 0..5" }; }
         ctx->requireScene();
+        ctx->requireWork();
         const Dev& d = ctx->d;
         const SceneHost& h = ctx->scenes[0];
         ctx->sync();
@@ -2345,6 +2388,7 @@ int tsp_get_neighbors(tsp_ctx* ctx, int rel, uint32_t* counts, uint32_t* idx, ui
             if (total) { *total = tot; }
             if (idx && cap >= tot && tot)
             {
+                if (!ctx->listsValid) { throw Error{ TSP_ERR_STATE, "the lists of the last search were not stored" }; }
                 const uint32_t* offs = rel == 3 ? d.rfOff : (rel == 4 ? d.rbOff : d.rrOff);
                 const uint32_t* list = rel == 3 ? d.rfIdx : (rel == 4 ? d.rbIdx : d.rrIdx);
                 if (rel != 3 && !ctx->contactLists) { throw Error{ TSP_ERR_STATE, "RB/RR lists were not stored" }; }
@@ -2375,6 +2419,7 @@ int tsp_get_neighbors(tsp_ctx* ctx, int rel, uint32_t* counts, uint32_t* idx, ui
         for (uint32_t i = 0; i < n; i++) { tot += cnt[i] & mask; if (counts) { counts[i] = cnt[i] & mask; } }
         if (total) { *total = tot; }
         if (!idx || cap < tot || !tot) { return TSP_OK; }
+        if (!ctx->listsValid) { throw Error{ TSP_ERR_STATE, "the lists of the last search were not stored" }; }
         const uint64_t units = ctx->last.poolUnits[rel];
         std::vector<uint16_t> pool(units);
         if (units) { hipCheck(hipMemcpy(pool.data(), d.pool[rel], sizeof(uint16_t) * units, hipMemcpyDeviceToHost), "D2H"); }
@@ -2417,6 +2462,7 @@ int tsp_get_sort(tsp_ctx* ctx, uint32_t* orderF, uint64_t* keysF, uint32_t* orde
 {
     return guarded(ctx, [&]() {
         ctx->requireScene();
+        ctx->requireWork();
         const Dev& d = ctx->d;
         const SceneHost& h = ctx->scenes[0];
         ctx->sync();
@@ -2712,6 +2758,7 @@ int tsp_batch_step(tsp_ctx* ctx, uint32_t n_steps)
 {
     return guarded(ctx, [&]() {
         ctx->requireScene();
+        ctx->requireWork();
         ctx->steps(n_steps);
         return TSP_OK;
     });
