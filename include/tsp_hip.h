@@ -325,7 +325,8 @@ int tsp_batch_export_snapshot(tsp_ctx *ctx, uint32_t scene_id, uint32_t surface_
 /* advances every scene n_steps IISPH steps (ExecuteFullSimStep of each scene's backend) */
 int tsp_batch_step(tsp_ctx *ctx, uint32_t n_steps);
 /* device bytes a scene of these counts holds while resident (an upper estimate at the initial
-   list pool sizes), for admission against an HBM budget */
+   list pool sizes), for admission against an HBM budget. Without its cell tables: 24 bytes per cell
+   of its frame (tsp_set_cell_limit caps a context's) */
 uint64_t tsp_batch_footprint(uint32_t n_fluid, uint32_t n_boundary, uint32_t n_rigid,
                              uint32_t n_bodies);
 

@@ -316,6 +316,7 @@ struct tsp_ctx
     std::vector<void*> poolAllocs;  // SELL-32 pools and the RF list
     std::vector<void*> solveAllocs; // the FB records of a solve in one launch
     uint64_t fbCap = 0;
+    bool solveRefused = false;      // no memory for them
     std::vector<void*> contactAllocs; // RB/RR lists and the contact boundary arrays (grown on demand)
     uint64_t cellCap = 0;
     uint64_t cellLimit = 0xffffffffull;   // most cells of all scenes' frames (tsp_set_cell_limit)
@@ -600,26 +601,29 @@ struct tsp_ctx
         d.rfCap = rfCap;
     }
 
-    // The FB records of a solve in one launch, for contexts of few blocks: as long as the FB pool, but no
-    // more than 64 units per particle (the pool may be a larger scene's that the context held before; a
-    // search that uses more solves launch by launch, and so does a context without the memory).
-    void allocSolve()
+    // The FB records of a solve in one launch, for contexts of few blocks, at an offset like the FB pool's:
+    // as long as that pool is to begin with (it may be a larger scene's that the context held before), then
+    // as a search's FB lists need (units), up to 64 units per particle. A search that uses more solves
+    // launch by launch, and so does a context without the memory.
+    void allocSolve(uint64_t units)
     {
         const bool few = d.nF != 0u && d.nF / kBlock <= kSolveBlocksMost;
-        const uint64_t want = few ? std::min<uint64_t>(d.poolCap[1], 64ull * d.nF + 1024u) : 0u;
-        if (want == 0u || want > fbCap)
-        {
-            releaseList(solveAllocs);
-            d.fbGrad = nullptr;
-            fbCap = 0;
-        }
-        if (want == 0u || d.fbGrad) { return; }
+        const uint64_t most = 64ull * d.nF + 1024u;
+        const uint64_t want = few && units <= most ? std::min(most, std::max<uint64_t>(16ull * d.nF + 1024u, units + units / 8u)) : 0u;
+        if (few && want <= fbCap) { return; }
+        releaseList(solveAllocs);
+        d.fbGrad = nullptr;
+        fbCap = 0;
+        if (want == 0u) { return; }
         try
         {
             d.fbGrad = alloc<float4>(want, solveAllocs, MEM_LF);
             fbCap = want;
         }
-        catch (const Error&) { (void)hipGetLastError(); }
+        catch (const Error&)
+        {
+            solveRefused = true;   // (until the next layout)
+        }
     }
 
     // the fluid fields of a scene in the records of n (missing fields are left out)
@@ -1086,7 +1090,8 @@ struct tsp_ctx
                 }
                 allocPools(cap, rfCap);
             }
-            allocSolve();
+            solveRefused = false;
+            allocSolve(0);
         }
         // world records of the rigid particles from the body state
         launchRigidUpdate(stream, d, false);
@@ -1458,9 +1463,9 @@ struct tsp_ctx
                 }
                 const uint64_t rfCap = std::max<uint64_t>(d.rfCap, last.rfTotal + last.rfTotal / 8 + 64);
                 allocPools(cap, rfCap);
-                allocSolve();
                 for (SceneHost& h : scenes) { h.flags |= TSP_FLAG_LIST_REGROWN; }
             }
+            if (last.poolUnits[1] > fbCap && !solveRefused) { allocSolve(last.poolUnits[1]); }
             // the contact solve's RB and RR lists are stored when some scene has entries
             contactLists = last.rbTotal + last.rrTotal > 0;
             contactRB = last.rbTotal;
@@ -2766,14 +2771,17 @@ int tsp_batch_step(tsp_ctx* ctx, uint32_t n_steps)
 
 uint64_t tsp_batch_footprint(uint32_t n_fluid, uint32_t n_boundary, uint32_t n_rigid, uint32_t n_bodies)
 {
-    // device bytes a scene holds while resident: per fluid slot (segment rounded to 256) about
-    // 190 B of records and second buffers, 16 B of sort keys, 160 B of SELL-32 lists at the
-    // initial pool sizes, 66 B of halo, counts, list heads and boundary hit masks, and up to
-    // 24 B of cell tables; per boundary particle 64 B; per rigid particle about 400 B (records,
-    // keys, the RF list); per body 256 B
+    // device bytes a scene holds while resident: per fluid slot (segment rounded to 256) 160 B of
+    // records and second buffers, 24 B of sort keys and indices, 160 B of lists at the initial pool
+    // sizes, 76 B of hit masks, 38 B of halo, counts and list heads; in a context of so few blocks that
+    // the solve runs in one launch 256 B of wall records; per boundary particle 64 B; per rigid particle
+    // about 400 B (records, keys, the RF list); per body 256 B. The cell tables come on top: 24 B per
+    // cell of the scene's frame, which follows from where the particles are (a context's cells are
+    // capped by its cell limit).
     const uint64_t f = static_cast<uint64_t>(roundUp(n_fluid, kBlock));
-    return f * 456ull + static_cast<uint64_t>(n_boundary) * 64ull + static_cast<uint64_t>(n_rigid) * 400ull
-         + static_cast<uint64_t>(n_bodies) * 256ull + (64ull << 10);
+    const uint64_t slot = 458ull + (f / kBlock <= kSolveBlocksMost ? 256ull : 0ull);
+    return f * slot + static_cast<uint64_t>(n_boundary) * 64ull + static_cast<uint64_t>(n_rigid) * 400ull
+         + static_cast<uint64_t>(n_bodies) * 256ull + (256ull << 10);
 }
 
 } // extern "C"
