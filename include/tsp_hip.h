@@ -139,6 +139,15 @@ const char *tsp_name(void);
 int tsp_set_params(tsp_ctx *ctx, const tsp_params *params);
 /* I_SimBackend::SetSimDomainBounds (core/backend_sim.h:204) */
 int tsp_set_domain(tsp_ctx *ctx, const float mn[3], const float mx[3]);
+/* which form the pressure solves of the context's steps took: steps[0] in one launch (contexts of up
+   to 256 blocks of 256 fluid particles and one per compute unit), steps[1] so begun and finished launch
+   by launch because some scene's blocks were not all on the chip at once, steps[2] launch by launch
+   (steps as captured graphs are not counted). All forms give the same bits. No reference counterpart. */
+int tsp_get_solve_forms(tsp_ctx *ctx, uint64_t steps[3]);
+/* the next solve in one launch waits for one block more than the scene has and so gives that scene
+   up, as on a GPU that other work keeps busy (0: no scene). For tests of what follows. */
+int tsp_hold_solve(tsp_ctx *ctx, uint32_t scene_id);
+
 /* the most cells the cell frames of the context's scenes may hold together (the dense cell
    tables take 24 bytes per cell); default and maximum 2^32 - 1. A layout beyond it (a pull, an
    admission or a frame rebuild) fails with TSP_ERR_CAPACITY and leaves the resident scenes as

@@ -159,6 +159,8 @@ def _declare_hip(lib):
         "tsp_set_domain": (i, [vp, _fp, _fp]),
         "tsp_set_cell_limit": (i, [vp, ctypes.c_uint64]),
         "tsp_set_step_graph": (i, [vp, i]),
+        "tsp_get_solve_forms": (i, [vp, _u64p]),
+        "tsp_hold_solve": (i, [vp, ctypes.c_uint32]),
         "tsp_pull": (i, [vp, ctypes.POINTER(TspStateView)]),
         "tsp_push": (i, [vp, ctypes.POINTER(TspStateView)]),
         "tsp_neighbor_search": (i, [vp]),

@@ -57,6 +57,17 @@ class HipBackend:
         """Steps as captured graphs or launch by launch (tsp_set_step_graph)."""
         self._check(self.lib.tsp_set_step_graph(self.h, 1 if enable else 0), "tsp_set_step_graph")
 
+    def solve_forms(self):
+        """Steps by the form of their pressure solve: in one launch, given up there, launch by launch
+        (tsp_get_solve_forms)."""
+        n = np.zeros(3, np.uint64)
+        self._check(self.lib.tsp_get_solve_forms(self.h, _capi.u64ptr(n)), "tsp_get_solve_forms")
+        return tuple(int(v) for v in n)
+
+    def hold_solve(self, scene_id=1):
+        """The next solve in one launch gives the scene up at its entry (tsp_hold_solve)."""
+        self._check(self.lib.tsp_hold_solve(self.h, scene_id), "tsp_hold_solve")
+
     def set_cell_limit(self, max_cells):
         """The most cells the context's cell frames may hold (tsp_set_cell_limit)."""
         self._check(self.lib.tsp_set_cell_limit(self.h, int(max_cells)), "tsp_set_cell_limit")
@@ -362,6 +373,10 @@ class HipBatch:
     memory = HipBackend.memory
     trim = HipBackend.trim
     set_memory_limit = HipBackend.set_memory_limit
+
+    # the forms of the solve (HipBackend.solve_forms, hold_solve)
+    solve_forms = HipBackend.solve_forms
+    hold_solve = HipBackend.hold_solve
 
     @staticmethod
     def footprint(n):

@@ -983,8 +983,9 @@ namespace tsp
         }
     };
 
+    // held: a scene whose entry waits for one block more than it has, and so gives up (none: kEmpty32)
     template <bool kFast>
-    __global__ void __launch_bounds__(kSweepThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) kSolve(Dev d)
+    __global__ void __launch_bounds__(kSweepThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) kSolve(Dev d, uint32_t held)
     {
         __shared__ double red[3][kSweepThreads / 64];
         __shared__ double part[3][kSolveBlocksMost];
@@ -1009,7 +1010,7 @@ namespace tsp
         // the state that solverInit left; every thread keeps it (nothing of it is read here again)
         Solve s = uniformLoad(&d.solve[sc]);
         uint32_t* bar = d.solveBar + static_cast<size_t>(sc) * kBarWords;
-        if (!enterScene(bar, S.nBlk)) { return; }   // (a barrier: the halo is staged)
+        if (!enterScene(bar, S.nBlk + (sc == held ? 1u : 0u))) { return; }   // (a barrier: the halo is staged)
         Kept kept;
         const bool keep = h.any && __ballot(active && l.n[REL_FF] > kKeepFF) == 0ull;
         if (keep && active) { kept.fill<kFast>(d, l, slots, h, hp, fbRows + t, k, p4); }
@@ -1414,11 +1415,11 @@ namespace tsp
         if (d.fastPairs) { kJacobi<true><<<n, kSweepThreads, 0, s>>>(d, n); }
         else { kJacobi<false><<<n, kSweepThreads, 0, s>>>(d, n); }
     }
-    void launchSolve(hipStream_t s, const Dev& d)
+    void launchSolve(hipStream_t s, const Dev& d, uint32_t held)
     {
         if (!d.nF) { return; }
-        if (d.fastPairs) { kSolve<true><<<blocksOf(d.nF), kSweepThreads, 0, s>>>(d); }
-        else { kSolve<false><<<blocksOf(d.nF), kSweepThreads, 0, s>>>(d); }
+        if (d.fastPairs) { kSolve<true><<<blocksOf(d.nF), kSweepThreads, 0, s>>>(d, held); }
+        else { kSolve<false><<<blocksOf(d.nF), kSweepThreads, 0, s>>>(d, held); }
     }
     void launchFinalize(hipStream_t s, const Dev& d)
     {

@@ -60,7 +60,7 @@ namespace tsp
     void launchPressureAcc(hipStream_t, const Dev&, bool);
     void launchJacobi(hipStream_t, const Dev&);
     void launchFinalize(hipStream_t, const Dev&);
-    void launchSolve(hipStream_t, const Dev&);
+    void launchSolve(hipStream_t, const Dev&, uint32_t);
     void launchIntegration(hipStream_t, const Dev&);
     void launchRigidUpdate(hipStream_t, const Dev&, bool);
     void launchRigidForces(hipStream_t, const Dev&, bool);
@@ -308,6 +308,8 @@ struct tsp_ctx
     uint32_t cuCount = 0;           // of the device
     uint32_t solveHold = 0;         // steps until a solve in one launch is tried again (one gave up)
     static constexpr uint32_t kSolveHold = 256;
+    uint64_t solveForms[3] = {};    // steps by the form of their solve (tsp_get_solve_forms)
+    uint32_t heldScene = 0;         // id of the scene that the next solve in one launch holds at its entry
     uint32_t* radixState = nullptr;
     uint32_t* aabb = nullptr;       // 6 per scene
     std::vector<void*> arena;       // particle and body arrays (replaced by a relayout)
@@ -1805,12 +1807,19 @@ struct tsp_ctx
         bool solved = false;
         if (anyFluid && solveInOne())
         {
-            launchSolve(stream, d);
+            const int held = heldScene ? indexOf(heldScene) : -1;
+            heldScene = 0;
+            launchSolve(stream, d, held >= 0 ? static_cast<uint32_t>(held) : kEmpty32);
             readStatus();
             solved = allSolved();
+            solveForms[solved ? 0 : 1]++;
             if (!solved) { solveHold = kSolveHold; }
         }
-        else if (solveHold) { solveHold--; }
+        else
+        {
+            if (solveHold) { solveHold--; }
+            if (anyFluid) { solveForms[2]++; }
+        }
         if (!anyFluid) { readStatus(); }
         else if (!solved) { solveLoop(0, group, maxSweeps); }
         tailLaunches(solved);
@@ -2238,6 +2247,24 @@ int tsp_set_step_graph(tsp_ctx* ctx, int enable)
 {
     return guarded(ctx, [&]() {
         ctx->stepGraphOn = enable != 0;
+        return TSP_OK;
+    });
+}
+
+int tsp_get_solve_forms(tsp_ctx* ctx, uint64_t steps[3])
+{
+    return guarded(ctx, [&]() {
+        if (!steps) { throw Error{ TSP_ERR_INVALID, "null counts" }; }
+        for (int q = 0; q < 3; q++) { steps[q] = ctx->solveForms[q]; }
+        return TSP_OK;
+    });
+}
+
+int tsp_hold_solve(tsp_ctx* ctx, uint32_t scene_id)
+{
+    return guarded(ctx, [&]() {
+        if (scene_id) { (void)ctx->sceneAt(scene_id); }
+        ctx->heldScene = scene_id;
         return TSP_OK;
     });
 }
