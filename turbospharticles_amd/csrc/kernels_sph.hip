@@ -217,7 +217,7 @@ namespace tsp
         const uint32_t blk = xcdBlock(nTiles);
         const Lists l = listsAt(d, blk);
         const SlotList slots = slotsOf(d, l);
-        const Halo h = haloOf(d, blk);
+        const Halo h = haloOf<false>(d, blk);   // (this kernel writes ulps)
         const uint32_t sc = uniformLoad(&d.blockScene[blk]);
         const Consts k = uniformLoad(&d.consts[sc]);
         const Scene S = uniformLoad(&d.scenes[sc]);
@@ -1007,8 +1007,10 @@ namespace tsp
         const float src = d.source[i], diag = d.diag[i];
         const bool active = i - S.offF < S.nF;
         stageHalo(h, [&](uint32_t j) { return d.pos[j]; }, [&](uint32_t q, const float4& r) { hp[q] = r; hw[q] = r.w; });
-        // the state that solverInit left; every thread keeps it (nothing of it is read here again)
-        Solve s = uniformLoad(&d.solve[sc]);
+        // the state that solverInit left (the rest of it is 0); every thread keeps it
+        Solve s{};
+        s.iters = d.solve[sc].iters;
+        s.compute = d.solve[sc].compute;
         uint32_t* bar = d.solveBar + static_cast<size_t>(sc) * kBarWords;
         if (!enterScene(bar, S.nBlk + (sc == held ? 1u : 0u))) { return; }   // (a barrier: the halo is staged)
         Kept kept;

@@ -871,6 +871,8 @@ namespace tsp
         uint32_t j[kPer];
     };
 
+    // (without kUlps the flag is not read: the kernel may write it)
+    template <bool kUlps = true>
     __device__ __forceinline__ Halo haloOf(const Dev& d, uint32_t blk)
     {
         Halo h;
@@ -880,10 +882,11 @@ namespace tsp
             const uint32_t q = u * kBlock + threadIdx.x;
             h.j[u] = (u + 1u < Halo::kPer || q < kHaloMax) ? idx[q] : 0u;
         }
-        const HaloInfo info = uniformLoad(&d.haloInfo[blk]);
-        h.any = info.count <= kHaloMax;
-        h.ulps = h.any && info.ulps != 0u;
-        h.count = h.any ? info.count : 0u;
+        const HaloInfo* info = &d.haloInfo[blk];
+        const uint32_t count = uniformLoad(&info->count), ulps = kUlps ? uniformLoad(&info->ulps) : 0u;
+        h.any = count <= kHaloMax;
+        h.ulps = h.any && ulps != 0u;
+        h.count = h.any ? count : 0u;
         return h;
     }
 
