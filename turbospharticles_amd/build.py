@@ -3,8 +3,8 @@
   lib/libtsp_hip.so   hipcc --offload-arch=gfx950: csrc/*.hip (kernels + C ABI)
   lib/libtsp_host.so  g++: host/*.cpp (scene builder, SimBackend_HIP), linked to libtsp_hip.so
   lib/sim_backend_roundtrip  g++: the C++ driver of SimBackend_HIP that the tests run
-  lib/math_selftest, lib/pair_selftest  hipcc: GPU checks of the short exact root, quotient and
-                      gradient factor against the general lowering
+  lib/math_selftest, lib/pair_selftest, lib/quotient_selftest  hipcc: GPU checks of the short exact
+                      root, quotient and gradient factor against the general lowering
 
 Floating point: -ffp-contract=off everywhere (the reference's ISO C++ build contracts nothing;
 every fused multiply-add is an explicit fmaf), correctly rounded f32 division and square root,
@@ -109,12 +109,18 @@ def build_pair_selftest(verbose=False):
     return _build_selftest("pair_selftest", verbose)
 
 
+def build_quotient_selftest(verbose=False):
+    """lib/quotient_selftest: the GPU check of the pair kernels' quotient over the allowed range"""
+    return _build_selftest("quotient_selftest", verbose)
+
+
 def build_all(verbose=False):
     build_hip(verbose)
     build_host(verbose)
     build_driver(verbose)
     build_math_selftest(verbose)
     build_pair_selftest(verbose)
+    build_quotient_selftest(verbose)
 
 
 if __name__ == "__main__":

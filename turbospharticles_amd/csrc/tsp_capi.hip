@@ -578,9 +578,11 @@ struct tsp_ctx
         for (uint32_t s = 0; s < nScenes(); s++)
         {
             k[s] = makeConsts(scenes[s].params, scenes[s].nF);
-            // the short exact quotient of the gradient factor needs its operands in range
+            // the short exact quotient of the gradient factor needs its operands in range, and koutScale no
+            // power of two (quotFrom)
             const float a = std::fabs(k[s].koutScale);
-            fast = fast && a >= 0x1p-60f && a <= 0x1p60f && k[s].ksize >= 0x1p-30f && k[s].ktwo <= 0x1p31f;
+            int e;
+            fast = fast && a >= 0x1p-60f && a <= 0x1p60f && std::frexp(a, &e) != 0.5f && k[s].ksize >= 0x1p-30f && k[s].ktwo <= 0x1p31f;
         }
         d.fastDiv = fast ? 1u : 0u;
         h2d(d.consts, k.data(), sizeof(Consts) * k.size());

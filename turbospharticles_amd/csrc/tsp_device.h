@@ -321,8 +321,8 @@ namespace tsp
     {
         uint32_t nF, nB, nR, nRB;    // array lengths over all scenes (nF counts padding slots)
         uint32_t nScenes;
-        uint32_t fastDiv;            // every scene's kernel constants lie in divCR's range
-        uint32_t fastPairs;          // this search's FF and FB pairs may take sqrtCR / divCR (kgFactor<true>)
+        uint32_t fastDiv;            // every scene's kernel constants lie in quotFrom's range
+        uint32_t fastPairs;          // this search's FF and FB pairs may take sqrtCR, rootRcp and quotFrom (kgFactor<true>)
         Scene *scenes;
         Frame *frames;
         Consts *consts;
@@ -531,8 +531,14 @@ namespace tsp
     // corrections of the quotient -- the general lowering's core, which is the whole computation
     // when it needs no operand scaling. Callers guarantee 2^-60 <= |a| <= 2^60 and
     // 2^-30 <= |b| <= 2^31 (the exponents then differ by less than the 96 that trigger
-    // scaling, and every intermediate is a normal number); checked bit for bit against the
-    // general lowering over such operands.
+    // scaling, and every intermediate is a normal number). The last correction's error is |r / b| times the
+    // relative error of y, half an ulp of the quotient times at most 2^-24, so it rounds correctly unless
+    // the quotient lies that near a midpoint; it can only where b's mantissa is next to 2 and y has the largest
+    // error. With rootRcp's estimate (b = sqrt(x)) that is one pair: a a power of two, b the float below
+    // one; every other pair gives the general lowering's bits (checked for every a at the last 4,096 floats x of
+    // a binade, over 2^33 random pairs of this range and every float of the outer branch at particle sizes of
+    // the whole range). The host keeps the general lowering where koutScale is a power of two (which it
+    // is for no float h).
     __device__ __forceinline__ float quotFrom(float a, float b, float y)
     {
         const float e = __builtin_fmaf(-b, y, 1.0f);
@@ -544,6 +550,7 @@ namespace tsp
         return __builtin_fmaf(r, y, q);
     }
 
+    // (what quotFrom's estimate took the place of: its check against the general lowering stays)
     __device__ __forceinline__ float divCR(float a, float b) { return quotFrom(a, b, __builtin_amdgcn_rcpf(b)); }
 
     // sqrt(x) for x = 0 or 2^-96 <= x < inf, and an estimate y of 1 / sqrt(x) (2^60 for x = 0):
