@@ -519,8 +519,7 @@ struct tsp_ctx
                 if (n)
                 {
                     const uint32_t q = b.count++;
-                    b.piece[q] = XferPiece{ f.dev, f.stride, f.comps, static_cast<uint32_t>(done), static_cast<uint32_t>(n),
-                                            static_cast<uint32_t>(at), 0u };
+                    b.piece[q] = pieceOf(f, done, static_cast<uint32_t>(n), static_cast<uint32_t>(at));
                     b.block[q + 1u] = b.block[q] + static_cast<uint32_t>((n + kXferBlock - 1u) / kXferBlock);
                     copies[k].push_back(StageCopy{ f.host + done * 4u, static_cast<size_t>(at) * 4u, static_cast<size_t>(n) * 4u });
                     at += (n + 3ull) & ~3ull;

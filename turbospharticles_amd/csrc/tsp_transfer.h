@@ -39,6 +39,14 @@ namespace tsp
         uint64_t n;
     };
 
+    // words [done, done + n) of a field, at stage[at ...]. The piece starts at the record of its first word,
+    // so that its word numbers stay small however long the field is (three words each of 2^31 records pass 2^32).
+    inline XferPiece pieceOf(const XferField& f, uint64_t done, uint32_t n, uint32_t at)
+    {
+        const uint64_t rec = done / f.comps;
+        return XferPiece{ f.dev + rec * f.stride, f.stride, f.comps, static_cast<uint32_t>(done - rec * f.comps), n, at, 0u };
+    }
+
     // a range of the stage and where it belongs in the caller's memory
     struct StageCopy
     {
