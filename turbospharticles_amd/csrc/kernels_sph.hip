@@ -1357,8 +1357,10 @@ namespace tsp
 
     // A body's part of a step in one block: the force sums, the prediction, the integration and the body's
     // particles, whichever `parts` asks for, in this order. Each was a launch of 4 to 10 us of which little
-    // more than the launch was needed. More than kBodyParticles in the context are updated by a launch of
-    // their own: one block takes about 2 us per thousand (6,364 particles: 22 us together, 16 apart).
+    // more than the launch was needed. Where a body has more than kBodyParticles, the particles are updated by a
+    // launch of their own: a block takes about 2 us per thousand of its body's. A step with one body of 2,044 /
+    // 2,368 / 3,088 / 3,904 / 6,364 particles: 557 / 605 / 687 / 799 / 1,256 us together, 559 / 605 / 686 / 796 /
+    // 1,246 apart; several bodies share the time of the largest: ten of 1,468 take 371 us together, 390 apart.
     constexpr uint32_t kBodyParticles = 2048;
     enum BodyParts { kBodySums = 1, kBodyPredict = 2, kBodyIntegrate = 4, kBodyUpdate = 8, kBodyUpdatePredicted = 16 };
 
@@ -1437,7 +1439,7 @@ namespace tsp
     static void launchRigidBody(hipStream_t s, const Dev& d, uint32_t parts)
     {
         if (!d.nRB) { return; }
-        const bool alone = d.nR > kBodyParticles;
+        const bool alone = d.mostR > kBodyParticles;
         constexpr uint32_t kUpdates = kBodyUpdate | kBodyUpdatePredicted;
         kRigidBody<<<d.nRB, kBodyThreads, 0, s>>>(d, alone ? parts & ~kUpdates : parts);
         if (alone && (parts & kUpdates)) { launchRigidUpdate(s, d, (parts & kBodyUpdatePredicted) != 0u); }

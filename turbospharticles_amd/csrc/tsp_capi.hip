@@ -942,6 +942,7 @@ struct tsp_ctx
                 for (uint32_t i = 0; i < h.nB; i++) { sceneB[h.offB + i] = static_cast<uint16_t>(s); }
             }
             for (uint32_t i = 0; i < nR; i++) { off[rbody[i] + 1]++; }
+            n.mostR = *std::max_element(off.begin(), off.end());   // (off holds the bodies' counts so far)
             for (uint32_t b = 0; b < nRB; b++) { off[b + 1] += off[b]; }
             std::vector<uint32_t> w(off);
             for (uint32_t i = 0; i < nR; i++) { idx[w[rbody[i]]++] = i; }

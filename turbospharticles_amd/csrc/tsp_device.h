@@ -321,6 +321,7 @@ namespace tsp
     {
         uint32_t nF, nB, nR, nRB;    // array lengths over all scenes (nF counts padding slots)
         uint32_t nScenes;
+        uint32_t mostR;              // rigid particles of the largest body
         uint32_t fastDiv;            // every scene's kernel constants lie in quotFrom's range
         uint32_t fastPairs;          // this search's FF and FB pairs may take sqrtCR, rootRcp and quotFrom (kgFactor<true>)
         Scene *scenes;
