@@ -13,7 +13,7 @@
 //   count     per particle: FF/FB/FR hit masks and counts over the 27-cell stencil (inclusive
 //             cutoff, distance fma(dx,dx,fma(dy,dy,dz*dz)), neighbor_search.cpp:1130-1249); per
 //             64-position slice: pitch, base, u16/u32 format and storage
-//   scan      multi-block exclusive scans (radix digit offsets, RF offsets)
+//   scan      one-pass exclusive scans of many blocks (RF, RB and RR offsets, the surface flags of an export)
 //   fill      writes the entries in the reference's iteration order: z-y-x stencil raster,
 //             ascending index within a cell (CPU/backend/neighbor_lists.h:171-197 for wide lists),
 //             and builds the FF halo of each 256-particle block
@@ -267,9 +267,8 @@ namespace tsp
         }
     }
 
-    // keys and indices of a population; passes > 0 adds
-    // the digit counts of all sort passes to the sort state (particles in motion are nearly in
-    // order, so a block meets few digits and adds few words)
+    // keys and indices of a population; passes > 0 adds the digit counts of all sort passes to the sort
+    // state (particles in motion are nearly in order, so a block meets few digits and adds few words)
     template <typename K>
     __global__ void __launch_bounds__(kBlock) kKeys(Dev d, int pop, const float4* __restrict__ p, uint32_t n, bool check,
         K* __restrict__ key, uint32_t* __restrict__ idx, uint32_t* __restrict__ state, uint32_t passes)
@@ -764,9 +763,10 @@ namespace tsp
     // third as long. The fill always runs so. The count pass does for up to kShareBlocks blocks (two per
     // CU: the chain is what its time consists of); beyond that one wave walks all nine rows, because
     // what the waves of a particle repeat, and their barriers, cost more than the shorter chain gains.
-    // kQueryCount, against one lane walking all rows candidate by candidate: 16 blocks 66 to 33 us, 250
-    // blocks 65 to 34 (one wave: 50), 432 blocks 82 to 49 (one wave: 67); 3,907 blocks 215 to 206 (three waves: 228),
-    // 31,250 blocks 1,333 to 1,205 (three waves: 1,446). What bounds the large launches is the vector
+    // kQueryCount on a resting lattice, three waves / one wave: 16 blocks 30 / 49 us, 250 blocks 30 / 48, 311 blocks
+    // 40 / 51, 432 blocks 42 / 50, 519 blocks 55 / 56, 686 blocks 60 / 56, 977 blocks 67 / 65, 2,000 blocks 111 /
+    // 108, 3,907 blocks 202 / 179; against one lane walking all rows candidate by candidate: 16 blocks 66 to 33,
+    // 432 blocks 82 to 49, 3,907 blocks 215 to 206, 31,250 blocks 1,333 to 1,205. What bounds the large launches is the vector
     // memory path: 240 scattered 12-byte records per lane, about 20 cycles a wave each. (Candidates
     // staged in LDS per 64 particles, in cell order: 250 us at 3,907 blocks, more barriers than loads
     // saved.)
@@ -1673,8 +1673,7 @@ namespace tsp
     }
 
     // per-scene bounds of one population: out[6 s + a] holds the ordered bits of the min x, y, z
-    // and then the max; a wave whose valid lanes share one scene reduces before its atomics
-    // per-scene bounds: each wave walks a contiguous range of 64-particle chunks, keeps per-lane
+    // and then the max. Each wave walks a contiguous range of 64-particle chunks, keeps per-lane
     // running bounds while the chunks belong to one scene, and reduces them into that scene's
     // bounds with one set of atomics when the scene changes or the range ends (chunks that mix
     // scenes update lane by lane)
@@ -1750,7 +1749,6 @@ namespace tsp
     bool radixSortSingleBlock(uint32_t n) { return n <= kSmallSort; }
 
     static uint32_t radixPasses(uint32_t bits) { return (bits + kRadixBits - 1u) / kRadixBits; }
-
 
     // cells: the cell tables hold the runs of the sorted keys, which are cleared
     void launchResetSearch(hipStream_t s, const Dev& d, bool cells)

@@ -480,10 +480,8 @@ namespace tsp
         a[0] = 0.0f - ax; a[1] = 0.0f - ay; a[2] = 0.0f - az;
     }
 
-    // a sweep's pressure accelerations; block 0 of a sweep launch first finishes the bookkeeping of
-    // the previous Jacobi sweep, which the next Jacobi launch reads. Blocks that see the solve
-    // converged skip their particles: the final launch (sweep = false) recomputes every a^p.
-    // one tile of a sweep's pressure accelerations
+    // one tile of a sweep's pressure accelerations. Blocks that see the solve converged skip their
+    // particles: the final launch (sweep = false) recomputes every a^p.
     template <bool kFast>
     __device__ __forceinline__ void pressureAccTile(const Dev& d, uint32_t blk, bool sweep)
     {
@@ -516,14 +514,14 @@ namespace tsp
     __global__ void __launch_bounds__(kSweepThreads) TSP_WAVES_ATTR(TSP_TUNE_PA_WAVES) kPressureAcc(Dev d, bool sweep, uint32_t nTiles)
     {
         if (stopped(d)) { return; }
-        // block b of the launch finishes the previous sweep of scenes b, b + grid, ...
+        // a sweep launch first finishes the bookkeeping of the previous Jacobi sweep, which the next Jacobi
+        // launch reads: block b that of scenes b, b + grid, ...
         if (sweep)
         {
             for (uint32_t q = blockIdx.x; q < d.nScenes; q += gridDim.x) { finalizeSweep(d, q, nTiles); }
         }
         pressureAccTile<kFast>(d, xcdBlock(), sweep);
     }
-
 
     __device__ __forceinline__ void addError(float pred, const Consts& k, double& eRaw, double& ePos, double& eAbs)
     {

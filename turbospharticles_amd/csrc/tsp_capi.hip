@@ -1330,9 +1330,10 @@ struct tsp_ctx
     }
 
     // the rigid particles' part of a search phase on the side stream, the fluid's beside it (they read the
-    // same sorted particles and write different lists), while the fluid's leaves room on the chip: 432
-    // blocks hide 30 us of rigid launches; with 3,907 the small launches wait behind them, and a step of
-    // 2.8 ms is 1% slower
+    // same sorted particles and write different lists), while the fluid's leaves room on the chip. A landing
+    // cube's step, beside / in turn: 128 blocks 544 / 553 us, 432 blocks 755 / 768, 686 blocks 642 / 649, 977
+    // blocks 604 / 608, 1,520 blocks 694 / 691, 2,000 blocks 844 / 832 (the small launches wait behind the
+    // fluid's); a body that touches nothing has little to hide and gains or loses up to 1%
     static constexpr uint32_t kBesideBlocks = 1024;
 
     template <typename Rigid, typename Fluid>
@@ -1888,7 +1889,6 @@ struct tsp_ctx
         addField(fields, s->rigid_id, idR + h.offR, h.nR);
         for (size_t f = 0; f < TSP_RB_COUNT; f++) { addField(fields, s->body[f], d.rb + f * nRB1 + h.offRB, h.nRB); }
         transfer(fields, true);
-        sync();
         if (s->rigid_body) { for (uint32_t i = 0; i < h.nR; i++) { s->rigid_body[i] = h.rbodyLocal[i]; } }
         for (uint32_t b = 0; b < h.nRB; b++)
         {

@@ -1,10 +1,9 @@
 """Autotuner of the build-time variants of the step (the TSP_TUNE_* switches in csrc/tsp_device.h).
 
-Every variant gives the same bits; they differ in how the work maps onto the GPU: the radix sort's
-digit width (8, 6 or 4 bits: 4 to 8 passes over 28-bit keys), the size of a step's first sweep
-group against the previous step's sweep count, the whole step as one graph launch or launch by
-launch, 24- or 32-byte Jacobi halo records, the halo cap (LDS per sweep block), register budgets of the sweep
-kernels, sweep groups as HIP graphs. The
+Every variant gives the same bits; they differ in how the work maps onto the GPU: the size of a step's
+first sweep group against the previous step's sweep count, the whole step as captured graphs or launch by
+launch, sweep groups as HIP graphs, the halo cap (LDS per sweep block), and the register budgets of the two
+sweep kernels. The
 tuner walks the switches one at a time from the current settings (coordinate descent), keeping a
 change when it shortens the measured step.
 
