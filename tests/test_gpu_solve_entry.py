@@ -64,6 +64,20 @@ def test_form_by_the_number_of_blocks(counts, one):
     same_report(g.info(), timed.info())
 
 
+def test_walls_that_need_longer_records():
+    # 250 particles in a tube one particle wide: more than the 16 wall entries per slot (and 1,024) that the
+    # records have room for to begin with
+    print("case: 250 particles in a tube", flush=True)
+    st = dam_break(250, H, counts=(250, 1, 1), tank=(2.51, 0.01, 0.01))
+    g, timed = backend(st), backend(st, timed=True)
+    for b in (g, timed):
+        b.step(3)
+    assert g.info().n_fb > 16 * 256 + 1024
+    assert g.solve_forms() == (3, 0, 0)
+    same(g.push(), timed.push())
+    same_report(g.info(), timed.info())
+
+
 @pytest.mark.parametrize("name", ["one block", "not full", "256 blocks", "body", "abs"])
 def test_given_up_scene_is_solved_launch_by_launch(name):
     print(f"case: {name}", flush=True)

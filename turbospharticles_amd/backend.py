@@ -64,8 +64,12 @@ class HipBackend:
         self._check(self.lib.tsp_get_solve_forms(self.h, _capi.u64ptr(n)), "tsp_get_solve_forms")
         return tuple(int(v) for v in n)
 
-    def hold_solve(self, scene_id=1):
-        """The next solve in one launch gives the scene up at its entry (tsp_hold_solve)."""
+    def hold_solve(self, scene_id=None):
+        """The next solve in one launch gives the scene (by default the first) up at its entry (tsp_hold_solve)."""
+        if scene_id is None:
+            first = np.zeros(1, np.uint32)
+            self._check(self.lib.tsp_batch_scene_ids(self.h, _capi.u32ptr(first), 1, None), "tsp_batch_scene_ids")
+            scene_id = int(first[0])
         self._check(self.lib.tsp_hold_solve(self.h, scene_id), "tsp_hold_solve")
 
     def set_cell_limit(self, max_cells):

@@ -612,7 +612,8 @@ struct tsp_ctx
     {
         const bool few = d.nF != 0u && d.nF / kBlock <= kSolveBlocksMost;
         const uint64_t most = 64ull * d.nF + 1024u;
-        const uint64_t want = few && units <= most ? std::min(most, std::max<uint64_t>(16ull * d.nF + 1024u, units + units / 8u)) : 0u;
+        if (few && units > most) { return; }
+        const uint64_t want = few ? std::min(most, std::max<uint64_t>(16ull * d.nF + 1024u, units + units / 8u)) : 0u;
         if (few && want <= fbCap) { return; }
         releaseList(solveAllocs);
         d.fbGrad = nullptr;
@@ -1947,6 +1948,7 @@ struct tsp_ctx
     // context's buffers, and nothing is allocated
     void statistics(uint32_t si, tsp_statistics* out, bool noAlloc = false)
     {
+        if (noAlloc && !workReady) { throw Error{ TSP_ERR_STATE, "the last layout found no memory for its buffers" }; }
         requireWork();
         const SceneHost& h = scenes[si];
         const uint64_t nb = (static_cast<uint64_t>(h.nF) + kBlock - 1) / kBlock;
